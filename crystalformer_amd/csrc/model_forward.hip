@@ -1,0 +1,171 @@
+// A whole inference forward of the encoder in one host call: every launch of the blocks issued from
+// here, all intermediate tensors carved from one buffer.
+//
+// Issued operator by operator from Python a forward of the four-block model is about 40 launches at
+// some 14 us of host time each, which is what a small batch costs whatever the GPU does (0.65 ms for
+// one crystal of 12 atoms whose kernels take 0.20 ms); from here a launch costs 2-3 us.
+#include "cf_common.h"
+
+namespace {
+
+using namespace cf;
+
+struct Carver {
+    char *base;
+    int64_t used;
+    template <typename T>
+    T *take(int64_t count)
+    {
+        used = (used + 255) & ~(int64_t)255;
+        T *p = base ? reinterpret_cast<T *>(base + used) : nullptr;
+        used += count * (int64_t)sizeof(T);
+        return p;
+    }
+};
+
+struct Buffers {
+    float *rvlen, *rpos, *x[2], *h, *q, *k, *v, *qs, *a, *att, *z, *val, *prob, *rings, *pooled, *hidden;
+    void *stats, *flags;
+    int64_t stats_bytes, flag_bytes;
+};
+
+// Whether the blocks with value bins start from staged rings, and the bytes these take.
+bool use_rings(const cf_forward_args &f, int64_t U)
+{
+    if (!f.staged_rings || U < 1) return false;
+    const int64_t edge = 2 * (int64_t)f.lattice_range + 1;
+    return edge * edge * edge <= 128 && cf_real_enc_ring_bytes(U) <= f.ring_limit_bytes;
+}
+
+int64_t carve(const cf_forward_args &f, const cf_forward_block *blocks, char *base, Buffers &b)
+{
+    Carver c{base, 0};
+    const int64_t N = f.N, E = f.E, U = (N + E) / 2, W = f.width;
+    bool rings = false, bins = false;
+    for (int64_t l = 0; l < f.layers; l++) bins = bins || blocks[l].bins > 0;
+    rings = bins && use_rings(f, U);
+    b.rvlen = c.take<float>(3 * f.B);
+    b.rpos = c.take<float>(3 * E);
+    for (int i = 0; i < 2; i++) b.x[i] = c.take<float>(N * W);
+    b.h = c.take<float>(N * f.ff);
+    b.q = c.take<float>(N * W);
+    b.k = c.take<float>(N * W);
+    b.v = c.take<float>(N * W);
+    b.qs = c.take<float>(N * W);
+    b.a = c.take<float>(N * f.H);
+    b.att = c.take<float>(N * W);
+    b.z = c.take<float>(E * f.H);
+    b.prob = c.take<float>(E * f.H);
+    b.val = bins ? c.take<float>(E * W) : nullptr;
+    b.stats_bytes = cf_gauss_exponents_workspace(N, f.H);
+    b.stats = c.take<char>(b.stats_bytes);
+    b.flag_bytes = rings ? cf_real_enc_flag_bytes(U, f.H) : 0;
+    b.flags = rings ? c.take<char>(b.flag_bytes) : nullptr;
+    b.rings = rings ? c.take<float>(cf_real_enc_ring_bytes(U) / 4) : nullptr;
+    b.pooled = c.take<float>(f.B * W);
+    b.hidden = c.take<float>(f.B * (f.hidden > 0 ? f.hidden : 1));
+    return c.used;
+}
+
+int check_args(const cf_forward_args *f, const cf_forward_block *blocks)
+{
+    CF_REQUIRE(f && blocks, CF_ERR_INVALID_ARGUMENT, "cf_forward: null arguments");
+    CF_REQUIRE(f->N >= 1 && f->E >= f->N && (f->N + f->E) % 2 == 0 && f->B >= 1 && f->layers >= 1, CF_ERR_INVALID_ARGUMENT,
+               "cf_forward: bad sizes N=%lld E=%lld B=%lld layers=%lld", (long long)f->N, (long long)f->E,
+               (long long)f->B, (long long)f->layers);
+    CF_REQUIRE((f->H == 1 || f->H == 2 || f->H == 4 || f->H == 8 || f->H == 16) && f->width % 16 == 0 &&
+                   f->ff % 16 == 0 && f->ff >= 16 && f->width >= 16 && f->width % f->H == 0 && f->width / f->H <= 32,
+               CF_ERR_UNSUPPORTED, "cf_forward: width %lld, heads %lld, feed-forward %lld not served",
+               (long long)f->width, (long long)f->H, (long long)f->ff);
+    for (int64_t l = 0; l < f->layers; l++)
+        CF_REQUIRE(blocks[l].bins >= 0 && blocks[l].bins <= 128 && (blocks[l].bins == 0 || blocks[l].w_pe),
+                   CF_ERR_UNSUPPORTED, "cf_forward: block %lld: value bins outside 0..128 or without a projection",
+                   (long long)l);
+    return CF_OK;
+}
+
+}  // namespace
+
+extern "C" int64_t cf_forward_workspace(const cf_forward_args *f, const cf_forward_block *blocks)
+{
+    if (check_args(f, blocks)) return -1;
+    Buffers b;
+    return carve(*f, blocks, nullptr, b);
+}
+
+extern "C" int cf_forward(const cf_forward_args *f_, const cf_forward_block *blocks, void *workspace,
+                          int64_t workspace_bytes, void *stream)
+{
+    int rc = check_args(f_, blocks);
+    if (rc) return rc;
+    const cf_forward_args &f = *f_;
+    Buffers b;
+    const int64_t need = carve(f, blocks, (char *)workspace, b);
+    CF_REQUIRE(workspace && workspace_bytes >= need, CF_ERR_INVALID_ARGUMENT,
+               "cf_forward: workspace of %lld bytes needed", (long long)need);
+    CF_REQUIRE(f.x && f.pos && f.tvecs && f.batch && f.atom_start && f.edge_start && f.edges && f.e_start && f.pairs &&
+                   f.out && (f.targets == 0 || (f.w_last && (f.hidden == 0 || f.w_head))),
+               CF_ERR_INVALID_ARGUMENT, "cf_forward: null pointer");
+    const int64_t N = f.N, E = f.E, U = (N + E) / 2, W = f.width, H = f.H, D = W / H;
+    const bool adaptive_any = f.adaptive != 0;
+    if ((rc = cf_lattice_geometry(f.tvecs, f.B, nullptr, nullptr, b.rvlen, stream))) return rc;
+    if ((rc = cf_edge_index(f.atom_start, f.edge_start, f.B, E, f.pos, nullptr, b.rpos, stream))) return rc;
+    const cf_forward_block *staged = nullptr;      // the block whose grid the rings in b.rings hold
+    const float *x = f.x;
+    int side = 0;
+    for (int64_t l = 0; l < f.layers; l++) {
+        const cf_forward_block &p = blocks[l];
+        if ((rc = cf_linear_rows(x, N, W, p.wq, p.wk, p.wv, 3, W, p.b_in, nullptr, 0, b.q, b.k, b.v, stream))) return rc;
+        if ((rc = cf_gauss_exponents(b.q, p.w_pos, p.gauss_scale, N, H, D, p.normalize, f.update_stats, p.positive_func,
+                                     (float)p.beta, (float)p.lower_bound, (float)p.coef, (float)p.q_scale, b.stats,
+                                     b.stats_bytes, nullptr, b.a, b.qs, stream)))
+            return rc;
+        const float *rvlen = adaptive_any && p.cutoff != 0.0 ? b.rvlen : nullptr;
+        const bool adaptive = rvlen != nullptr;
+        if (p.bins > 0 && b.rings && (!adaptive || (f.adaptive_rings && H <= 8))) {
+            if (!staged || staged->bins != p.bins || staged->dist_max != p.dist_max || staged->wscale != p.wscale ||
+                staged->weakest != p.weakest) {
+                if ((rc = cf_real_enc_ring_stage(b.rpos, f.tvecs, f.pairs, U, p.bins, p.dist_max, p.wscale,
+                                                 f.lattice_range, p.weakest, b.rings, stream)))
+                    return rc;
+                staged = &p;
+            }
+            rc = cf_real_enc_fwd_rings(b.a, adaptive ? b.rpos : nullptr, adaptive ? f.tvecs : nullptr,
+                                       adaptive ? f.batch : nullptr, f.edges, f.pairs, U, N, H, E, p.bins, D, p.dist_max,
+                                       p.wscale, p.w_pe, rvlen, p.cutoff, f.lattice_range, f.minimum_range, b.rings,
+                                       b.flags, b.flag_bytes, b.z, b.val, stream);
+        } else {
+            rc = cf_real_enc_fwd(b.a, b.rpos, f.tvecs, f.batch, f.edges, N, H, E, f.B, p.bins, p.bins > 0 ? D : 0,
+                                 p.dist_max, p.wscale, p.bins > 0 ? p.w_pe : nullptr, p.bins > 0 ? 1 : 0, rvlen,
+                                 adaptive ? p.cutoff : 0.0, f.lattice_range, f.minimum_range, f.pairs, U, f.sched, b.z,
+                                 p.bins > 0 ? b.val : nullptr, stream);
+        }
+        if (rc) return rc;
+        if ((rc = cf_fused_dpa_fwd(b.qs, b.k, b.v, b.z, p.bins > 0 ? b.val : nullptr, f.edges, f.e_start, N, H, E, D, D,
+                                   b.prob, b.att, stream)))
+            return rc;
+        float *y = f.targets == 0 && l + 1 == f.layers ? f.out : b.x[side];
+        if ((rc = cf_linear_rows(b.att, N, W, p.wo, nullptr, nullptr, 1, W, p.bo, x, 0, b.qs, nullptr, nullptr, stream)))
+            return rc;                              // (the scaled query is spent: its buffer takes the sum)
+        if ((rc = cf_linear_rows(b.qs, N, W, p.w1, nullptr, nullptr, 1, f.ff, p.b1, nullptr, 1, b.h, nullptr, nullptr,
+                                 stream)))
+            return rc;
+        if ((rc = cf_linear_rows(b.h, N, f.ff, p.w2, nullptr, nullptr, 1, W, p.b2, b.qs, 0, y, nullptr, nullptr, stream)))
+            return rc;
+        x = y;
+        side ^= 1;
+    }
+    if (f.targets == 0) return CF_OK;
+    if ((rc = cf_irregular_mean_fwd(x, f.atom_start, f.B, W, b.pooled, stream))) return rc;
+    const float *top = b.pooled;
+    int64_t top_width = W;
+    if (f.hidden > 0) {
+        if ((rc = cf_linear_rows(b.pooled, f.B, W, f.w_head, nullptr, nullptr, 1, f.hidden, f.b_head, nullptr, 1, b.hidden,
+                                 nullptr, nullptr, stream)))
+            return rc;
+        top = b.hidden;
+        top_width = f.hidden;
+    }
+    return cf_linear_rows(top, f.B, top_width, f.w_last, nullptr, nullptr, 1, f.targets, f.b_last, nullptr, 0, f.out,
+                          nullptr, nullptr, stream);
+}

@@ -203,6 +203,10 @@ class CrystalformerEncoderCUDA(Module):
                 onehot: Optional[Tensor] = None) -> Tensor:
         if src.size(-1) != self.d_model:
             raise RuntimeError("the feature number of src and tgt must be equal to d_model")
+        from . import executor
+        out = executor.encode(self, src, pos, batch, trans, sizes)     # inference, plain blocks: one native call
+        if out is not None:
+            return out
         P = self.lattice_params
         # geometry prologue of compute_lattice_distances_for_cuda, plus the lengths of the
         # reciprocal vectors (all a block needs of them), in two launches

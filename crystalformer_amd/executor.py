@@ -1,0 +1,198 @@
+"""Inference forwards as one native call.
+
+:func:`encode` and :func:`forward` run the encoder -- the latter with pooling and the regression
+head behind it -- through ``cf_forward``, which issues every launch from C++.  They serve the plain
+case (real domain, no norm layers, ReLU, softmax attention, exponents from the query, one value
+projection per head) without autograd and return ``None`` for everything else: other options,
+modules replaced by a user's own, forward hooks (which must see the intermediate outputs), kernel
+timing and counting.  The callers then run the modules one by one, with the same operators.
+"""
+from __future__ import annotations
+
+import math
+from typing import Optional, Tuple
+
+import torch
+from torch import Tensor, nn
+from torch.nn.modules import module as _torch_module
+
+from . import global_config as config
+from . import hip_funcs
+from . import lib as _lib
+from . import ops
+from . import pooling
+from .lib import CrystalformerHipError, device_guard, stream_handle
+
+
+def _hooked(module: nn.Module) -> bool:
+    return bool(module._forward_hooks or module._forward_pre_hooks)
+
+
+def _any_hooked(module: nn.Module) -> bool:
+    if _hooked(module):
+        return True
+    for child in module._modules.values():
+        if child is not None and _any_hooked(child):
+            return True
+    return False
+
+
+def _ready(t: Optional[Tensor], numel: int, device_index: int) -> bool:
+    """A parameter the kernels can read as it is (absent ones are fine)."""
+    return t is None or (t.dtype is torch.float32 and t.get_device() == device_index and t.is_contiguous()
+                         and t.numel() == numel)
+
+
+def _address(t: Optional[Tensor]) -> Optional[int]:
+    return None if t is None else t.data_ptr()
+
+
+def _block(layer: nn.Module, width: int, device_index: int):
+    """(``cf_forward_block`` fields, heads, feed-forward width) of a layer, or None when it is not the plain case."""
+    from .attention import CrystalformerMultiheadAttentionCUDA, fused_exponents_spec
+    from .encoder import CrystalformerEncoderLayerCUDA
+    if type(layer) is not CrystalformerEncoderLayerCUDA:
+        return None
+    mods = layer._modules
+    attn, lin1, lin2 = mods["self_attn"], mods["linear1"], mods["linear2"]
+    if type(attn) is not CrystalformerMultiheadAttentionCUDA or type(lin1) is not nn.Linear or type(lin2) is not nn.Linear:
+        return None
+    if type(mods["norm1"]) is not nn.Identity or type(mods["norm2"]) is not nn.Identity \
+            or layer.activation is not torch.nn.functional.relu:
+        return None
+    P = attn.params
+    if layer.training and (attn.dropout > 0 or any(type(mods[d]) is not nn.Identity
+                                                   for d in ("dropout", "dropout1", "dropout2"))):
+        return None
+    spec = fused_exponents_spec(P)
+    if P.domain != "real" or P.norm_func_mode not in (0, "default") or spec is None \
+            or attn.kdim != width or attn.vdim != width or attn.embed_dim != width:
+        return None
+    H = attn.num_heads
+    D = width // H
+    bins = max(int(P.value_pe_dist_real), 0)
+    if bins == 0 and not hip_funcs.KernelManager.FUSE_ENCODING_ATTENTION:
+        return None                                    # (the two operators asked for one by one)
+    if bins > 0 and (P.value_pe_condproj != "no" or not P.value_pe_headed or not P.use_low_memory):
+        return None
+    own = attn._parameters
+    out, w1, w2 = attn._modules["out_proj"]._parameters, lin1._parameters, lin2._parameters
+    ff = lin1.out_features
+    tensors = (own["q_proj_weight"], own["k_proj_weight"], own["v_proj_weight"], own["in_proj_bias"],
+               own["lattice_pos_weights"], own["gauss_scale"], own["pe_dist_proj"] if bins > 0 else None,
+               out["weight"], out["bias"], w1["weight"], w1["bias"], w2["weight"], w2["bias"])
+    sq = width * width
+    counts = (sq, sq, sq, 3 * width, width, 2, H * D * bins, sq, width, width * ff, ff, width * ff, width)
+    if bins > 0 and tensors[6] is None:
+        return None
+    for t, n in zip(tensors, counts):
+        if not _ready(t, n, device_index):
+            return None
+    dist_max = P.value_pe_dist_max
+    if dist_max < 0:
+        dist_max = (-dist_max) * P.scale_real
+    cutoff = P.adaptive_cutoff_sigma
+    if cutoff > 0:
+        cutoff = P.scale_real * P.gauss_lb_real ** (-0.5) * cutoff
+    fields = [_address(t) for t in tensors]
+    fields += [bins, int(bool(P.normalize_gauss)), ops.POSITIVE_FUNCS[spec[0]], dist_max, P.value_pe_width_scale,
+               cutoff, -0.5 * P.gauss_lb_real * P.scale_real ** -2 * (1 - 1e-5), -0.5 * P.scale_real ** -2,
+               P.gauss_lb_real, spec[1], 1.0 / math.sqrt(D)]
+    return fields, H, ff
+
+
+def _head(mlp: nn.Module, width: int, device_index: int) -> Optional[Tuple[tuple, int, int]]:
+    """((w_head, b_head, w_last, b_last), hidden, targets) of a head ``Linear, ReLU, Linear`` or ``Linear``
+    (identities in between do not count), else None."""
+    mods = [m for m in mlp._modules.values() if type(m) is not nn.Identity]
+    kinds = [type(m) for m in mods]
+    if kinds == [nn.Linear, nn.ReLU, nn.Linear]:
+        first, last = mods[0]._parameters, mods[2]._parameters
+        hidden = mods[0].out_features
+        if hidden % 16 or mods[2].in_features != hidden \
+                or not _ready(first["weight"], hidden * width, device_index) \
+                or not _ready(first["bias"], hidden, device_index):
+            return None
+        head = (first["weight"], first["bias"])
+    elif kinds == [nn.Linear]:
+        last, hidden, head = mods[0]._parameters, 0, (None, None)
+    else:
+        return None
+    targets = mods[-1].out_features
+    if not _ready(last["weight"], targets * (hidden or width), device_index) \
+            or not _ready(last["bias"], targets, device_index):
+        return None
+    return head + (last["weight"], last["bias"]), hidden, targets
+
+
+def _run(encoder: nn.Module, src: Tensor, pos: Tensor, batch: Tensor, trans: Tensor, sizes: Tensor,
+         head=None) -> Optional[Tensor]:
+    KM = hip_funcs.KernelManager
+    if torch.is_grad_enabled() or config.REPRODUCIBLITY_STATE < 2 or not KM.DENSE_EDGE_BLOCKS \
+            or ops.instrumented() or encoder._modules.get("norm") is not None \
+            or _torch_module._global_forward_hooks or _torch_module._global_forward_pre_hooks or _any_hooked(encoder):
+        return None
+    width = encoder.d_model
+    index = src.get_device()
+    N = src.shape[0]
+    B = trans.shape[0]
+    if index < 0 or src.dim() != 2 or N == 0 or not _ready(src, N * width, index) or not _ready(pos, 3 * N, index) \
+            or not _ready(trans, 9 * B, index) or batch.get_device() != index or batch.dtype is not torch.int64:
+        return None
+    blocks = []
+    H = ff = None
+    for layer in encoder._modules["layers"]._modules.values():
+        got = _block(layer, width, index)
+        if got is None or (blocks and (got[1] != H or got[2] != ff)):
+            return None
+        fields, H, ff = got
+        blocks.append(fields)
+    if not blocks:
+        return None
+    dev = src.device
+    from .encoder import _sizes_on_device
+    if not torch.is_tensor(sizes) or sizes.device != dev or sizes.dtype != torch.long:
+        sizes = _sizes_on_device(sizes, batch, B, dev)
+    layout = ops.batch_layout(sizes, batch)            # index structure: built once per batch
+    if layout.pairs is None or layout.num_edges == 0 or layout.num_atoms != N or sizes.numel() > B:
+        return None
+    tensors, hidden, targets = head if head is not None else ((None,) * 4, 0, 0)
+    out = torch.empty((sizes.numel(), targets) if targets else (N, width), dtype=torch.float32, device=dev)
+    L = _lib.load()
+    sched = ops._scheduling_words(dev) if ops.DYNAMIC_ROUNDS else None
+    args = _lib.ForwardArgs(
+        N, layout.num_edges, sizes.numel(), len(blocks), H, width, ff, KM.LATTICE_RANGE, KM.MINIMUM_RANGE, 1,
+        int(encoder.training), int(KM.STAGED_RINGS), int(KM.ADAPTIVE_RINGS), ops.STAGED_RINGS_MAX_BYTES, hidden,
+        targets, src.data_ptr(), pos.data_ptr(), trans.data_ptr(), layout.batch.data_ptr(), layout.atom_start.data_ptr(),
+        layout.edge_start.data_ptr(), layout.edges.data_ptr(), layout.e_start.data_ptr(), layout.pairs.data_ptr(),
+        _address(sched), *(_address(t) for t in tensors), out.data_ptr())
+    table = (_lib.ForwardBlock * len(blocks))(*(tuple(f) for f in blocks))
+    need = L.cf_forward_workspace(_lib.ctypes.byref(args), table)
+    if need < 0:
+        return None
+    ws = torch.empty(need, dtype=torch.uint8, device=dev)
+    with device_guard(dev):
+        rc = L.cf_forward(_lib.ctypes.byref(args), table, ws.data_ptr(), need, stream_handle(dev))
+    if rc == -2:                                       # a shape some kernel does not serve: module by module
+        return None
+    _lib.check(rc, "cf_forward")
+    return out
+
+
+def encode(encoder: nn.Module, src: Tensor, pos: Tensor, batch: Tensor, trans: Tensor, sizes) -> Optional[Tensor]:
+    """The output of ``CrystalformerEncoderCUDA.forward``, or None where it has to run module by module."""
+    return _run(encoder, src, pos, batch, trans, sizes)
+
+
+def forward(model: nn.Module, src: Tensor, data) -> Optional[Tensor]:
+    """The output of ``Latticeformer.forward`` behind the embedding, or None."""
+    if torch.is_grad_enabled():
+        return None
+    mods = model._modules
+    if type(mods["proj_before_pooling"]) is not nn.Identity or model.pooling_layer is not pooling.avr_pool \
+            or _hooked(mods["proj_before_pooling"]) or _any_hooked(mods["mlp"]):
+        return None
+    head = _head(mods["mlp"], mods["encoder"].d_model, src.get_device())
+    if head is None:
+        return None
+    return _run(mods["encoder"], src, data.pos, data.batch, data.trans_vec, data.sizes, head)

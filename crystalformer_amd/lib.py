@@ -24,6 +24,25 @@ _dbl = ctypes.c_double
 _f32 = ctypes.c_float
 _ptr = ctypes.c_void_p
 
+
+class ForwardBlock(ctypes.Structure):
+    """``cf_forward_block`` of include/crystalformer_hip.h."""
+    _fields_ = ([(n, _ptr) for n in ("wq", "wk", "wv", "b_in", "w_pos", "gauss_scale", "w_pe", "wo", "bo", "w1", "b1",
+                                     "w2", "b2")]
+                + [(n, _i64) for n in ("bins", "normalize", "positive_func")]
+                + [(n, _dbl) for n in ("dist_max", "wscale", "cutoff", "weakest", "coef", "lower_bound", "beta",
+                                       "q_scale")])
+
+
+class ForwardArgs(ctypes.Structure):
+    """``cf_forward_args`` of include/crystalformer_hip.h."""
+    _fields_ = ([(n, _i64) for n in ("N", "E", "B", "layers", "H", "width", "ff", "lattice_range", "minimum_range",
+                                     "adaptive", "update_stats", "staged_rings", "adaptive_rings", "ring_limit_bytes",
+                                     "hidden", "targets")]
+                + [(n, _ptr) for n in ("x", "pos", "tvecs", "batch", "atom_start", "edge_start", "edges", "e_start",
+                                       "pairs", "sched", "w_head", "b_head", "w_last", "b_last", "out")])
+
+
 # name -> (restype, argtypes); mirrors include/crystalformer_hip.h
 SIGNATURES = {
     "cf_version": (_int, []),
@@ -67,6 +86,8 @@ SIGNATURES = {
     "cf_gauss_exponents_bwd_workspace": (_i64, [_i64, _i64, _i64]),
     "cf_gauss_exponents_bwd": (_int, [_ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _i64, _i64, _i64, _int, _f32, _f32, _f32,
                                       _f32, _ptr, _i64, _ptr, _ptr, _ptr]),
+    "cf_forward_workspace": (_i64, [_ptr, _ptr]),
+    "cf_forward": (_int, [_ptr, _ptr, _ptr, _i64, _ptr]),
     "cf_kr_base": (_int, [_ptr, _ptr, _ptr, _ptr, _i64, _ptr, _ptr]),
     "cf_reci_enc_fwd": (_int, [_ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _i64, _i64, _i64, _int, _ptr, _ptr, _ptr]),
     "cf_reci_enc_bwd": (_int, [_ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _i64, _i64, _i64, _int, _int, _ptr, _ptr]),

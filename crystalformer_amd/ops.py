@@ -37,6 +37,11 @@ def set_eval_counter(counter: Optional[list]) -> None:
     _eval_counter = counter
 
 
+def instrumented() -> bool:
+    """Whether launches are being timed or counted one by one."""
+    return _event_log is not None or _eval_counter is not None
+
+
 def count_translation_evals(a_ik: Tensor, rvlen_n: Optional[Tensor], batch_i: Tensor, edge_ij_e: Tensor,
                             cutoff: float, lattice_range: int, minimum_range: int) -> float:
     E = edge_ij_e.shape[1]

@@ -478,6 +478,50 @@ int cf_linear_weight_grad(const float *g, const float *x, int64_t N, int64_t C, 
                           void *workspace, int64_t workspace_bytes, float *gW, float *gb, void *stream);
 
 /*
+ * Inference forward of the encoder -- and, with targets > 0, of mean pooling and the regression head --
+ * in one call that issues every launch: what CrystalformerEncoderCUDA.forward
+ * (models/indexed_latticeformer_encoder.py:872-890) and Latticeformer.forward
+ * (models/latticeformer.py:291-302) do operator by operator, for blocks in the real domain without norm
+ * layers (t-fixup), with ReLU, the plain softmax, one value projection per head and exponents from the
+ * query.  The index structure of the batch (edges, row offsets, pair list) comes from cf_batch_layout.
+ * With a size header set, N and E are the capacities (see cf_set_size_header).
+ */
+typedef struct {
+    const float *wq, *wk, *wv;        /* (width, width) each */
+    const float *b_in;                /* (3 width), nullable */
+    const float *w_pos;               /* (width): exponent weights per head */
+    float *gauss_scale;               /* (2): stored statistics, written when update_stats */
+    const float *w_pe;                /* (H, D, bins), NULL without value bins */
+    const float *wo, *bo;             /* (width, width), (width) nullable */
+    const float *w1, *b1;             /* (ff, width), (ff) nullable */
+    const float *w2, *b2;             /* (width, ff), (width) nullable */
+    int64_t bins, normalize, positive_func;     /* positive_func as in cf_gauss_exponents */
+    double dist_max, wscale;          /* bin grid */
+    double cutoff;                    /* adaptive boxes (as cutoff_radius of cf_real_enc_fwd), 0: fixed cube */
+    double weakest;                   /* upper bound (<= 0) of the exponents (cf_real_enc_ring_stage) */
+    double coef, lower_bound, beta, q_scale;    /* as in cf_gauss_exponents */
+} cf_forward_block;
+
+typedef struct {
+    int64_t N, E, B, layers, H, width, ff;
+    int64_t lattice_range, minimum_range;
+    int64_t adaptive;                 /* 0: cutoffs are ignored, every box is the fixed cube */
+    int64_t update_stats;             /* training mode without gradients: store the exponent statistics */
+    int64_t staged_rings, adaptive_rings, ring_limit_bytes;   /* whether and up to what size blocks share staged rings */
+    int64_t hidden, targets;          /* head: width -> hidden (ReLU) -> targets; hidden 0: width -> targets;
+                                         targets 0: out takes the encoder's output (N, width) */
+    const float *x, *pos, *tvecs;     /* (N, width) embedded atoms, (N, 3), (B, 3, 3) */
+    const int64_t *batch, *atom_start, *edge_start, *edges, *e_start, *pairs;
+    int32_t *sched;                   /* two zeroed words (as sched_2 of cf_real_enc_fwd), nullable */
+    const float *w_head, *b_head, *w_last, *b_last;
+    float *out;                       /* (B, targets) or (N, width) */
+} cf_forward_args;
+
+int64_t cf_forward_workspace(const cf_forward_args *args, const cf_forward_block *blocks);
+int cf_forward(const cf_forward_args *args, const cf_forward_block *blocks, void *workspace,
+               int64_t workspace_bytes, void *stream);
+
+/*
  * Reciprocal-space periodic encoding (ReciPeriodicEncodingFuncCUDA, models/cuda_funcs/reci_space_enc.py:17-99;
  * kernels models/kernels/reci_enc_fwd.cu:3-68, reci_enc_bwd.cu:3-71), LATTICE_RANGE passed at run time:
  *   S[e,h] = sum over n1 in [0,R] (weight 2 for n1 != 0), n2, n3 in [-R,R] of

@@ -1,0 +1,126 @@
+"""The native inference forward (``executor``) against the same model run module by module, and
+against the CPU oracle: the sizes at which its kernels can go wrong (one atom, row tiles and their
+remainders, empty crystals), the options it serves and those it leaves to the modules."""
+import pytest
+import torch
+
+from crystalformer_amd import executor, hip_funcs
+from crystalformer_amd.latticeformer import Latticeformer, default_params
+from crystalformer_amd.synthetic import CrystalBatch, make_batch
+from oracle import torch_model as om
+from tests.helpers import RTOL, assert_close, atol_rows
+
+pytestmark = pytest.mark.gpu
+
+
+def batch_of(sizes, seed=3):
+    """Crystals of exactly these sizes (zeros allowed)."""
+    full = make_batch(len(sizes), (max(sizes), max(sizes)), False, (3.0, 11.0), (65.0, 115.0), seed=seed)
+    keep = torch.cat([torch.arange(max(sizes)) < n for n in sizes])
+    s = torch.tensor(sizes)
+    return CrystalBatch(full.x[keep], full.pos[keep].contiguous(), torch.repeat_interleave(torch.arange(len(s)), s),
+                        full.trans_vec, s)
+
+
+def both_ways(model, b):
+    """(native, module by module) outputs of the encoder: a forward hook sends it through the modules."""
+    x = torch.nn.functional.linear(b.x, model.input_embeddings.weight)
+    args = (x, b.pos, b.batch, b.trans_vec, b.sizes)
+    with torch.no_grad():
+        native = executor.encode(model.encoder, *args)
+        assert native is not None
+        handle = model.encoder.layers[0].linear1.register_forward_hook(lambda m, i, o: None)
+        try:
+            assert executor.encode(model.encoder, *args) is None
+            return native, model.encoder(*args)
+        finally:
+            handle.remove()
+
+
+def scaled(cfg, seed=5):
+    torch.manual_seed(seed)
+    model = Latticeformer(cfg)
+    with torch.no_grad():
+        model.input_embeddings.weight.normal_()            # (the initialisation's features are near zero)
+        for layer in model.encoder.layers:
+            for p in (layer.self_attn.in_proj_bias, layer.self_attn.out_proj.bias, layer.linear1.bias,
+                      layer.linear2.bias):
+                p.normal_(0.0, 0.3)
+    return model
+
+
+# sizes: one atom; a tile of rows less one, exactly, plus one; more than one tile; empty crystals
+@pytest.mark.parametrize("sizes", [[1], [15], [16], [17], [1, 2, 30], [5, 0, 0, 64, 3], [200]])
+@pytest.mark.parametrize("options", [dict(), dict(adaptive_cutoff_sigma=0.0), dict(value_pe_dist_real=0),
+                                     dict(value_pe_dist_real=24, head_num=4, positive_func="abs"),
+                                     dict(model_dim=64, embedding_dim=[64], ff_dim=96, normalize_gauss=False)])
+def test_native_forward_equals_the_modules(dev, sizes, options):
+    model = scaled(default_params(num_layers=2, **options)).to(dev).eval()
+    b = batch_of(sizes).to(dev)
+    native, modules = both_ways(model, b)
+    # every output element is a chain of sums over up to 512 products of its row
+    assert_close(native, modules, "encoder", rtol=RTOL, atol=atol_rows(modules))
+    with torch.no_grad():
+        for layer in model.encoder.layers:                 # stored statistics instead of the batch's
+            layer.self_attn.gauss_scale.copy_(torch.tensor([0.7, -0.2]))
+    native, modules = both_ways(model, b)
+    assert_close(native, modules, "encoder, stored statistics", rtol=RTOL, atol=atol_rows(modules))
+
+
+@pytest.mark.parametrize("options", [dict(), dict(targets=["a", "b", "c"]), dict(embedding_dim=[128, 64]),
+                                     dict(pre_pooling_op="w+relu", embedding_dim=[128, 128])])
+def test_native_forward_with_its_head(dev, options):
+    """Whole model, one or several targets and heads the native call does not take, against the oracle."""
+    cfg = default_params(num_layers=2, adaptive_cutoff_sigma=0.0, **options)
+    model = scaled(cfg)
+    b = batch_of([3, 1, 40, 17])
+    with torch.no_grad():
+        if "pre_pooling_op" in options or len(cfg.embedding_dim) > 1:
+            got = model.to(dev).eval()(b.to(dev))
+            model.encoder.register_forward_hook(lambda m, i, o: None)
+            want = model(b.to(dev)).cpu()
+        else:
+            want = om.latticeformer_forward({k: v.detach() for k, v in model.state_dict().items()}, cfg, b,
+                                            training=False)
+            got = model.to(dev).eval()(b.to(dev))
+    assert_close(got, want, "model", rtol=RTOL)
+
+
+def test_training_mode_without_gradients_stores_the_statistics(dev):
+    cfg = default_params(num_layers=2)
+    one, two = scaled(cfg).to(dev).train(), scaled(cfg).to(dev).train()
+    b = batch_of([9, 20]).to(dev)
+    handle = two.encoder.layers[0].register_forward_hook(lambda m, i, o: None)
+    with torch.no_grad():
+        y1, y2 = one(b), two(b)
+    handle.remove()
+    assert_close(y1, y2, "first pass")
+    for l1, l2 in zip(one.encoder.layers, two.encoder.layers):
+        assert float(l1.self_attn.gauss_scale[0]) > 0
+        assert_close(l1.self_attn.gauss_scale, l2.self_attn.gauss_scale, "statistics")
+    stored = [layer.self_attn.gauss_scale.clone() for layer in one.encoder.layers]
+    with torch.no_grad():
+        one(batch_of([4, 31], seed=8).to(dev))
+    for layer, s in zip(one.encoder.layers, stored):
+        assert torch.equal(layer.self_attn.gauss_scale, s)         # written once
+
+
+def test_native_forward_leaves_other_models_to_the_modules(dev):
+    b = batch_of([4, 6]).to(dev)
+    for options in (dict(domain="multihead"), dict(value_pe_condproj="i"), dict(gauss_state="1"),
+                    dict(t_fixup_init=False), dict(norm_func_mode=2), dict(use_low_memory=False),
+                    dict(t_activation="gelu")):
+        model = scaled(default_params(num_layers=1, **options)).to(dev).eval()
+        x = torch.nn.functional.linear(b.x, model.input_embeddings.weight)
+        with torch.no_grad():
+            assert executor.encode(model.encoder, x, b.pos, b.batch, b.trans_vec, b.sizes) is None, options
+            assert torch.isfinite(model(b)).all()
+    model = scaled(default_params(num_layers=1)).to(dev).eval()
+    x = torch.nn.functional.linear(b.x, model.input_embeddings.weight)
+    assert executor.encode(model.encoder, x, b.pos, b.batch, b.trans_vec, b.sizes) is None      # gradients wanted
+    hip_funcs.KernelManager.DENSE_EDGE_BLOCKS = False
+    try:
+        with torch.no_grad():
+            assert executor.encode(model.encoder, x, b.pos, b.batch, b.trans_vec, b.sizes) is None
+    finally:
+        hip_funcs.KernelManager.DENSE_EDGE_BLOCKS = True

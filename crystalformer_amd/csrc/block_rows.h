@@ -1,0 +1,54 @@
+// Arguments and launchers of block_rows.hip (row-wise parts of a forward, used by cf_forward).
+#pragma once
+#include "cf_common.h"
+
+namespace cf {
+
+struct RowsArgs {
+    int64_t N;
+    int H, embed_width;
+    const float *att, *x;                     // attention output; block input (or the rows to embed)
+    const float *packed_tail, *packed_head;   // packed weights of the block each belongs to, null: no such part
+    const float *bo, *b1, *b2;                // tail
+    const float *packed_embed, *b_embed;      // null: x is the block input itself
+    float *y;                                 // tail or embedding: the rows behind it
+    const float *b_in, *w_pos;                // head
+    float *gauss_scale;
+    int normalize, update_stats, func;
+    float beta, lb, coef, q_scale;
+    float *qs, *k, *v, *a;
+    float *part;                              // statistics without stored ones: 3 floats per 256 values of a
+    unsigned *counter;                        // zeroed word
+    const int64_t *live_N;                    // set by the launcher
+};
+
+constexpr int PACK_BLOCKS = 32;               // blocks per packing launch (48 bytes of kernel arguments each)
+constexpr int64_t PACKED_BLOCK = 12 * 128 * 128;   // floats a block
+struct PackSource {
+    const float *wo, *w1, *w2, *wq, *wk, *wv;
+};
+struct PackArgs {
+    PackSource block[PACK_BLOCKS];
+    int blocks, embed_width;
+    const float *w_embed;                     // (128, embed_width <= 128), nullable
+    float *packed, *packed_embed;             // blocks x PACKED_BLOCK floats; 128 x 128
+};
+int launch_pack_weights(const PackArgs &p, hipStream_t st);
+
+struct PoolHeadArgs {
+    const float *x;
+    const int64_t *start_n;
+    const float *w_head, *b_head, *w_last, *b_last;
+    int64_t hidden, targets;
+    float *out;
+};
+
+bool block_rows_served(int64_t width, int64_t ff, int64_t H);
+int launch_block_rows(RowsArgs p, hipStream_t st);
+bool pool_head_served(int64_t width, int64_t hidden);
+int launch_pool_head(const PoolHeadArgs &p, int64_t B, hipStream_t st);
+// cf_lattice_geometry that also clears `words` 32-bit words at `zero` (counters of later launches).
+int launch_lattice_geometry(const float *trans, int64_t B, float *vcell, float *recip, float *rvlen, unsigned *zero,
+                            int words, hipStream_t st);
+
+}  // namespace cf

@@ -1,0 +1,499 @@
+// Everything between one block's attention and the next block's that works row by row, in one launch:
+//
+//   tail   s = att Wo^T + bo + x,  h = relu(s W1^T + b1),  y = h W2^T + b2 + s
+//   head   q, k, v = y Wq^T, y Wk^T, y Wv^T (+ b),  a = coef rho(norm(<q, w_pos>)),  q scaled
+//
+// for the 128-wide blocks with 512 hidden units; the embedding of the atoms can stand in front of the
+// first head.  As four linear launches and two for the exponents this was 6.6 and 4.5 us each at the 1.8
+// thousand rows of a batch, none of it arithmetic: 0.35 GFLOP a block take 2.2 us at the fp32 matrix rate.
+//
+// A work-group of 8 wavefronts owns 4 R rows; the rows and all intermediates stay in LDS, the weights
+// (786 KB a block) stream from the L2, a 16-column tile per wavefront, two tiles ahead of their use.  At 64
+// bytes a clock a CU reads the weights in 5 us, and at 4 R = 8 rows the matrix cores (256 FLOP a clock and
+// CU) need as long; measured 14.2 us a launch with tail and head at 1774 rows (R 2), 10.1 at 12 rows (R 1), 20.3
+// at 4096 (R 4), against 35 us as six launches.  Variants: weights read from the matrices as they are 24 us (see
+// pack_weights_kernel); every 16-column tile with its own read of the rows, its own epilogue and a barrier 16.5 us.
+//
+// v_mfma_f32_4x4x1_16b_f32: sixteen independent 4 x 4 blocks, here 4 column groups x 4 reduction slots.
+//   B: lane (kq, c) = (lane / 16, lane % 16) holds W[col c][k0 + 4 kq + s], one component of a 16-byte load
+//      (16 rows of W, 64 consecutive bytes of each);
+//   A: lane l holds x[row l % 4][k0 + l / 4], one 4-byte LDS read for four steps: step s broadcasts block
+//      4 kq + s of each group of four (CBSZ 2, ABID s) to the group;
+//   D: lane (kq, c), register r: row r, column c, summed over the reduction slots 4 kq .. 4 kq + 3 of every
+//      16; two lane swaps at the end add the four slots and leave row kq, column c in each lane.
+// A row's sums do not depend on R or on the tile it falls in.
+#include "cf_common.h"
+#include "block_rows.h"
+#include "gauss_maps.h"
+
+#include <math.h>
+
+namespace {
+
+using namespace cf;
+
+typedef float float4_t __attribute__((ext_vector_type(4)));
+
+constexpr int RW = 128, RF = 512;            // block width, hidden units
+constexpr int LDX = RW + 16, LDH = RF + 16;  // LDS row strides: 16 mod 64, so the four rows of an A read and
+                                             // the four rows of a D write fall into disjoint banks
+constexpr int RT = 512;                      // threads
+
+enum Source { ROWS_PLAIN = 0, ROWS_EMBED = 1, ROWS_TAIL = 2 };
+
+struct Weights {
+    float4_t w[8];                           // 128 reduction steps of a 16-column tile
+};
+
+// `p` is wave-uniform and `off` this lane's byte offset: one address register for all units.
+__device__ __forceinline__ void load_weights(Weights &b, const float *__restrict__ p, unsigned off)
+{
+#pragma unroll
+    for (int c = 0; c < 8; c++)
+        b.w[c] = *reinterpret_cast<const float4_t *>(reinterpret_cast<const char *>(p + 256 * c) + off);
+}
+
+// The rows' values of 128 reduction steps as A operands.
+template <int R>
+struct Rows {
+    float x[8][R];
+};
+
+template <int R>
+__device__ __forceinline__ void read_rows(Rows<R> &a, const float *xs, int ld, int lane)
+{
+    const float *xr = xs + (lane & 3) * ld + (lane >> 2);
+#pragma unroll
+    for (int c = 0; c < 8; c++)
+#pragma unroll
+        for (int r = 0; r < R; r++) a.x[c][r] = xr[4 * r * ld + 16 * c];
+}
+
+template <int R>
+__device__ __forceinline__ void multiply(float4_t (&acc)[R], const Weights &b, const Rows<R> &a)
+{
+#pragma unroll
+    for (int c = 0; c < 8; c++) {
+#pragma unroll
+        for (int r = 0; r < R; r++) acc[r] = __builtin_amdgcn_mfma_f32_4x4x1f32(a.x[c][r], b.w[c][0], acc[r], 2, 0, 0);
+#pragma unroll
+        for (int r = 0; r < R; r++) acc[r] = __builtin_amdgcn_mfma_f32_4x4x1f32(a.x[c][r], b.w[c][1], acc[r], 2, 1, 0);
+#pragma unroll
+        for (int r = 0; r < R; r++) acc[r] = __builtin_amdgcn_mfma_f32_4x4x1f32(a.x[c][r], b.w[c][2], acc[r], 2, 2, 0);
+#pragma unroll
+        for (int r = 0; r < R; r++) acc[r] = __builtin_amdgcn_mfma_f32_4x4x1f32(a.x[c][r], b.w[c][3], acc[r], 2, 3, 0);
+    }
+    // (the products belong here: left to itself the compiler moves them to where the sums are used, and keeps
+    // every weight until then)
+#pragma unroll
+    for (int r = 0; r < R; r++) asm volatile("" : "+v"(acc[r]));
+}
+
+__device__ __forceinline__ float lo_f(uint2_cf r) { return __int_as_float((int)r[0]) + __int_as_float((int)r[1]); }
+
+// Sum over the four reduction slots: lane (g, c) gets row g of the tile.
+__device__ __forceinline__ float slot_sum(float4_t a)
+{
+    const float u = lo_f(__builtin_amdgcn_permlane32_swap(__float_as_int(a[0]), __float_as_int(a[2]), false, false));
+    const float v = lo_f(__builtin_amdgcn_permlane32_swap(__float_as_int(a[1]), __float_as_int(a[3]), false, false));
+    return lo_f(__builtin_amdgcn_permlane16_swap(__float_as_int(u), __float_as_int(v), false, false));
+}
+
+template <int R>
+__device__ __forceinline__ void clear(float4_t (&acc)[R])
+{
+#pragma unroll
+    for (int r = 0; r < R; r++) acc[r] = float4_t{0.f, 0.f, 0.f, 0.f};
+}
+
+// Rows row0 .. of a (N, 128) matrix into LDS (rows past the end repeat the last one).
+template <int R>
+__device__ __forceinline__ void stage_rows(float *dst, const float *__restrict__ src, int64_t row0, int64_t N)
+{
+    for (int t = threadIdx.x; t < 4 * R * (RW / 4); t += RT) {
+        const int r = t / (RW / 4), c = t % (RW / 4);
+        const int64_t row = min(row0 + r, N - 1);
+        *reinterpret_cast<float4_t *>(dst + r * LDX + 4 * c) =
+            *reinterpret_cast<const float4_t *>(src + row * RW + 4 * c);
+    }
+}
+
+// The exponents where no statistics are stored: the last work-group to finish merges the statistics of
+// all raw values (a holds them) as the two exponent kernels do -- groups of 256 values, mean first, then
+// the squared deviations, groups merged by Chan's formula in the same order -- and maps them in place.
+__device__ void finish_exponents(const RowsArgs &p, int64_t total, float *red)
+{
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t blocks = (total + 255) / 256;
+    for (int64_t b = wave; b < blocks; b += RT / WAVE) {
+        float v[4], s[4];
+        const float cnt = (float)min((int64_t)256, total - 256 * b);
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const int64_t t = 256 * b + 64 * u + lane;
+            v[u] = t < total ? p.a[t] : 0.f;
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u++) s[u] = wave_sum(v[u]);
+        const float mean = (((0.f + s[0]) + s[1]) + s[2] + s[3]) / cnt;
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const float dv = 256 * b + 64 * u + lane < total ? v[u] - mean : 0.f;
+            s[u] = wave_sum(dv * dv);
+        }
+        if (lane == 0) {
+            p.part[3 * b] = cnt;
+            p.part[3 * b + 1] = mean;
+            p.part[3 * b + 2] = ((0.f + s[0]) + s[1]) + s[2] + s[3];
+        }
+    }
+    __syncthreads();
+    if (wave == 0) {
+        float n, mean, m2;
+        merge_statistics(p.part, (int)blocks, lane, n, mean, m2);
+        if (lane == 0) {
+            const float scale = 1.0f / sqrtf(m2 / (n - 1.0f));
+            red[0] = scale;
+            red[1] = -mean;
+            if (p.update_stats) {
+                p.gauss_scale[0] = scale;
+                p.gauss_scale[1] = -mean;
+            }
+        }
+    }
+    __syncthreads();
+    const float scale = red[0], shift = red[1];
+    for (int64_t t = threadIdx.x; t < total; t += RT)
+        p.a[t] = positive_map((p.a[t] + shift) * scale, p.func, p.beta, p.lb) * p.coef;
+}
+
+// The matrices as a sequence of units, 16 columns a wavefront x 128 reduction steps each:
+// 0 output projection, 1-4 hidden units, 5-8 their reduction (or 8 the embedding), 9-11 query, key, value.
+constexpr int UNIT_FF1 = 1, UNIT_FF2 = 5, UNIT_EMBED = 8, UNIT_QUERY = 9, UNIT_END = 12, UNIT_FLOATS = RW * RW;
+
+// The weights of up to PACK_BLOCKS blocks in the order the row kernel reads them: per unit and wavefront eight
+// 1 KB pieces, one per 16 reduction steps, in lane order.  Read from the matrices themselves every load
+// of a wavefront takes 64 bytes of 16 rows, 512 or 2048 bytes apart, which fall into a few of the L2's
+// channels: 24 us a launch.
+__global__ __launch_bounds__(256) void pack_weights_kernel(PackArgs p)
+{
+    const int l = blockIdx.y, u = blockIdx.x / (UNIT_FLOATS / 1024);
+    if (l == p.blocks && u > 0) return;
+    const int at = 4 * (int)(blockIdx.x % (UNIT_FLOATS / 1024) * 256 + threadIdx.x);     // first of four floats of the unit
+    const int wave = at / 2048, k = at / 256 % 8 * 16 + at / 64 % 4 * 4, col = 16 * wave + at / 4 % 16;
+    if (l == p.blocks) {                                        // the embedding, filled up with zeros
+        const float *we = p.w_embed + col * p.embed_width;
+        float4_t v;
+#pragma unroll
+        for (int i = 0; i < 4; i++) v[i] = k + i < p.embed_width ? we[k + i] : 0.f;
+        *reinterpret_cast<float4_t *>(p.packed_embed + at) = v;
+        return;
+    }
+    const PackSource &w = p.block[l];
+    const float *src;
+    if (u == 0) src = w.wo + col * RW + k;
+    else if (u < UNIT_FF2) src = w.w1 + ((u - UNIT_FF1) * RW + col) * RW + k;
+    else if (u < UNIT_QUERY) src = w.w2 + col * RF + (u - UNIT_FF2) * RW + k;
+    else src = (u == UNIT_QUERY ? w.wq : u == UNIT_QUERY + 1 ? w.wk : w.wv) + col * RW + k;
+    *reinterpret_cast<float4_t *>(p.packed + (int64_t)l * PACKED_BLOCK + u * UNIT_FLOATS + at) =
+        *reinterpret_cast<const float4_t *>(src);
+}
+
+template <int R, int SRC, bool HEAD>
+__global__ __launch_bounds__(RT) void block_rows_kernel(RowsArgs p)
+{
+    constexpr int M = 4 * R;
+    constexpr int FIRST = SRC == ROWS_TAIL ? 0 : SRC == ROWS_EMBED ? UNIT_EMBED : UNIT_QUERY;
+    constexpr int END = HEAD ? UNIT_END : UNIT_QUERY;
+    __shared__ __align__(16) float b0[M * LDX];
+    __shared__ __align__(16) float b1[M * LDX];
+    __shared__ __align__(16) float hs[M * LDH];                 // hidden units, then query, key, value
+    __shared__ float biases[UNIT_END * RW], w_pos[RW];
+    __shared__ float red[2];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int kq = lane >> 4, c = lane & 15;
+    const int col = 16 * wave + c;
+    const int64_t N = live_count(p.live_N, p.N);
+    bool stored = true;
+    float scale = 1.f, shift = 0.f;
+    if (HEAD && p.normalize) {
+        scale = p.gauss_scale[0];
+        shift = p.gauss_scale[1];
+        stored = scale > 0.f;
+    }
+    auto unit_weights = [&](int u) -> const float * {
+        if (SRC == ROWS_EMBED && u == UNIT_EMBED) return p.packed_embed;
+        return (u < UNIT_QUERY ? p.packed_tail : p.packed_head) + u * UNIT_FLOATS;
+    };
+    // (one tile per work-group unless the grid was cut short: with a live row count it covers a capacity)
+    bool first = true;
+    for (int64_t row0 = (int64_t)blockIdx.x * M; row0 < N; row0 += (int64_t)gridDim.x * M) {
+        float4_t acc[R];
+        Weights wa, wb, wc;
+        unsigned woff = (unsigned)(wave * 2048 + lane * 4) * 4u;
+        asm volatile("" : "+v"(woff));       // (not a constant of this loop: else a hundred registers hold addresses)
+        load_weights(wa, unit_weights(FIRST), woff);
+        if (SRC == ROWS_TAIL) {
+            stage_rows<R>(b0, p.att, row0, N);
+            stage_rows<R>(b1, p.x, row0, N);
+        } else if (SRC == ROWS_PLAIN) {
+            stage_rows<R>(b0, p.x, row0, N);
+        } else {
+            const int K = p.embed_width;
+            for (int t = threadIdx.x; t < M * RW; t += RT) {
+                const int r = t / RW, k = t % RW;
+                b1[r * LDX + k] = k < K ? p.x[min(row0 + r, N - 1) * K + k] : 0.f;
+            }
+        }
+        if (first) {
+            first = false;
+            for (int t = threadIdx.x; t < (END - FIRST) * RW; t += RT) {
+                const int u = FIRST + t / RW, k = t % RW;
+                const float *src = u >= UNIT_QUERY ? p.b_in : SRC == ROWS_EMBED ? p.b_embed : u == 0 ? p.bo
+                                   : u < UNIT_FF2 ? p.b1 : p.b2;
+                const int at = u >= UNIT_QUERY ? u - UNIT_QUERY : u >= UNIT_FF1 && u < UNIT_FF2 ? u - UNIT_FF1 : 0;
+                biases[u * RW + k] = src ? src[at * RW + k] : 0.f;
+            }
+            if (HEAD && threadIdx.x < RW) w_pos[threadIdx.x] = p.w_pos[threadIdx.x];
+        }
+        load_weights(wb, unit_weights(FIRST + 1), woff);
+        __syncthreads();
+        const int at = kq * LDX + col, at_h = kq * LDH + col;   // this lane's results: rows 4 r + kq
+        Rows<R> x;
+        if (SRC == ROWS_TAIL) {
+            // output projection and residual: s replaces x in place
+            load_weights(wc, unit_weights(2), woff);
+            read_rows(x, b0, LDX, lane);
+            clear(acc);
+            multiply(acc, wa, x);
+#pragma unroll
+            for (int r = 0; r < R; r++) b1[at + 4 * r * LDX] += slot_sum(acc[r]) + biases[col];
+            __syncthreads();
+            // hidden units, four tiles on one read of the rows
+            read_rows(x, b1, LDX, lane);
+            float4_t hid[4][R];
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                Weights &cur = u % 3 == 0 ? wb : u % 3 == 1 ? wc : wa, &nxt = u % 3 == 0 ? wa : u % 3 == 1 ? wb : wc;
+                load_weights(nxt, unit_weights(UNIT_FF1 + 2 + u), woff);
+                clear(hid[u]);
+                multiply(hid[u], cur, x);
+            }
+#pragma unroll
+            for (int u = 0; u < 4; u++)
+#pragma unroll
+                for (int r = 0; r < R; r++) {
+                    const float v = slot_sum(hid[u][r]) + biases[(UNIT_FF1 + u) * RW + col];
+                    hs[at_h + 4 * r * LDH + u * RW] = v < 0.f ? 0.f : v;          // (a NaN stays one, as in torch.relu)
+                }
+            __syncthreads();
+            clear(acc);
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                Weights &cur = u % 3 == 0 ? wc : u % 3 == 1 ? wa : wb, &nxt = u % 3 == 0 ? wb : u % 3 == 1 ? wc : wa;
+                if (UNIT_FF2 + 2 + u < END) load_weights(nxt, unit_weights(UNIT_FF2 + 2 + u), woff);
+                read_rows(x, hs + u * RW, LDH, lane);
+                multiply(acc, cur, x);
+            }
+#pragma unroll
+            for (int r = 0; r < R; r++)
+                b0[at + 4 * r * LDX] = slot_sum(acc[r]) + biases[UNIT_FF2 * RW + col] + b1[at + 4 * r * LDX];
+            __syncthreads();
+        } else if (SRC == ROWS_EMBED) {
+            load_weights(wc, unit_weights(UNIT_QUERY + 1), woff);
+            read_rows(x, b1, LDX, lane);
+            clear(acc);
+            multiply(acc, wa, x);
+#pragma unroll
+            for (int r = 0; r < R; r++) b0[at + 4 * r * LDX] = slot_sum(acc[r]) + biases[UNIT_EMBED * RW + col];
+            __syncthreads();
+        }
+        if (HEAD) {
+            float4_t proj[3][R];
+            read_rows(x, b0, LDX, lane);
+            constexpr int S = SRC == ROWS_EMBED ? 1 : 0;         // (the buffer that holds the query weights)
+#pragma unroll
+            for (int u = 0; u < 3; u++) {
+                Weights &cur = (u + S) % 3 == 0 ? wa : (u + S) % 3 == 1 ? wb : wc;
+                Weights &nxt = (u + S) % 3 == 0 ? wc : (u + S) % 3 == 1 ? wa : wb;
+                if (u == 0) load_weights(nxt, unit_weights(UNIT_QUERY + 2), woff);
+                clear(proj[u]);
+                multiply(proj[u], cur, x);
+            }
+#pragma unroll
+            for (int u = 0; u < 3; u++)
+#pragma unroll
+                for (int r = 0; r < R; r++)
+                    hs[at_h + 4 * r * LDH + u * RW] = slot_sum(proj[u][r]) + biases[(UNIT_QUERY + u) * RW + col];
+        }
+        if (HEAD) __syncthreads();
+        // results leave LDS in whole rows once the loop has no more loads to wait for
+        for (int t = threadIdx.x; t < M * (RW / 4); t += RT) {
+            const int r = t / (RW / 4), d = 4 * (t % (RW / 4));
+            const int64_t at = (row0 + r) * RW + d;
+            if (row0 + r >= N) break;
+            if (SRC != ROWS_PLAIN)
+                *reinterpret_cast<float4_t *>(p.y + at) = *reinterpret_cast<const float4_t *>(b0 + r * LDX + d);
+            if (HEAD) {
+                const float *out = hs + r * LDH + d;
+                *reinterpret_cast<float4_t *>(p.qs + at) = *reinterpret_cast<const float4_t *>(out) * p.q_scale;
+                *reinterpret_cast<float4_t *>(p.k + at) = *reinterpret_cast<const float4_t *>(out + RW);
+                *reinterpret_cast<float4_t *>(p.v + at) = *reinterpret_cast<const float4_t *>(out + 2 * RW);
+            }
+        }
+        if (HEAD) {
+            const int D = RW / p.H;
+            for (int t = threadIdx.x; t < M * p.H; t += RT) {
+                const int r = t / p.H, h = t - r * p.H;
+                const float *q = hs + r * LDH + h * D, *w = w_pos + h * D;
+                float alpha = 0.f;
+                for (int d = 0; d < D; d += 4)                  // (the order of the exponent kernel)
+                    alpha += (q[d] * w[d] + q[d + 1] * w[d + 1]) + (q[d + 2] * w[d + 2] + q[d + 3] * w[d + 3]);
+                if (p.normalize && stored) alpha = (alpha + shift) * scale;
+                if (!p.normalize || stored) alpha = positive_map(alpha, p.func, p.beta, p.lb) * p.coef;
+                if (row0 + r < N) p.a[(row0 + r) * p.H + h] = alpha;
+            }
+        }
+        __syncthreads();                                        // the next tile overwrites the rows
+    }
+    if (HEAD && !stored) {
+        // a work-group that had rows counts itself; the last one finishes the exponents of all
+        const int64_t active = min((int64_t)gridDim.x, (N + M - 1) / M);
+        if ((int64_t)blockIdx.x >= active) return;
+        __threadfence();
+        __syncthreads();
+        if (threadIdx.x == 0) red[0] = atomicAdd(p.counter, 1u) + 1u == (unsigned)active ? 1.f : 0.f;
+        __syncthreads();
+        const bool last = red[0] != 0.f;
+        __syncthreads();
+        if (last) {
+            __threadfence();
+            finish_exponents(p, N * p.H, red);
+        }
+    }
+}
+
+// Mean over a crystal's atoms and the regression head, one work-group per crystal: 32 lanes x 16 bytes
+// read an atom's row, sixteen atoms side by side; a row of a head matrix is one 512-byte read of half a
+// wavefront, requested before the mean so that nothing but the atoms' rows is waited for.  (As a mean and
+// two linear launches 17 us at 128 crystals, all latency.)
+constexpr int PH_T = 512, PH_G = PH_T / 32;
+__global__ __launch_bounds__(PH_T) void pool_head_kernel(PoolHeadArgs p)
+{
+    __shared__ __align__(16) float part[PH_G][RW];
+    __shared__ __align__(16) float top[RW];
+    const int64_t b = blockIdx.x;
+    const int g = threadIdx.x >> 5, piece = threadIdx.x & 31;
+    const int64_t r0 = p.start_n[b], r1 = p.start_n[b + 1];
+    float4_t wh[RW / PH_G];
+    float bh[RW / PH_G];
+    if (p.hidden) {
+#pragma unroll
+        for (int i = 0; i < RW / PH_G; i++) {
+            wh[i] = *reinterpret_cast<const float4_t *>(p.w_head + (i * PH_G + g) * RW + 4 * piece);
+            bh[i] = p.b_head ? p.b_head[i * PH_G + g] : 0.f;
+        }
+    }
+    float4_t s[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) s[u] = float4_t{0.f, 0.f, 0.f, 0.f};
+    int64_t r = r0 + g;
+    for (; r + 3 * PH_G < r1; r += 4 * PH_G)
+#pragma unroll
+        for (int u = 0; u < 4; u++) s[u] += *reinterpret_cast<const float4_t *>(p.x + (r + PH_G * u) * RW + 4 * piece);
+#pragma unroll
+    for (int u = 0; u < 3; u++)
+        if (r + PH_G * u < r1) s[u] += *reinterpret_cast<const float4_t *>(p.x + (r + PH_G * u) * RW + 4 * piece);
+    *reinterpret_cast<float4_t *>(&part[g][4 * piece]) = (s[0] + s[1]) + (s[2] + s[3]);
+    __syncthreads();
+    if (threadIdx.x < RW) {
+        float t = part[0][threadIdx.x];
+#pragma unroll
+        for (int i = 1; i < PH_G; i++) t += part[i][threadIdx.x];
+        top[threadIdx.x] = t / (float)(r1 - r0);
+    }
+    __syncthreads();
+    float4_t xv = *reinterpret_cast<const float4_t *>(&top[4 * piece]);
+    auto dot = [&](const float4_t wv) {
+        float d = (xv[0] * wv[0] + xv[1] * wv[1]) + (xv[2] * wv[2] + xv[3] * wv[3]);
+        d += dpp_f<DPP_QUAD_1032, 0xF>(0.f, d);
+        d += dpp_f<DPP_QUAD_2301, 0xF>(0.f, d);
+        d += dpp_f<DPP_ROW_ROR4, 0xF>(0.f, d);
+        d += dpp_f<DPP_ROW_ROR8, 0xF>(0.f, d);
+        return d + __shfl_xor(d, 16, 32);
+    };
+    if (p.hidden) {
+        __syncthreads();                                        // everyone holds its piece of the mean
+#pragma unroll
+        for (int i = 0; i < RW / PH_G; i++) {
+            const float v = dot(wh[i]) + bh[i];
+            if (piece == 0) top[i * PH_G + g] = v < 0.f ? 0.f : v;
+        }
+        __syncthreads();
+        xv = *reinterpret_cast<const float4_t *>(&top[4 * piece]);
+    }
+    for (int64_t o = g; o < p.targets; o += PH_G) {
+        const float v = dot(*reinterpret_cast<const float4_t *>(p.w_last + o * RW + 4 * piece))
+                        + (p.b_last ? p.b_last[o] : 0.f);
+        if (piece == 0) p.out[b * p.targets + o] = v;
+    }
+}
+
+template <int R>
+void launch_rows(const RowsArgs &p, int source, bool head, unsigned grid, hipStream_t st)
+{
+    if (source == ROWS_TAIL && head) block_rows_kernel<R, ROWS_TAIL, true><<<grid, RT, 0, st>>>(p);
+    else if (source == ROWS_TAIL) block_rows_kernel<R, ROWS_TAIL, false><<<grid, RT, 0, st>>>(p);
+    else if (source == ROWS_EMBED) block_rows_kernel<R, ROWS_EMBED, true><<<grid, RT, 0, st>>>(p);
+    else block_rows_kernel<R, ROWS_PLAIN, true><<<grid, RT, 0, st>>>(p);
+}
+
+}  // namespace
+
+namespace cf {
+
+bool block_rows_served(int64_t width, int64_t ff, int64_t H)
+{
+    return width == RW && ff == RF && H >= 1 && RW % H == 0 && (RW / H) % 4 == 0;
+}
+
+int launch_pack_weights(const PackArgs &p, hipStream_t st)
+{
+    pack_weights_kernel<<<dim3(UNIT_END * UNIT_FLOATS / 1024, (unsigned)(p.blocks + (p.w_embed ? 1 : 0))), 256, 0, st>>>(p);
+    CF_CHECK_LAUNCH("packing of the weights");
+    return CF_OK;
+}
+
+int launch_block_rows(RowsArgs p, hipStream_t st)
+{
+    const int source = p.packed_tail ? ROWS_TAIL : (p.packed_embed ? ROWS_EMBED : ROWS_PLAIN);
+    const bool head = p.packed_head != nullptr;
+    p.live_N = live_atoms(p.N);
+    const int64_t cus = device_cu_count();
+    // Rows per work-group.  Four while that gives a CU at most one tile, eight while that does.  Beyond, sixteen rows
+    // cost 20 us a round of tiles (one per CU), eight rows 23.5 us per two tiles and CU, side by side: sixteen
+    // where the last round is full enough (4096 rows 20.3 against 23.3 us, 5600 rows 37.8 against 32.5).  A live
+    // row count is somewhere below the capacity: eight rows.
+    const double rounds = (double)p.N / (double)(16 * cus);
+    const int R = p.live_N ? 2 : p.N <= 4 * cus ? 1 : ceil(rounds) * 0.85 <= rounds ? 4 : 2;
+    int64_t grid = (p.N + 4 * R - 1) / (4 * R);
+    if (p.live_N && grid > 2 * cus) grid = 2 * cus;             // a capacity: stride over the tiles that exist
+    CF_REQUIRE(grid < (1ll << 31), CF_ERR_UNSUPPORTED, "block rows: too many atoms");
+    if (R == 1) launch_rows<1>(p, source, head, (unsigned)grid, st);
+    else if (R == 2) launch_rows<2>(p, source, head, (unsigned)grid, st);
+    else launch_rows<4>(p, source, head, (unsigned)grid, st);
+    CF_CHECK_LAUNCH("block rows");
+    return CF_OK;
+}
+
+bool pool_head_served(int64_t width, int64_t hidden) { return width == RW && (hidden == 0 || hidden == RW); }
+
+int launch_pool_head(const PoolHeadArgs &p, int64_t B, hipStream_t st)
+{
+    CF_REQUIRE(B >= 1 && B < (1ll << 31), CF_ERR_UNSUPPORTED, "pooling and head: bad crystal count");
+    pool_head_kernel<<<(unsigned)B, PH_T, 0, st>>>(p);
+    CF_CHECK_LAUNCH("pooling and head");
+    return CF_OK;
+}
+
+}  // namespace cf

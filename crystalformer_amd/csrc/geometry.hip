@@ -5,6 +5,8 @@
 //     normalisation over the batch, the positive map and the final
 //     a = -rho / (2 r0^2), plus the scaled query for the attention.
 #include "cf_common.h"
+#include "block_rows.h"
+#include "gauss_maps.h"
 
 namespace {
 
@@ -14,9 +16,11 @@ using namespace cf;
 // term order of models/indexed_latticeformer_encoder.py:34-44 so the volume is
 // the one the stock elementwise expression gives.
 __global__ void lattice_geometry_kernel(const float *trans, int64_t B, float *vcell, float *recip,
-                                        float *rvlen)
+                                        float *rvlen, unsigned *zero, int words)
 {
 #pragma clang fp contract(off)
+    if (blockIdx.x == 0)
+        for (int w = threadIdx.x; w < words; w += blockDim.x) zero[w] = 0u;
     const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (b >= B) return;
     const float *m = trans + b * 9;
@@ -80,28 +84,6 @@ __device__ __forceinline__ int64_t live_total(const GaussArgs &p, int &blocks)
     const int64_t total = live_count(p.live_N, p.N) * p.H;
     blocks = (int)((total + GE_THREADS - 1) / GE_THREADS);
     return total;
-}
-
-__device__ __forceinline__ float positive_map(float x, int func, float beta, float lb)
-{
-    // models/indexed_lattice_multi_head_attention_cuda.py:675-692
-    if (func == 0) {            // elu
-        const float t = x * (beta / (1.0f - lb));
-        return (1.0f - lb) * (t > 0.f ? t : expf(t) - 1.0f) + 1.0f;
-    }
-    if (func == 1) return (1.0f - lb) * fabsf(x) + lb;           // abs
-    return (1.0f - lb) * expf(x * (beta / (1.0f - lb))) + lb;   // exp
-}
-
-// Chan's pairwise update of (count, mean, M2).
-__device__ __forceinline__ void stat_merge(float &n, float &mean, float &m2, float nb, float meanb, float m2b)
-{
-    const float nt = n + nb;
-    if (nt == 0.f) return;
-    const float delta = meanb - mean;
-    mean += delta * (nb / nt);
-    m2 += m2b + delta * delta * (n * nb / nt);
-    n = nt;
 }
 
 // One thread per (atom, head): alpha = <q, w_head>; the block leaves its
@@ -182,19 +164,8 @@ __global__ __launch_bounds__(GE_THREADS) void gauss_exponents_final_kernel(Gauss
     if ((int)blockIdx.x >= live_blocks) return;
     if (threadIdx.x < WAVE) {
         const int lane = threadIdx.x;
-        float n = 0.f, mean = 0.f, m2 = 0.f;
-        for (int b = lane; b < live_blocks; b += WAVE)
-            stat_merge(n, mean, m2, p.part[3 * b], p.part[3 * b + 1], p.part[3 * b + 2]);
-#pragma unroll
-        for (int off = 1; off < WAVE; off <<= 1) {
-            const float nb = __shfl_xor(n, off, WAVE), mb = __shfl_xor(mean, off, WAVE),
-                        qb = __shfl_xor(m2, off, WAVE);
-            // lower lane first on both sides so partners agree bit for bit
-            float n0 = (lane & off) ? nb : n, m0 = (lane & off) ? mb : mean, q0 = (lane & off) ? qb : m2;
-            const float n1 = (lane & off) ? n : nb, m1 = (lane & off) ? mean : mb, q1 = (lane & off) ? m2 : qb;
-            stat_merge(n0, m0, q0, n1, m1, q1);
-            n = n0; mean = m0; m2 = q0;
-        }
+        float n, mean, m2;
+        merge_statistics(p.part, live_blocks, lane, n, mean, m2);
         if (lane == 0) {
             const float stored_scale = p.part[3 * p.blocks + 2], stored_shift = p.part[3 * p.blocks + 3];
             const bool stored = stored_scale > 0.f;
@@ -388,19 +359,24 @@ extern "C" int cf_gauss_exponents_bwd(const float *ga, const float *gqs, const f
     return CF_OK;
 }
 
-extern "C" int cf_lattice_geometry(const float *trans, int64_t B, float *vcell, float *recip, float *rvlen,
-                                   void *stream_)
+int cf::launch_lattice_geometry(const float *trans, int64_t B, float *vcell, float *recip, float *rvlen, unsigned *zero,
+                                int words, hipStream_t st)
 {
-    hipStream_t stream = (hipStream_t)stream_;
+    const int threads = 128;
+    lattice_geometry_kernel<<<(int)((B + threads - 1) / threads), threads, 0, st>>>(trans, B, vcell, recip, rvlen, zero,
+                                                                                    words);
+    CF_CHECK_LAUNCH("cf_lattice_geometry");
+    return CF_OK;
+}
+
+extern "C" int cf_lattice_geometry(const float *trans, int64_t B, float *vcell, float *recip, float *rvlen,
+                                   void *stream)
+{
     CF_REQUIRE(B >= 0, CF_ERR_INVALID_ARGUMENT, "cf_lattice_geometry: negative crystal count");
     if (B == 0) return CF_OK;
     CF_REQUIRE(trans, CF_ERR_INVALID_ARGUMENT, "cf_lattice_geometry: trans is NULL");
     CF_REQUIRE(vcell || recip || rvlen, CF_ERR_INVALID_ARGUMENT, "cf_lattice_geometry: no output requested");
-    const int threads = 128;
-    lattice_geometry_kernel<<<(int)((B + threads - 1) / threads), threads, 0, stream>>>(trans, B, vcell, recip,
-                                                                                         rvlen);
-    CF_CHECK_LAUNCH("cf_lattice_geometry");
-    return CF_OK;
+    return cf::launch_lattice_geometry(trans, B, vcell, recip, rvlen, nullptr, 0, (hipStream_t)stream);
 }
 
 extern "C" int64_t cf_gauss_exponents_workspace(int64_t N, int64_t H)

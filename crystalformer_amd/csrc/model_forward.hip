@@ -5,6 +5,7 @@
 // some 14 us of host time each, which is what a small batch costs whatever the GPU does (0.65 ms for
 // one crystal of 12 atoms whose kernels take 0.20 ms); from here a launch costs 2-3 us.
 #include "cf_common.h"
+#include "block_rows.h"
 
 namespace {
 
@@ -26,6 +27,8 @@ struct Carver {
 struct Buffers {
     float *rvlen, *rpos, *x[2], *h, *q, *k, *v, *qs, *a, *att, *z, *val, *prob, *rings, *pooled, *hidden;
     void *stats, *flags;
+    unsigned *counters;
+    float *packed;
     int64_t stats_bytes, flag_bytes;
 };
 
@@ -37,6 +40,21 @@ bool use_rings(const cf_forward_args &f, int64_t U)
     return edge * edge * edge <= 128 && cf_real_enc_ring_bytes(U) <= f.ring_limit_bytes;
 }
 
+// Whether everything between two attentions runs as one launch.
+bool use_rows(const cf_forward_args &f) { return block_rows_served(f.width, f.ff, f.H); }
+
+// The head of block l: projections and exponents.
+void head_of(RowsArgs &r, const cf_forward_args &f, const cf_forward_block &p, const Buffers &b, int64_t l)
+{
+    r.packed_head = b.packed + l * PACKED_BLOCK; r.b_in = p.b_in; r.w_pos = p.w_pos;
+    r.gauss_scale = p.gauss_scale;
+    r.normalize = (int)p.normalize; r.update_stats = (int)f.update_stats; r.func = (int)p.positive_func;
+    r.beta = (float)p.beta; r.lb = (float)p.lower_bound; r.coef = (float)p.coef; r.q_scale = (float)p.q_scale;
+    r.qs = b.qs; r.k = b.k; r.v = b.v; r.a = b.a;
+    r.part = (float *)b.stats;
+    r.counter = b.counters + l;
+}
+
 int64_t carve(const cf_forward_args &f, const cf_forward_block *blocks, char *base, Buffers &b)
 {
     Carver c{base, 0};
@@ -44,11 +62,12 @@ int64_t carve(const cf_forward_args &f, const cf_forward_block *blocks, char *ba
     bool rings = false, bins = false;
     for (int64_t l = 0; l < f.layers; l++) bins = bins || blocks[l].bins > 0;
     rings = bins && use_rings(f, U);
+    const bool rows = use_rows(f);
     b.rvlen = c.take<float>(3 * f.B);
     b.rpos = c.take<float>(3 * E);
     for (int i = 0; i < 2; i++) b.x[i] = c.take<float>(N * W);
-    b.h = c.take<float>(N * f.ff);
-    b.q = c.take<float>(N * W);
+    b.h = rows ? nullptr : c.take<float>(N * f.ff);
+    b.q = rows ? nullptr : c.take<float>(N * W);
     b.k = c.take<float>(N * W);
     b.v = c.take<float>(N * W);
     b.qs = c.take<float>(N * W);
@@ -59,6 +78,8 @@ int64_t carve(const cf_forward_args &f, const cf_forward_block *blocks, char *ba
     b.val = bins ? c.take<float>(E * W) : nullptr;
     b.stats_bytes = cf_gauss_exponents_workspace(N, f.H);
     b.stats = c.take<char>(b.stats_bytes);
+    b.packed = rows ? c.take<float>(f.layers * PACKED_BLOCK + W * W) : nullptr;
+    b.counters = c.take<unsigned>(f.layers);
     b.flag_bytes = rings ? cf_real_enc_flag_bytes(U, f.H) : 0;
     b.flags = rings ? c.take<char>(b.flag_bytes) : nullptr;
     b.rings = rings ? c.take<float>(cf_real_enc_ring_bytes(U) / 4) : nullptr;
@@ -77,6 +98,11 @@ int check_args(const cf_forward_args *f, const cf_forward_block *blocks)
                    f->ff % 16 == 0 && f->ff >= 16 && f->width >= 16 && f->width % f->H == 0 && f->width / f->H <= 32,
                CF_ERR_UNSUPPORTED, "cf_forward: width %lld, heads %lld, feed-forward %lld not served",
                (long long)f->width, (long long)f->H, (long long)f->ff);
+    CF_REQUIRE(!f->w_embed || (use_rows(*f) && f->embed_width >= 1 && f->embed_width <= f->width), CF_ERR_UNSUPPORTED,
+               "cf_forward: an embedding of %lld features is not served", (long long)f->embed_width);
+    for (int64_t l = 0; l < f->layers; l++)
+        CF_REQUIRE(blocks[l].positive_func >= 0 && blocks[l].positive_func <= 2 && blocks[l].lower_bound < 1.0,
+                   CF_ERR_UNSUPPORTED, "cf_forward: block %lld: positive map not served", (long long)l);
     for (int64_t l = 0; l < f->layers; l++)
         CF_REQUIRE(blocks[l].bins >= 0 && blocks[l].bins <= 128 && (blocks[l].bins == 0 || blocks[l].w_pe),
                    CF_ERR_UNSUPPORTED, "cf_forward: block %lld: value bins outside 0..128 or without a projection",
@@ -108,15 +134,45 @@ extern "C" int cf_forward(const cf_forward_args *f_, const cf_forward_block *blo
                CF_ERR_INVALID_ARGUMENT, "cf_forward: null pointer");
     const int64_t N = f.N, E = f.E, U = (N + E) / 2, W = f.width, H = f.H, D = W / H;
     const bool adaptive_any = f.adaptive != 0;
-    if ((rc = cf_lattice_geometry(f.tvecs, f.B, nullptr, nullptr, b.rvlen, stream))) return rc;
+    const bool rows = use_rows(f);
+    if ((rc = launch_lattice_geometry(f.tvecs, f.B, nullptr, nullptr, b.rvlen, b.counters, (int)f.layers,
+                                      (hipStream_t)stream)))
+        return rc;
     if ((rc = cf_edge_index(f.atom_start, f.edge_start, f.B, E, f.pos, nullptr, b.rpos, stream))) return rc;
     const cf_forward_block *staged = nullptr;      // the block whose grid the rings in b.rings hold
     const float *x = f.x;
     int side = 0;
+    if (rows) {
+        for (int64_t first = 0; first < f.layers; first += PACK_BLOCKS) {
+            PackArgs a{};
+            a.blocks = (int)(f.layers - first < PACK_BLOCKS ? f.layers - first : PACK_BLOCKS);
+            for (int i = 0; i < a.blocks; i++) {
+                const cf_forward_block &p = blocks[first + i];
+                a.block[i] = PackSource{p.wo, p.w1, p.w2, p.wq, p.wk, p.wv};
+            }
+            a.packed = b.packed + first * PACKED_BLOCK;
+            if (first == 0 && f.w_embed) {
+                a.w_embed = f.w_embed;
+                a.embed_width = (int)f.embed_width;
+                a.packed_embed = b.packed + f.layers * PACKED_BLOCK;
+            }
+            if ((rc = launch_pack_weights(a, (hipStream_t)stream))) return rc;
+        }
+        RowsArgs r{};
+        r.N = N; r.H = (int)H; r.x = f.x;
+        head_of(r, f, blocks[0], b, 0);
+        if (f.w_embed) {
+            r.packed_embed = b.packed + f.layers * PACKED_BLOCK; r.b_embed = f.b_embed; r.embed_width = (int)f.embed_width;
+            r.y = b.x[1];
+            x = b.x[1];
+        }
+        if ((rc = launch_block_rows(r, (hipStream_t)stream))) return rc;
+    }
     for (int64_t l = 0; l < f.layers; l++) {
         const cf_forward_block &p = blocks[l];
-        if ((rc = cf_linear_rows(x, N, W, p.wq, p.wk, p.wv, 3, W, p.b_in, nullptr, 0, b.q, b.k, b.v, stream))) return rc;
-        if ((rc = cf_gauss_exponents(b.q, p.w_pos, p.gauss_scale, N, H, D, p.normalize, f.update_stats, p.positive_func,
+        if (!rows && (rc = cf_linear_rows(x, N, W, p.wq, p.wk, p.wv, 3, W, p.b_in, nullptr, 0, b.q, b.k, b.v, stream)))
+            return rc;
+        if (!rows && (rc = cf_gauss_exponents(b.q, p.w_pos, p.gauss_scale, N, H, D, p.normalize, f.update_stats, p.positive_func,
                                      (float)p.beta, (float)p.lower_bound, (float)p.coef, (float)p.q_scale, b.stats,
                                      b.stats_bytes, nullptr, b.a, b.qs, stream)))
             return rc;
@@ -145,6 +201,16 @@ extern "C" int cf_forward(const cf_forward_args *f_, const cf_forward_block *blo
                                    b.prob, b.att, stream)))
             return rc;
         float *y = f.targets == 0 && l + 1 == f.layers ? f.out : b.x[side];
+        if (rows) {
+            RowsArgs r{};
+            r.N = N; r.H = (int)H; r.att = b.att; r.x = x; r.y = y;
+            r.packed_tail = b.packed + l * PACKED_BLOCK; r.bo = p.bo; r.b1 = p.b1; r.b2 = p.b2;
+            if (l + 1 < f.layers) head_of(r, f, blocks[l + 1], b, l + 1);
+            if ((rc = launch_block_rows(r, (hipStream_t)stream))) return rc;
+            x = y;
+            side ^= 1;
+            continue;
+        }
         if ((rc = cf_linear_rows(b.att, N, W, p.wo, nullptr, nullptr, 1, W, p.bo, x, 0, b.qs, nullptr, nullptr, stream)))
             return rc;                              // (the scaled query is spent: its buffer takes the sum)
         if ((rc = cf_linear_rows(b.qs, N, W, p.w1, nullptr, nullptr, 1, f.ff, p.b1, nullptr, 1, b.h, nullptr, nullptr,
@@ -156,6 +222,10 @@ extern "C" int cf_forward(const cf_forward_args *f_, const cf_forward_block *blo
         side ^= 1;
     }
     if (f.targets == 0) return CF_OK;
+    if (pool_head_served(W, f.hidden)) {
+        const PoolHeadArgs h{x, f.atom_start, f.w_head, f.b_head, f.w_last, f.b_last, f.hidden, f.targets, f.out};
+        return launch_pool_head(h, f.B, (hipStream_t)stream);
+    }
     if ((rc = cf_irregular_mean_fwd(x, f.atom_start, f.B, W, b.pooled, stream))) return rc;
     const float *top = b.pooled;
     int64_t top_width = W;

@@ -125,8 +125,22 @@ def _head(mlp: nn.Module, width: int, device_index: int) -> Optional[Tuple[tuple
     return head + (last["weight"], last["bias"]), hidden, targets
 
 
+def _embeds(model: nn.Module, x: Tensor):
+    """Whether the native call can embed the atoms itself: a plain, unhooked projection of contiguous rows into
+    the one block width that has the kernel, without autocast (which would run it in another type)."""
+    embed = model._modules["input_embeddings"]
+    layers = model._modules["encoder"]._modules["layers"]
+    return (type(embed) is nn.Linear and not _hooked(embed) and embed.out_features == 128 and len(layers) > 0
+            and getattr(layers[0], "linear1", None) is not None and layers[0].linear1.out_features == 512
+            and type(x) is Tensor and x.dim() == 2 and x.shape[1] == embed.in_features <= 128
+            and not torch.is_autocast_enabled("cuda") and x.get_device() >= 0
+            and _ready(x, x.numel(), x.get_device())
+            and _ready(embed.weight, embed.in_features * 128, x.get_device())
+            and _ready(embed.bias, 128, x.get_device()))
+
+
 def _run(encoder: nn.Module, src: Tensor, pos: Tensor, batch: Tensor, trans: Tensor, sizes: Tensor,
-         head=None) -> Optional[Tensor]:
+         head=None, embed: Optional[nn.Module] = None) -> Optional[Tensor]:
     KM = hip_funcs.KernelManager
     if torch.is_grad_enabled() or config.REPRODUCIBLITY_STATE < 2 or not KM.DENSE_EDGE_BLOCKS \
             or ops.instrumented() or encoder._modules.get("norm") is not None \
@@ -136,7 +150,7 @@ def _run(encoder: nn.Module, src: Tensor, pos: Tensor, batch: Tensor, trans: Ten
     index = src.get_device()
     N = src.shape[0]
     B = trans.shape[0]
-    if index < 0 or src.dim() != 2 or N == 0 or not _ready(src, N * width, index) or not _ready(pos, 3 * N, index) \
+    if index < 0 or src.dim() != 2 or N == 0 or not _ready(src, N * (embed.in_features if embed else width), index) or not _ready(pos, 3 * N, index) \
             or not _ready(trans, 9 * B, index) or batch.get_device() != index or batch.dtype is not torch.int64:
         return None
     blocks = []
@@ -163,9 +177,10 @@ def _run(encoder: nn.Module, src: Tensor, pos: Tensor, batch: Tensor, trans: Ten
     args = _lib.ForwardArgs(
         N, layout.num_edges, sizes.numel(), len(blocks), H, width, ff, KM.LATTICE_RANGE, KM.MINIMUM_RANGE, 1,
         int(encoder.training), int(KM.STAGED_RINGS), int(KM.ADAPTIVE_RINGS), ops.STAGED_RINGS_MAX_BYTES, hidden,
-        targets, src.data_ptr(), pos.data_ptr(), trans.data_ptr(), layout.batch.data_ptr(), layout.atom_start.data_ptr(),
+        targets, embed.in_features if embed else 0, src.data_ptr(), pos.data_ptr(), trans.data_ptr(), layout.batch.data_ptr(), layout.atom_start.data_ptr(),
         layout.edge_start.data_ptr(), layout.edges.data_ptr(), layout.e_start.data_ptr(), layout.pairs.data_ptr(),
-        _address(sched), *(_address(t) for t in tensors), out.data_ptr())
+        _address(sched), *(_address(t) for t in tensors),
+        *((_address(embed.weight), _address(embed.bias)) if embed else (None, None)), out.data_ptr())
     table = (_lib.ForwardBlock * len(blocks))(*(tuple(f) for f in blocks))
     need = L.cf_forward_workspace(_lib.ctypes.byref(args), table)
     if need < 0:
@@ -184,15 +199,20 @@ def encode(encoder: nn.Module, src: Tensor, pos: Tensor, batch: Tensor, trans: T
     return _run(encoder, src, pos, batch, trans, sizes)
 
 
-def forward(model: nn.Module, src: Tensor, data) -> Optional[Tensor]:
-    """The output of ``Latticeformer.forward`` behind the embedding, or None."""
+def forward(model: nn.Module, data) -> Tuple[Optional[Tensor], Optional[Tensor]]:
+    """The output of ``Latticeformer.forward``, or None and the embedded atoms if they are there already."""
     if torch.is_grad_enabled():
-        return None
+        return None, None
     mods = model._modules
     if type(mods["proj_before_pooling"]) is not nn.Identity or model.pooling_layer is not pooling.avr_pool \
             or _hooked(mods["proj_before_pooling"]) or _any_hooked(mods["mlp"]):
-        return None
-    head = _head(mods["mlp"], mods["encoder"].d_model, src.get_device())
+        return None, None
+    x = data.x
+    head = _head(mods["mlp"], mods["encoder"].d_model, x.get_device())
     if head is None:
-        return None
-    return _run(mods["encoder"], src, data.pos, data.batch, data.trans_vec, data.sizes, head)
+        return None, None
+    where = data.pos, data.batch, data.trans_vec, data.sizes, head
+    if _embeds(model, x):
+        return _run(mods["encoder"], x, *where, mods["input_embeddings"]), None
+    x = hip_funcs.linear(x, model.input_embeddings.weight, model.input_embeddings.bias)
+    return _run(mods["encoder"], x, *where), x

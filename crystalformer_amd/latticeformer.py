@@ -115,10 +115,11 @@ class Latticeformer(nn.Module):
         # (inside a fused training step the embedding's and the head's weight gradients join the
         # grouped weight-gradient launch; otherwise these are the stock linear ops)
         from . import executor, hip_funcs
-        x = hip_funcs.linear(data.x, self.input_embeddings.weight, self.input_embeddings.bias)
-        out = executor.forward(self, x, data)          # inference: one native call where it serves the model
+        out, x = executor.forward(self, data)          # inference: one native call where it serves the model
         if out is not None:
             return out
+        if x is None:
+            x = hip_funcs.linear(data.x, self.input_embeddings.weight, self.input_embeddings.bias)
         x = self.encoder(x, data.pos, data.batch, data.trans_vec, data.sizes, data.x)
         x = self.proj_before_pooling(x)
         x = self.pooling_layer(x, data.batch, data.sizes)

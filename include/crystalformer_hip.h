@@ -510,10 +510,13 @@ typedef struct {
     int64_t staged_rings, adaptive_rings, ring_limit_bytes;   /* whether and up to what size blocks share staged rings */
     int64_t hidden, targets;          /* head: width -> hidden (ReLU) -> targets; hidden 0: width -> targets;
                                          targets 0: out takes the encoder's output (N, width) */
-    const float *x, *pos, *tvecs;     /* (N, width) embedded atoms, (N, 3), (B, 3, 3) */
+    int64_t embed_width;
+    const float *x, *pos, *tvecs;     /* (N, width) embedded atoms, (N, 3), (B, 3, 3); with w_embed (width,
+                                         embed_width) x is (N, embed_width) and x w_embed^T + b_embed is embedded */
     const int64_t *batch, *atom_start, *edge_start, *edges, *e_start, *pairs;
     int32_t *sched;                   /* two zeroed words (as sched_2 of cf_real_enc_fwd), nullable */
     const float *w_head, *b_head, *w_last, *b_last;
+    const float *w_embed, *b_embed;   /* nullable; width 128 with ff 512 only (CF_ERR_UNSUPPORTED otherwise) */
     float *out;                       /* (B, targets) or (N, width) */
 } cf_forward_args;
 

@@ -86,6 +86,34 @@ def test_native_forward_with_its_head(dev, options):
     assert_close(got, want, "model", rtol=RTOL)
 
 
+# rows: one work-group's tile of 4, 8 and 16 rows less one, exactly, plus one; either side of the row counts at
+# which the tile grows (four and eight rows per CU, one full round of sixteen)
+@pytest.mark.parametrize("atoms", [1, 3, 4, 5, 1023, 1025, 2047, 2049, 3480, 3490, 4097])
+def test_row_kernel_tiles_against_float64(dev, atoms):
+    """Embedding, tail and head of the 128-wide blocks on crystals of up to 16 atoms, encoder against the module
+    path and the last block's row-wise half against float64."""
+    torch.manual_seed(atoms)
+    sizes = [16] * (atoms // 16) + ([atoms % 16] if atoms % 16 else [])
+    model = scaled(default_params(num_layers=2, value_pe_dist_real=0)).to(dev).eval()
+    b = batch_of(sizes).to(dev)
+    native, modules = both_ways(model, b)
+    assert_close(native, modules, "encoder", rtol=RTOL, atol=atol_rows(modules))
+    with torch.no_grad():
+        y = model(b)
+        last = {}
+        hooks = [m.register_forward_hook(lambda m, i, o, k=k: last.__setitem__(k, o)) for k, m in
+                 (("encoder", model.encoder), ("pool", model.mlp))]
+        want = model(b)
+        for h in hooks:
+            h.remove()
+        pooled = torch.stack([e.double().mean(0) for e in last["encoder"].split(sizes)])
+        ref = pooled
+        for m in model.mlp:
+            ref = torch.nn.functional.linear(ref, m.weight.double(), m.bias.double()) if hasattr(m, "weight") else m(ref)
+    assert_close(y, want, "model", rtol=RTOL)
+    assert_close(y, ref.float(), "head", rtol=RTOL)
+
+
 def test_training_mode_without_gradients_stores_the_statistics(dev):
     cfg = default_params(num_layers=2)
     one, two = scaled(cfg).to(dev).train(), scaled(cfg).to(dev).train()

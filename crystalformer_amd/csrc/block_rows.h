@@ -16,6 +16,8 @@ struct RowsArgs {
     float *gauss_scale;
     int normalize, update_stats, func;
     float beta, lb, coef, q_scale;
+    int split;                                // heads from H/2 on: factor coef_second, their exponents behind all
+    float coef_second;                        //   of the first half's, (N, H/2) each
     float *qs, *k, *v, *a;
     float *part;                              // statistics without stored ones: 3 floats per 256 values of a
     unsigned *counter;                        // zeroed word

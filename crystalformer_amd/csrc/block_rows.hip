@@ -164,7 +164,8 @@ __device__ void finish_exponents(const RowsArgs &p, int64_t total, float *red)
     __syncthreads();
     const float scale = red[0], shift = red[1];
     for (int64_t t = threadIdx.x; t < total; t += RT)
-        p.a[t] = positive_map((p.a[t] + shift) * scale, p.func, p.beta, p.lb) * p.coef;
+        p.a[t] = positive_map((p.a[t] + shift) * scale, p.func, p.beta, p.lb) *
+                 (p.split && 2 * t >= total ? p.coef_second : p.coef);
 }
 
 // The matrices as a sequence of units, 16 columns a wavefront x 128 reduction steps each:
@@ -350,8 +351,13 @@ __global__ __launch_bounds__(RT) void block_rows_kernel(RowsArgs p)
                 for (int d = 0; d < D; d += 4)                  // (the order of the exponent kernel)
                     alpha += (q[d] * w[d] + q[d + 1] * w[d + 1]) + (q[d + 2] * w[d + 2] + q[d + 3] * w[d + 3]);
                 if (p.normalize && stored) alpha = (alpha + shift) * scale;
-                if (!p.normalize || stored) alpha = positive_map(alpha, p.func, p.beta, p.lb) * p.coef;
-                if (row0 + r < N) p.a[(row0 + r) * p.H + h] = alpha;
+                const int half = p.H >> 1;
+                const bool second = p.split && h >= half;
+                if (!p.normalize || stored)
+                    alpha = positive_map(alpha, p.func, p.beta, p.lb) * (second ? p.coef_second : p.coef);
+                if (row0 + r < N)
+                    p.a[p.split ? (second ? N : 0) * half + (row0 + r) * half + h - (second ? half : 0)
+                                : (row0 + r) * p.H + h] = alpha;
             }
         }
         __syncthreads();                                        // the next tile overwrites the rows

@@ -25,6 +25,7 @@ struct DpaArgs {
     float *gque, *gkey, *gval, *gaij, *gbij;
     int64_t N, E;
     int H, Dk, Dv;
+    uint32_t aij_second;     // two halves of heads: floats from aij to the second half's bias, 0: one array
     const int64_t *live_N;   // forward only, nullable: live atom count on the device (N is then the capacity)
 };
 
@@ -173,7 +174,10 @@ __device__ __forceinline__ void st1(void *base, uint32_t byte_off, float v)
 // register budget is that of 8 resident wavefronts per SIMD, which the compiler meets by
 // fetching the value rows after the key rows have been used: one more round trip, and all
 // rows of a small batch resident at once.
-template <int DV4, bool HAS_A, bool HAS_B, bool PREFETCH>
+// SPLIT: the heads come in two halves with a bias of their own each, (E, H/2) at aij and at aij + aij_second, and
+// only the first half has a b_ij, (E, H/2, Dv): a block half of whose heads are in reciprocal space.
+// Without prob (inference) the weights are not kept: no parked logits, no closing sweep.
+template <int DV4, bool HAS_A, bool HAS_B, bool PREFETCH, bool SPLIT = false>
 __global__ __launch_bounds__(256, (PREFETCH ? 6 : 7)) void fused_dpa_fwd_stream_kernel(DpaArgs p, int LPE)
 {
     __shared__ float part[DPA_WPQ][WAVE][6];
@@ -203,10 +207,16 @@ __global__ __launch_bounds__(256, (PREFETCH ? 6 : 7)) void fused_dpa_fwd_stream_
     float4_v acc = {0.f, 0.f, 0.f, 0.f};
     float4_v k4[4], v4[4], b4[4];
     float av[4];
+    const uint32_t a_lane = SPLIT && h >= H / 2 ? p.aij_second + h - H / 2 : h, a_edge = SPLIT ? H / 2 : H;
+    const uint32_t b_edge = SPLIT ? HD4 / 2 : HD4;
+    const bool has_b = HAS_B && (!SPLIT || piece < b_edge);
     auto fetch = [&](int u, uint32_t e, uint32_t j) {
         // (independent of the key index: first; long rows: a stream that is read once)
-        if (HAS_B) b4[u] = PREFETCH ? ld4_stream(p.bij, (e * HD4 + piece) * 16u) : ld4(p.bij, (e * HD4 + piece) * 16u);
-        if (HAS_A) av[u] = ld1(p.aij, (e * H + h) * 4u);
+        if (SPLIT && HAS_B) {
+            b4[u] = float4_v{0.f, 0.f, 0.f, 0.f};
+            if (has_b) b4[u] = PREFETCH ? ld4_stream(p.bij, (e * b_edge + piece) * 16u) : ld4(p.bij, (e * b_edge + piece) * 16u);
+        } else if (HAS_B) b4[u] = PREFETCH ? ld4_stream(p.bij, (e * HD4 + piece) * 16u) : ld4(p.bij, (e * HD4 + piece) * 16u);
+        if (HAS_A) av[u] = ld1(p.aij, (e * a_edge + a_lane) * 4u);
         k4[u] = ld4(p.key, (j * HD4 + piece) * 16u);
         v4[u] = ld4(p.val, (j * HD4 + piece) * 16u);
     };
@@ -250,7 +260,7 @@ __global__ __launch_bounds__(256, (PREFETCH ? 6 : 7)) void fused_dpa_fwd_stream_
 #pragma unroll
         for (int u = 0; u < 4; u++) s_tail[u] = fold(u, e + u * stride < e1);
         if (last) break;
-        if (lead) {
+        if (lead && p.prob) {
 #pragma unroll
             for (int u = 0; u < 4; u++) st1(p.prob, ((e + u * stride) * H + h) * 4u, s_tail[u]);
         }
@@ -298,6 +308,7 @@ __global__ __launch_bounds__(256, (PREFETCH ? 6 : 7)) void fused_dpa_fwd_stream_
     }
     __syncthreads();
     if (closer) reinterpret_cast<float4_v *>(p.out)[i * HD4 + piece] = acc;   // after the barrier: nothing waits for it
+    if (!p.prob) return;
     // normalise: the partial step from registers, the parked logits in place (element x of the
     // row's (n,H) block belongs to head x % H)
     if (lead) {
@@ -598,7 +609,9 @@ template <int DV4, bool PREFETCH>
 void launch_fwd_stream_dv(const DpaArgs &p, int lpe, hipStream_t st)
 {
     const dim3 grid((unsigned)p.N), block(DPA_WPQ * WAVE);
-    if (p.aij && p.bij) fused_dpa_fwd_stream_kernel<DV4, true, true, PREFETCH><<<grid, block, 0, st>>>(p, lpe);
+    if (p.aij_second && p.bij) fused_dpa_fwd_stream_kernel<DV4, true, true, PREFETCH, true><<<grid, block, 0, st>>>(p, lpe);
+    else if (p.aij_second) fused_dpa_fwd_stream_kernel<DV4, true, false, PREFETCH, true><<<grid, block, 0, st>>>(p, lpe);
+    else if (p.aij && p.bij) fused_dpa_fwd_stream_kernel<DV4, true, true, PREFETCH><<<grid, block, 0, st>>>(p, lpe);
     else if (p.aij) fused_dpa_fwd_stream_kernel<DV4, true, false, PREFETCH><<<grid, block, 0, st>>>(p, lpe);
     else if (p.bij) fused_dpa_fwd_stream_kernel<DV4, false, true, PREFETCH><<<grid, block, 0, st>>>(p, lpe);
     else fused_dpa_fwd_stream_kernel<DV4, false, false, PREFETCH><<<grid, block, 0, st>>>(p, lpe);
@@ -653,7 +666,38 @@ void launch_bwd_stream(const DpaArgs &p, int dv4, int lpe, hipStream_t st)
     }
 }
 
+// streaming kernels where a head's components split into 16-byte pieces that tile a wavefront
+bool streams(int64_t N, int64_t H, int64_t E, int64_t Dk, int64_t Dv)
+{
+    const int64_t dv4 = Dv / 4, lpe = H * dv4;
+    const bool pow2 = (dv4 & (dv4 - 1)) == 0 && (H & (H - 1)) == 0;
+    const bool fits32 = (E + 1) * H * Dv * 4 < (1ll << 32) && (N + 1) * H * Dv * 4 < (1ll << 32);
+    return Dk == Dv && Dv % 4 == 0 && pow2 && lpe >= 1 && lpe <= 64 && dv4 <= 16 && fits32;
+}
+
 }  // namespace
+
+namespace cf {
+
+bool dpa_streams(int64_t N, int64_t H, int64_t E, int64_t D) { return H <= MAXH && streams(N, H, E, D, D); }
+
+int launch_dpa_inference(const float *que, const float *key, const float *val, const float *aij, int64_t aij_second,
+                         const float *bij, const int64_t *edges, const int64_t *e_start, int64_t N, int64_t H, int64_t E,
+                         int64_t D, float *out, hipStream_t st)
+{
+    CF_REQUIRE(dpa_streams(N, H, E, D) && (aij_second == 0 || H % 2 == 0), CF_ERR_UNSUPPORTED,
+               "attention: shape not served");
+    DpaArgs p{};
+    p.que = que; p.key = key; p.val = val; p.aij = aij; p.bij = bij; p.aij_second = (uint32_t)aij_second;
+    p.edges = edges; p.e_start = e_start; p.out = out;
+    p.N = N; p.E = E; p.H = (int)H; p.Dk = (int)D; p.Dv = (int)D;
+    p.live_N = live_atoms(N);
+    launch_fwd_stream(p, (int)(D / 4), (int)(H * (D / 4)), st);
+    CF_CHECK_LAUNCH("attention");
+    return CF_OK;
+}
+
+}  // namespace cf
 
 extern "C" int cf_fused_dpa_fwd(const float *que, const float *key, const float *val,
                                 const float *aij_eh, const float *bij_ehd, const int64_t *edge_ij_e,
@@ -672,11 +716,8 @@ extern "C" int cf_fused_dpa_fwd(const float *que, const float *key, const float 
     p.N = N; p.E = E; p.H = (int)H; p.Dk = (int)Dk; p.Dv = (int)Dv;
     p.live_N = cf::live_atoms(N);
     hipStream_t st = (hipStream_t)stream;
-    // streaming kernel when a head's components split into 16-byte pieces that tile a wavefront
-    const int64_t dv4 = Dv / 4, lpe = H * dv4;
-    const bool pow2 = (dv4 & (dv4 - 1)) == 0 && (H & (H - 1)) == 0;
-    const bool fits32 = (E + 1) * H * Dv * 4 < (1ll << 32) && (N + 1) * H * Dv * 4 < (1ll << 32);
-    if (Dk == Dv && Dv % 4 == 0 && pow2 && lpe >= 1 && lpe <= 64 && dv4 <= 16 && fits32) {
+    if (streams(N, H, E, Dk, Dv)) {
+        const int64_t dv4 = Dv / 4, lpe = H * dv4;
         launch_fwd_stream(p, (int)dv4, (int)lpe, st);
         CF_CHECK_LAUNCH("cf_fused_dpa_fwd");
         return CF_OK;
@@ -720,15 +761,10 @@ extern "C" int cf_fused_dpa_bwd(const float *que, const float *key, const float 
     p.gque = gque; p.gkey = gkey; p.gval = gval; p.gaij = gaij; p.gbij = gbij;
     p.N = N; p.E = E; p.H = (int)H; p.Dk = (int)Dk; p.Dv = (int)Dv;
     hipStream_t st = (hipStream_t)stream;
-    {
-        const int64_t dv4 = Dv / 4, lpe = H * dv4;
-        const bool pow2 = (dv4 & (dv4 - 1)) == 0 && (H & (H - 1)) == 0;
-        const bool fits32 = (E + 1) * H * Dv * 4 < (1ll << 32) && (N + 1) * H * Dv * 4 < (1ll << 32);
-        if (Dk == Dv && Dv % 4 == 0 && pow2 && lpe >= 1 && lpe <= 64 && dv4 <= 16 && fits32) {
-            launch_bwd_stream(p, (int)dv4, (int)lpe, st);
-            CF_CHECK_LAUNCH("cf_fused_dpa_bwd: streaming kernels");
-            return CF_OK;
-        }
+    if (streams(N, H, E, Dk, Dv)) {
+        launch_bwd_stream(p, (int)(Dv / 4), (int)(H * (Dv / 4)), st);
+        CF_CHECK_LAUNCH("cf_fused_dpa_bwd: streaming kernels");
+        return CF_OK;
     }
     const int wpb = 4;
     const int grid = (int)((N + wpb - 1) / wpb);

@@ -29,6 +29,7 @@ struct Buffers {
     void *stats, *flags;
     unsigned *counters;
     float *packed;
+    float *vcell, *recip, *kr, *sumexp;
     int64_t stats_bytes, flag_bytes;
 };
 
@@ -50,6 +51,7 @@ void head_of(RowsArgs &r, const cf_forward_args &f, const cf_forward_block &p, c
     r.gauss_scale = p.gauss_scale;
     r.normalize = (int)p.normalize; r.update_stats = (int)f.update_stats; r.func = (int)p.positive_func;
     r.beta = (float)p.beta; r.lb = (float)p.lower_bound; r.coef = (float)p.coef; r.q_scale = (float)p.q_scale;
+    r.split = p.coef_reci != 0.0; r.coef_second = (float)p.coef_reci;
     r.qs = b.qs; r.k = b.k; r.v = b.v; r.a = b.a;
     r.part = (float *)b.stats;
     r.counter = b.counters + l;
@@ -74,7 +76,13 @@ int64_t carve(const cf_forward_args &f, const cf_forward_block *blocks, char *ba
     b.a = c.take<float>(N * f.H);
     b.att = c.take<float>(N * W);
     b.z = c.take<float>(E * f.H);
-    b.prob = c.take<float>(E * f.H);
+    b.prob = dpa_streams(N, f.H, E, W / f.H) ? nullptr : c.take<float>(E * f.H);
+    bool reci = false;
+    for (int64_t l = 0; l < f.layers; l++) reci = reci || blocks[l].coef_reci != 0.0;
+    b.vcell = reci ? c.take<float>(f.B) : nullptr;
+    b.recip = reci ? c.take<float>(9 * f.B) : nullptr;
+    b.kr = reci ? c.take<float>(3 * E) : nullptr;
+    b.sumexp = reci ? c.take<float>(E * (f.H / 2)) : nullptr;
     b.val = bins ? c.take<float>(E * W) : nullptr;
     b.stats_bytes = cf_gauss_exponents_workspace(N, f.H);
     b.stats = c.take<char>(b.stats_bytes);
@@ -100,6 +108,10 @@ int check_args(const cf_forward_args *f, const cf_forward_block *blocks)
                (long long)f->width, (long long)f->H, (long long)f->ff);
     CF_REQUIRE(!f->w_embed || (use_rows(*f) && f->embed_width >= 1 && f->embed_width <= f->width), CF_ERR_UNSUPPORTED,
                "cf_forward: an embedding of %lld features is not served", (long long)f->embed_width);
+    for (int64_t l = 0; l < f->layers; l++)
+        CF_REQUIRE(blocks[l].coef_reci == 0.0 ||
+                       (use_rows(*f) && f->H % 2 == 0 && dpa_streams(f->N, f->H, f->E, f->width / f->H) && !live_atoms(f->N)),
+                   CF_ERR_UNSUPPORTED, "cf_forward: block %lld: two domains not served", (long long)l);
     for (int64_t l = 0; l < f->layers; l++)
         CF_REQUIRE(blocks[l].positive_func >= 0 && blocks[l].positive_func <= 2 && blocks[l].lower_bound < 1.0,
                    CF_ERR_UNSUPPORTED, "cf_forward: block %lld: positive map not served", (long long)l);
@@ -135,10 +147,11 @@ extern "C" int cf_forward(const cf_forward_args *f_, const cf_forward_block *blo
     const int64_t N = f.N, E = f.E, U = (N + E) / 2, W = f.width, H = f.H, D = W / H;
     const bool adaptive_any = f.adaptive != 0;
     const bool rows = use_rows(f);
-    if ((rc = launch_lattice_geometry(f.tvecs, f.B, nullptr, nullptr, b.rvlen, b.counters, (int)f.layers,
+    if ((rc = launch_lattice_geometry(f.tvecs, f.B, b.vcell, b.recip, b.rvlen, b.counters, (int)f.layers,
                                       (hipStream_t)stream)))
         return rc;
     if ((rc = cf_edge_index(f.atom_start, f.edge_start, f.B, E, f.pos, nullptr, b.rpos, stream))) return rc;
+    if (b.kr && (rc = cf_kr_base(b.rpos, b.recip, f.batch, f.edges, E, b.kr, stream))) return rc;
     const cf_forward_block *staged = nullptr;      // the block whose grid the rings in b.rings hold
     const float *x = f.x;
     int side = 0;
@@ -178,7 +191,9 @@ extern "C" int cf_forward(const cf_forward_args *f_, const cf_forward_block *blo
             return rc;
         const float *rvlen = adaptive_any && p.cutoff != 0.0 ? b.rvlen : nullptr;
         const bool adaptive = rvlen != nullptr;
-        if (p.bins > 0 && b.rings && (!adaptive || (f.adaptive_rings && H <= 8))) {
+        const bool split = p.coef_reci != 0.0;                  // real space: the first half of the heads
+        const int64_t HR = split ? H / 2 : H;
+        if (p.bins > 0 && b.rings && (!adaptive || (f.adaptive_rings && HR <= 8))) {
             if (!staged || staged->bins != p.bins || staged->dist_max != p.dist_max || staged->wscale != p.wscale ||
                 staged->weakest != p.weakest) {
                 if ((rc = cf_real_enc_ring_stage(b.rpos, f.tvecs, f.pairs, U, p.bins, p.dist_max, p.wscale,
@@ -187,19 +202,24 @@ extern "C" int cf_forward(const cf_forward_args *f_, const cf_forward_block *blo
                 staged = &p;
             }
             rc = cf_real_enc_fwd_rings(b.a, adaptive ? b.rpos : nullptr, adaptive ? f.tvecs : nullptr,
-                                       adaptive ? f.batch : nullptr, f.edges, f.pairs, U, N, H, E, p.bins, D, p.dist_max,
+                                       adaptive ? f.batch : nullptr, f.edges, f.pairs, U, N, HR, E, p.bins, D, p.dist_max,
                                        p.wscale, p.w_pe, rvlen, p.cutoff, f.lattice_range, f.minimum_range, b.rings,
                                        b.flags, b.flag_bytes, b.z, b.val, stream);
         } else {
-            rc = cf_real_enc_fwd(b.a, b.rpos, f.tvecs, f.batch, f.edges, N, H, E, f.B, p.bins, p.bins > 0 ? D : 0,
+            rc = cf_real_enc_fwd(b.a, b.rpos, f.tvecs, f.batch, f.edges, N, HR, E, f.B, p.bins, p.bins > 0 ? D : 0,
                                  p.dist_max, p.wscale, p.bins > 0 ? p.w_pe : nullptr, p.bins > 0 ? 1 : 0, rvlen,
                                  adaptive ? p.cutoff : 0.0, f.lattice_range, f.minimum_range, f.pairs, U, f.sched, b.z,
                                  p.bins > 0 ? b.val : nullptr, stream);
         }
         if (rc) return rc;
-        if ((rc = cf_fused_dpa_fwd(b.qs, b.k, b.v, b.z, p.bins > 0 ? b.val : nullptr, f.edges, f.e_start, N, H, E, D, D,
-                                   b.prob, b.att, stream)))
+        if (split && (rc = cf_reci_enc_fwd(b.a + N * HR, b.kr, b.recip, b.vcell, f.batch, f.e_start, N, HR, E,
+                                           (int)f.lattice_range, b.z + E * HR, b.sumexp, stream)))
             return rc;
+        const float *val = p.bins > 0 ? b.val : nullptr;
+        rc = b.prob ? cf_fused_dpa_fwd(b.qs, b.k, b.v, b.z, val, f.edges, f.e_start, N, H, E, D, D, b.prob, b.att, stream)
+                    : launch_dpa_inference(b.qs, b.k, b.v, b.z, split ? E * HR : 0, val, f.edges, f.e_start, N, H, E, D,
+                                           b.att, (hipStream_t)stream);
+        if (rc) return rc;
         float *y = f.targets == 0 && l + 1 == f.layers ? f.out : b.x[side];
         if (rows) {
             RowsArgs r{};

@@ -65,13 +65,17 @@ def _block(layer: nn.Module, width: int, device_index: int):
                                                    for d in ("dropout", "dropout1", "dropout2"))):
         return None
     spec = fused_exponents_spec(P)
-    if P.domain != "real" or P.norm_func_mode not in (0, "default") or spec is None \
+    halves = P.domain == "multihead"               # half of the heads in reciprocal space
+    if halves and (P.gauss_lb_real != P.gauss_lb_reci or attn.num_heads % 2 or width != 128 or lin1.out_features != 512
+                   or ops.current_live_sizes() is not None):
+        return None
+    if (P.domain != "real" and not halves) or P.norm_func_mode not in (0, "default") or spec is None \
             or attn.kdim != width or attn.vdim != width or attn.embed_dim != width:
         return None
     H = attn.num_heads
     D = width // H
     bins = max(int(P.value_pe_dist_real), 0)
-    if bins == 0 and not hip_funcs.KernelManager.FUSE_ENCODING_ATTENTION:
+    if bins == 0 and not halves and not hip_funcs.KernelManager.FUSE_ENCODING_ATTENTION:
         return None                                    # (the two operators asked for one by one)
     if bins > 0 and (P.value_pe_condproj != "no" or not P.value_pe_headed or not P.use_low_memory):
         return None
@@ -97,7 +101,7 @@ def _block(layer: nn.Module, width: int, device_index: int):
     fields = [_address(t) for t in tensors]
     fields += [bins, int(bool(P.normalize_gauss)), ops.POSITIVE_FUNCS[spec[0]], dist_max, P.value_pe_width_scale,
                cutoff, -0.5 * P.gauss_lb_real * P.scale_real ** -2 * (1 - 1e-5), -0.5 * P.scale_real ** -2,
-               P.gauss_lb_real, spec[1], 1.0 / math.sqrt(D)]
+               P.gauss_lb_real, spec[1], 1.0 / math.sqrt(D), -0.5 * P.scale_reci ** 2 if halves else 0.0]
     return fields, H, ff
 
 

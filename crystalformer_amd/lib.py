@@ -31,7 +31,7 @@ class ForwardBlock(ctypes.Structure):
                                      "w2", "b2")]
                 + [(n, _i64) for n in ("bins", "normalize", "positive_func")]
                 + [(n, _dbl) for n in ("dist_max", "wscale", "cutoff", "weakest", "coef", "lower_bound", "beta",
-                                       "q_scale")])
+                                       "q_scale", "coef_reci")])
 
 
 class ForwardArgs(ctypes.Structure):

@@ -500,6 +500,8 @@ typedef struct {
     double cutoff;                    /* adaptive boxes (as cutoff_radius of cf_real_enc_fwd), 0: fixed cube */
     double weakest;                   /* upper bound (<= 0) of the exponents (cf_real_enc_ring_stage) */
     double coef, lower_bound, beta, q_scale;    /* as in cf_gauss_exponents */
+    double coef_reci;                 /* != 0: heads from H/2 on are in reciprocal space, coef for theirs; width 128
+                                         with ff 512 only, not under a size header (CF_ERR_UNSUPPORTED) */
 } cf_forward_block;
 
 typedef struct {

@@ -53,7 +53,9 @@ def scaled(cfg, seed=5):
 @pytest.mark.parametrize("sizes", [[1], [15], [16], [17], [1, 2, 30], [5, 0, 0, 64, 3], [200]])
 @pytest.mark.parametrize("options", [dict(), dict(adaptive_cutoff_sigma=0.0), dict(value_pe_dist_real=0),
                                      dict(value_pe_dist_real=24, head_num=4, positive_func="abs"),
-                                     dict(model_dim=64, embedding_dim=[64], ff_dim=96, normalize_gauss=False)])
+                                     dict(model_dim=64, embedding_dim=[64], ff_dim=96, normalize_gauss=False),
+                                     dict(domain="multihead"), dict(domain="multihead-real", head_num=4),
+                                     dict(domain="multihead", value_pe_dist_real=0, adaptive_cutoff_sigma=0.0)])
 def test_native_forward_equals_the_modules(dev, sizes, options):
     model = scaled(default_params(num_layers=2, **options)).to(dev).eval()
     b = batch_of(sizes).to(dev)
@@ -135,7 +137,7 @@ def test_training_mode_without_gradients_stores_the_statistics(dev):
 
 def test_native_forward_leaves_other_models_to_the_modules(dev):
     b = batch_of([4, 6]).to(dev)
-    for options in (dict(domain="multihead"), dict(value_pe_condproj="i"), dict(gauss_state="1"),
+    for options in (dict(domain="reci"), dict(domain="multihead", gauss_lb_reci=0.3), dict(value_pe_condproj="i"), dict(gauss_state="1"),
                     dict(t_fixup_init=False), dict(norm_func_mode=2), dict(use_low_memory=False),
                     dict(t_activation="gelu")):
         model = scaled(default_params(num_layers=1, **options)).to(dev).eval()

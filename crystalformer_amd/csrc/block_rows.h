@@ -1,4 +1,4 @@
-// Arguments and launchers of block_rows.hip (row-wise parts of a forward, used by cf_forward).
+// Arguments and launchers that cf_forward uses beside the C entry points: block_rows.hip and parts of others.
 #pragma once
 #include "cf_common.h"
 
@@ -49,6 +49,12 @@ bool block_rows_served(int64_t width, int64_t ff, int64_t H);
 int launch_block_rows(RowsArgs p, hipStream_t st);
 bool pool_head_served(int64_t width, int64_t hidden);
 int launch_pool_head(const PoolHeadArgs &p, int64_t B, hipStream_t st);
+// fused_dpa.hip: attention whose weights nobody reads.  aij_second != 0: the heads come in two halves with a
+// bias (E, H/2) each, the second aij_second floats behind the first, and bij (E, H/2, D) is the first half's.
+bool dpa_streams(int64_t N, int64_t H, int64_t E, int64_t D);
+int launch_dpa_inference(const float *que, const float *key, const float *val, const float *aij, int64_t aij_second,
+                         const float *bij, const int64_t *edges, const int64_t *e_start, int64_t N, int64_t H, int64_t E,
+                         int64_t D, float *out, hipStream_t st);
 // cf_lattice_geometry that also clears `words` 32-bit words at `zero` (counters of later launches).
 int launch_lattice_geometry(const float *trans, int64_t B, float *vcell, float *recip, float *rvlen, unsigned *zero,
                             int words, hipStream_t st);

@@ -57,12 +57,6 @@ int launch_real_enc_fwd_rings(const float *a_ik, const int64_t *pairs, int64_t U
                               int64_t K, int64_t D, float bin_step, float s_scale, const float *W,
                               const float *cache, const int *order, const int64_t *n_units,
                               float *z, float *v, hipStream_t st);
-// fused_dpa.hip: attention whose weights nobody reads.  aij_second != 0: the heads come in two halves with a
-// bias (E, H/2) each, the second aij_second floats behind the first, and bij (E, H/2, D) is the first half's.
-bool dpa_streams(int64_t N, int64_t H, int64_t E, int64_t D);
-int launch_dpa_inference(const float *que, const float *key, const float *val, const float *aij, int64_t aij_second,
-                         const float *bij, const int64_t *edges, const int64_t *e_start, int64_t N, int64_t H, int64_t E,
-                         int64_t D, float *out, hipStream_t st);
 int64_t unit_partition_bytes(int64_t U);
 int launch_unit_partition(const float *a_ik, const float *rvlen, const int64_t *pairs, int64_t U, int64_t N, int64_t H,
                           float cutoff, int lattice_range, int min_range, void *scratch, int64_t **counts_out,

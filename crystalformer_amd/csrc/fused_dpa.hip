@@ -12,6 +12,7 @@
 //   keys    (per key)  : gv_j = sum_i gb_ij, gk_j = sum_i gs_ij q_i, walking a
 //                        column of the crystal's dense n x n edge block.
 #include "cf_common.h"
+#include "block_rows.h"
 
 namespace {
 

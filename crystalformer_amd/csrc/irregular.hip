@@ -143,6 +143,54 @@ __global__ void layout_rows_kernel(const int64_t *atom_start, const int64_t *edg
     if (batch) batch[i] = lo;
 }
 
+// ---- is an edge list the dense per-crystal block list? ---------------------------
+// An edge list comes from someone else's model as plain tensors, and every new batch brings new ones, so the check
+// is part of a first pass on each.  As some twenty torch launches (a counting scatter over the edges, repeat_interleave,
+// index arithmetic in 64 bits, a comparison) it took 190 us at 4.5e5 edges; here three launches and 15 us.
+//
+// words {unsorted, first id, last id, differs}, zeroed by the caller
+__global__ __launch_bounds__(256) void dense_head_kernel(const int64_t *__restrict__ batch, int64_t N, int64_t *words)
+{
+    const int64_t tid = (int64_t)blockIdx.x * 256 + threadIdx.x, step = (int64_t)gridDim.x * 256;
+    bool bad = false;
+    for (int64_t i = tid; i + 1 < N; i += step) bad = bad || batch[i + 1] < batch[i];
+    if (bad) words[0] = 1;                                      // (every writer writes the same)
+    if (tid == 0) {
+        words[1] = batch[0];
+        words[2] = batch[N - 1];
+    }
+}
+
+// sizes of crystals 0 .. B - 1 from the sorted crystal ids of the atoms
+__global__ __launch_bounds__(256) void crystal_sizes_kernel(const int64_t *__restrict__ batch, int64_t N, int64_t B,
+                                                            int64_t *__restrict__ sizes)
+{
+    const int64_t b = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (b >= B) return;
+    auto first_at_least = [&](int64_t id) -> int64_t {
+        int64_t lo = 0, hi = N;
+        while (lo < hi) {
+            const int64_t mid = (lo + hi) >> 1;
+            if (batch[mid] < id) lo = mid + 1;
+            else hi = mid;
+        }
+        return lo;
+    };
+    sizes[b] = first_at_least(b + 1) - first_at_least(b);
+}
+
+__global__ __launch_bounds__(256) void dense_check_kernel(const int64_t *atom_start, const int64_t *edge_start, int64_t B,
+                                                          int64_t E, const int64_t *__restrict__ edges, int64_t *words)
+{
+    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    bool bad = edge_start[B] != E;
+    if (!bad && e < E) {
+        const EdgeEnds r = edge_ends(atom_start, edge_start, B, e);
+        bad = edges[e] != r.i || edges[E + e] != r.j;
+    }
+    if (bad) words[3] = 1;
+}
+
 // Up to COPY_SEGMENTS device-to-device copies (or zero fills, src == NULL) in one launch: a
 // work-group strides over the 16-byte pieces of every segment, bytes beyond the last whole piece
 // (and segments that are not 16-byte aligned) go one at a time.
@@ -261,4 +309,52 @@ extern "C" int cf_batch_layout(const int64_t *sizes_n, int64_t B, int64_t N, int
     if (rc) return rc;
     if (pairs_u) rc = cf_edge_pairs(atom_start_n, edge_start_n, unit_start_n, B, E, pairs_u, stream);
     return rc;
+}
+
+extern "C" int cf_layout_scan(const int64_t *sizes_n, int64_t B, int64_t *atom_start_n, int64_t *edge_start_n,
+                              int64_t *unit_start_n, void *stream)
+{
+    CF_REQUIRE(B >= 1 && sizes_n && atom_start_n && edge_start_n && unit_start_n, CF_ERR_INVALID_ARGUMENT,
+               "cf_layout_scan: null pointer or no crystals");
+    layout_scan_kernel<<<1, SCAN_THREADS, 0, (hipStream_t)stream>>>(sizes_n, B, atom_start_n, edge_start_n, unit_start_n,
+                                                                    nullptr, 0, 0);
+    CF_CHECK_LAUNCH("cf_layout_scan");
+    return CF_OK;
+}
+
+extern "C" int cf_dense_head(const int64_t *batch_i, int64_t N, int64_t *words_4, void *stream)
+{
+    CF_REQUIRE(N >= 1 && batch_i && words_4, CF_ERR_INVALID_ARGUMENT, "cf_dense_head: null pointer or no atoms");
+    const int64_t blocks = (N + 255) / 256;
+    dense_head_kernel<<<(unsigned)(blocks < 1024 ? blocks : 1024), 256, 0, (hipStream_t)stream>>>(batch_i, N, words_4);
+    CF_CHECK_LAUNCH("cf_dense_head");
+    return CF_OK;
+}
+
+extern "C" int cf_dense_check(const int64_t *batch_i, int64_t N, int64_t B, const int64_t *edge_ij_e, int64_t E,
+                              int64_t *sizes_n, int64_t *atom_start_n, int64_t *edge_start_n, int64_t *unit_start_n,
+                              int64_t *words_4, void *stream)
+{
+    CF_REQUIRE(N >= 1 && B >= 1 && E >= 0 && E < (1ll << 31) * 256 && batch_i && sizes_n && atom_start_n && edge_start_n &&
+                   unit_start_n && words_4 && (E == 0 || edge_ij_e),
+               CF_ERR_INVALID_ARGUMENT, "cf_dense_check: null pointer or bad size");
+    hipStream_t st = (hipStream_t)stream;
+    crystal_sizes_kernel<<<(unsigned)((B + 255) / 256), 256, 0, st>>>(batch_i, N, B, sizes_n);
+    CF_CHECK_LAUNCH("cf_dense_check: sizes");
+    const int rc = cf_layout_scan(sizes_n, B, atom_start_n, edge_start_n, unit_start_n, stream);
+    if (rc) return rc;
+    dense_check_kernel<<<(unsigned)((E + 256) / 256), 256, 0, st>>>(atom_start_n, edge_start_n, B, E, edge_ij_e, words_4);
+    CF_CHECK_LAUNCH("cf_dense_check");
+    return CF_OK;
+}
+
+extern "C" int cf_dense_rows(const int64_t *atom_start_n, const int64_t *edge_start_n, int64_t B, int64_t N,
+                             int64_t *e_start_i, void *stream)
+{
+    CF_REQUIRE(B >= 1 && N >= 0 && N < (1ll << 31) * 256 && atom_start_n && edge_start_n && e_start_i,
+               CF_ERR_INVALID_ARGUMENT, "cf_dense_rows: null pointer or bad size");
+    layout_rows_kernel<<<(unsigned)((N + 1 + 255) / 256), 256, 0, (hipStream_t)stream>>>(atom_start_n, edge_start_n, B, N,
+                                                                                         nullptr, e_start_i, nullptr);
+    CF_CHECK_LAUNCH("cf_dense_rows");
+    return CF_OK;
 }

@@ -87,6 +87,10 @@ SIGNATURES = {
     "cf_gauss_exponents_bwd": (_int, [_ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _i64, _i64, _i64, _int, _f32, _f32, _f32,
                                       _f32, _ptr, _i64, _ptr, _ptr, _ptr]),
     "cf_forward_workspace": (_i64, [_ptr, _ptr]),
+    "cf_layout_scan": (_int, [_ptr, _i64, _ptr, _ptr, _ptr, _ptr]),
+    "cf_dense_head": (_int, [_ptr, _i64, _ptr, _ptr]),
+    "cf_dense_check": (_int, [_ptr, _i64, _i64, _ptr, _i64, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr]),
+    "cf_dense_rows": (_int, [_ptr, _ptr, _i64, _i64, _ptr, _ptr]),
     "cf_forward": (_int, [_ptr, _ptr, _ptr, _i64, _ptr]),
     "cf_kr_base": (_int, [_ptr, _ptr, _ptr, _ptr, _i64, _ptr, _ptr]),
     "cf_reci_enc_fwd": (_int, [_ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _i64, _i64, _i64, _int, _ptr, _ptr, _ptr]),

@@ -608,6 +608,20 @@ def minimum_distance(rpos_ij_e: Tensor, tvecs_n: Tensor, batch_i: Tensor, edge_i
     return out
 
 
+def _layout_starts(sizes: Tensor) -> Tuple[Tensor, Tensor, Tensor]:
+    """Leading-zero prefix sums (B+1) of the sizes n, of n^2 and of n (n + 1) / 2."""
+    B = sizes.numel()
+    if B == 0:
+        zero = torch.zeros(1, dtype=torch.int64, device=sizes.device)
+        return zero, zero, zero
+    starts = torch.empty((3, B + 1), dtype=torch.int64, device=sizes.device)
+    with device_guard(sizes.device):
+        rc = _lib.load().cf_layout_scan(ptr(sizes), B, ptr(starts[0]), ptr(starts[1]), ptr(starts[2]),
+                                        stream_handle(sizes.device))
+    check(rc, "cf_layout_scan")
+    return starts[0], starts[1], starts[2]
+
+
 def edge_index(sizes: Tensor, pos: Optional[Tensor] = None,
                num_edges: Optional[int] = None) -> Tuple[Tensor, Optional[Tensor]]:
     """Dense intra-crystal edge list (2,E) and, with ``pos``, p_j - p_i (E,3),
@@ -617,8 +631,7 @@ def edge_index(sizes: Tensor, pos: Optional[Tensor] = None,
     sizes = _i64(sizes, "sizes")
     pos = _f32(pos, "pos")
     B = sizes.numel()
-    atom_start = F.pad(sizes.cumsum(0), (1, 0))
-    edge_start = F.pad((sizes * sizes).cumsum(0), (1, 0))
+    atom_start, edge_start, _ = _layout_starts(sizes)
     if num_edges is None:
         # one host read per distinct ``sizes`` tensor; repeated forwards over the same batch
         # (and stream capture after a warm-up) find the count in the cache
@@ -647,14 +660,16 @@ def edge_pairs(sizes: Tensor, num_atoms: Optional[int] = None, num_edges: Option
     dev = require_device(sizes)
     sizes = _i64(sizes, "sizes")
     B = sizes.numel()
-    atom_start = F.pad(sizes.cumsum(0), (1, 0))
-    edge_start = F.pad((sizes * sizes).cumsum(0), (1, 0))
-    unit_start = F.pad((sizes * (sizes + 1) // 2).cumsum(0), (1, 0))
+    atom_start, edge_start, unit_start = _layout_starts(sizes)
     if num_atoms is None or num_edges is None:
         tail = torch.stack([atom_start[-1], edge_start[-1]]).tolist() if B > 0 else [0, 0]
         num_atoms, num_edges = int(tail[0]), int(tail[1])
-    U = (num_edges + num_atoms) // 2
-    pairs = torch.empty((U, PAIR_FIELDS), dtype=torch.int64, device=dev)
+    return _edge_pairs_of(atom_start, edge_start, unit_start, num_atoms, num_edges)
+
+
+def _edge_pairs_of(atom_start: Tensor, edge_start: Tensor, unit_start: Tensor, num_atoms: int, num_edges: int) -> Tensor:
+    dev, B = atom_start.device, atom_start.numel() - 1
+    pairs = torch.empty(((num_edges + num_atoms) // 2, PAIR_FIELDS), dtype=torch.int64, device=dev)
     with device_guard(dev):
         rc = _lib.load().cf_edge_pairs(ptr(atom_start), ptr(edge_start), ptr(unit_start), B, num_edges,
                                        ptr(pairs), stream_handle(dev))
@@ -672,13 +687,41 @@ def cached_edge_row_offsets(edge_ij_e: Tensor, num_atoms: int) -> Tensor:
 def dense_block_layout(batch_i: Tensor, edge_ij_e: Tensor) -> Optional[Tensor]:
     """Crystal sizes (B,) if ``edge_ij_e`` is exactly the dense per-crystal block list of
     ``get_edge_index`` for the crystals of ``batch_i`` (atoms of a crystal contiguous, edge
-    (i,j) of a crystal with n atoms at e0 + i*n + j), else ``None``.  Plain torch ops on the
-    tensors' own device; reads three small results back to the host, so it is meant for the
-    first sight of a batch, not for every launch."""
-    N, E = batch_i.numel(), edge_ij_e.shape[1]
-    dev = batch_i.device
+    (i,j) of a crystal with n atoms at e0 + i*n + j), else ``None``.  Reads two small results
+    back to the host, so it is meant for the first sight of a batch, not for every launch."""
+    found = _dense_layout(batch_i, edge_ij_e)
+    return None if found is None else found[0]
+
+
+def _dense_layout(batch_i: Tensor, edge_ij_e: Tensor):
+    """``(sizes, starts)`` of :func:`dense_block_layout`, ``starts`` the prefix sums of :func:`_layout_starts` or None."""
     if edge_ij_e.dim() != 2 or edge_ij_e.shape[0] != 2:
         return None
+    if not (batch_i.is_cuda and edge_ij_e.device == batch_i.device and batch_i.dtype is torch.int64
+            and edge_ij_e.dtype is torch.int64 and batch_i.dim() == 1 and batch_i.is_contiguous()
+            and edge_ij_e.is_contiguous() and batch_i.numel() > 0):
+        sizes = _dense_sizes_torch(batch_i, edge_ij_e)
+        return None if sizes is None else (sizes, None)
+    N, E, dev, lib = batch_i.numel(), edge_ij_e.shape[1], batch_i.device, _lib.load()
+    words = torch.zeros(4, dtype=torch.int64, device=dev)
+    with device_guard(dev):
+        check(lib.cf_dense_head(ptr(batch_i), N, ptr(words), stream_handle(dev)), "cf_dense_head")
+    unsorted, first, last, _ = words.tolist()
+    if unsorted or first < 0 or last >= (1 << 24):
+        return None
+    B = last + 1                          # crystal ids index the lattices as they are
+    sizes = torch.empty(B, dtype=torch.int64, device=dev)
+    starts = torch.empty((3, B + 1), dtype=torch.int64, device=dev).unbind(0)
+    with device_guard(dev):
+        rc = lib.cf_dense_check(ptr(batch_i), N, B, ptr(edge_ij_e), E, ptr(sizes), ptr(starts[0]), ptr(starts[1]),
+                                ptr(starts[2]), ptr(words), stream_handle(dev))
+    check(rc, "cf_dense_check")
+    return None if words[3].item() else (sizes, starts)
+
+
+def _dense_sizes_torch(batch_i: Tensor, edge_ij_e: Tensor) -> Optional[Tensor]:
+    N, E = batch_i.numel(), edge_ij_e.shape[1]
+    dev = batch_i.device
     if N == 0:
         return torch.zeros(0, dtype=torch.int64, device=dev) if E == 0 else None
     head = torch.stack([(batch_i[1:] >= batch_i[:-1]).all().long(), batch_i[0], batch_i[-1]]).tolist()
@@ -700,14 +743,35 @@ def dense_block_layout(batch_i: Tensor, edge_ij_e: Tensor) -> Optional[Tensor]:
 
 def cached_dense_sizes(batch_i: Tensor, edge_ij_e: Tensor) -> Optional[Tensor]:
     """:func:`dense_block_layout`, verified once per (batch_i, edge_ij_e) pair."""
+    return _cached_dense(batch_i, edge_ij_e)[0]
+
+
+def _cached_dense(batch_i: Tensor, edge_ij_e: Tensor):
+    """(sizes or None, starts or None)"""
     sig, hit = _cache_lookup("dense", batch_i, edge_ij_e)
     if hit is not None:
-        return hit[0]
+        return hit if len(hit) == 2 else (hit[0], None)
     if batch_i.is_cuda and torch.cuda.is_current_stream_capturing():
         raise _lib.CrystalformerHipError(
             "an edge list first seen under stream capture cannot be checked for the dense block "
             "layout (the check reads back to the host): run one eager call on it first")
-    return _cache_store(sig, (batch_i, edge_ij_e), (dense_block_layout(batch_i, edge_ij_e),))[0]
+    found = _dense_layout(batch_i, edge_ij_e) or (None, None)
+    if found[1] is not None:
+        # the row offsets and prefix sums follow from the sizes: the attention looks them up under these keys
+        atom_start, edge_start, _ = found[1]
+        dev, N = batch_i.device, batch_i.numel()
+        e_start = torch.empty(N + 1, dtype=torch.int64, device=dev)
+        with device_guard(dev):
+            rc = _lib.load().cf_dense_rows(ptr(atom_start), ptr(edge_start), found[0].numel(), N, ptr(e_start),
+                                           stream_handle(dev))
+        check(rc, "cf_dense_rows")
+        s_, held = _cache_lookup("e_start", edge_ij_e)
+        if held is None:
+            _cache_store(s_, (edge_ij_e,), e_start)
+        s_, held = _cache_lookup("offsets", batch_i)
+        if held is None:
+            _cache_store(s_, (batch_i,), (atom_start, edge_start))
+    return _cache_store(sig, (batch_i, edge_ij_e), found)
 
 
 def cached_edge_pairs(batch_i: Tensor, edge_ij_e: Tensor, num_crystals: int) -> Optional[Tensor]:
@@ -717,13 +781,14 @@ def cached_edge_pairs(batch_i: Tensor, edge_ij_e: Tensor, num_crystals: int) -> 
     sig, hit = _cache_lookup("pairs", batch_i, edge_ij_e)
     if hit is not None:
         return hit
-    sizes = cached_dense_sizes(batch_i, edge_ij_e)
+    sizes, starts = _cached_dense(batch_i, edge_ij_e)
     if sizes is None:
         return None
     if sizes.numel() > num_crystals:
         raise _lib.CrystalformerHipError(
             f"batch_i names {sizes.numel()} crystals but only {num_crystals} lattices were given")
-    pairs = edge_pairs(sizes, batch_i.numel(), edge_ij_e.shape[1])
+    N, E = batch_i.numel(), edge_ij_e.shape[1]
+    pairs = edge_pairs(sizes, N, E) if starts is None else _edge_pairs_of(*starts, N, E)
     return _cache_store(sig, (batch_i, edge_ij_e), pairs)
 
 

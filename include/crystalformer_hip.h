@@ -527,6 +527,23 @@ int cf_forward(const cf_forward_args *args, const cf_forward_block *blocks, void
                int64_t workspace_bytes, void *stream);
 
 /*
+ * Is an edge list (2,E) the dense per-crystal block list of get_edge_index
+ * (models/indexed_latticeformer_encoder.py:15-32) for the atoms' crystal ids batch_i (N)?
+ *   cf_dense_head   words_4 (zeroed by the caller): [0] = 1 if the ids are not ascending, [1] / [2] first and last id
+ *   cf_dense_check  with B = last id + 1 of ascending ids >= 0: sizes_n (B), the prefix sums of cf_layout_scan, and
+ *                   words_4[3] = 1 unless the list is exactly the dense one
+ *   cf_dense_rows   row offsets (N+1) of a list that is
+ * cf_layout_scan: leading-zero prefix sums (B+1) of n, n^2 and n (n + 1) / 2.
+ */
+int cf_layout_scan(const int64_t *sizes_n, int64_t B, int64_t *atom_start_n, int64_t *edge_start_n,
+                   int64_t *unit_start_n, void *stream);
+int cf_dense_head(const int64_t *batch_i, int64_t N, int64_t *words_4, void *stream);
+int cf_dense_check(const int64_t *batch_i, int64_t N, int64_t B, const int64_t *edge_ij_e, int64_t E, int64_t *sizes_n,
+                   int64_t *atom_start_n, int64_t *edge_start_n, int64_t *unit_start_n, int64_t *words_4, void *stream);
+int cf_dense_rows(const int64_t *atom_start_n, const int64_t *edge_start_n, int64_t B, int64_t N, int64_t *e_start_i,
+                  void *stream);
+
+/*
  * Reciprocal-space periodic encoding (ReciPeriodicEncodingFuncCUDA, models/cuda_funcs/reci_space_enc.py:17-99;
  * kernels models/kernels/reci_enc_fwd.cu:3-68, reci_enc_bwd.cu:3-71), LATTICE_RANGE passed at run time:
  *   S[e,h] = sum over n1 in [0,R] (weight 2 for n1 != 0), n2, n3 in [-R,R] of

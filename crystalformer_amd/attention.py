@@ -406,6 +406,35 @@ class CrystalformerMultiheadAttentionCUDA(Module):
         return self._project_output(attn, n, vd, fused_linear, fused_train, residual, need_weights,
                                     weights if need_weights else values)
 
+    def exponent_settings(self):
+        """(normalize, update_stats, positive_func, beta, lower_bound, coef, q_scale) of a real-space block."""
+        P = self.params
+        spec = fused_exponents_spec(P)
+        return (P.normalize_gauss, self.training, spec[0], spec[1], P.gauss_lb_real, -0.5 * P.scale_real ** -2,
+                1.0 / math.sqrt(self.head_dim))
+
+    def encode_and_attend(self, a, qs, k, v, batch, edges, points, dist2_min, tvecs, rvecs) -> Tensor:
+        """Periodic encoding and attention of a plain real-space block, from its exponents and its (N, embed_dim)
+        scaled query, key and value."""
+        P = self.params
+        n, H, D = qs.shape[0], self.num_heads, self.head_dim
+        dist_max = P.value_pe_dist_max
+        if dist_max < 0:
+            dist_max = (-dist_max) * P.scale_real
+        adaptive = (None, None)
+        if P.adaptive_cutoff_sigma != 0:
+            rvlen = rvecs if rvecs.dim() == 2 else torch.norm(rvecs, 2, dim=-1)
+            cutoff = P.adaptive_cutoff_sigma if P.adaptive_cutoff_sigma < 0 else \
+                P.scale_real * P.gauss_lb_real ** (-0.5) * P.adaptive_cutoff_sigma
+            adaptive = (rvlen, cutoff)
+        enc = RealPeriodicEncodingWithProjFuncCUDA if P.use_low_memory else RealPeriodicEncodingFuncCUDA
+        # (an upper bound of the exponents, as in forward)
+        weakest = -0.5 * P.gauss_lb_real * P.scale_real ** -2 * (1 - 1e-5)
+        out = enc.apply(a, points, dist2_min, tvecs, batch, edges, P.value_pe_dist_real, dist_max,
+                        P.value_pe_width_scale, self.pe_dist_proj, *adaptive, weakest)
+        return FusedDotProductAttentionCUDA.apply(qs.view(n, H, D), k.view(n, H, D), v.view(n, H, D), out[0],
+                                                  out[1] if len(out) >= 2 else None, batch, edges)
+
     def _attention_scale(self, prob: Tensor, batch_q: Tensor) -> Tensor:
         """Negative norm_func_mode: outputs times the stored scale, or the reciprocal of the mean (over
         crystals, of the mean over queries and heads) total |weight| per query, stored once in training

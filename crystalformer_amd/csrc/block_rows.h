@@ -19,6 +19,8 @@ struct RowsArgs {
     int split;                                // heads from H/2 on: factor coef_second, their exponents behind all
     float coef_second;                        //   of the first half's, (N, H/2) each
     float *qs, *k, *v, *a;
+    float *s, *h;                             // training: the sum behind the attention, the hidden units,
+    float *q, *alpha_n, *used;                //   the query, the normalised alpha, the (scale, shift) applied
     float *part;                              // statistics without stored ones: 3 floats per 256 values of a
     unsigned *counter;                        // zeroed word
     const int64_t *live_N;                    // set by the launcher
@@ -34,8 +36,26 @@ struct PackArgs {
     int blocks, embed_width;
     const float *w_embed;                     // (128, embed_width <= 128), nullable
     float *packed, *packed_embed;             // blocks x PACKED_BLOCK floats; 128 x 128
+    float *packed_bwd;                        // nullable: as packed, for the backward kernels
+    unsigned *zero;                           // words to clear, nullable
+    int words;
 };
 int launch_pack_weights(const PackArgs &p, hipStream_t st);
+
+struct TailBwdArgs {
+    int64_t N;
+    const float *gy, *h, *packed;
+    float *gh, *gs, *gatt;
+};
+
+struct HeadBwdArgs {
+    int64_t N;
+    int H, func;
+    float beta, lb, coef, q_scale;
+    const float *ga, *gqs, *gk, *gv, *carry;  // nullable each
+    const float *w_pos, *alpha_n, *used, *packed;
+    float *g_alpha, *gq, *gx;
+};
 
 struct PoolHeadArgs {
     const float *x;

@@ -155,6 +155,10 @@ __device__ void finish_exponents(const RowsArgs &p, int64_t total, float *red)
             const float scale = 1.0f / sqrtf(m2 / (n - 1.0f));
             red[0] = scale;
             red[1] = -mean;
+            if (p.used) {
+                p.used[0] = scale;
+                p.used[1] = -mean;
+            }
             if (p.update_stats) {
                 p.gauss_scale[0] = scale;
                 p.gauss_scale[1] = -mean;
@@ -163,9 +167,28 @@ __device__ void finish_exponents(const RowsArgs &p, int64_t total, float *red)
     }
     __syncthreads();
     const float scale = red[0], shift = red[1];
-    for (int64_t t = threadIdx.x; t < total; t += RT)
-        p.a[t] = positive_map((p.a[t] + shift) * scale, p.func, p.beta, p.lb) *
-                 (p.split && 2 * t >= total ? p.coef_second : p.coef);
+    for (int64_t t = threadIdx.x; t < total; t += RT) {
+        const float alpha = (p.a[t] + shift) * scale;
+        if (p.alpha_n) p.alpha_n[t] = alpha;
+        p.a[t] = positive_map(alpha, p.func, p.beta, p.lb) * (p.split && 2 * t >= total ? p.coef_second : p.coef);
+    }
+}
+
+// A work-group that had rows (the first `tiles` of the grid) counts itself; the last one finishes the exponents of all.
+__device__ void finish_if_last(const RowsArgs &p, int64_t N, int64_t tiles, float *red)
+{
+    const int64_t active = min((int64_t)gridDim.x, tiles);
+    if ((int64_t)blockIdx.x >= active) return;
+    __threadfence();
+    __syncthreads();
+    if (threadIdx.x == 0) red[0] = atomicAdd(p.counter, 1u) + 1u == (unsigned)active ? 1.f : 0.f;
+    __syncthreads();
+    const bool last = red[0] != 0.f;
+    __syncthreads();
+    if (last) {
+        __threadfence();
+        finish_exponents(p, N * p.H, red);
+    }
 }
 
 // The matrices as a sequence of units, 16 columns a wavefront x 128 reduction steps each:
@@ -179,6 +202,8 @@ constexpr int UNIT_FF1 = 1, UNIT_FF2 = 5, UNIT_EMBED = 8, UNIT_QUERY = 9, UNIT_E
 __global__ __launch_bounds__(256) void pack_weights_kernel(PackArgs p)
 {
     const int l = blockIdx.y, u = blockIdx.x / (UNIT_FLOATS / 1024);
+    if (p.zero && blockIdx.x == 0 && l == 0 && blockIdx.z == 0)
+        for (int t = threadIdx.x; t < p.words; t += 256) p.zero[t] = 0u;
     if (l == p.blocks && u > 0) return;
     const int at = 4 * (int)(blockIdx.x % (UNIT_FLOATS / 1024) * 256 + threadIdx.x);     // first of four floats of the unit
     const int wave = at / 2048, k = at / 256 % 8 * 16 + at / 64 % 4 * 4, col = 16 * wave + at / 4 % 16;
@@ -191,6 +216,18 @@ __global__ __launch_bounds__(256) void pack_weights_kernel(PackArgs p)
         return;
     }
     const PackSource &w = p.block[l];
+    if (blockIdx.z == 1) {                                      // transposed: units 0-3 W2, 4-7 W1, 8 Wo, 9-11 Wq, Wk, Wv
+        const float *t;
+        int ld = RW;
+        if (u < 4) t = w.w2 + u * RW, ld = RF;
+        else if (u < 8) t = w.w1 + (u - 4) * RW * RW;
+        else t = u == 8 ? w.wo : u == 9 ? w.wq : u == 10 ? w.wk : w.wv;
+        float4_t v;
+#pragma unroll
+        for (int i = 0; i < 4; i++) v[i] = t[(k + i) * ld + col];
+        *reinterpret_cast<float4_t *>(p.packed_bwd + (int64_t)l * PACKED_BLOCK + u * UNIT_FLOATS + at) = v;
+        return;
+    }
     const float *src;
     if (u == 0) src = w.wo + col * RW + k;
     else if (u < UNIT_FF2) src = w.w1 + ((u - UNIT_FF1) * RW + col) * RW + k;
@@ -362,21 +399,313 @@ __global__ __launch_bounds__(RT) void block_rows_kernel(RowsArgs p)
         }
         __syncthreads();                                        // the next tile overwrites the rows
     }
-    if (HEAD && !stored) {
-        // a work-group that had rows counts itself; the last one finishes the exponents of all
-        const int64_t active = min((int64_t)gridDim.x, (N + M - 1) / M);
-        if ((int64_t)blockIdx.x >= active) return;
-        __threadfence();
-        __syncthreads();
-        if (threadIdx.x == 0) red[0] = atomicAdd(p.counter, 1u) + 1u == (unsigned)active ? 1.f : 0.f;
-        __syncthreads();
-        const bool last = red[0] != 0.f;
-        __syncthreads();
-        if (last) {
-            __threadfence();
-            finish_exponents(p, N * p.H, red);
+    if (HEAD && !stored) finish_if_last(p, N, (N + M - 1) / M, red);
+}
+
+// ---- training ------------------------------------------------------------------
+// The same parts with what their backward passes need, and these, on v_mfma_f32_16x16x4_f32 with sixteen rows a
+// work-group: every sum of linear_rows_kernel, linear_rows_nn_kernel and the exponent kernels in their order, so that
+// a training step is the same to the bit.  (It has to be: after the optimiser's first steps biases come back to zero
+// but for rounding, a hidden unit's ReLU then opens or shuts for all atoms at once, and gradients of any other
+// order of summation drift apart by 5% within ten steps.)  What bounds a launch is the matrix cores of the CUs that
+// have a tile: 7.7 us of a tail.  Measured at 1774 rows: tail 14.1 us forward and 15.0 backward, head 8.2 and 8.7 plus 8.5
+// for the gradient of w_pos, 54 us a block where the separate launches took 78.
+//   A: lane (q, c) reads 16 bytes of row c at k = 16 s + 4 q;  B: the packed weights as they are;
+//   D: lane (q, c), register r: row 4 q + r, column c.
+constexpr int TM = 16;
+constexpr int TLX = RW + 4, TLH = RF + 4;    // LDS row strides: 4 mod 64, so 16 rows' 16-byte reads cover all banks
+
+__device__ __forceinline__ void multiply16(float4_t &acc, const Weights &b, const float *xs, int ld, int lane)
+{
+    const float *xr = xs + (lane & 15) * ld + 4 * (lane >> 4);
+    float4_t x[8];
+#pragma unroll
+    for (int c = 0; c < 8; c++) x[c] = *reinterpret_cast<const float4_t *>(xr + 16 * c);
+#pragma unroll
+    for (int c = 0; c < 8; c++)
+#pragma unroll
+        for (int s = 0; s < 4; s++) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(x[c][s], b.w[c][s], acc, 0, 0, 0);
+    asm volatile("" : "+v"(acc));            // (as in multiply: the products belong here)
+}
+
+// rows row0 .. of a (N, 128) matrix into LDS and back: 512 threads are 16 rows x 32 pieces of 16 bytes
+__device__ __forceinline__ void stage16(float *dst, const float *__restrict__ src, int64_t row0, int64_t N)
+{
+    const int r = threadIdx.x / (RW / 4), c = threadIdx.x % (RW / 4);
+    *reinterpret_cast<float4_t *>(dst + r * TLX + 4 * c) =
+        *reinterpret_cast<const float4_t *>(src + min(row0 + r, N - 1) * RW + 4 * c);
+}
+
+__device__ __forceinline__ void unstage16(float *__restrict__ dst, int ld, const float *src, int lds_ld, int64_t row0,
+                                          int64_t N)
+{
+    const int r = threadIdx.x / (RW / 4), c = threadIdx.x % (RW / 4);
+    if (row0 + r < N)
+        *reinterpret_cast<float4_t *>(dst + (row0 + r) * ld + 4 * c) =
+            *reinterpret_cast<const float4_t *>(src + r * lds_ld + 4 * c);
+}
+
+__global__ __launch_bounds__(RT) void block_tail_train_kernel(RowsArgs p)
+{
+    __shared__ __align__(16) float b0[TM * TLX], b1[TM * TLX], hs[TM * TLH];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int q = lane >> 4, col = 16 * wave + (lane & 15);
+    const int64_t row0 = (int64_t)blockIdx.x * TM, N = p.N;
+    const unsigned woff = (unsigned)(wave * 2048 + lane * 4) * 4u;
+    const float *w = p.packed_tail;
+    Weights wa, wb, wc;
+    load_weights(wa, w, woff);
+    stage16(b0, p.att, row0, N);
+    stage16(b1, p.x, row0, N);
+    const float bo = p.bo ? p.bo[col] : 0.f, b2 = p.b2 ? p.b2[col] : 0.f;
+    float bh[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) bh[u] = p.b1 ? p.b1[u * RW + col] : 0.f;
+    load_weights(wb, w + UNIT_FLOATS, woff);
+    __syncthreads();
+    const float4_t zero4 = {0.f, 0.f, 0.f, 0.f};
+    float4_t acc = zero4;
+    load_weights(wc, w + 2 * UNIT_FLOATS, woff);
+    multiply16(acc, wa, b0, TLX, lane);
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        const float v = acc[r] + bo;
+        b1[(4 * q + r) * TLX + col] = v + b1[(4 * q + r) * TLX + col];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+        Weights &cur = u % 3 == 0 ? wb : u % 3 == 1 ? wc : wa, &nxt = u % 3 == 0 ? wa : u % 3 == 1 ? wb : wc;
+        load_weights(nxt, w + (UNIT_FF1 + 2 + u) * UNIT_FLOATS, woff);
+        acc = zero4;
+        multiply16(acc, cur, b1, TLX, lane);
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const float v = acc[r] + bh[u];
+            hs[(4 * q + r) * TLH + u * RW + col] = v < 0.f ? 0.f : v;            // (a NaN stays one)
         }
     }
+    __syncthreads();
+    acc = zero4;
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+        Weights &cur = u % 3 == 0 ? wc : u % 3 == 1 ? wa : wb, &nxt = u % 3 == 0 ? wb : u % 3 == 1 ? wc : wa;
+        if (u < 2) load_weights(nxt, w + (UNIT_FF2 + 2 + u) * UNIT_FLOATS, woff);
+        multiply16(acc, cur, hs + u * RW, TLH, lane);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        const float v = acc[r] + b2;
+        b0[(4 * q + r) * TLX + col] = v + b1[(4 * q + r) * TLX + col];
+    }
+    __syncthreads();
+    unstage16(p.y, RW, b0, TLX, row0, N);
+    unstage16(p.s, RW, b1, TLX, row0, N);
+#pragma unroll
+    for (int u = 0; u < 4; u++) unstage16(p.h + u * RW, RF, hs + u * RW, TLH, row0, N);
+}
+
+__global__ __launch_bounds__(RT) void block_head_train_kernel(RowsArgs p)
+{
+    __shared__ __align__(16) float b0[TM * TLX], out[3][TM * TLX];
+    __shared__ float red[2];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int q = lane >> 4, col = 16 * wave + (lane & 15);
+    const int64_t row0 = (int64_t)blockIdx.x * TM, N = p.N;
+    const unsigned woff = (unsigned)(wave * 2048 + lane * 4) * 4u;
+    const float *w = p.packed_head + UNIT_QUERY * UNIT_FLOATS;
+    Weights wt[3];
+    load_weights(wt[0], w, woff);
+    stage16(b0, p.x, row0, N);
+    load_weights(wt[1], w + UNIT_FLOATS, woff);
+    load_weights(wt[2], w + 2 * UNIT_FLOATS, woff);
+    bool stored = true;
+    float scale = 1.f, shift = 0.f;
+    if (p.normalize) {
+        scale = p.gauss_scale[0];
+        shift = p.gauss_scale[1];
+        stored = scale > 0.f;
+        if (p.used && stored && blockIdx.x == 0 && threadIdx.x == 0) {
+            p.used[0] = scale;
+            p.used[1] = shift;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < 3; u++) {
+        const float bias = p.b_in ? p.b_in[u * RW + col] : 0.f;
+        float4_t acc = {0.f, 0.f, 0.f, 0.f};
+        multiply16(acc, wt[u], b0, TLX, lane);
+#pragma unroll
+        for (int r = 0; r < 4; r++) out[u][(4 * q + r) * TLX + col] = acc[r] + bias;
+    }
+    __syncthreads();
+    unstage16(p.q, RW, out[0], TLX, row0, N);
+    unstage16(p.k, RW, out[1], TLX, row0, N);
+    unstage16(p.v, RW, out[2], TLX, row0, N);
+    {
+        const int r = threadIdx.x / (RW / 4), d = 4 * (threadIdx.x % (RW / 4));
+        if (row0 + r < N)
+            *reinterpret_cast<float4_t *>(p.qs + (row0 + r) * RW + d) =
+                *reinterpret_cast<const float4_t *>(out[0] + r * TLX + d) * p.q_scale;
+    }
+    const int D = RW / p.H;
+    for (int t = threadIdx.x; t < TM * p.H; t += RT) {
+        const int r = t / p.H, h = t - r * p.H;
+        if (row0 + r >= N) break;
+        float alpha = 0.f;
+        for (int d = 0; d < D; d += 4) {                        // (the order of the exponent kernel)
+            const float4 qv = *reinterpret_cast<const float4 *>(out[0] + r * TLX + h * D + d);
+            const float4 wv = *reinterpret_cast<const float4 *>(p.w_pos + h * D + d);
+            alpha += (qv.x * wv.x + qv.y * wv.y) + (qv.z * wv.z + qv.w * wv.w);
+        }
+        const int64_t at = (row0 + r) * p.H + h;
+        if (p.normalize && stored) alpha = (alpha + shift) * scale;
+        if (!p.normalize || stored) {
+            if (p.alpha_n) p.alpha_n[at] = alpha;
+            alpha = positive_map(alpha, p.func, p.beta, p.lb) * p.coef;
+        }
+        p.a[at] = alpha;
+    }
+    if (!stored) finish_if_last(p, N, (N + TM - 1) / TM, red);
+}
+
+// tail: from gy, the gradient behind the block,  gh = (gy W2) where h > 0,  gs = gh W1 + gy,  gatt = gs Wo
+__global__ __launch_bounds__(RT) void block_tail_bwd_kernel(TailBwdArgs p)
+{
+    __shared__ __align__(16) float b0[TM * TLX], b1[TM * TLX], hs[TM * TLH];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int q = lane >> 4, col = 16 * wave + (lane & 15);
+    const int64_t row0 = (int64_t)blockIdx.x * TM, N = p.N;
+    const unsigned woff = (unsigned)(wave * 2048 + lane * 4) * 4u;
+    Weights wa, wb, wc;
+    load_weights(wa, p.packed, woff);
+    stage16(b0, p.gy, row0, N);
+    float open[4][4];                                           // the hidden units of this lane's results
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) open[u][r] = p.h[min(row0 + 4 * q + r, N - 1) * RF + u * RW + col];
+    load_weights(wb, p.packed + UNIT_FLOATS, woff);
+    __syncthreads();
+    const float4_t zero4 = {0.f, 0.f, 0.f, 0.f};
+    float4_t acc;
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+        Weights &cur = u % 3 == 0 ? wa : u % 3 == 1 ? wb : wc, &nxt = u % 3 == 0 ? wc : u % 3 == 1 ? wa : wb;
+        load_weights(nxt, p.packed + (u + 2) * UNIT_FLOATS, woff);
+        acc = zero4;
+        multiply16(acc, cur, b0, TLX, lane);
+#pragma unroll
+        for (int r = 0; r < 4; r++) hs[(4 * q + r) * TLH + u * RW + col] = open[u][r] > 0.f ? acc[r] : 0.f;
+    }
+    __syncthreads();
+    acc = zero4;
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+        Weights &cur = u % 3 == 0 ? wb : u % 3 == 1 ? wc : wa, &nxt = u % 3 == 0 ? wa : u % 3 == 1 ? wb : wc;
+        if (u < 3) load_weights(nxt, p.packed + (6 + u) * UNIT_FLOATS, woff);
+        multiply16(acc, cur, hs + u * RW, TLH, lane);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; r++) b1[(4 * q + r) * TLX + col] = acc[r] + b0[(4 * q + r) * TLX + col];
+    __syncthreads();
+    acc = zero4;
+    multiply16(acc, wc, b1, TLX, lane);                         // (unit 8)
+#pragma unroll
+    for (int r = 0; r < 4; r++) b0[(4 * q + r) * TLX + col] = acc[r];
+    __syncthreads();
+    unstage16(p.gatt, RW, b0, TLX, row0, N);
+    unstage16(p.gs, RW, b1, TLX, row0, N);
+#pragma unroll
+    for (int u = 0; u < 4; u++) unstage16(p.gh + u * RW, RF, hs + u * RW, TLH, row0, N);
+}
+
+// head: g_alpha = ga rho'(alpha_n) coef scale,  gq = g_alpha w_pos + gqs q_scale,  gx = gq Wq + gk Wk + gv Wv + carry
+__global__ __launch_bounds__(RT) void block_head_bwd_kernel(HeadBwdArgs p)
+{
+    __shared__ __align__(16) float b[3][TM * TLX];              // gq, gk, gv
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int q = lane >> 4, col = 16 * wave + (lane & 15);
+    const int64_t row0 = (int64_t)blockIdx.x * TM, N = p.N;
+    const unsigned woff = (unsigned)(wave * 2048 + lane * 4) * 4u;
+    const float *packed = p.packed + UNIT_QUERY * UNIT_FLOATS;
+    Weights wt[3];
+    load_weights(wt[0], packed, woff);
+    const float4_t zero4 = {0.f, 0.f, 0.f, 0.f};
+    const int r_ = threadIdx.x / (RW / 4), d = 4 * (threadIdx.x % (RW / 4));
+    const bool on = row0 + r_ < N;
+    const int64_t row = min(row0 + r_, N - 1), in = row * RW + d;
+    const int D = RW / p.H;
+    {
+        const float4_t sv = p.gqs ? *reinterpret_cast<const float4_t *>(p.gqs + in) : zero4;
+        const float4_t wv = *reinterpret_cast<const float4_t *>(p.w_pos + d);
+        float g_alpha = 0.f;
+        if (p.ga) {
+            const int64_t ah = row * p.H + d / D;               // (D is a multiple of 4)
+            g_alpha = p.ga[ah] * positive_map_slope(p.alpha_n[ah], p.func, p.beta, p.lb) * p.coef;
+            if (p.used) g_alpha *= p.used[0];
+            if (on && d % D == 0) p.g_alpha[ah] = g_alpha;
+        }
+        float4_t gq = sv * p.q_scale;
+#pragma unroll
+        for (int i = 0; i < 4; i++) gq[i] = fmaf(wv[i], g_alpha, gq[i]);     // (rounded as gauss_exponents_bwd_kernel does)
+        *reinterpret_cast<float4_t *>(&b[0][r_ * TLX + d]) = gq;
+        if (on) *reinterpret_cast<float4_t *>(p.gq + in) = gq;
+        *reinterpret_cast<float4_t *>(&b[1][r_ * TLX + d]) = p.gk ? *reinterpret_cast<const float4_t *>(p.gk + in) : zero4;
+        *reinterpret_cast<float4_t *>(&b[2][r_ * TLX + d]) = p.gv ? *reinterpret_cast<const float4_t *>(p.gv + in) : zero4;
+    }
+    load_weights(wt[1], packed + UNIT_FLOATS, woff);
+    load_weights(wt[2], packed + 2 * UNIT_FLOATS, woff);
+    __syncthreads();
+    float4_t acc = zero4;
+#pragma unroll
+    for (int u = 0; u < 3; u++) multiply16(acc, wt[u], b[u], TLX, lane);
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < 4; r++) b[0][(4 * q + r) * TLX + col] = acc[r];
+    __syncthreads();
+    if (on) {
+        float4_t v = *reinterpret_cast<const float4_t *>(&b[0][r_ * TLX + d]);
+        if (p.carry) v += *reinterpret_cast<const float4_t *>(p.carry + in);
+        *reinterpret_cast<float4_t *>(p.gx + in) = v;
+    }
+}
+
+// gw_pos = sum over atoms of g_alpha q: 16 columns a work-group; shares of 256 / H atoms each, 64 side by side, their
+// atoms in ascending order, the even and the odd shares added up in order (as the exponent kernels' backward does).
+__global__ __launch_bounds__(1024) void head_weight_grad_kernel(const float *__restrict__ g_alpha, const float *__restrict__ q,
+                                                                int64_t N, int H, float *__restrict__ gw)
+{
+#pragma clang fp contract(off)
+    __shared__ float run[64][17];
+    const int c = threadIdx.x & 15, g = threadIdx.x >> 4, col = blockIdx.x * 16 + c;
+    const int h = col / (RW / H);
+    const int64_t atoms = 256 / H;
+    float s0 = 0.f, s1 = 0.f;
+    for (int64_t first = 0; first < N; first += 64 * atoms) {
+        const int64_t i0 = first + g * atoms, i1 = min(i0 + atoms, N);
+        float s = 0.f;
+        int64_t i = i0;
+        for (; i + 8 <= i1; i += 8) {        // (sixteen at a time: 15.6 instead of 8.5 us at 1774 atoms)
+            float v[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) v[u] = g_alpha[(i + u) * H + h] * q[(i + u) * RW + col];
+#pragma unroll
+            for (int u = 0; u < 8; u++) s += v[u];
+        }
+        for (; i < i1; i++) s += g_alpha[i * H + h] * q[i * RW + col];
+        __syncthreads();
+        run[g][c] = s;                       // (shares past the end: zero)
+        __syncthreads();
+        if (g == 0) {
+            for (int k = 0; k < 64; k += 2) {
+                s0 += run[k][c];
+                s1 += run[k + 1][c];
+            }
+        }
+    }
+    if (g == 0) gw[col] = s0 + s1;
 }
 
 // Mean over a crystal's atoms and the regression head, one work-group per crystal: 32 lanes x 16 bytes
@@ -445,6 +774,16 @@ __global__ __launch_bounds__(PH_T) void pool_head_kernel(PoolHeadArgs p)
     }
 }
 
+// Rows per work-group over four.  One while that gives a CU at most one tile, two while that does.  Beyond, sixteen
+// rows cost 20 us a round of tiles (one per CU), eight rows 23.5 us per two tiles and CU, side by side: sixteen
+// where the last round is full enough (4096 rows 20.3 against 23.3 us, 5600 rows 37.8 against 32.5).
+int rows_per_quad(int64_t N)
+{
+    const int64_t cus = device_cu_count();
+    const double rounds = (double)N / (double)(16 * cus);
+    return N <= 4 * cus ? 1 : N <= 8 * cus ? 2 : ceil(rounds) * 0.85 <= rounds ? 4 : 2;
+}
+
 template <int R>
 void launch_rows(const RowsArgs &p, int source, bool head, unsigned grid, hipStream_t st)
 {
@@ -465,7 +804,8 @@ bool block_rows_served(int64_t width, int64_t ff, int64_t H)
 
 int launch_pack_weights(const PackArgs &p, hipStream_t st)
 {
-    pack_weights_kernel<<<dim3(UNIT_END * UNIT_FLOATS / 1024, (unsigned)(p.blocks + (p.w_embed ? 1 : 0))), 256, 0, st>>>(p);
+    const dim3 grid(UNIT_END * UNIT_FLOATS / 1024, (unsigned)(p.blocks + (p.w_embed ? 1 : 0)), p.packed_bwd ? 2 : 1);
+    pack_weights_kernel<<<grid, 256, 0, st>>>(p);
     CF_CHECK_LAUNCH("packing of the weights");
     return CF_OK;
 }
@@ -476,12 +816,7 @@ int launch_block_rows(RowsArgs p, hipStream_t st)
     const bool head = p.packed_head != nullptr;
     p.live_N = live_atoms(p.N);
     const int64_t cus = device_cu_count();
-    // Rows per work-group.  Four while that gives a CU at most one tile, eight while that does.  Beyond, sixteen rows
-    // cost 20 us a round of tiles (one per CU), eight rows 23.5 us per two tiles and CU, side by side: sixteen
-    // where the last round is full enough (4096 rows 20.3 against 23.3 us, 5600 rows 37.8 against 32.5).  A live
-    // row count is somewhere below the capacity: eight rows.
-    const double rounds = (double)p.N / (double)(16 * cus);
-    const int R = p.live_N ? 2 : p.N <= 4 * cus ? 1 : ceil(rounds) * 0.85 <= rounds ? 4 : 2;
+    const int R = p.live_N ? 2 : rows_per_quad(p.N);            // (live rows are somewhere below the capacity)
     int64_t grid = (p.N + 4 * R - 1) / (4 * R);
     if (p.live_N && grid > 2 * cus) grid = 2 * cus;             // a capacity: stride over the tiles that exist
     CF_REQUIRE(grid < (1ll << 31), CF_ERR_UNSUPPORTED, "block rows: too many atoms");
@@ -503,3 +838,114 @@ int launch_pool_head(const PoolHeadArgs &p, int64_t B, hipStream_t st)
 }
 
 }  // namespace cf
+
+extern "C" int64_t cf_pack_blocks_floats(int64_t blocks) { return blocks < 0 ? -1 : blocks * cf::PACKED_BLOCK; }
+
+extern "C" int cf_pack_blocks(int64_t blocks, const float *const *weights, float *packed, float *packed_bwd,
+                              int32_t *zero_words, int64_t words, void *stream)
+{
+    CF_REQUIRE(blocks >= 0 && words >= 0, CF_ERR_INVALID_ARGUMENT, "cf_pack_blocks: negative size");
+    if (blocks == 0) return CF_OK;
+    CF_REQUIRE(weights && packed && (words == 0 || zero_words), CF_ERR_INVALID_ARGUMENT, "cf_pack_blocks: null pointer");
+    for (int64_t first = 0; first < blocks; first += cf::PACK_BLOCKS) {
+        cf::PackArgs a{};
+        a.blocks = (int)(blocks - first < cf::PACK_BLOCKS ? blocks - first : cf::PACK_BLOCKS);
+        for (int i = 0; i < a.blocks; i++) {
+            const float *const *w = weights + 6 * (first + i);
+            for (int k = 0; k < 6; k++)
+                CF_REQUIRE(w[k], CF_ERR_INVALID_ARGUMENT, "cf_pack_blocks: null weight in block %lld", (long long)(first + i));
+            a.block[i] = cf::PackSource{w[0], w[1], w[2], w[3], w[4], w[5]};
+        }
+        a.packed = packed + first * cf::PACKED_BLOCK;
+        a.packed_bwd = packed_bwd ? packed_bwd + first * cf::PACKED_BLOCK : nullptr;
+        if (first == 0) {
+            a.zero = (unsigned *)zero_words;
+            a.words = (int)words;
+        }
+        const int rc = cf::launch_pack_weights(a, (hipStream_t)stream);
+        if (rc) return rc;
+    }
+    return CF_OK;
+}
+
+extern "C" int cf_block_head(const float *x, int64_t N, int64_t H, const float *packed, const float *b_in,
+                             const float *w_pos, float *gauss_scale, int normalize, int update_stats, int positive_func,
+                             float beta, float lower_bound, float coef, float q_scale, float *part, int32_t *counter,
+                             float *q, float *qs, float *k, float *v, float *a, float *alpha_n, float *used, void *stream)
+{
+    CF_REQUIRE(N >= 0 && cf::block_rows_served(RW, RF, H), CF_ERR_UNSUPPORTED, "cf_block_head: N=%lld H=%lld not served",
+               (long long)N, (long long)H);
+    CF_REQUIRE(positive_func >= 0 && positive_func <= 2 && lower_bound < 1.0f, CF_ERR_UNSUPPORTED,
+               "cf_block_head: positive map not served");
+    if (N == 0) return CF_OK;
+    CF_REQUIRE(x && packed && w_pos && q && qs && k && v && a && (!normalize || (gauss_scale && part && counter)),
+               CF_ERR_INVALID_ARGUMENT, "cf_block_head: null pointer");
+    const int64_t grid = (N + TM - 1) / TM;
+    CF_REQUIRE(grid < (1ll << 31), CF_ERR_UNSUPPORTED, "cf_block_head: too many rows");
+    cf::RowsArgs r{};
+    r.N = N; r.H = (int)H; r.x = x; r.packed_head = packed; r.b_in = b_in; r.w_pos = w_pos; r.gauss_scale = gauss_scale;
+    r.normalize = normalize; r.update_stats = update_stats; r.func = positive_func;
+    r.beta = beta; r.lb = lower_bound; r.coef = coef; r.q_scale = q_scale;
+    r.part = part; r.counter = (unsigned *)counter;
+    r.q = q; r.qs = qs; r.k = k; r.v = v; r.a = a; r.alpha_n = alpha_n; r.used = used;
+    block_head_train_kernel<<<(unsigned)grid, RT, 0, (hipStream_t)stream>>>(r);
+    CF_CHECK_LAUNCH("cf_block_head");
+    return CF_OK;
+}
+
+extern "C" int cf_block_tail(const float *att, const float *x, int64_t N, const float *packed, const float *bo,
+                             const float *b1, const float *b2, float *s, float *h, float *y, void *stream)
+{
+    CF_REQUIRE(N >= 0, CF_ERR_INVALID_ARGUMENT, "cf_block_tail: negative size");
+    if (N == 0) return CF_OK;
+    CF_REQUIRE(att && x && packed && s && h && y, CF_ERR_INVALID_ARGUMENT, "cf_block_tail: null pointer");
+    const int64_t grid = (N + TM - 1) / TM;
+    CF_REQUIRE(grid < (1ll << 31), CF_ERR_UNSUPPORTED, "cf_block_tail: too many rows");
+    cf::RowsArgs r{};
+    r.N = N; r.H = 1; r.att = att; r.x = x; r.packed_tail = packed; r.bo = bo; r.b1 = b1; r.b2 = b2;
+    r.s = s; r.h = h; r.y = y;
+    block_tail_train_kernel<<<(unsigned)grid, RT, 0, (hipStream_t)stream>>>(r);
+    CF_CHECK_LAUNCH("cf_block_tail");
+    return CF_OK;
+}
+
+extern "C" int cf_block_tail_bwd(const float *gy, const float *h, int64_t N, const float *packed_bwd, float *gh, float *gs,
+                                 float *gatt, void *stream)
+{
+    CF_REQUIRE(N >= 0, CF_ERR_INVALID_ARGUMENT, "cf_block_tail_bwd: negative size");
+    if (N == 0) return CF_OK;
+    CF_REQUIRE(gy && h && packed_bwd && gh && gs && gatt, CF_ERR_INVALID_ARGUMENT, "cf_block_tail_bwd: null pointer");
+    const cf::TailBwdArgs p{N, gy, h, packed_bwd, gh, gs, gatt};
+    const int64_t grid = (N + TM - 1) / TM;
+    CF_REQUIRE(grid < (1ll << 31), CF_ERR_UNSUPPORTED, "cf_block_tail_bwd: too many rows");
+    block_tail_bwd_kernel<<<(unsigned)grid, RT, 0, (hipStream_t)stream>>>(p);
+    CF_CHECK_LAUNCH("cf_block_tail_bwd");
+    return CF_OK;
+}
+
+extern "C" int cf_block_head_bwd(const float *ga, const float *gqs, const float *gk, const float *gv, const float *carry,
+                                 const float *q, const float *w_pos, const float *alpha_n, const float *used, int64_t N,
+                                 int64_t H, const float *packed_bwd, int positive_func, float beta, float lower_bound,
+                                 float coef, float q_scale, float *g_alpha, float *gq, float *gx, float *gw_pos,
+                                 void *stream)
+{
+    CF_REQUIRE(N >= 0 && cf::block_rows_served(RW, RF, H), CF_ERR_UNSUPPORTED,
+               "cf_block_head_bwd: N=%lld H=%lld not served", (long long)N, (long long)H);
+    CF_REQUIRE(positive_func >= 0 && positive_func <= 2 && lower_bound < 1.0f, CF_ERR_UNSUPPORTED,
+               "cf_block_head_bwd: positive map not served");
+    CF_REQUIRE((N == 0 || (w_pos && packed_bwd && gq && gx)) && (!ga || (q && alpha_n && g_alpha && gw_pos)),
+               CF_ERR_INVALID_ARGUMENT, "cf_block_head_bwd: null pointer");
+    if (N == 0) return CF_OK;
+    hipStream_t st = (hipStream_t)stream;
+    const int64_t grid = (N + TM - 1) / TM;
+    CF_REQUIRE(grid < (1ll << 31), CF_ERR_UNSUPPORTED, "cf_block_head_bwd: too many rows");
+    const cf::HeadBwdArgs p{N, (int)H, positive_func, beta, lower_bound, coef, q_scale, ga, gqs, gk, gv, carry, w_pos,
+                            alpha_n, used, packed_bwd, g_alpha, gq, gx};
+    block_head_bwd_kernel<<<(unsigned)grid, RT, 0, st>>>(p);
+    CF_CHECK_LAUNCH("cf_block_head_bwd");
+    if (ga) {
+        head_weight_grad_kernel<<<RW / 16, 1024, 0, st>>>(g_alpha, q, N, (int)H, gw_pos);
+        CF_CHECK_LAUNCH("cf_block_head_bwd: weight gradient");
+    }
+    return CF_OK;
+}

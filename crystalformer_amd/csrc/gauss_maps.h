@@ -15,6 +15,16 @@ __device__ __forceinline__ float positive_map(float x, int func, float beta, flo
     return (1.0f - lb) * expf(x * (beta / (1.0f - lb))) + lb;   // exp
 }
 
+__device__ __forceinline__ float positive_map_slope(float x, int func, float beta, float lb)
+{
+    if (func == 0) {            // elu
+        const float t = x * (beta / (1.0f - lb));
+        return (t > 0.f ? 1.0f : expf(t)) * beta;
+    }
+    if (func == 1) return (x > 0.f ? 1.0f : (x < 0.f ? -1.0f : 0.f)) * (1.0f - lb);   // abs
+    return expf(x * (beta / (1.0f - lb))) * beta;                                      // exp
+}
+
 // Chan's pairwise update of (count, mean, M2).
 __device__ __forceinline__ void stat_merge(float &n, float &mean, float &m2, float nb, float meanb, float m2b)
 {

@@ -203,16 +203,6 @@ struct GaussBwdArgs {
     float *gq, *gw;
 };
 
-__device__ __forceinline__ float positive_map_slope(float x, int func, float beta, float lb)
-{
-    if (func == 0) {            // elu
-        const float t = x * (beta / (1.0f - lb));
-        return (t > 0.f ? 1.0f : expf(t)) * beta;
-    }
-    if (func == 1) return (x > 0.f ? 1.0f : (x < 0.f ? -1.0f : 0.f)) * (1.0f - lb);   // abs
-    return expf(x * (beta / (1.0f - lb))) * beta;                                      // exp
-}
-
 // One thread per (atom, head): g_alpha = ga * rho'(alpha_n) * coef * scale;
 // gq = g_alpha w_head + gqs * q_scale; the block leaves sum_atoms g_alpha q per (head, d),
 // 16 columns of d at a time through LDS, atoms added in ascending order.

@@ -118,12 +118,23 @@ class CrystalformerEncoderLayerCUDA(Module):
 
     def forward(self, src: Tensor, batch: Tensor, edges: Tensor, pos_ij: Tensor = None,
                 dist2_min: Tensor = None, trans: Tensor = None, kr_base: Tensor = None,
-                rvecs: Tensor = None, vcell: Tensor = None, onehot: Tensor = None) -> Tensor:
+                rvecs: Tensor = None, vcell: Tensor = None, onehot: Tensor = None, packed=None) -> Tensor:
+        """``packed`` (an extension): this block's weights as the one-launch row kernels read them, from the
+        encoder in a fused training step."""
         if self.domain in ("real", "multihead"):
             assert pos_ij is not None and trans is not None
         if self.domain in ("reci", "multihead", "RECI"):
             assert kr_base is not None and rvecs is not None and rvecs.dim() == 3 and vcell is not None
         x = src
+        if packed is not None:
+            attn, W = self.self_attn, self.linear1.in_features
+            a, qs, k, v, x = hip_funcs.BlockHeadHIP.apply(
+                x, attn.q_proj_weight, attn.k_proj_weight, attn.v_proj_weight, attn.in_proj_bias,
+                attn.lattice_pos_weights, attn.gauss_scale, attn.num_heads, packed, *attn.exponent_settings())
+            att = attn.encode_and_attend(a, qs, k, v, batch, edges, pos_ij, dist2_min, trans, rvecs)
+            return hip_funcs.BlockTailHIP.apply(att.view(-1, W), x, attn.out_proj.weight, attn.out_proj.bias,
+                                                self.linear1.weight, self.linear1.bias, self.linear2.weight,
+                                                self.linear2.bias, packed)
         if self._fused_tail(x):
             # inference without norm layers: residuals, bias and ReLU ride in the epilogues of
             # three row-block linear launches (out_proj, linear1, linear2)
@@ -223,7 +234,12 @@ class CrystalformerEncoderCUDA(Module):
             rvecs = recip
             kr_base = ops.kr_base(pos_ij, recip, batch, edges)
         output = src
-        for layer in self.layers:
+        pack = executor.pack_for_training(self, src)
+        for i, layer in enumerate(self.layers):
+            if pack is not None:
+                output = layer(output, batch, edges, pos_ij, dist2_min, trans, kr_base, rvecs, vcell, onehot,
+                               packed=pack.block(i))
+                continue
             output = layer(output, batch, edges, pos_ij, dist2_min, trans, kr_base, rvecs, vcell, onehot)
         if self.norm is not None:
             output = self.norm(output)

@@ -105,6 +105,35 @@ def _block(layer: nn.Module, width: int, device_index: int):
     return fields, H, ff
 
 
+def _backward_hooked(module: nn.Module) -> bool:
+    return bool(module._backward_hooks or module._backward_pre_hooks) or \
+        any(c is not None and _backward_hooked(c) for c in module._modules.values())
+
+
+def pack_for_training(encoder: nn.Module, src: Tensor) -> Optional["ops.PackedBlocks"]:
+    """The blocks' weights packed for the one-launch row kernels if every block of a fused training step is one
+    they serve (the plain case of this module, 128 wide with 512 hidden units, real domain) and nobody looks into
+    the blocks; else None: the blocks then run their operators one by one."""
+    if not (hip_funcs.USE_LINEAR_FUNCTION and torch.is_grad_enabled()) or type(src) is not Tensor or src.dim() != 2 \
+            or config.REPRODUCIBLITY_STATE < 2 or encoder.d_model != 128 or ops.current_live_sizes() is not None \
+            or not _ready(src, src.shape[0] * 128, src.get_device()) or src.get_device() < 0 or src.shape[0] == 0 \
+            or _torch_module._global_forward_hooks or _torch_module._global_forward_pre_hooks \
+            or _torch_module._global_backward_hooks or _torch_module._global_backward_pre_hooks:
+        return None
+    blocks = []
+    for layer in encoder._modules["layers"]._modules.values():
+        mods = layer._modules
+        if any(c is not None and (_any_hooked(c) or _backward_hooked(c)) for c in mods.values()):
+            return None
+        got = _block(layer, 128, src.get_device())
+        if got is None or got[2] != 512 or layer.self_attn.params.domain != "real" or 128 // got[1] % 4:
+            return None
+        attn = mods["self_attn"]
+        blocks.append((attn.out_proj.weight, mods["linear1"].weight, mods["linear2"].weight, attn.q_proj_weight,
+                       attn.k_proj_weight, attn.v_proj_weight))
+    return ops.PackedBlocks(blocks) if blocks else None
+
+
 def _head(mlp: nn.Module, width: int, device_index: int) -> Optional[Tuple[tuple, int, int]]:
     """((w_head, b_head, w_last, b_last), hidden, targets) of a head ``Linear, ReLU, Linear`` or ``Linear``
     (identities in between do not count), else None."""

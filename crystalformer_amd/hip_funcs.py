@@ -620,6 +620,92 @@ class FusedLinearHIP(torch.autograd.Function):
         return (gx, gb, g_res, None, None, *gws)
 
 
+def _weight_gradients(layers):
+    """``(gw, gb)`` per layer of ``(g, x, w, w_leaf, b_leaf, b_off, want_w, want_b)``: None where they are deferred to the
+    end of the backward pass or not wanted.  ``b_leaf`` may own several layers' biases, ``b_off`` is the first."""
+    out, immediate = [(None, None)] * len(layers), []
+    for i, (g, x, w, w_leaf, b_leaf, b_off, want_w, want_b) in enumerate(layers):
+        if not want_w and not want_b:
+            continue
+        if _deferred is not None and want_w and w_leaf is not None and w_leaf.grad is None and \
+                (b_leaf is None or (want_b and b_leaf.grad is None)):
+            _deferred.append((g, x, w_leaf, b_leaf if want_b else None, b_off))
+            continue
+        gw = torch.empty_like(w, memory_format=torch.contiguous_format)
+        gb = torch.empty(w.shape[0], dtype=w.dtype, device=w.device) if want_b else None
+        immediate.append((g, x, gw, gb))
+        out[i] = (gw if want_w else None), gb
+    if immediate:
+        ops.linear_weight_grad_grouped(immediate)
+    return out
+
+
+def _leaf(t):
+    return t if (t is not None and t.is_leaf) else None
+
+
+class BlockHeadHIP(torch.autograd.Function):
+    """``(a, qs, k, v, x)`` of a 128-wide block: the three projections of ``x`` and the Gaussian exponents in one
+    launch (:func:`ops.block_head`), one more and a short reduction backward.  ``x`` itself is handed on (an identity
+    whose gradient is added in the backward launch) for the residual that leaves here; the statistics are
+    constants of the backward pass, as in :class:`GaussianExponentsHIP`."""
+
+    @staticmethod
+    def forward(ctx, x, wq, wk, wv, b_in, w_pos, gauss_scale, heads, packed, normalize, update_stats, positive_func, beta,
+                lower_bound, coef, q_scale):
+        conf = (positive_func, beta, lower_bound, coef, q_scale)
+        a, qs, k, v, q, alpha_n, used = ops.block_head(x.detach(), heads, packed[0], packed[2], b_in, w_pos.detach(),
+                                                       gauss_scale, normalize, update_stats, *conf)
+        ctx.save_for_backward(x, wq, wk, wv, w_pos, q, alpha_n, used, packed[1])
+        ctx.conf = conf
+        ctx.leaves = (_leaf(wq), _leaf(wk), _leaf(wv)), _leaf(b_in), b_in is not None
+        return a, qs, k, v, x
+
+    @staticmethod
+    def backward(ctx, ga, gqs, gk, gv, carry):
+        x, wq, wk, wv, w_pos, q, alpha_n, used, packed_bwd = ctx.saved_tensors
+        gq, gx, gw_pos = ops.block_head_bwd(ga, gqs, gk, gv, carry, q, w_pos, alpha_n, used, packed_bwd, *ctx.conf)
+        need = ctx.needs_input_grad
+        weights, bias, has_bias = ctx.leaves
+        want_b = has_bias and need[4]
+        W = wq.shape[0]
+        gs = [gq] + [g.contiguous() if g is not None else torch.zeros_like(gq) for g in (gk, gv)]
+        # (one bias vector for the three layers: all of them deferred, or none)
+        together = not has_bias or (bias is not None and bias.grad is None and want_b)
+        if not (together and all(need[1:4]) and all(w is not None and w.grad is None for w in weights)):
+            weights = (None, None, None)
+        got = _weight_gradients([(g, x, w, leaf, bias, i * W, need[1 + i], want_b)
+                                 for i, (g, w, leaf) in enumerate(zip(gs, (wq, wk, wv), weights))])
+        gb = torch.cat([b for _, b in got]) if want_b and got[0][1] is not None else None
+        return (gx if need[0] else None, *(w for w, _ in got), gb, gw_pos.view(w_pos.shape) if need[5] and gw_pos is not None else None,
+                *(None,) * 10)
+
+
+class BlockTailHIP(torch.autograd.Function):
+    """``y = s + W2 relu(W1 s + b1) + b2`` with ``s = x + Wo att + bo`` of a 128-wide block with 512 hidden units: one
+    launch forward, one backward, the weight and bias gradients from the grouped kernel (deferred inside
+    :class:`deferred_weight_grads`)."""
+
+    @staticmethod
+    def forward(ctx, att, x, wo, bo, w1, b1, w2, b2, packed):
+        y, s, h = ops.block_tail(att.detach(), x.detach(), packed[0], bo, b1, b2)
+        ctx.save_for_backward(att, s, h, wo, w1, w2, packed[1])
+        ctx.leaves = tuple(_leaf(t) for t in (wo, bo, w1, b1, w2, b2))
+        ctx.has_bias = (bo is not None, b1 is not None, b2 is not None)
+        return y
+
+    @staticmethod
+    def backward(ctx, gy):
+        att, s, h, wo, w1, w2, packed_bwd = ctx.saved_tensors
+        gy = gy.contiguous()
+        gh, gs, gatt = ops.block_tail_bwd(gy, h, packed_bwd)
+        need, leaves, has = ctx.needs_input_grad, ctx.leaves, ctx.has_bias
+        got = _weight_gradients([(g, x, w, leaves[2 * i] if not has[i] or leaves[2 * i + 1] is not None else None,
+                                  leaves[2 * i + 1], 0, need[2 + 2 * i], has[i] and need[3 + 2 * i])
+                                 for i, (g, x, w) in enumerate(((gs, att, wo), (gh, s, w1), (gy, h, w2)))])
+        return (gatt if need[0] else None, gs if need[1] else None, *(t for pair in got for t in pair), None)
+
+
 # A list while a training step defers its linear layers' weight gradients (see
 # :func:`deferred_weight_grads`), else None.
 _deferred = None

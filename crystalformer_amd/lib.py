@@ -91,6 +91,14 @@ SIGNATURES = {
     "cf_dense_head": (_int, [_ptr, _i64, _ptr, _ptr]),
     "cf_dense_check": (_int, [_ptr, _i64, _i64, _ptr, _i64, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr]),
     "cf_dense_rows": (_int, [_ptr, _ptr, _i64, _i64, _ptr, _ptr]),
+    "cf_pack_blocks_floats": (_i64, [_i64]),
+    "cf_pack_blocks": (_int, [_i64, _ptr, _ptr, _ptr, _ptr, _i64, _ptr]),
+    "cf_block_head": (_int, [_ptr, _i64, _i64, _ptr, _ptr, _ptr, _ptr, _int, _int, _int, _f32, _f32, _f32, _f32, _ptr,
+                             _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr]),
+    "cf_block_tail": (_int, [_ptr, _ptr, _i64, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr]),
+    "cf_block_tail_bwd": (_int, [_ptr, _ptr, _i64, _ptr, _ptr, _ptr, _ptr, _ptr]),
+    "cf_block_head_bwd": (_int, [_ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _i64, _i64, _ptr, _int, _f32, _f32,
+                                 _f32, _f32, _ptr, _ptr, _ptr, _ptr, _ptr]),
     "cf_forward": (_int, [_ptr, _ptr, _ptr, _i64, _ptr]),
     "cf_kr_base": (_int, [_ptr, _ptr, _ptr, _ptr, _i64, _ptr, _ptr]),
     "cf_reci_enc_fwd": (_int, [_ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _i64, _i64, _i64, _int, _ptr, _ptr, _ptr]),

@@ -1105,6 +1105,118 @@ def gauss_exponents_bwd(ga: Optional[Tensor], gqs: Optional[Tensor], q_ihd: Tens
     return gq, gw
 
 
+class PackedBlocks:
+    """Weights of a stack of blocks in the order the one-launch row kernels read them, forward and backward
+    form, and a zeroed counter per block; made anew for every forward pass."""
+
+    __slots__ = ("forward", "backward", "counters", "floats")
+
+    def __init__(self, blocks):
+        """``blocks``: (Wo, W1, W2, Wq, Wk, Wv) per block, contiguous float32 on one GPU."""
+        import ctypes
+        dev = require_device(*(w for b in blocks for w in b))
+        for b in blocks:
+            if len(b) != 6 or any(not _plain_f32(w, dev) or w.shape != shape for w, shape in
+                                  zip(b, ((128, 128), (512, 128), (128, 512)) + ((128, 128),) * 3)):
+                raise _lib.CrystalformerHipError("PackedBlocks: contiguous float32 weights of 128-wide blocks with 512 "
+                                                 "hidden units expected")
+        lib = _lib.load()
+        L = len(blocks)
+        self.floats = int(lib.cf_pack_blocks_floats(1))
+        self.forward = torch.empty(L * self.floats, dtype=torch.float32, device=dev)
+        self.backward = torch.empty(L * self.floats, dtype=torch.float32, device=dev)
+        self.counters = torch.empty(L, dtype=torch.int32, device=dev)
+        table = (ctypes.c_void_p * (6 * L))(*[w.data_ptr() for b in blocks for w in b])
+        with device_guard(dev):
+            rc = lib.cf_pack_blocks(L, table, ptr(self.forward), ptr(self.backward), ptr(self.counters), L,
+                                    stream_handle(dev))
+        check(rc, "cf_pack_blocks")
+
+    def block(self, index: int):
+        """(forward, backward, counter) of a block."""
+        n = self.floats
+        return (self.forward[index * n:(index + 1) * n], self.backward[index * n:(index + 1) * n],
+                self.counters[index:index + 1])
+
+
+def block_head(x: Tensor, heads: int, packed: Tensor, counter: Tensor, b_in: Optional[Tensor], w_pos: Tensor,
+               gauss_scale: Tensor, normalize: bool, update_stats: bool, positive_func: str, beta: float,
+               lower_bound: float, coef: float, q_scale: float):
+    """Query, key and value projections and the Gaussian exponents of a 128-wide block in one launch:
+    ``(a, qs, k, v, q, alpha_n, used)`` as :func:`linear_rows` and :func:`gauss_exponents` give them."""
+    dev = require_device(x, packed, b_in, w_pos, gauss_scale)
+    N, W = x.shape
+    if W != 128 or not _plain_f32(x, dev) or positive_func not in POSITIVE_FUNCS or w_pos.numel() != W \
+            or not _plain_f32(w_pos, dev) or not _plain_f32(gauss_scale, dev) or gauss_scale.numel() != 2 \
+            or not (b_in is None or (_plain_f32(b_in, dev) and b_in.numel() == 3 * W)):
+        raise _lib.CrystalformerHipError("block_head: contiguous float32 rows of 128 and their block's parameters expected")
+    lib = _lib.load()
+    q, qs, k, v = torch.empty((4, N, W), dtype=torch.float32, device=dev).unbind(0)
+    a, alpha_n = torch.empty((2, N, heads), dtype=torch.float32, device=dev).unbind(0)
+    used = torch.empty(2, dtype=torch.float32, device=dev) if normalize else None
+    part = torch.empty(int(lib.cf_gauss_exponents_workspace(N, heads)) // 4, dtype=torch.float32,
+                       device=dev) if normalize else None
+    with device_guard(dev):
+        rc = lib.cf_block_head(x.data_ptr(), N, heads, ptr(packed), ptr(b_in), ptr(w_pos), ptr(gauss_scale),
+                               int(bool(normalize)), int(bool(update_stats)), POSITIVE_FUNCS[positive_func], float(beta),
+                               float(lower_bound), float(coef), float(q_scale), ptr(part), ptr(counter), ptr(q), ptr(qs),
+                               ptr(k), ptr(v), ptr(a), ptr(alpha_n), ptr(used), stream_handle(dev))
+    check(rc, "cf_block_head")
+    return a, qs, k, v, q, alpha_n, used
+
+
+def block_head_bwd(ga, gqs, gk, gv, carry, q: Tensor, w_pos: Tensor, alpha_n: Tensor, used: Optional[Tensor],
+                   packed_bwd: Tensor, positive_func: str, beta: float, lower_bound: float, coef: float, q_scale: float):
+    """(gq, gx, gw_pos) from the gradients of :func:`block_head`'s ``a``, ``qs``, ``k``, ``v`` and of the input's other
+    uses (``carry``), None where there is none."""
+    dev = require_device(ga, gqs, gk, gv, carry, q, packed_bwd)
+    ga, gqs, gk, gv, carry = (_f32(t, "gradient") for t in (ga, gqs, gk, gv, carry))
+    N, W = q.shape
+    lib = _lib.load()
+    gq, gx = torch.empty((2, N, W), dtype=torch.float32, device=dev).unbind(0)
+    gw = torch.empty(W, dtype=torch.float32, device=dev) if ga is not None else None
+    g_alpha = torch.empty_like(alpha_n)
+    with device_guard(dev):
+        rc = lib.cf_block_head_bwd(ptr(ga), ptr(gqs), ptr(gk), ptr(gv), ptr(carry), ptr(q), ptr(w_pos), ptr(alpha_n),
+                                   ptr(used), N, alpha_n.shape[1], ptr(packed_bwd), POSITIVE_FUNCS[positive_func],
+                                   float(beta), float(lower_bound), float(coef), float(q_scale), ptr(g_alpha), ptr(gq),
+                                   ptr(gx), ptr(gw), stream_handle(dev))
+    check(rc, "cf_block_head_bwd")
+    return gq, gx, gw
+
+
+def block_tail(att: Tensor, x: Tensor, packed: Tensor, bo: Optional[Tensor], b1: Optional[Tensor],
+               b2: Optional[Tensor]) -> Tuple[Tensor, Tensor, Tensor]:
+    """(y, s, h): output projection with the residual ``x`` (s), hidden units (h) and the block's output of a
+    128-wide block with 512 hidden units, in one launch."""
+    dev = require_device(att, x, packed, bo, b1, b2)
+    N, W = x.shape
+    if W != 128 or att.shape != x.shape or not _plain_f32(x, dev) or not _plain_f32(att, dev) or any(
+            b is not None and (not _plain_f32(b, dev) or b.numel() != n) for b, n in ((bo, W), (b1, 512), (b2, W))):
+        raise _lib.CrystalformerHipError("block_tail: contiguous float32 rows of 128 and their block's biases expected")
+    s, y = torch.empty((2, N, W), dtype=torch.float32, device=dev).unbind(0)
+    h = torch.empty((N, 512), dtype=torch.float32, device=dev)
+    with device_guard(dev):
+        rc = _lib.load().cf_block_tail(ptr(att), ptr(x), N, ptr(packed), ptr(bo), ptr(b1), ptr(b2), ptr(s), ptr(h), ptr(y),
+                                       stream_handle(dev))
+    check(rc, "cf_block_tail")
+    return y, s, h
+
+
+def block_tail_bwd(gy: Tensor, h: Tensor, packed_bwd: Tensor) -> Tuple[Tensor, Tensor, Tensor]:
+    """(gh, gs, gatt): gradients of :func:`block_tail`'s hidden units (before the ReLU), of s and of att."""
+    dev = require_device(gy, h, packed_bwd)
+    gy = _f32(gy, "gy")
+    N, W = gy.shape
+    gs, gatt = torch.empty((2, N, W), dtype=torch.float32, device=dev).unbind(0)
+    gh = torch.empty_like(h)
+    with device_guard(dev):
+        rc = _lib.load().cf_block_tail_bwd(ptr(gy), ptr(h), N, ptr(packed_bwd), ptr(gh), ptr(gs), ptr(gatt),
+                                           stream_handle(dev))
+    check(rc, "cf_block_tail_bwd")
+    return gh, gs, gatt
+
+
 def linear_rows_supported(x: Tensor, *weights: Tensor) -> bool:
     """True when :func:`linear_rows` serves these operands (float32 on the GPU, input
     width a multiple of 16, equal weight shapes)."""

@@ -544,6 +544,39 @@ int cf_dense_rows(const int64_t *atom_start_n, const int64_t *edge_start_n, int6
                   void *stream);
 
 /*
+ * The row-wise parts of a 128-wide block with 512 hidden units as one launch each, forward and backward
+ * (models/indexed_lattice_multi_head_attention_cuda.py:636-722 and the encoder layer around it):
+ *   head   q, k, v = x W^T + b_in (split in three),  qs = q q_scale,  a = coef rho(norm(<q, w_pos>))  as cf_gauss_exponents
+ *   tail   s = att Wo^T + bo + x,  h = relu(s W1^T + b1),  y = h W2^T + b2 + s
+ * cf_pack_blocks puts the weights of `blocks` blocks (weights: HOST array of 6 device pointers per block: Wo, W1,
+ * W2, Wq, Wk, Wv) into the order the kernels read, cf_pack_blocks_floats(1) floats per block in `packed` and, for
+ * the backward calls, in `packed_bwd` (nullable), and clears `words` 32-bit words.  The other calls take the
+ * packed weights of their block.
+ *   counter   one of the cleared words;  part: cf_gauss_exponents_workspace(N, H) bytes
+ *   alpha_n, used (2 floats): nullable; q, s and h are for the backward calls
+ *   tail_bwd  gh = (gy W2) where h > 0,  gs = gh W1 + gy,  gatt = gs Wo
+ *   head_bwd  g_alpha (N,H) = ga da/dalpha,  gq = g_alpha w_pos + gqs q_scale,  gx = gq Wq + gk Wk + gv Wv + carry,  gw_pos (128);
+ *             ga, gqs, gk, gv, carry nullable (zero; without ga gw_pos is not written); the statistics are constants
+ * The sums are those of cf_linear_rows, cf_linear_rows_nn, cf_gauss_exponents and cf_gauss_exponents_bwd, in their
+ * order: results are the same to the bit.
+ */
+int64_t cf_pack_blocks_floats(int64_t blocks);
+int cf_pack_blocks(int64_t blocks, const float *const *weights, float *packed, float *packed_bwd, int32_t *zero_words,
+                   int64_t words, void *stream);
+int cf_block_head(const float *x, int64_t N, int64_t H, const float *packed, const float *b_in, const float *w_pos,
+                  float *gauss_scale, int normalize, int update_stats, int positive_func, float beta, float lower_bound,
+                  float coef, float q_scale, float *part, int32_t *counter, float *q, float *qs, float *k, float *v,
+                  float *a, float *alpha_n, float *used, void *stream);
+int cf_block_tail(const float *att, const float *x, int64_t N, const float *packed, const float *bo, const float *b1,
+                  const float *b2, float *s, float *h, float *y, void *stream);
+int cf_block_tail_bwd(const float *gy, const float *h, int64_t N, const float *packed_bwd, float *gh, float *gs, float *gatt,
+                      void *stream);
+int cf_block_head_bwd(const float *ga, const float *gqs, const float *gk, const float *gv, const float *carry,
+                      const float *q, const float *w_pos, const float *alpha_n, const float *used, int64_t N, int64_t H,
+                      const float *packed_bwd, int positive_func, float beta, float lower_bound, float coef, float q_scale,
+                      float *g_alpha, float *gq, float *gx, float *gw_pos, void *stream);
+
+/*
  * Reciprocal-space periodic encoding (ReciPeriodicEncodingFuncCUDA, models/cuda_funcs/reci_space_enc.py:17-99;
  * kernels models/kernels/reci_enc_fwd.cu:3-68, reci_enc_bwd.cu:3-71), LATTICE_RANGE passed at run time:
  *   S[e,h] = sum over n1 in [0,R] (weight 2 for n1 != 0), n2, n3 in [-R,R] of

@@ -41,6 +41,12 @@ bool use_rings(const cf_forward_args &f, int64_t U)
     return edge * edge * edge <= 128 && cf_real_enc_ring_bytes(U) <= f.ring_limit_bytes;
 }
 
+// Adaptive boxes from staged rings are three launches, of which the range rule per pair and the two lists cost 8.5 us
+// whatever the batch; the pair kernel, which stages for itself, is one.  From three rounds of the whole chip on (a
+// unit per wavefront, 16 a CU) the rings' cheaper rounds make up for it: with all pairs in the cube 18 against 21 us at
+// 4.1 thousand pairs, 33 against 32.5 at 12.7, 61 against 52 at 29; with fewer in the cube the pair kernel gains.
+bool adaptive_rings_pay(int64_t U) { return U > 48 * (int64_t)device_cu_count(); }
+
 // Whether everything between two attentions runs as one launch.
 bool use_rows(const cf_forward_args &f) { return block_rows_served(f.width, f.ff, f.H); }
 
@@ -193,7 +199,7 @@ extern "C" int cf_forward(const cf_forward_args *f_, const cf_forward_block *blo
         const bool adaptive = rvlen != nullptr;
         const bool split = p.coef_reci != 0.0;                  // real space: the first half of the heads
         const int64_t HR = split ? H / 2 : H;
-        if (p.bins > 0 && b.rings && (!adaptive || (f.adaptive_rings && HR <= 8))) {
+        if (p.bins > 0 && b.rings && (!adaptive || (f.adaptive_rings && HR <= 8 && adaptive_rings_pay(U)))) {
             if (!staged || staged->bins != p.bins || staged->dist_max != p.dist_max || staged->wscale != p.wscale ||
                 staged->weakest != p.weakest) {
                 if ((rc = cf_real_enc_ring_stage(b.rpos, f.tvecs, f.pairs, U, p.bins, p.dist_max, p.wscale,

@@ -105,9 +105,14 @@ def _block(layer: nn.Module, width: int, device_index: int):
     return fields, H, ff
 
 
-def _backward_hooked(module: nn.Module) -> bool:
-    return bool(module._backward_hooks or module._backward_pre_hooks) or \
-        any(c is not None and _backward_hooked(c) for c in module._modules.values())
+def _watched(module: nn.Module) -> bool:
+    """A hook of any kind on the module or one below it."""
+    if module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks:
+        return True
+    for child in module._modules.values():
+        if child is not None and _watched(child):
+            return True
+    return False
 
 
 def pack_for_training(encoder: nn.Module, src: Tensor) -> Optional["ops.PackedBlocks"]:
@@ -123,7 +128,7 @@ def pack_for_training(encoder: nn.Module, src: Tensor) -> Optional["ops.PackedBl
     blocks = []
     for layer in encoder._modules["layers"]._modules.values():
         mods = layer._modules
-        if any(c is not None and (_any_hooked(c) or _backward_hooked(c)) for c in mods.values()):
+        if any(c is not None and _watched(c) for c in mods.values()):
             return None
         got = _block(layer, 128, src.get_device())
         if got is None or got[2] != 512 or layer.self_attn.params.domain != "real" or 128 // got[1] % 4:

@@ -69,6 +69,18 @@ def test_native_forward_equals_the_modules(dev, sizes, options):
     assert_close(native, modules, "encoder, stored statistics", rtol=RTOL, atol=atol_rows(modules))
 
 
+def test_adaptive_boxes_either_side_of_the_staged_rings(dev):
+    """Below three rounds of the chip the blocks stage for themselves, above they share staged rings: both are the
+    module path's results, which always uses the rings."""
+    per_round = 16 * torch.cuda.get_device_properties(0).multi_processor_count
+    for units in (3 * per_round - 10, 3 * per_round, 3 * per_round + 10):
+        crystals, rest = divmod(units, 16 * 17 // 2)
+        b = batch_of([16] * crystals + [1] * rest).to(dev)
+        model = scaled(default_params(num_layers=2)).to(dev).eval()
+        native, modules = both_ways(model, b)
+        assert_close(native, modules, str(units), rtol=RTOL, atol=atol_rows(modules))
+
+
 @pytest.mark.parametrize("options", [dict(), dict(targets=["a", "b", "c"]), dict(embedding_dim=[128, 64]),
                                      dict(pre_pooling_op="w+relu", embedding_dim=[128, 128])])
 def test_native_forward_with_its_head(dev, options):

@@ -42,6 +42,16 @@ struct PackArgs {
 };
 int launch_pack_weights(const PackArgs &p, hipStream_t st);
 
+struct PrologueArgs {
+    int64_t B, E;
+    const int64_t *atom_start, *edge_start;
+    const float *pos, *trans;
+    float *rpos, *vcell, *recip, *rvlen;      // vcell, recip nullable
+    const int64_t *live_E;                    // set by the launcher
+};
+// packing, edge offsets (cf_edge_index) and lattice geometry (cf_lattice_geometry) at once
+int launch_forward_prologue(const PackArgs &k, PrologueArgs p, hipStream_t st);
+
 struct TailBwdArgs {
     int64_t N;
     const float *gy, *h, *packed;
@@ -75,8 +85,5 @@ bool dpa_streams(int64_t N, int64_t H, int64_t E, int64_t D);
 int launch_dpa_inference(const float *que, const float *key, const float *val, const float *aij, int64_t aij_second,
                          const float *bij, const int64_t *edges, const int64_t *e_start, int64_t N, int64_t H, int64_t E,
                          int64_t D, float *out, hipStream_t st);
-// cf_lattice_geometry that also clears `words` 32-bit words at `zero` (counters of later launches).
-int launch_lattice_geometry(const float *trans, int64_t B, float *vcell, float *recip, float *rvlen, unsigned *zero,
-                            int words, hipStream_t st);
 
 }  // namespace cf

@@ -5,57 +5,18 @@
 //     normalisation over the batch, the positive map and the final
 //     a = -rho / (2 r0^2), plus the scaled query for the attention.
 #include "cf_common.h"
-#include "block_rows.h"
 #include "gauss_maps.h"
+#include "lattice_geometry.h"
 
 namespace {
 
 using namespace cf;
 
-// One thread per crystal.  Products and sums are kept un-contracted and in the
-// term order of models/indexed_latticeformer_encoder.py:34-44 so the volume is
-// the one the stock elementwise expression gives.
 __global__ void lattice_geometry_kernel(const float *trans, int64_t B, float *vcell, float *recip,
-                                        float *rvlen, unsigned *zero, int words)
+                                        float *rvlen)
 {
-#pragma clang fp contract(off)
-    if (blockIdx.x == 0)
-        for (int w = threadIdx.x; w < words; w += blockDim.x) zero[w] = 0u;
     const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= B) return;
-    const float *m = trans + b * 9;
-    const float m00 = m[0], m01 = m[1], m02 = m[2];
-    const float m10 = m[3], m11 = m[4], m12 = m[5];
-    const float m20 = m[6], m21 = m[7], m22 = m[8];
-    float det = m00 * m11 * m22;
-    det = det + m01 * m12 * m20;
-    det = det + m02 * m10 * m21;
-    det = det - m02 * m11 * m20;
-    det = det - m00 * m12 * m21;
-    det = det - m01 * m10 * m22;
-    if (vcell) vcell[b] = det;
-    // b1 = 2 pi (a2 x a3) / V and cyclic (models/indexed_latticeformer_encoder.py:206-212)
-    const float s = (1.0f / det) * 6.283185307179586f;
-    float c[9];
-    c[0] = m11 * m22 - m12 * m21;
-    c[1] = m12 * m20 - m10 * m22;
-    c[2] = m10 * m21 - m11 * m20;
-    c[3] = m21 * m02 - m22 * m01;
-    c[4] = m22 * m00 - m20 * m02;
-    c[5] = m20 * m01 - m21 * m00;
-    c[6] = m01 * m12 - m02 * m11;
-    c[7] = m02 * m10 - m00 * m12;
-    c[8] = m00 * m11 - m01 * m10;
-#pragma unroll
-    for (int r = 0; r < 3; r++) {
-        const float x = c[3 * r] * s, y = c[3 * r + 1] * s, z = c[3 * r + 2] * s;
-        if (recip) {
-            recip[b * 9 + 3 * r] = x;
-            recip[b * 9 + 3 * r + 1] = y;
-            recip[b * 9 + 3 * r + 2] = z;
-        }
-        if (rvlen) rvlen[b * 3 + r] = sqrtf(x * x + y * y + z * z);
-    }
+    if (b < B) lattice_geometry_of(trans, b, vcell, recip, rvlen);
 }
 
 // ---- Gaussian exponents -----------------------------------------------------
@@ -349,16 +310,6 @@ extern "C" int cf_gauss_exponents_bwd(const float *ga, const float *gqs, const f
     return CF_OK;
 }
 
-int cf::launch_lattice_geometry(const float *trans, int64_t B, float *vcell, float *recip, float *rvlen, unsigned *zero,
-                                int words, hipStream_t st)
-{
-    const int threads = 128;
-    lattice_geometry_kernel<<<(int)((B + threads - 1) / threads), threads, 0, st>>>(trans, B, vcell, recip, rvlen, zero,
-                                                                                    words);
-    CF_CHECK_LAUNCH("cf_lattice_geometry");
-    return CF_OK;
-}
-
 extern "C" int cf_lattice_geometry(const float *trans, int64_t B, float *vcell, float *recip, float *rvlen,
                                    void *stream)
 {
@@ -366,7 +317,11 @@ extern "C" int cf_lattice_geometry(const float *trans, int64_t B, float *vcell, 
     if (B == 0) return CF_OK;
     CF_REQUIRE(trans, CF_ERR_INVALID_ARGUMENT, "cf_lattice_geometry: trans is NULL");
     CF_REQUIRE(vcell || recip || rvlen, CF_ERR_INVALID_ARGUMENT, "cf_lattice_geometry: no output requested");
-    return cf::launch_lattice_geometry(trans, B, vcell, recip, rvlen, nullptr, 0, (hipStream_t)stream);
+    const int threads = 128;
+    lattice_geometry_kernel<<<(int)((B + threads - 1) / threads), threads, 0, (hipStream_t)stream>>>(trans, B, vcell, recip,
+                                                                                                     rvlen);
+    CF_CHECK_LAUNCH("cf_lattice_geometry");
+    return CF_OK;
 }
 
 extern "C" int64_t cf_gauss_exponents_workspace(int64_t N, int64_t H)

@@ -153,14 +153,6 @@ extern "C" int cf_forward(const cf_forward_args *f_, const cf_forward_block *blo
     const int64_t N = f.N, E = f.E, U = (N + E) / 2, W = f.width, H = f.H, D = W / H;
     const bool adaptive_any = f.adaptive != 0;
     const bool rows = use_rows(f);
-    if ((rc = launch_lattice_geometry(f.tvecs, f.B, b.vcell, b.recip, b.rvlen, b.counters, (int)f.layers,
-                                      (hipStream_t)stream)))
-        return rc;
-    if ((rc = cf_edge_index(f.atom_start, f.edge_start, f.B, E, f.pos, nullptr, b.rpos, stream))) return rc;
-    if (b.kr && (rc = cf_kr_base(b.rpos, b.recip, f.batch, f.edges, E, b.kr, stream))) return rc;
-    const cf_forward_block *staged = nullptr;      // the block whose grid the rings in b.rings hold
-    const float *x = f.x;
-    int side = 0;
     if (rows) {
         for (int64_t first = 0; first < f.layers; first += PACK_BLOCKS) {
             PackArgs a{};
@@ -170,13 +162,29 @@ extern "C" int cf_forward(const cf_forward_args *f_, const cf_forward_block *blo
                 a.block[i] = PackSource{p.wo, p.w1, p.w2, p.wq, p.wk, p.wv};
             }
             a.packed = b.packed + first * PACKED_BLOCK;
-            if (first == 0 && f.w_embed) {
+            if (first > 0) {
+                if ((rc = launch_pack_weights(a, (hipStream_t)stream))) return rc;
+                continue;
+            }
+            if (f.w_embed) {
                 a.w_embed = f.w_embed;
                 a.embed_width = (int)f.embed_width;
                 a.packed_embed = b.packed + f.layers * PACKED_BLOCK;
             }
-            if ((rc = launch_pack_weights(a, (hipStream_t)stream))) return rc;
+            a.zero = b.counters;
+            a.words = (int)f.layers;
+            const PrologueArgs g{f.B, E, f.atom_start, f.edge_start, f.pos, f.tvecs, b.rpos, b.vcell, b.recip, b.rvlen, nullptr};
+            if ((rc = launch_forward_prologue(a, g, (hipStream_t)stream))) return rc;
         }
+    } else {
+        if ((rc = cf_lattice_geometry(f.tvecs, f.B, nullptr, nullptr, b.rvlen, stream))) return rc;
+        if ((rc = cf_edge_index(f.atom_start, f.edge_start, f.B, E, f.pos, nullptr, b.rpos, stream))) return rc;
+    }
+    if (b.kr && (rc = cf_kr_base(b.rpos, b.recip, f.batch, f.edges, E, b.kr, stream))) return rc;
+    const cf_forward_block *staged = nullptr;      // the block whose grid the rings in b.rings hold
+    const float *x = f.x;
+    int side = 0;
+    if (rows) {
         RowsArgs r{};
         r.N = N; r.H = (int)H; r.x = f.x;
         head_of(r, f, blocks[0], b, 0);

@@ -5,7 +5,7 @@
 //
 // for the 128-wide blocks with 512 hidden units; the embedding of the atoms can stand in front of the
 // first head.  As four linear launches and two for the exponents this was 6.6 and 4.5 us each at the 1.8
-// thousand rows of a batch, none of it arithmetic: 0.35 GFLOP a block take 2.2 us at the fp32 matrix rate.
+// thousand rows of a batch, most of it not arithmetic: 0.7 GFLOP a block take 4.8 us at the fp32 matrix rate.
 //
 // A work-group of 8 wavefronts owns 4 R rows; the rows and all intermediates stay in LDS, the weights
 // (786 KB a block) stream from the L2, a 16-column tile per wavefront, two tiles ahead of their use.  At 64

@@ -42,9 +42,10 @@ bool use_rings(const cf_forward_args &f, int64_t U)
 }
 
 // Adaptive boxes from staged rings are three launches, of which the range rule per pair and the two lists cost 8.5 us
-// whatever the batch; the pair kernel, which stages for itself, is one.  From three rounds of the whole chip on (a
-// unit per wavefront, 16 a CU) the rings' cheaper rounds make up for it: with all pairs in the cube 18 against 21 us at
-// 4.1 thousand pairs, 33 against 32.5 at 12.7, 61 against 52 at 29; with fewer in the cube the pair kernel gains.
+// whatever the batch; the pair kernel, which stages for itself, is one.  Against that the rings' rounds are cheaper: 11.2
+// for 14.7 us at 4.1 thousand pairs in the fixed cube, 21.7 for 28.4 at 12.7 thousand, and at 29 thousand with nearly all
+// pairs in the cube 52 for 61 with everything counted.  So the rings from three rounds of the whole chip on (a unit per
+// wavefront, 16 a CU).  Where many pairs leave the cube the pair kernel stays ahead: 36.6 for 45.5 us at 12.7 thousand.
 bool adaptive_rings_pay(int64_t U) { return U > 48 * (int64_t)device_cu_count(); }
 
 // Whether everything between two attentions runs as one launch.

@@ -69,14 +69,15 @@ def test_native_forward_equals_the_modules(dev, sizes, options):
     assert_close(native, modules, "encoder, stored statistics", rtol=RTOL, atol=atol_rows(modules))
 
 
-def test_adaptive_boxes_either_side_of_the_staged_rings(dev):
+@pytest.mark.parametrize("r0", [1.4, 3.0])               # nearly all pairs keep the cube; most leave it
+def test_adaptive_boxes_either_side_of_the_staged_rings(dev, r0):
     """Below three rounds of the chip the blocks stage for themselves, above they share staged rings: both are the
     module path's results, which always uses the rings."""
     per_round = 16 * torch.cuda.get_device_properties(0).multi_processor_count
-    for units in (3 * per_round - 10, 3 * per_round, 3 * per_round + 10):
+    for units in (3 * per_round - 10, 3 * per_round, 3 * per_round + 1, 3 * per_round + 127, 5 * per_round):
         crystals, rest = divmod(units, 16 * 17 // 2)
         b = batch_of([16] * crystals + [1] * rest).to(dev)
-        model = scaled(default_params(num_layers=2)).to(dev).eval()
+        model = scaled(default_params(num_layers=2, scale_real=[r0])).to(dev).eval()
         native, modules = both_ways(model, b)
         assert_close(native, modules, str(units), rtol=RTOL, atol=atol_rows(modules))
 

@@ -119,39 +119,72 @@ __device__ __forceinline__ void stage_rows(float *dst, const float *__restrict__
     }
 }
 
+// Raw exponents on their way to the work-group that finishes them: written through and read past the L2 of an XCD, so that
+// no work-group has to write back or invalidate a cache (a fence each cost 35 us a block in all).
+__device__ __forceinline__ void put_raw(float *p, float v)
+{
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ float get_raw(const float *p)
+{
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // The exponents where no statistics are stored: the last work-group to finish merges the statistics of
 // all raw values (a holds them) as the two exponent kernels do -- groups of 256 values, mean first, then
-// the squared deviations, groups merged by Chan's formula in the same order -- and maps them in place.
+// the squared deviations, groups merged by Chan's formula in the same order -- and maps them in place.  Up to
+// KEPT groups a wavefront it holds the values in registers meanwhile.
+constexpr int KEPT = 8;                      // (all values of 2048 atoms with 8 heads)
+
+__device__ __forceinline__ void group_statistics(const float (&v)[4], int64_t b, int64_t total, int lane, float *out)
+{
+    const float cnt = (float)min((int64_t)256, total - 256 * b);
+    float s[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) s[u] = wave_sum(v[u]);
+    const float mean = (((0.f + s[0]) + s[1]) + s[2] + s[3]) / cnt;
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+        const float dv = 256 * b + 64 * u + lane < total ? v[u] - mean : 0.f;
+        s[u] = wave_sum(dv * dv);
+    }
+    if (lane == 0) {
+        out[3 * b] = cnt;
+        out[3 * b + 1] = mean;
+        out[3 * b + 2] = ((0.f + s[0]) + s[1]) + s[2] + s[3];
+    }
+}
+
 __device__ void finish_exponents(const RowsArgs &p, int64_t total, float *red)
 {
+    constexpr int WAVES = RT / WAVE;
+    __shared__ float stats[3 * KEPT * WAVES];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int64_t blocks = (total + 255) / 256;
-    for (int64_t b = wave; b < blocks; b += RT / WAVE) {
-        float v[4], s[4];
-        const float cnt = (float)min((int64_t)256, total - 256 * b);
+    const bool kept = blocks <= KEPT * WAVES;
+    float v[KEPT][4];
+    auto fetch = [&](int64_t b0) {                              // this wavefront's groups b0 + wave, + 8, ...: 32 loads in flight
 #pragma unroll
-        for (int u = 0; u < 4; u++) {
-            const int64_t t = 256 * b + 64 * u + lane;
-            v[u] = t < total ? p.a[t] : 0.f;
-        }
+        for (int k = 0; k < KEPT; k++)
 #pragma unroll
-        for (int u = 0; u < 4; u++) s[u] = wave_sum(v[u]);
-        const float mean = (((0.f + s[0]) + s[1]) + s[2] + s[3]) / cnt;
+            for (int u = 0; u < 4; u++) {
+                const int64_t t = 256 * (b0 + wave + WAVES * k) + 64 * u + lane;
+                v[k][u] = t < total ? get_raw(p.a + t) : 0.f;
+            }
+    };
+    for (int64_t b0 = 0; b0 < blocks; b0 += KEPT * WAVES) {
+        fetch(b0);
 #pragma unroll
-        for (int u = 0; u < 4; u++) {
-            const float dv = 256 * b + 64 * u + lane < total ? v[u] - mean : 0.f;
-            s[u] = wave_sum(dv * dv);
-        }
-        if (lane == 0) {
-            p.part[3 * b] = cnt;
-            p.part[3 * b + 1] = mean;
-            p.part[3 * b + 2] = ((0.f + s[0]) + s[1]) + s[2] + s[3];
+        for (int k = 0; k < KEPT; k++) {
+            const int64_t b = b0 + wave + WAVES * k;
+            if (b < blocks) group_statistics(v[k], b, total, lane, kept ? stats : p.part);
         }
     }
     __syncthreads();
     if (wave == 0) {
         float n, mean, m2;
-        merge_statistics(p.part, (int)blocks, lane, n, mean, m2);
+        if (kept) merge_statistics(stats, (int)blocks, lane, n, mean, m2);
+        else merge_statistics(p.part, (int)blocks, lane, n, mean, m2);
         if (lane == 0) {
             const float scale = 1.0f / sqrtf(m2 / (n - 1.0f));
             red[0] = scale;
@@ -168,10 +201,20 @@ __device__ void finish_exponents(const RowsArgs &p, int64_t total, float *red)
     }
     __syncthreads();
     const float scale = red[0], shift = red[1];
-    for (int64_t t = threadIdx.x; t < total; t += RT) {
-        const float alpha = (p.a[t] + shift) * scale;
+    auto finish = [&](int64_t t, float raw) {
+        const float alpha = (raw + shift) * scale;
         if (p.alpha_n) p.alpha_n[t] = alpha;
         p.a[t] = positive_map(alpha, p.func, p.beta, p.lb) * (p.split && 2 * t >= total ? p.coef_second : p.coef);
+    };
+    for (int64_t b0 = 0; b0 < blocks; b0 += KEPT * WAVES) {
+        if (!kept) fetch(b0);
+#pragma unroll
+        for (int k = 0; k < KEPT; k++)
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const int64_t t = 256 * (b0 + wave + WAVES * k) + 64 * u + lane;
+                if (t < total) finish(t, v[k][u]);
+            }
     }
 }
 
@@ -180,14 +223,14 @@ __device__ void finish_if_last(const RowsArgs &p, int64_t N, int64_t tiles, floa
 {
     const int64_t active = min((int64_t)gridDim.x, tiles);
     if ((int64_t)blockIdx.x >= active) return;
-    __threadfence();
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");           // this wavefront's raw values have arrived
     __syncthreads();
     if (threadIdx.x == 0) red[0] = atomicAdd(p.counter, 1u) + 1u == (unsigned)active ? 1.f : 0.f;
     __syncthreads();
     const bool last = red[0] != 0.f;
     __syncthreads();
     if (last) {
-        __threadfence();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
         finish_exponents(p, N * p.H, red);
     }
 }
@@ -423,9 +466,12 @@ __global__ __launch_bounds__(RT) void block_rows_kernel(RowsArgs p)
                 const bool second = p.split && h >= half;
                 if (!p.normalize || stored)
                     alpha = positive_map(alpha, p.func, p.beta, p.lb) * (second ? p.coef_second : p.coef);
-                if (row0 + r < N)
-                    p.a[p.split ? (second ? N : 0) * half + (row0 + r) * half + h - (second ? half : 0)
-                                : (row0 + r) * p.H + h] = alpha;
+                if (row0 + r < N) {
+                    float *out = p.a + (p.split ? (second ? N : 0) * half + (row0 + r) * half + h - (second ? half : 0)
+                                                : (row0 + r) * p.H + h);
+                    if (stored) *out = alpha;
+                    else put_raw(out, alpha);
+                }
             }
         }
         __syncthreads();                                        // the next tile overwrites the rows
@@ -594,9 +640,10 @@ __global__ __launch_bounds__(RT) void block_head_train_kernel(RowsArgs p)
         if (p.normalize && stored) alpha = (alpha + shift) * scale;
         if (!p.normalize || stored) {
             if (p.alpha_n) p.alpha_n[at] = alpha;
-            alpha = positive_map(alpha, p.func, p.beta, p.lb) * p.coef;
+            p.a[at] = positive_map(alpha, p.func, p.beta, p.lb) * p.coef;
+        } else {
+            put_raw(p.a + at, alpha);
         }
-        p.a[at] = alpha;
     }
     if (!stored) finish_if_last(p, N, (N + TM - 1) / TM, red);
 }

@@ -133,7 +133,11 @@ __device__ __forceinline__ float get_raw(const float *p)
 // The exponents where no statistics are stored: the last work-group to finish merges the statistics of
 // all raw values (a holds them) as the two exponent kernels do -- groups of 256 values, mean first, then
 // the squared deviations, groups merged by Chan's formula in the same order -- and maps them in place.  Up to
-// KEPT groups a wavefront it holds the values in registers meanwhile.
+// KEPT groups a wavefront it holds the values in registers meanwhile.  An inference forward of more rows has them
+// mapped by a launch of its own (apart): the map alone keeps one work-group busy for 26 us at 8 thousand atoms
+// (seven blocks 4243 us, with the launch 4061).  With stored statistics that launch ends at once, 1% of such a forward;
+// a capacity, whose live rows are mostly fewer, and training, which has stored statistics from its second step on, do
+// without it.
 constexpr int KEPT = 8;                      // (all values of 2048 atoms with 8 heads)
 
 __device__ __forceinline__ void group_statistics(const float (&v)[4], int64_t b, int64_t total, int lane, float *out)
@@ -189,6 +193,10 @@ __device__ void finish_exponents(const RowsArgs &p, int64_t total, float *red)
             const float scale = 1.0f / sqrtf(m2 / (n - 1.0f));
             red[0] = scale;
             red[1] = -mean;
+            if (p.apart) {                                      // (the groups' statistics are merged)
+                p.part[0] = scale;
+                p.part[1] = -mean;
+            }
             if (p.used) {
                 p.used[0] = scale;
                 p.used[1] = -mean;
@@ -199,6 +207,7 @@ __device__ void finish_exponents(const RowsArgs &p, int64_t total, float *red)
             }
         }
     }
+    if (p.apart) return;
     __syncthreads();
     const float scale = red[0], shift = red[1];
     auto finish = [&](int64_t t, float raw) {
@@ -232,6 +241,21 @@ __device__ void finish_if_last(const RowsArgs &p, int64_t N, int64_t tiles, floa
     if (last) {
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
         finish_exponents(p, N * p.H, red);
+    }
+}
+
+constexpr int FINISH_T = 256, FINISH_VALUES = 4 * FINISH_T;
+__global__ __launch_bounds__(FINISH_T) void finish_exponents_kernel(RowsArgs p)
+{
+    if (*p.counter == 0) return;                                // stored statistics: mapped already
+    const int64_t total = p.N * p.H;
+    const float scale = p.part[0], shift = p.part[1];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+        const int64_t t = (int64_t)blockIdx.x * FINISH_VALUES + u * FINISH_T + threadIdx.x;
+        if (t < total)
+            p.a[t] = positive_map((p.a[t] + shift) * scale, p.func, p.beta, p.lb) *
+                     (p.split && 2 * t >= total ? p.coef_second : p.coef);
     }
 }
 
@@ -908,10 +932,15 @@ int launch_block_rows(RowsArgs p, hipStream_t st)
     int64_t grid = (p.N + 4 * R - 1) / (4 * R);
     if (p.live_N && grid > 2 * cus) grid = 2 * cus;             // a capacity: stride over the tiles that exist
     CF_REQUIRE(grid < (1ll << 31), CF_ERR_UNSUPPORTED, "block rows: too many atoms");
+    p.apart = head && p.normalize && !p.live_N && p.N * p.H > 256 * KEPT * (RT / WAVE);
     if (R == 1) launch_rows<1>(p, source, head, (unsigned)grid, st);
     else if (R == 2) launch_rows<2>(p, source, head, (unsigned)grid, st);
     else launch_rows<4>(p, source, head, (unsigned)grid, st);
     CF_CHECK_LAUNCH("block rows");
+    if (p.apart) {
+        finish_exponents_kernel<<<(unsigned)((p.N * p.H + FINISH_VALUES - 1) / FINISH_VALUES), FINISH_T, 0, st>>>(p);
+        CF_CHECK_LAUNCH("block rows: exponents");
+    }
     return CF_OK;
 }
 

@@ -129,6 +129,18 @@ def test_row_kernel_tiles_against_float64(dev, atoms):
     assert_close(y, ref.float(), "head", rtol=RTOL)
 
 
+@pytest.mark.parametrize("domain", ["real", "multihead"])
+@pytest.mark.parametrize("atoms", [2040, 2048, 2049, 2100, 5000])   # 64 groups of 256 exponents are kept in registers
+def test_batch_statistics_of_many_atoms(dev, atoms, domain):
+    """Exponents under the batch's own statistics, finished by one work-group or by a launch of their own."""
+    sizes = [8] * (atoms // 8) + ([atoms % 8] if atoms % 8 else [])
+    model = scaled(default_params(num_layers=3, value_pe_dist_real=0, domain=domain, adaptive_cutoff_sigma=0.0))
+    model = model.to(dev).eval()
+    b = batch_of(sizes).to(dev)
+    native, modules = both_ways(model, b)
+    assert_close(native, modules, "encoder", rtol=RTOL, atol=atol_rows(modules))
+
+
 def test_training_mode_without_gradients_stores_the_statistics(dev):
     cfg = default_params(num_layers=2)
     one, two = scaled(cfg).to(dev).train(), scaled(cfg).to(dev).train()

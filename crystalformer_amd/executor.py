@@ -166,7 +166,7 @@ def _head(mlp: nn.Module, width: int, device_index: int) -> Optional[Tuple[tuple
 def _embeds(model: nn.Module, x: Tensor):
     """Whether the native call can embed the atoms itself: a plain, unhooked projection of contiguous rows into
     the one block width that has the kernel, without autocast (which would run it in another type)."""
-    embed = model._modules["input_embeddings"]
+    embed = model._modules.get("input_embeddings")
     layers = model._modules["encoder"]._modules["layers"]
     return (type(embed) is nn.Linear and not _hooked(embed) and embed.out_features == 128 and len(layers) > 0
             and getattr(layers[0], "linear1", None) is not None and layers[0].linear1.out_features == 512
@@ -239,18 +239,23 @@ def encode(encoder: nn.Module, src: Tensor, pos: Tensor, batch: Tensor, trans: T
 
 def forward(model: nn.Module, data) -> Tuple[Optional[Tensor], Optional[Tensor]]:
     """The output of ``Latticeformer.forward``, or None and the embedded atoms if they are there already."""
+    from .encoder import CrystalformerEncoderCUDA
     if torch.is_grad_enabled():
         return None, None
     mods = model._modules
-    if type(mods["proj_before_pooling"]) is not nn.Identity or model.pooling_layer is not pooling.avr_pool \
-            or _hooked(mods["proj_before_pooling"]) or _any_hooked(mods["mlp"]):
+    encoder, proj = mods.get("encoder"), mods.get("proj_before_pooling")
+    # (an encoder of another class, or with a forward of its own, computes something else than its layers say)
+    if type(encoder) is not CrystalformerEncoderCUDA or "forward" in encoder.__dict__:
+        return None, None
+    if type(proj) is not nn.Identity or model.pooling_layer is not pooling.avr_pool \
+            or _hooked(proj) or _any_hooked(mods["mlp"]):
         return None, None
     x = data.x
-    head = _head(mods["mlp"], mods["encoder"].d_model, x.get_device())
+    head = _head(mods["mlp"], encoder.d_model, x.get_device())
     if head is None:
         return None, None
     where = data.pos, data.batch, data.trans_vec, data.sizes, head
     if _embeds(model, x):
-        return _run(mods["encoder"], x, *where, mods["input_embeddings"]), None
+        return _run(encoder, x, *where, mods["input_embeddings"]), None
     x = hip_funcs.linear(x, model.input_embeddings.weight, model.input_embeddings.bias)
-    return _run(mods["encoder"], x, *where), x
+    return _run(encoder, x, *where), x

@@ -1,0 +1,90 @@
+"""Which models, batches and settings the native inference call is chosen for, on the CPU (the call itself is
+replaced by a marker), and on the GPU that everything it leaves alone computes what its modules say."""
+import pytest
+import torch
+from torch import nn
+
+from crystalformer_amd import executor
+from crystalformer_amd.encoder import CrystalformerEncoderCUDA
+from crystalformer_amd.latticeformer import Latticeformer, default_params
+from crystalformer_amd.synthetic import make_batch
+from tests.helpers import RTOL, assert_close
+
+
+def small_model(**options):
+    torch.manual_seed(2)
+    model = Latticeformer(default_params(num_layers=2, **options)).eval()
+    with torch.no_grad():
+        model.input_embeddings.weight.normal_()            # (the initialisation's features are near zero)
+        for layer in model.encoder.layers:                 # trained: stored statistics
+            layer.self_attn.gauss_scale.copy_(torch.tensor([0.7, -0.2]))
+    return model
+
+
+def small_batch():
+    return make_batch(3, (4, 9), False, (3.0, 11.0), (65.0, 115.0), seed=3)
+
+
+@pytest.fixture
+def natively(monkeypatch):
+    """Whether a model's forward would take the native call: ``_run`` answers with a marker."""
+    marker = torch.zeros(())
+    monkeypatch.setattr(executor, "_run", lambda *args: marker)
+
+    def ask(model):
+        with torch.no_grad():
+            return executor.forward(model, small_batch())[0] is marker
+    assert ask(small_model())
+    return ask
+
+
+def same_with_and_without_gradients(model, dev):
+    """Under ``no_grad`` the model computes what it computes with gradients enabled, which is module by module."""
+    model, b = model.to(dev), small_batch().to(dev)
+    with torch.no_grad():
+        got = model(b)
+    assert_close(got, model(b).detach(), "model", rtol=RTOL)
+    return got
+
+
+class HalvingEncoder(CrystalformerEncoderCUDA):
+    def forward(self, *args):
+        return super().forward(*args) * 0.5
+
+
+class ForeignEncoder(nn.Module):                           # (no layers, no d_model)
+    def __init__(self, width=128):
+        super().__init__()
+        self.proj = nn.Linear(width, width)
+
+    def forward(self, src, pos, batch, trans, sizes, onehot=None):
+        return self.proj(src)
+
+
+def subclassed_encoder(model):
+    model.encoder.__class__ = HalvingEncoder
+
+
+def foreign_encoder(model):
+    model.encoder = ForeignEncoder()
+
+
+def replaced_forward(model):
+    plain = model.encoder.forward
+    model.encoder.forward = lambda *args: plain(*args) * 0.5
+
+
+@pytest.mark.parametrize("change", [subclassed_encoder, foreign_encoder, replaced_forward])
+def test_encoders_of_the_users_own(natively, change):
+    model = small_model()
+    change(model)
+    assert not natively(model)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("change", [subclassed_encoder, foreign_encoder, replaced_forward])
+def test_encoders_of_the_users_own_are_called(dev, change):
+    model = small_model()
+    plain = same_with_and_without_gradients(small_model(), dev)
+    change(model)
+    assert not torch.equal(same_with_and_without_gradients(model, dev), plain)

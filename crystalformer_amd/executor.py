@@ -240,18 +240,20 @@ def encode(encoder: nn.Module, src: Tensor, pos: Tensor, batch: Tensor, trans: T
 def forward(model: nn.Module, data) -> Tuple[Optional[Tensor], Optional[Tensor]]:
     """The output of ``Latticeformer.forward``, or None and the embedded atoms if they are there already."""
     from .encoder import CrystalformerEncoderCUDA
+    from .latticeformer import Latticeformer, is_plain_head
     if torch.is_grad_enabled():
         return None, None
     mods = model._modules
-    encoder, proj = mods.get("encoder"), mods.get("proj_before_pooling")
+    encoder, proj, mlp = mods.get("encoder"), mods.get("proj_before_pooling"), mods.get("mlp")
     # (an encoder of another class, or with a forward of its own, computes something else than its layers say)
     if type(encoder) is not CrystalformerEncoderCUDA or "forward" in encoder.__dict__:
         return None, None
     if type(proj) is not nn.Identity or model.pooling_layer is not pooling.avr_pool \
-            or _hooked(proj) or _any_hooked(mods["mlp"]):
+            or _hooked(proj) or not is_plain_head(mlp) or _any_hooked(mlp) \
+            or type(model)._head is not Latticeformer._head or "_head" in model.__dict__:
         return None, None
     x = data.x
-    head = _head(mods["mlp"], encoder.d_model, x.get_device())
+    head = _head(mlp, encoder.d_model, x.get_device())
     if head is None:
         return None, None
     where = data.pos, data.batch, data.trans_vec, data.sizes, head

@@ -38,6 +38,12 @@ def default_params(**overrides) -> SimpleNamespace:
     return SimpleNamespace(**cfg)
 
 
+def is_plain_head(mlp) -> bool:
+    """Whether a regression head is its children one after the other: a Sequential without a forward of its own."""
+    return isinstance(mlp, nn.Sequential) and type(mlp).forward is nn.Sequential.forward \
+        and "forward" not in mlp.__dict__
+
+
 class Latticeformer(nn.Module):
     def __init__(self, params):
         super().__init__()
@@ -130,6 +136,8 @@ class Latticeformer(nn.Module):
         norm layers is one row-block launch instead of a library GEMM plus elementwise launches."""
         from . import ops
         from .attention import inference_only
+        if not is_plain_head(self.mlp):
+            return self.mlp(x)
         mods = list(self.mlp)
         plain = all(isinstance(m, (nn.Linear, nn.ReLU, nn.Identity)) for m in mods)
         if not (plain and x.is_cuda and inference_only(x, self.mlp.parameters)):

@@ -88,3 +88,69 @@ def test_encoders_of_the_users_own_are_called(dev, change):
     plain = same_with_and_without_gradients(small_model(), dev)
     change(model)
     assert not torch.equal(same_with_and_without_gradients(model, dev), plain)
+
+
+class Residual(nn.Module):                                 # (the children of the usual head, used differently)
+    def __init__(self):
+        super().__init__()
+        torch.manual_seed(4)
+        self.a, self.r, self.b = nn.Linear(128, 128), nn.ReLU(), nn.Linear(128, 1)
+
+    def forward(self, x):
+        return self.b(x + self.r(self.a(x)))
+
+
+class ResidualSequential(nn.Sequential):
+    def __init__(self):
+        torch.manual_seed(4)
+        super().__init__(nn.Linear(128, 128), nn.ReLU(), nn.Linear(128, 1))
+
+    def forward(self, x):
+        return self[2](x + self[1](self[0](x)))
+
+
+class DoublingModel(Latticeformer):
+    def _head(self, x):
+        return super()._head(x) * 2.0
+
+
+def residual_head(model):
+    model.mlp = Residual()
+
+
+def residual_sequential_head(model):
+    model.mlp = ResidualSequential()
+
+
+def residual_instance_head(model):
+    model.mlp = nn.Sequential(*ResidualSequential())
+    model.mlp.forward = ResidualSequential.forward.__get__(model.mlp)
+
+
+def overridden_head(model):
+    model.__class__ = DoublingModel
+
+
+HEADS = [residual_head, residual_sequential_head, residual_instance_head, overridden_head]
+
+
+@pytest.mark.parametrize("change", HEADS)
+def test_heads_of_the_users_own(natively, change):
+    model = small_model()
+    change(model)
+    assert not natively(model)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("change", HEADS)
+def test_heads_of_the_users_own_are_called(dev, change):
+    model = small_model()
+    b = small_batch().to(dev)
+    change(model)
+    got = same_with_and_without_gradients(model, dev)
+    with torch.no_grad():
+        x = torch.nn.functional.linear(b.x, model.input_embeddings.weight)
+        x = model.encoder(x, b.pos, b.batch, b.trans_vec, b.sizes)
+        pooled = torch.stack([p.double().mean(0) for p in x.split(b.sizes.tolist())]).float()
+        want = 2.0 * model.mlp(pooled) if change is overridden_head else model.mlp(pooled)
+    assert_close(got, want, "head", rtol=RTOL)

@@ -55,7 +55,8 @@ def _block(layer: nn.Module, width: int, device_index: int):
         return None
     mods = layer._modules
     attn, lin1, lin2 = mods["self_attn"], mods["linear1"], mods["linear2"]
-    if type(attn) is not CrystalformerMultiheadAttentionCUDA or type(lin1) is not nn.Linear or type(lin2) is not nn.Linear:
+    if type(attn) is not CrystalformerMultiheadAttentionCUDA or type(lin1) is not nn.Linear \
+            or type(lin2) is not nn.Linear or type(attn._modules.get("out_proj")) is not nn.Linear:
         return None
     if type(mods["norm1"]) is not nn.Identity or type(mods["norm2"]) is not nn.Identity \
             or layer.activation is not torch.nn.functional.relu:
@@ -82,9 +83,12 @@ def _block(layer: nn.Module, width: int, device_index: int):
     own = attn._parameters
     out, w1, w2 = attn._modules["out_proj"]._parameters, lin1._parameters, lin2._parameters
     ff = lin1.out_features
-    tensors = (own["q_proj_weight"], own["k_proj_weight"], own["v_proj_weight"], own["in_proj_bias"],
-               own["lattice_pos_weights"], own["gauss_scale"], own["pe_dist_proj"] if bins > 0 else None,
-               out["weight"], out["bias"], w1["weight"], w1["bias"], w2["weight"], w2["bias"])
+    try:
+        tensors = (own["q_proj_weight"], own["k_proj_weight"], own["v_proj_weight"], own["in_proj_bias"],
+                   own["lattice_pos_weights"], own["gauss_scale"], own["pe_dist_proj"] if bins > 0 else None,
+                   out["weight"], out["bias"], w1["weight"], w1["bias"], w2["weight"], w2["bias"])
+    except KeyError:                                       # (worked out from others whenever it is read)
+        return None
     sq = width * width
     counts = (sq, sq, sq, 3 * width, width, 2, H * D * bins, sq, width, width * ff, ff, width * ff, width)
     if bins > 0 and tensors[6] is None:
@@ -144,6 +148,8 @@ def _head(mlp: nn.Module, width: int, device_index: int) -> Optional[Tuple[tuple
     (identities in between do not count), else None."""
     mods = [m for m in mlp._modules.values() if type(m) is not nn.Identity]
     kinds = [type(m) for m in mods]
+    if any(t is nn.Linear and not m._parameters.keys() >= {"weight", "bias"} for t, m in zip(kinds, mods)):
+        return None                                        # (as in _block)
     if kinds == [nn.Linear, nn.ReLU, nn.Linear]:
         first, last = mods[0]._parameters, mods[2]._parameters
         hidden = mods[0].out_features

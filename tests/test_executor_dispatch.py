@@ -8,6 +8,7 @@ from crystalformer_amd import executor
 from crystalformer_amd.encoder import CrystalformerEncoderCUDA
 from crystalformer_amd.latticeformer import Latticeformer, default_params
 from crystalformer_amd.synthetic import make_batch
+from crystalformer_amd.training import fused_training_step, training_step
 from tests.helpers import RTOL, assert_close
 
 
@@ -154,3 +155,76 @@ def test_heads_of_the_users_own_are_called(dev, change):
         pooled = torch.stack([p.double().mean(0) for p in x.split(b.sizes.tolist())]).float()
         want = 2.0 * model.mlp(pooled) if change is overridden_head else model.mlp(pooled)
     assert_close(got, want, "head", rtol=RTOL)
+
+
+def weight_norm(module):
+    torch.nn.utils.parametrizations.weight_norm(module)
+
+
+def plain_attributes(module):
+    """Weight and bias worked out elsewhere and set as plain tensors, as reparametrising code does."""
+    for name in ("weight", "bias"):
+        value = getattr(module, name).detach().clone() * 1.5 + 0.01
+        delattr(module, name)
+        setattr(module, name, value)
+
+
+MODULES = [lambda m: m.encoder.layers[1].self_attn.out_proj, lambda m: m.encoder.layers[0].linear1,
+           lambda m: m.encoder.layers[1].linear2, lambda m: m.mlp[0], lambda m: m.mlp[-1]]
+
+
+@pytest.mark.parametrize("where", range(len(MODULES)))
+@pytest.mark.parametrize("change", [weight_norm, plain_attributes])
+def test_blocks_with_parameters_worked_out_are_declined(where, change):
+    model = small_model()
+    change(MODULES[where](model))
+    blocks = [executor._block(layer, 128, -1) for layer in model.encoder.layers]
+    head = executor._head(model.mlp, 128, -1)
+    assert [blocks[1], blocks[0], blocks[1], head, head][where] is None
+    assert sum(b is None for b in blocks) + (head is None) == 1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("where", range(len(MODULES)))
+@pytest.mark.parametrize("change", [weight_norm, plain_attributes])
+def test_blocks_with_parameters_worked_out(dev, where, change):
+    model = small_model().to(dev)
+    change(MODULES[where](model))
+    same_with_and_without_gradients(model, dev)
+
+
+class PlainSGD:
+    """An optimiser with the interface the training steps use, which leaves the parameters alone."""
+    def __init__(self, model):
+        self.params = list(model.parameters())
+
+    def zero_grad(self, set_to_none=True):
+        for p in self.params:
+            p.grad = None
+
+    def step(self):
+        pass
+
+
+def step_gradients(model, dev, fused):
+    """Loss and gradients of one training step: from the fused step, or of the plain one."""
+    b = make_batch(3, (4, 9), False, (3.0, 11.0), (65.0, 115.0), seed=3, with_targets=True).to(dev)
+    opt = PlainSGD(model)
+    loss = fused_training_step(model, b, opt) if fused else training_step(model, b, opt, clip_norm=0)
+    return [loss] + [p.grad for p in opt.params if p.requires_grad]
+
+
+def fused_step_equals_the_plain_one(model, dev):
+    model = model.to(dev)
+    plain = step_gradients(model, dev, False)
+    for got, want in zip(step_gradients(model, dev, True), plain):
+        # (sums over the atoms in another order: relative to the whole tensor)
+        assert float((got - want).norm()) <= RTOL * float(want.norm().clamp_min(1e-12))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("where", range(3))
+def test_training_with_parameters_worked_out(dev, where):
+    model = small_model()
+    weight_norm(MODULES[where](model))
+    fused_step_equals_the_plain_one(model, dev)

@@ -192,9 +192,12 @@ def _run(encoder: nn.Module, src: Tensor, pos: Tensor, batch: Tensor, trans: Ten
         return None
     width = encoder.d_model
     index = src.get_device()
-    N = src.shape[0]
-    B = trans.shape[0]
-    if index < 0 or src.dim() != 2 or N == 0 or not _ready(src, N * (embed.in_features if embed else width), index) or not _ready(pos, 3 * N, index) \
+    if index < 0 or src.dim() != 2 or trans.dim() != 3 or batch.dim() != 1:
+        return None
+    N, B = src.shape[0], trans.shape[0]
+    # (shapes and not counts: what the operators refuse one by one is theirs to refuse)
+    if N == 0 or src.shape[1] != (embed.in_features if embed else width) or pos.shape != (N, 3) \
+            or trans.shape != (B, 3, 3) or not _ready(src, src.numel(), index) or not _ready(pos, 3 * N, index) \
             or not _ready(trans, 9 * B, index) or batch.get_device() != index or batch.dtype is not torch.int64:
         return None
     blocks = []

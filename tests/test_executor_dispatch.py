@@ -1,11 +1,14 @@
 """Which models, batches and settings the native inference call is chosen for, on the CPU (the call itself is
 replaced by a marker), and on the GPU that everything it leaves alone computes what its modules say."""
+import dataclasses
+
 import pytest
 import torch
 from torch import nn
 
 from crystalformer_amd import executor
 from crystalformer_amd.encoder import CrystalformerEncoderCUDA
+from crystalformer_amd.lib import CrystalformerHipError
 from crystalformer_amd.latticeformer import Latticeformer, default_params
 from crystalformer_amd.synthetic import make_batch
 from crystalformer_amd.training import fused_training_step, training_step
@@ -228,3 +231,33 @@ def test_training_with_parameters_worked_out(dev, where):
     model = small_model()
     weight_norm(MODULES[where](model))
     fused_step_equals_the_plain_one(model, dev)
+
+
+# as many numbers in another shape: what the operators refuse one by one
+SHAPES = {"pos": lambda b: dict(pos=b.pos.T.contiguous()), "pos_flat": lambda b: dict(pos=b.pos.reshape(-1)),
+          "trans": lambda b: dict(trans_vec=b.trans_vec.reshape(-1, 9)),
+          "trans_one": lambda b: dict(trans_vec=b.trans_vec.reshape(1, -1, 3)),
+          "trans_rows": lambda b: dict(trans_vec=b.trans_vec.reshape(-1, 1, 9))}
+
+
+def test_shapes_are_looked_at(monkeypatch):
+    """Every batch of these shapes is declined before anything is laid out for it."""
+    monkeypatch.setattr(torch.Tensor, "get_device", lambda t: 0)
+    monkeypatch.setattr(executor, "_block", lambda *args: pytest.fail("accepted"))
+    model, b = small_model(), small_batch()
+    for change in SHAPES.values():
+        c = dataclasses.replace(b, **change(b))
+        with torch.no_grad():
+            assert executor._run(model.encoder, b.x @ model.input_embeddings.weight.T, c.pos, c.batch, c.trans_vec,
+                                 c.sizes) is None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", SHAPES)
+def test_shapes_are_refused(dev, shape):
+    model, b = small_model().to(dev), small_batch().to(dev)
+    c = dataclasses.replace(b, **SHAPES[shape](b))
+    with torch.no_grad(), pytest.raises(CrystalformerHipError):
+        model(c)
+    with pytest.raises(CrystalformerHipError):
+        model(c)

@@ -48,7 +48,8 @@ def _address(t: Optional[Tensor]) -> Optional[int]:
 
 
 def _block(layer: nn.Module, width: int, device_index: int):
-    """(``cf_forward_block`` fields, heads, feed-forward width) of a layer, or None when it is not the plain case."""
+    """(``cf_forward_block`` fields, heads, feed-forward width, whether it stores its exponents' statistics) of a
+    layer, or None when it is not the plain case."""
     from .attention import CrystalformerMultiheadAttentionCUDA, fused_exponents_spec
     from .encoder import CrystalformerEncoderLayerCUDA
     if type(layer) is not CrystalformerEncoderLayerCUDA:
@@ -62,8 +63,9 @@ def _block(layer: nn.Module, width: int, device_index: int):
             or layer.activation is not torch.nn.functional.relu:
         return None
     P = attn.params
-    if layer.training and (attn.dropout > 0 or any(type(mods[d]) is not nn.Identity
-                                                   for d in ("dropout", "dropout1", "dropout2"))):
+    # (every module has a mode of its own: the attention's decides on its dropout and its statistics)
+    if (attn.training and attn.dropout > 0) or any(type(mods[d]) is not nn.Identity and (layer.training or mods[d].training)
+                                                   for d in ("dropout", "dropout1", "dropout2")):
         return None
     spec = fused_exponents_spec(P)
     halves = P.domain == "multihead"               # half of the heads in reciprocal space
@@ -106,7 +108,7 @@ def _block(layer: nn.Module, width: int, device_index: int):
     fields += [bins, int(bool(P.normalize_gauss)), ops.POSITIVE_FUNCS[spec[0]], dist_max, P.value_pe_width_scale,
                cutoff, -0.5 * P.gauss_lb_real * P.scale_real ** -2 * (1 - 1e-5), -0.5 * P.scale_real ** -2,
                P.gauss_lb_real, spec[1], 1.0 / math.sqrt(D), -0.5 * P.scale_reci ** 2 if halves else 0.0]
-    return fields, H, ff
+    return fields, H, ff, attn.training and bool(P.normalize_gauss)
 
 
 def _watched(module: nn.Module) -> bool:
@@ -201,12 +203,12 @@ def _run(encoder: nn.Module, src: Tensor, pos: Tensor, batch: Tensor, trans: Ten
             or not _ready(trans, 9 * B, index) or batch.get_device() != index or batch.dtype is not torch.int64:
         return None
     blocks = []
-    H = ff = None
+    H = ff = store = None
     for layer in encoder._modules["layers"]._modules.values():
         got = _block(layer, width, index)
-        if got is None or (blocks and (got[1] != H or got[2] != ff)):
-            return None
-        fields, H, ff = got
+        if got is None or (blocks and got[1:] != (H, ff, store)):
+            return None                                # (one setting for all blocks: some frozen, some not)
+        fields, H, ff, store = got
         blocks.append(fields)
     if not blocks:
         return None
@@ -223,7 +225,7 @@ def _run(encoder: nn.Module, src: Tensor, pos: Tensor, batch: Tensor, trans: Ten
     sched = ops._scheduling_words(dev) if ops.DYNAMIC_ROUNDS else None
     args = _lib.ForwardArgs(
         N, layout.num_edges, sizes.numel(), len(blocks), H, width, ff, KM.LATTICE_RANGE, KM.MINIMUM_RANGE, 1,
-        int(encoder.training), int(KM.STAGED_RINGS), int(KM.ADAPTIVE_RINGS), ops.STAGED_RINGS_MAX_BYTES, hidden,
+        int(store), int(KM.STAGED_RINGS), int(KM.ADAPTIVE_RINGS), ops.STAGED_RINGS_MAX_BYTES, hidden,
         targets, embed.in_features if embed else 0, src.data_ptr(), pos.data_ptr(), trans.data_ptr(), layout.batch.data_ptr(), layout.atom_start.data_ptr(),
         layout.edge_start.data_ptr(), layout.edges.data_ptr(), layout.e_start.data_ptr(), layout.pairs.data_ptr(),
         _address(sched), *(_address(t) for t in tensors),

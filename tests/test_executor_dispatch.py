@@ -261,3 +261,60 @@ def test_shapes_are_refused(dev, shape):
         model(c)
     with pytest.raises(CrystalformerHipError):
         model(c)
+
+
+def accepted(model):
+    """Blocks that the native call takes, with whether they store statistics."""
+    blocks = [executor._block(layer, 128, -1) for layer in model.encoder.layers]
+    return [b and b[3] for b in blocks]
+
+
+def test_modes_are_each_modules_own():
+    model = small_model()
+    assert accepted(model) == [False, False]
+    assert accepted(model.train()) == [True, True]
+    model.encoder.layers[0].eval()                         # (a frozen block)
+    assert accepted(model) == [False, True]
+    model.encoder.eval().training = True
+    assert accepted(model) == [False, False]
+    model = small_model(dropout=0.2)
+    assert accepted(model) == [False, False]
+    assert accepted(model.train()) == [None, None]
+    model.eval().encoder.layers[1].self_attn.train()       # dropout on the weights only
+    assert accepted(model) == [False, None]
+    model.eval().encoder.layers[1].dropout2.train()
+    assert accepted(model) == [False, None]
+    model = small_model(normalize_gauss=False)
+    model.encoder.layers[0].train()
+    assert accepted(model) == [False, False]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("frozen", [[0], [1], [0, 1]])
+def test_frozen_blocks_keep_their_statistics(dev, frozen):
+    model = small_model().to(dev).train()
+    for i, layer in enumerate(model.encoder.layers):
+        layer.self_attn.gauss_scale.data.zero_()
+        if i in frozen:
+            layer.eval()
+    with torch.no_grad():
+        model(small_batch().to(dev))
+    for i, layer in enumerate(model.encoder.layers):
+        assert bool(layer.self_attn.gauss_scale[0] > 0) == (i not in frozen)
+
+
+@pytest.mark.gpu
+def test_dropout_follows_the_modules_modes(dev):
+    """Dropout of an attention in training mode inside a block in evaluation mode, at inference; of a feed-forward
+    in training mode, in a fused training step."""
+    model, b = small_model(dropout=0.5).to(dev), small_batch().to(dev)
+    with torch.no_grad():
+        assert torch.equal(model(b), model(b))
+        model.encoder.layers[0].self_attn.train()
+        assert not torch.equal(model(b), model(b))
+    model.eval()
+    one, two = (step_gradients(model, dev, True)[0] for _ in range(2))
+    assert torch.equal(one, two)
+    model.encoder.layers[0].dropout2.train()
+    one, two = (step_gradients(model, dev, True)[0] for _ in range(2))
+    assert not torch.equal(one, two)

@@ -28,11 +28,13 @@ def _hooked(module: nn.Module) -> bool:
     return bool(module._forward_hooks or module._forward_pre_hooks)
 
 
-def _any_hooked(module: nn.Module) -> bool:
-    if _hooked(module):
+def _touched(module: nn.Module, backward: bool = False) -> bool:
+    """A forward hook (or, with ``backward``, a hook of any kind) or a forward of its own on the module or one below."""
+    if module._forward_hooks or module._forward_pre_hooks or "forward" in module.__dict__ \
+            or (backward and (module._backward_hooks or module._backward_pre_hooks)):
         return True
     for child in module._modules.values():
-        if child is not None and _any_hooked(child):
+        if child is not None and _touched(child, backward):
             return True
     return False
 
@@ -111,16 +113,6 @@ def _block(layer: nn.Module, width: int, device_index: int):
     return fields, H, ff, attn.training and bool(P.normalize_gauss)
 
 
-def _watched(module: nn.Module) -> bool:
-    """A hook of any kind on the module or one below it."""
-    if module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks:
-        return True
-    for child in module._modules.values():
-        if child is not None and _watched(child):
-            return True
-    return False
-
-
 def pack_for_training(encoder: nn.Module, src: Tensor) -> Optional["ops.PackedBlocks"]:
     """The blocks' weights packed for the one-launch row kernels if every block of a fused training step is one
     they serve (the plain case of this module, 128 wide with 512 hidden units, real domain) and nobody looks into
@@ -134,7 +126,7 @@ def pack_for_training(encoder: nn.Module, src: Tensor) -> Optional["ops.PackedBl
     blocks = []
     for layer in encoder._modules["layers"]._modules.values():
         mods = layer._modules
-        if any(c is not None and _watched(c) for c in mods.values()):
+        if _touched(layer, backward=True):
             return None
         got = _block(layer, 128, src.get_device())
         if got is None or got[2] != 512 or layer.self_attn.params.domain != "real" or 128 // got[1] % 4:
@@ -190,7 +182,7 @@ def _run(encoder: nn.Module, src: Tensor, pos: Tensor, batch: Tensor, trans: Ten
     KM = hip_funcs.KernelManager
     if torch.is_grad_enabled() or config.REPRODUCIBLITY_STATE < 2 or not KM.DENSE_EDGE_BLOCKS \
             or ops.instrumented() or encoder._modules.get("norm") is not None \
-            or _torch_module._global_forward_hooks or _torch_module._global_forward_pre_hooks or _any_hooked(encoder):
+            or _torch_module._global_forward_hooks or _torch_module._global_forward_pre_hooks or _touched(encoder):
         return None
     width = encoder.d_model
     index = src.get_device()
@@ -256,11 +248,11 @@ def forward(model: nn.Module, data) -> Tuple[Optional[Tensor], Optional[Tensor]]
         return None, None
     mods = model._modules
     encoder, proj, mlp = mods.get("encoder"), mods.get("proj_before_pooling"), mods.get("mlp")
-    # (an encoder of another class, or with a forward of its own, computes something else than its layers say)
+    # (an encoder of another class computes something else than its layers say)
     if type(encoder) is not CrystalformerEncoderCUDA or "forward" in encoder.__dict__:
         return None, None
     if type(proj) is not nn.Identity or model.pooling_layer is not pooling.avr_pool \
-            or _hooked(proj) or not is_plain_head(mlp) or _any_hooked(mlp) \
+            or _hooked(proj) or not is_plain_head(mlp) or _touched(mlp) \
             or type(model)._head is not Latticeformer._head or "_head" in model.__dict__:
         return None, None
     x = data.x

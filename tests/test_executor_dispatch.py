@@ -318,3 +318,49 @@ def test_dropout_follows_the_modules_modes(dev):
     model.encoder.layers[0].dropout2.train()
     one, two = (step_gradients(model, dev, True)[0] for _ in range(2))
     assert not torch.equal(one, two)
+
+
+def halved_offsets(attn):
+    """An attention whose offsets p_j - p_i are halved."""
+    plain = attn.forward
+    attn.forward = lambda *args, **kwargs: plain(*args[:6], 0.5 * args[6], *args[7:], **kwargs)
+
+
+def halved_output(layer):
+    plain = layer.forward
+    layer.forward = lambda src, *args, **kwargs: 0.5 * plain(src, *args, **kwargs)
+
+
+INNER = {"attention": lambda m: halved_offsets(m.encoder.layers[1].self_attn),
+         "layer": lambda m: halved_output(m.encoder.layers[0])}
+HOOKED = {"attention": lambda m: m.encoder.layers[1].self_attn, "layer": lambda m: m.encoder.layers[0]}
+
+
+@pytest.mark.parametrize("where", INNER)
+def test_forwards_replaced_below_the_encoder(where):
+    model = small_model()
+    assert not executor._touched(model.encoder)
+    INNER[where](model)
+    assert executor._touched(model.encoder)
+    model = small_model()
+    HOOKED[where](model).register_full_backward_hook(lambda *args: None)
+    assert not executor._touched(model.encoder) and executor._touched(model.encoder, backward=True)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("where", INNER)
+def test_forwards_replaced_below_the_encoder_are_called(dev, where):
+    """At inference and in a fused training step."""
+    model = small_model()
+    plain = same_with_and_without_gradients(small_model(), dev)
+    INNER[where](model)
+    assert not torch.equal(same_with_and_without_gradients(model, dev), plain)
+    fused_step_equals_the_plain_one(model, dev)
+
+
+@pytest.mark.gpu
+def test_hooks_of_a_layer_in_a_fused_step(dev):
+    """A hook may hand on what the row kernels do not take, rows that are not contiguous here."""
+    model = small_model()
+    model.encoder.layers[0].register_forward_hook(lambda m, args, out: (0.5 * out.T.contiguous()).T)
+    fused_step_equals_the_plain_one(model, dev)

@@ -40,7 +40,7 @@ def _refresh(moves) -> None:
     """``dst.copy_(src)`` for each pair, in one launch where the tensors are plain (each copy of its own is 2 us of
     transfer and as much of a gap in front of the graph)."""
     if all(type(s) is torch.Tensor and s.device == d.device and s.dtype is d.dtype and s.shape == d.shape
-           and s.is_contiguous() and not s.is_neg() and not s.is_conj() for d, s in moves):
+           and d.is_contiguous() and s.is_contiguous() and not s.is_neg() and not s.is_conj() for d, s in moves):
         ops.copy_segments(moves)
         return
     for d, s in moves:

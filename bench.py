@@ -193,6 +193,41 @@ def ingest_counters(directory: str, key: str, kernel: str) -> int:
     return 0
 
 
+def record_calls(ops, names, run) -> dict:
+    """``(args, kwargs)`` of every call of the operators ``names`` during ``run()``.  An event log keeps the native
+    forward out of the way, which issues the same launches without passing through the operators; blocks without
+    value bins take two launches there, so they do here."""
+    from crystalformer_amd import hip_funcs
+    KM = hip_funcs.KernelManager
+    calls = {name: [] for name in names}
+    originals = {name: getattr(ops, name) for name in names}
+    fuse = KM.FUSE_ENCODING_ATTENTION
+
+    def spy_on(name):
+        def spy(*a, **kw):
+            calls[name].append((a, kw))
+            return originals[name](*a, **kw)
+        return spy
+    try:
+        KM.FUSE_ENCODING_ATTENTION = False
+        ops.set_event_log([])
+        for name in names:
+            setattr(ops, name, spy_on(name))
+        run()
+    finally:
+        for name in names:
+            setattr(ops, name, originals[name])
+        ops.set_event_log(None)
+        KM.FUSE_ENCODING_ATTENTION = fuse
+    return calls
+
+
+def require_encodings(calls: dict, domain: str) -> None:
+    """Raise unless a model with real-space blocks was seen to encode."""
+    if domain != "reci" and not any(calls[name] for name in calls if name.startswith("real_enc")):
+        raise SystemExit("bench.py: no launch of the periodic encoding was recorded")
+
+
 def flop_per_eval(H: int, K: int) -> int:
     """Algorithmic work of one (edge, translation) evaluation, all heads and
     bins, geometry and Gaussians shared across heads: 23 (geometry) + 3H
@@ -490,30 +525,23 @@ def main() -> int:
         # plain copy of known size: 64 Mi floats read + 64 Mi floats written
         src = torch.ones(64 << 20, dtype=torch.float32, device=dev)
         dst = torch.empty_like(src)
-        captured = {}
         # --train: the backward kernel; otherwise the forward one, pair kernel or from staged rings
         names = ("real_enc_bwd",) if args.train else ("real_enc_fwd", "real_enc_fwd_rings", "staged_rings")
-        originals = {nm: getattr(ops, nm) for nm in names}
 
-        def spy_on(nm):
-            def spy(*a, **kw):
-                captured.setdefault(nm, (a, kw))
-                return originals[nm](*a, **kw)
-            return spy
-        for nm in names:
-            setattr(ops, nm, spy_on(nm))
-        if args.train:
-            model.train()
-            out = model(data)
-            torch.nn.functional.l1_loss(out[:, 0], data.y).backward()
-        else:
-            with torch.no_grad():
-                model(data)
-        for nm in names:
-            setattr(ops, nm, originals[nm])
+        def one_pass():
+            if args.train:
+                model.train()
+                out = model(data)
+                torch.nn.functional.l1_loss(out[:, 0], data.y).backward()
+            else:
+                with torch.no_grad():
+                    model(data)
+        originals = {nm: getattr(ops, nm) for nm in names}
+        captured = record_calls(ops, names, one_pass)
+        require_encodings(captured, args.domain)
         for _ in range(5):
             dst.copy_(src)
-        for nm, (a, kw) in captured.items():
+        for nm, (a, kw) in ((nm, seen[0]) for nm, seen in captured.items() if seen):
             for _ in range(5):
                 if nm == "staged_rings":
                     ops._ring_cache.clear()
@@ -534,20 +562,10 @@ def main() -> int:
         eager_elapsed, y_eager = timed(lambda: model(data), args.steps, args.warmup)
         # Kernel durations: the encoding / attention launches of one forward are re-issued back to
         # back (queue kept full), each bracketed by a pair of HIP events on the launch stream.
-        calls = {"real_enc_fwd": [], "real_enc_fwd_rings": [], "fused_dpa_fwd": [], "fused_enc_dpa_fwd": [],
-                 "staged_rings": []}
-        originals = {name: getattr(ops, name) for name in calls}
-
-        def spy_on(name):
-            def spy(*a, **kw):
-                calls[name].append((a, kw))
-                return originals[name](*a, **kw)
-            return spy
-        for name in calls:
-            setattr(ops, name, spy_on(name))
-        model(data)
-        for name in calls:
-            setattr(ops, name, originals[name])
+        names = ("real_enc_fwd", "real_enc_fwd_rings", "fused_dpa_fwd", "staged_rings")
+        originals = {name: getattr(ops, name) for name in names}
+        calls = record_calls(ops, names, lambda: model(data))
+        require_encodings(calls, args.domain)
         log: list = []
         ops.set_event_log(log)
         for name in calls:
@@ -588,11 +606,8 @@ def main() -> int:
 
     # ---- roofline of the dominant kernel (periodic encoding, forward)
     enc_ms = [s.elapsed_time(e) for (name, s, e, info) in log if name == "real_enc_fwd"]
-    one_launch_ms = [s.elapsed_time(e) for (name, s, e, info) in log if name == "fused_enc_dpa_fwd"]
     dpa_ms = [s.elapsed_time(e) for (name, s, e, info) in log if name == "fused_dpa_fwd"]
     stage_ms = [s.elapsed_time(e) for (name, s, e, info) in log if name == "real_enc_ring_stage"]
-    if not enc_ms and one_launch_ms:
-        enc_ms = one_launch_ms
     enc_avg_ms = sum(enc_ms) / max(len(enc_ms), 1)
     # translations walked per launch (all heads share a trip): one untimed forward with the counter on
     counts: list = []
@@ -614,7 +629,7 @@ def main() -> int:
                     "real_enc_fwd_two_role_kernel (periodic encoding forward, adaptive boxes: atom pairs that keep the "
                     "cube from the staged translations, the others staged in the same launch; with its two list-building "
                     "launches)") if calls["real_enc_fwd_rings"] else
-                   "real_enc_fwd_pair_kernel (periodic encoding forward, projection fused)"),
+                   f"real_enc_fwd_pair_kernel (periodic encoding forward, {'projection fused' if K > 0 else 'bias only'})"),
         "bound": "mfma",
         # executed fp32 work (instruction counters of a stored rocprofv3 --pmc run of this kernel
         # on this workload) over the launch time measured in this run
@@ -641,9 +656,6 @@ def main() -> int:
     }
     if stage_ms:           # once per forward: the translations all blocks start from
         roofline["ring_stage_avg_ms"] = round(sum(stage_ms) / len(stage_ms), 4)
-    if one_launch_ms:      # blocks without value bins, eager: bias + attention in one launch
-        roofline["kernel"] = "enc_dpa_row_kernel (lattice-sum bias + attention in one launch; eager launches only)"
-        roofline["fused_enc_dpa_fwd_avg_ms"] = round(sum(one_launch_ms) / len(one_launch_ms), 4)
     # the attention kernel is the memory-bound one: algorithmic bytes per edge 4 H (Dv + 2)
     # (b_ij and a_ij read, prob written) + the q/k/v/out rows once per atom
     dpa_avg_ms = sum(dpa_ms) / max(len(dpa_ms), 1)
@@ -652,7 +664,9 @@ def main() -> int:
         roofline["fused_dpa_fwd"] = {"bound": "hbm", "achieved": round(dpa_bytes / (dpa_avg_ms * 1e-3) / 1e9, 1),
                                      "peak": 8000.0, "unit": "GB/s",
                                      "frac": round(dpa_bytes / (dpa_avg_ms * 1e-3) / 1e9 / 8000.0, 4),
-                                     "avg_launch_ms": round(dpa_avg_ms, 4)}
+                                     "avg_launch_ms": round(dpa_avg_ms, 4),
+                                     "note": "the operator, which stores the weights; a forward without gradients "
+                                             "leaves them out"}
 
     # ---- forwards over batches never seen before: every step a batch with other crystal sizes.
     # One captured graph with capacity buffers serves them all (the index structure and the counts

@@ -1139,6 +1139,11 @@ class PackedBlocks:
                 self.counters[index:index + 1])
 
 
+def _require_packed(packed: Tensor, dev: torch.device) -> None:
+    if not _plain_f32(packed, dev) or packed.numel() != _lib.load().cf_pack_blocks_floats(1):
+        raise _lib.CrystalformerHipError("packed weights of one block expected (PackedBlocks.block)")
+
+
 def block_head(x: Tensor, heads: int, packed: Tensor, counter: Tensor, b_in: Optional[Tensor], w_pos: Tensor,
                gauss_scale: Tensor, normalize: bool, update_stats: bool, positive_func: str, beta: float,
                lower_bound: float, coef: float, q_scale: float):
@@ -1148,9 +1153,11 @@ def block_head(x: Tensor, heads: int, packed: Tensor, counter: Tensor, b_in: Opt
     N, W = x.shape
     if W != 128 or not _plain_f32(x, dev) or positive_func not in POSITIVE_FUNCS or w_pos.numel() != W \
             or not _plain_f32(w_pos, dev) or not _plain_f32(gauss_scale, dev) or gauss_scale.numel() != 2 \
-            or not (b_in is None or (_plain_f32(b_in, dev) and b_in.numel() == 3 * W)):
+            or not (b_in is None or (_plain_f32(b_in, dev) and b_in.numel() == 3 * W)) \
+            or counter.dtype is not torch.int32 or counter.get_device() != dev.index or counter.numel() < 1:
         raise _lib.CrystalformerHipError("block_head: contiguous float32 rows of 128 and their block's parameters expected")
     lib = _lib.load()
+    _require_packed(packed, dev)
     q, qs, k, v = torch.empty((4, N, W), dtype=torch.float32, device=dev).unbind(0)
     a, alpha_n = torch.empty((2, N, heads), dtype=torch.float32, device=dev).unbind(0)
     used = torch.empty(2, dtype=torch.float32, device=dev) if normalize else None
@@ -1172,6 +1179,13 @@ def block_head_bwd(ga, gqs, gk, gv, carry, q: Tensor, w_pos: Tensor, alpha_n: Te
     dev = require_device(ga, gqs, gk, gv, carry, q, packed_bwd)
     ga, gqs, gk, gv, carry = (_f32(t, "gradient") for t in (ga, gqs, gk, gv, carry))
     N, W = q.shape
+    if W != 128 or not _plain_f32(q, dev) or not _plain_f32(w_pos, dev) or w_pos.numel() != W \
+            or not _plain_f32(alpha_n, dev) or alpha_n.dim() != 2 or alpha_n.shape[0] != N \
+            or (ga is not None and ga.shape != alpha_n.shape) \
+            or any(t is not None and t.shape != q.shape for t in (gqs, gk, gv, carry)) \
+            or not (used is None or (_plain_f32(used, dev) and used.numel() == 2)):
+        raise _lib.CrystalformerHipError("block_head_bwd: operands of block_head and gradients of its outputs' shapes expected")
+    _require_packed(packed_bwd, dev)
     lib = _lib.load()
     gq, gx = torch.empty((2, N, W), dtype=torch.float32, device=dev).unbind(0)
     gw = torch.empty(W, dtype=torch.float32, device=dev) if ga is not None else None
@@ -1194,6 +1208,7 @@ def block_tail(att: Tensor, x: Tensor, packed: Tensor, bo: Optional[Tensor], b1:
     if W != 128 or att.shape != x.shape or not _plain_f32(x, dev) or not _plain_f32(att, dev) or any(
             b is not None and (not _plain_f32(b, dev) or b.numel() != n) for b, n in ((bo, W), (b1, 512), (b2, W))):
         raise _lib.CrystalformerHipError("block_tail: contiguous float32 rows of 128 and their block's biases expected")
+    _require_packed(packed, dev)
     s, y = torch.empty((2, N, W), dtype=torch.float32, device=dev).unbind(0)
     h = torch.empty((N, 512), dtype=torch.float32, device=dev)
     with device_guard(dev):
@@ -1208,6 +1223,9 @@ def block_tail_bwd(gy: Tensor, h: Tensor, packed_bwd: Tensor) -> Tuple[Tensor, T
     dev = require_device(gy, h, packed_bwd)
     gy = _f32(gy, "gy")
     N, W = gy.shape
+    if W != 128 or not _plain_f32(h, dev) or h.shape != (N, 512):
+        raise _lib.CrystalformerHipError("block_tail_bwd: a gradient (N,128) and the hidden units (N,512) expected")
+    _require_packed(packed_bwd, dev)
     gs, gatt = torch.empty((2, N, W), dtype=torch.float32, device=dev).unbind(0)
     gh = torch.empty_like(h)
     with device_guard(dev):

@@ -7,6 +7,7 @@ import torch
 
 from crystalformer_amd import hip_funcs, ops
 from crystalformer_amd.attention import make_positive_func
+from crystalformer_amd.lib import CrystalformerHipError
 
 pytestmark = pytest.mark.gpu
 
@@ -137,3 +138,32 @@ def test_same_bits_as_the_operators_one_by_one(dev, n, heads, func, normalize):
         for what, one, two in zip(names, torch.autograd.grad(y, (x, *head, *tail), g),
                                   torch.autograd.grad(y2, (x, *head, *tail), g)):
             assert torch.equal(one, two), what
+
+
+def test_operands_of_other_shapes_are_refused(dev):
+    """Before any launch: the kernels read whole rows, heads and weights by these counts."""
+    n = 20
+    w = [torch.randn(s, device=dev) for s in ((128, 128), (512, 128), (128, 512)) + ((128, 128),) * 3]
+    blocks = ops.PackedBlocks([tuple(w)] * 2)
+    fwd, bwd, counter = blocks.block(0)
+    x, w_pos, gauss = torch.randn(n, 128, device=dev), torch.randn(128, device=dev), torch.ones(2, device=dev)
+    conf = ("elu", 0.1, 0.5, -0.3, 0.25)
+    a, qs, k, v, q, alpha_n, used = ops.block_head(x, 8, fwd, counter, None, w_pos, gauss, True, False, *conf)
+    y, s, h = ops.block_tail(x, x, fwd, None, None, None)
+    refused = pytest.raises(CrystalformerHipError)
+    for packed, count in ((blocks.forward, counter), (fwd[:-1], counter), (fwd.double(), counter), (fwd, counter.long()),
+                          (fwd, counter.cpu())):
+        with refused:
+            ops.block_head(x, 8, packed, count, None, w_pos, gauss, True, False, *conf)
+    with refused:
+        ops.block_tail(x, x, blocks.forward, None, None, None)
+    good = dict(ga=a, gqs=qs, gk=k, gv=v, carry=x, q=q, w_pos=w_pos, alpha_n=alpha_n, used=used, packed_bwd=bwd)
+    ops.block_head_bwd(*good.values(), *conf)
+    for name, wrong in (("ga", a[1:]), ("gqs", qs[1:]), ("gk", k[:, 1:]), ("gv", v[1:]), ("carry", x[:-1]), ("q", q[1:]),
+                        ("q", q[:, :64]), ("w_pos", w_pos[1:]), ("alpha_n", alpha_n[1:]), ("used", used[:1]),
+                        ("packed_bwd", bwd[:-1])):
+        with refused:
+            ops.block_head_bwd(*dict(good, **{name: wrong}).values(), *conf)
+    for g, hidden, packed in ((y[1:], h, bwd), (y, h[1:], bwd), (y, h[:, 1:], bwd), (y[:, 1:], h, bwd), (y, h, bwd[:-1])):
+        with refused:
+            ops.block_tail_bwd(g, hidden, packed)

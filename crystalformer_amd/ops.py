@@ -1189,6 +1189,8 @@ def block_head_bwd(ga, gqs, gk, gv, carry, q: Tensor, w_pos: Tensor, alpha_n: Te
     lib = _lib.load()
     gq, gx = torch.empty((2, N, W), dtype=torch.float32, device=dev).unbind(0)
     gw = torch.empty(W, dtype=torch.float32, device=dev) if ga is not None else None
+    if gw is not None and N == 0:
+        gw.zero_()                                     # (a sum over no atoms: nothing is launched)
     g_alpha = torch.empty_like(alpha_n)
     with device_guard(dev):
         rc = lib.cf_block_head_bwd(ptr(ga), ptr(gqs), ptr(gk), ptr(gv), ptr(carry), ptr(q), ptr(w_pos), ptr(alpha_n),

@@ -167,3 +167,16 @@ def test_operands_of_other_shapes_are_refused(dev):
     for g, hidden, packed in ((y[1:], h, bwd), (y, h[1:], bwd), (y, h[:, 1:], bwd), (y[:, 1:], h, bwd), (y, h, bwd[:-1])):
         with refused:
             ops.block_tail_bwd(g, hidden, packed)
+
+
+def test_no_atoms(dev):
+    x, = leaves(dev, (0, 128))
+    wq, wk, wv, b_in, w_pos = leaves(dev, (128, 128), (128, 128), (128, 128), (384,), (128,))
+    big = torch.zeros(512, 128, device=dev)
+    packed = packed_of(wq, big, big.T.contiguous(), wq, wk, wv)
+    full = torch.full((1 << 16,), 7.0, device=dev)         # (what a freed buffer may hold)
+    del full
+    out = hip_funcs.BlockHeadHIP.apply(x, wq, wk, wv, b_in, w_pos, torch.tensor([0.8, -0.1], device=dev), 8, packed, True,
+                                       False, "elu", 0.1, 0.5, -0.3, 0.25)
+    for g in torch.autograd.grad([t.sum() for t in out], (wq, wk, wv, b_in, w_pos)):
+        assert torch.equal(g, torch.zeros_like(g))

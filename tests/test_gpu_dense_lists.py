@@ -55,3 +55,29 @@ def test_other_lists_are_not(dev, sizes):
     spread = torch.empty(2, 2 * E, dtype=torch.int64, device=dev)[:, ::2]
     spread.copy_(edges)
     assert ops.dense_block_layout(batch, spread).tolist() == sizes
+
+
+# either side of the crystal counts up to which one work-group scans them
+@pytest.mark.parametrize("crystals", [ops.SCAN_TWO, ops.SCAN_TWO + 1, ops.SCAN_THREE + 1, ops.SCAN_DENSE + 1])
+def test_many_crystals(dev, crystals, monkeypatch):
+    g = torch.Generator().manual_seed(crystals)
+    sizes = torch.randint(0, 4, (crystals,), generator=g)
+    sizes[-1] = 3
+    batch = torch.repeat_interleave(torch.arange(crystals), sizes).to(dev)
+    scans = []
+    scan = ops._lib.load().cf_layout_scan
+    monkeypatch.setattr(ops._lib.load(), "cf_layout_scan", lambda *a: scans.append(a[1]) or scan(*a))
+    edges, _ = ops.edge_index(sizes.to(dev))
+    assert len(scans) == (crystals <= ops.SCAN_TWO)
+    pairs = ops.edge_pairs(sizes.to(dev))
+    assert len(scans) == (crystals <= ops.SCAN_TWO) + (crystals <= ops.SCAN_THREE)
+    N = batch.numel()
+    start = torch.cat([torch.zeros(1, dtype=torch.int64), sizes.cumsum(0)])[batch.cpu()]
+    rows = torch.repeat_interleave(torch.arange(N), sizes[batch.cpu()])
+    first = torch.cat([torch.zeros(1, dtype=torch.int64), sizes[batch.cpu()].cumsum(0)])[:-1]
+    assert torch.equal(edges[0].cpu(), rows)
+    assert torch.equal(edges[1].cpu(), start[rows] + torch.arange(rows.numel()) - first[rows])
+    assert ops.dense_block_layout(batch, edges).tolist() == sizes.tolist()
+    assert torch.equal(ops.cached_edge_pairs(batch, edges, crystals), pairs)
+    edges[1, 5] += 1
+    assert ops.dense_block_layout(batch, edges) is None

@@ -21,7 +21,10 @@ from . import hip_funcs
 from . import lib as _lib
 from . import ops
 from . import pooling
-from .lib import CrystalformerHipError, device_guard, stream_handle
+from .attention import CrystalformerMultiheadAttentionCUDA, fused_exponents_spec
+from .encoder import CrystalformerEncoderCUDA, CrystalformerEncoderLayerCUDA, _sizes_on_device
+from .latticeformer import Latticeformer, is_plain_head
+from .lib import device_guard, stream_handle
 
 
 def _hooked(module: nn.Module) -> bool:
@@ -49,41 +52,48 @@ def _address(t: Optional[Tensor]) -> Optional[int]:
     return None if t is None else t.data_ptr()
 
 
-def _block(layer: nn.Module, width: int, device_index: int):
-    """(``cf_forward_block`` fields, heads, feed-forward width, whether it stores its exponents' statistics) of a
-    layer, or None when it is not the plain case."""
-    from .attention import CrystalformerMultiheadAttentionCUDA, fused_exponents_spec
-    from .encoder import CrystalformerEncoderLayerCUDA
+def _plain(layer: nn.Module, width: int) -> bool:
+    """Whether a layer's classes, modes and options are those of the plain case: what costs little to look at, and
+    first, so that a model of another kind hardly pays for being asked."""
     if type(layer) is not CrystalformerEncoderLayerCUDA:
-        return None
+        return False
     mods = layer._modules
     attn, lin1, lin2 = mods["self_attn"], mods["linear1"], mods["linear2"]
     if type(attn) is not CrystalformerMultiheadAttentionCUDA or type(lin1) is not nn.Linear \
             or type(lin2) is not nn.Linear or type(attn._modules.get("out_proj")) is not nn.Linear:
-        return None
+        return False
     if type(mods["norm1"]) is not nn.Identity or type(mods["norm2"]) is not nn.Identity \
             or layer.activation is not torch.nn.functional.relu:
-        return None
+        return False
     P = attn.params
     # (every module has a mode of its own: the attention's decides on its dropout and its statistics)
     if (attn.training and attn.dropout > 0) or any(type(mods[d]) is not nn.Identity and (layer.training or mods[d].training)
                                                    for d in ("dropout", "dropout1", "dropout2")):
-        return None
-    spec = fused_exponents_spec(P)
+        return False
     halves = P.domain == "multihead"               # half of the heads in reciprocal space
     if halves and (P.gauss_lb_real != P.gauss_lb_reci or attn.num_heads % 2 or width != 128 or lin1.out_features != 512
                    or ops.current_live_sizes() is not None):
-        return None
-    if (P.domain != "real" and not halves) or P.norm_func_mode not in (0, "default") or spec is None \
+        return False
+    if (P.domain != "real" and not halves) or P.norm_func_mode not in (0, "default") or fused_exponents_spec(P) is None \
             or attn.kdim != width or attn.vdim != width or attn.embed_dim != width:
+        return False
+    if P.value_pe_dist_real <= 0:                      # (without FUSE_..: the two operators asked for one by one)
+        return halves or hip_funcs.KernelManager.FUSE_ENCODING_ATTENTION
+    return P.value_pe_condproj == "no" and P.value_pe_headed and P.use_low_memory
+
+
+def _block(layer: nn.Module, width: int, device_index: int):
+    """(``cf_forward_block`` fields, heads, feed-forward width, whether it stores its exponents' statistics) of a
+    layer, or None when it is not the plain case."""
+    if not _plain(layer, width):
         return None
+    mods = layer._modules
+    attn, lin1, lin2 = mods["self_attn"], mods["linear1"], mods["linear2"]
+    P = attn.params
+    spec, halves = fused_exponents_spec(P), P.domain == "multihead"
     H = attn.num_heads
     D = width // H
     bins = max(int(P.value_pe_dist_real), 0)
-    if bins == 0 and not halves and not hip_funcs.KernelManager.FUSE_ENCODING_ATTENTION:
-        return None                                    # (the two operators asked for one by one)
-    if bins > 0 and (P.value_pe_condproj != "no" or not P.value_pe_headed or not P.use_low_memory):
-        return None
     own = attn._parameters
     out, w1, w2 = attn._modules["out_proj"]._parameters, lin1._parameters, lin2._parameters
     ff = lin1.out_features
@@ -177,13 +187,30 @@ def _embeds(model: nn.Module, x: Tensor):
             and _ready(embed.bias, 128, x.get_device()))
 
 
-def _run(encoder: nn.Module, src: Tensor, pos: Tensor, batch: Tensor, trans: Tensor, sizes: Tensor,
-         head=None, embed: Optional[nn.Module] = None) -> Optional[Tensor]:
-    KM = hip_funcs.KernelManager
-    if torch.is_grad_enabled() or config.REPRODUCIBLITY_STATE < 2 or not KM.DENSE_EDGE_BLOCKS \
-            or ops.instrumented() or encoder._modules.get("norm") is not None \
-            or _torch_module._global_forward_hooks or _torch_module._global_forward_pre_hooks or _touched(encoder):
+def _blocks(encoder: nn.Module, device_index: int):
+    """(fields of all blocks, heads, feed-forward width, whether they store statistics) or None."""
+    if torch.is_grad_enabled() or config.REPRODUCIBLITY_STATE < 2 or not hip_funcs.KernelManager.DENSE_EDGE_BLOCKS \
+            or ops.instrumented() or encoder._modules.get("norm") is not None:
         return None
+    blocks, common = [], None
+    for layer in encoder._modules["layers"]._modules.values():
+        got = _block(layer, encoder.d_model, device_index)
+        if got is None or (blocks and got[1:] != common):
+            return None                                # (one setting for all blocks: some frozen, some not)
+        blocks.append(got[0])
+        common = got[1:]
+    if not blocks or _torch_module._global_forward_hooks or _torch_module._global_forward_pre_hooks or _touched(encoder):
+        return None
+    return (blocks, *common)
+
+
+def _run(encoder: nn.Module, src: Tensor, pos: Tensor, batch: Tensor, trans: Tensor, sizes: Tensor,
+         blocks, head=None, embed: Optional[nn.Module] = None) -> Optional[Tensor]:
+    """``blocks`` from :func:`_blocks`, ``head`` from :func:`_head`; ``embed`` where ``src`` is still to be embedded."""
+    if blocks is None:
+        return None
+    blocks, H, ff, store = blocks
+    KM = hip_funcs.KernelManager
     width = encoder.d_model
     index = src.get_device()
     if index < 0 or src.dim() != 2 or trans.dim() != 3 or batch.dim() != 1:
@@ -194,18 +221,7 @@ def _run(encoder: nn.Module, src: Tensor, pos: Tensor, batch: Tensor, trans: Ten
             or trans.shape != (B, 3, 3) or not _ready(src, src.numel(), index) or not _ready(pos, 3 * N, index) \
             or not _ready(trans, 9 * B, index) or batch.get_device() != index or batch.dtype is not torch.int64:
         return None
-    blocks = []
-    H = ff = store = None
-    for layer in encoder._modules["layers"]._modules.values():
-        got = _block(layer, width, index)
-        if got is None or (blocks and got[1:] != (H, ff, store)):
-            return None                                # (one setting for all blocks: some frozen, some not)
-        fields, H, ff, store = got
-        blocks.append(fields)
-    if not blocks:
-        return None
     dev = src.device
-    from .encoder import _sizes_on_device
     if not torch.is_tensor(sizes) or sizes.device != dev or sizes.dtype != torch.long:
         sizes = _sizes_on_device(sizes, batch, B, dev)
     layout = ops.batch_layout(sizes, batch)            # index structure: built once per batch
@@ -237,13 +253,11 @@ def _run(encoder: nn.Module, src: Tensor, pos: Tensor, batch: Tensor, trans: Ten
 
 def encode(encoder: nn.Module, src: Tensor, pos: Tensor, batch: Tensor, trans: Tensor, sizes) -> Optional[Tensor]:
     """The output of ``CrystalformerEncoderCUDA.forward``, or None where it has to run module by module."""
-    return _run(encoder, src, pos, batch, trans, sizes)
+    return _run(encoder, src, pos, batch, trans, sizes, _blocks(encoder, src.get_device()))
 
 
 def forward(model: nn.Module, data) -> Tuple[Optional[Tensor], Optional[Tensor]]:
     """The output of ``Latticeformer.forward``, or None and the embedded atoms if they are there already."""
-    from .encoder import CrystalformerEncoderCUDA
-    from .latticeformer import Latticeformer, is_plain_head
     if torch.is_grad_enabled():
         return None, None
     mods = model._modules
@@ -252,14 +266,17 @@ def forward(model: nn.Module, data) -> Tuple[Optional[Tensor], Optional[Tensor]]
     if type(encoder) is not CrystalformerEncoderCUDA or "forward" in encoder.__dict__:
         return None, None
     if type(proj) is not nn.Identity or model.pooling_layer is not pooling.avr_pool \
-            or _hooked(proj) or not is_plain_head(mlp) or _touched(mlp) \
+            or _hooked(proj) or not is_plain_head(mlp) \
             or type(model)._head is not Latticeformer._head or "_head" in model.__dict__:
         return None, None
     x = data.x
+    blocks = _blocks(encoder, x.get_device())
+    if blocks is None or _touched(mlp):
+        return None, None
     head = _head(mlp, encoder.d_model, x.get_device())
     if head is None:
         return None, None
-    where = data.pos, data.batch, data.trans_vec, data.sizes, head
+    where = data.pos, data.batch, data.trans_vec, data.sizes, blocks, head
     if _embeds(model, x):
         return _run(encoder, x, *where, mods["input_embeddings"]), None
     x = hip_funcs.linear(x, model.input_embeddings.weight, model.input_embeddings.bias)

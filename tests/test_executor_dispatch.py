@@ -33,7 +33,7 @@ def small_batch():
 def natively(monkeypatch):
     """Whether a model's forward would take the native call: ``_run`` answers with a marker."""
     marker = torch.zeros(())
-    monkeypatch.setattr(executor, "_run", lambda *args: marker)
+    monkeypatch.setattr(executor, "_run", lambda *args: None if args[6] is None else marker)
 
     def ask(model):
         with torch.no_grad():
@@ -243,13 +243,13 @@ SHAPES = {"pos": lambda b: dict(pos=b.pos.T.contiguous()), "pos_flat": lambda b:
 def test_shapes_are_looked_at(monkeypatch):
     """Every batch of these shapes is declined before anything is laid out for it."""
     monkeypatch.setattr(torch.Tensor, "get_device", lambda t: 0)
-    monkeypatch.setattr(executor, "_block", lambda *args: pytest.fail("accepted"))
+    monkeypatch.setattr(executor.ops, "batch_layout", lambda *args: pytest.fail("accepted"))
     model, b = small_model(), small_batch()
     for change in SHAPES.values():
         c = dataclasses.replace(b, **change(b))
         with torch.no_grad():
-            assert executor._run(model.encoder, b.x @ model.input_embeddings.weight.T, c.pos, c.batch, c.trans_vec,
-                                 c.sizes) is None
+            assert executor.encode(model.encoder, b.x @ model.input_embeddings.weight.T, c.pos, c.batch, c.trans_vec,
+                                   c.sizes) is None
 
 
 @pytest.mark.gpu
@@ -364,3 +364,17 @@ def test_hooks_of_a_layer_in_a_fused_step(dev):
     model = small_model()
     model.encoder.layers[0].register_forward_hook(lambda m, args, out: (0.5 * out.T.contiguous()).T)
     fused_step_equals_the_plain_one(model, dev)
+
+
+def test_declined_models_are_hardly_looked_at(monkeypatch):
+    """Options decide before anything is walked or counted: a model of another kind is asked at every forward."""
+    looked = []
+    monkeypatch.setattr(executor, "_touched", lambda *args: looked.append(args) or False)
+    monkeypatch.setattr(executor, "_ready", lambda *args: looked.append(args) or True)
+    for options in (dict(domain="reci"), dict(t_fixup_init=False), dict(t_activation="gelu"),
+                    dict(value_pe_condproj="i")):
+        model, b = small_model(**options), small_batch()
+        with torch.no_grad():
+            assert executor.forward(model, b) == (None, None)
+            assert executor.encode(model.encoder, b.x, b.pos, b.batch, b.trans_vec, b.sizes) is None
+        assert not looked, options

@@ -130,17 +130,25 @@ __device__ __forceinline__ float get_raw(const float *p)
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// The exponents where no statistics are stored: the last work-group to finish merges the statistics of
-// all raw values (a holds them) as the two exponent kernels do -- groups of 256 values, mean first, then
-// the squared deviations, groups merged by Chan's formula in the same order -- and maps them in place.  Up to
-// KEPT groups a wavefront it holds the values in registers meanwhile.  An inference forward of more rows has them
-// mapped by a launch of its own (apart): the map alone keeps one work-group busy for 26 us at 8 thousand atoms
-// (seven blocks 4243 us, with the launch 4061).  With stored statistics that launch ends at once, 1% of such a forward;
-// a capacity, whose live rows are mostly fewer, and training, which has stored statistics from its second step on, do
-// without it.
+// The exponents where no statistics are stored: a holds the raw values, whose statistics are formed as the two
+// exponent kernels do -- groups of 256 values, mean first, then the squared deviations, groups merged by Chan's formula
+// in the same order.  Up to KEPT groups a wavefront the last work-group to finish holds all values in registers, forms the
+// groups' statistics, merges and maps them: 18 us a block at 2048 atoms.  Beyond, the work-group that completes a group
+// forms its statistics and the last one only merges: 10 us a block at 8192 atoms with the map, where the last work-group
+// took 33 for all of it (forwards of four blocks without value bins 712 for 797 us, 2617 for 2956 at 32768 atoms; 666 and
+// 2486 where statistics are stored).
+// The map beyond KEPT groups is a launch of its own (apart): it keeps one work-group busy for 39 us at 8192 atoms.  With
+// stored statistics that launch ends at once, 1.8 us a block.  A capacity, whose live rows are mostly fewer, takes it
+// from four times that size on (32768 atoms, all live, 2637 for 3299 us); training, which has stored statistics from its
+// second step on, does without it.
 constexpr int KEPT = 8;                      // (all values of 2048 atoms with 8 heads)
+constexpr int WAVES = RT / WAVE;
 
-__device__ __forceinline__ void group_statistics(const float (&v)[4], int64_t b, int64_t total, int lane, float *out)
+// (a kernel of its own where all values can be kept: the code costs the others 1% of a launch)
+__host__ __device__ __forceinline__ bool spread_groups(int64_t total) { return total > 256 * KEPT * WAVES; }
+
+// (count, mean, squared deviations) of group b, one wavefront.
+__device__ __forceinline__ void group_statistics(const float (&v)[4], int64_t b, int64_t total, int lane, float (&out)[3])
 {
     const float cnt = (float)min((int64_t)256, total - 256 * b);
     float s[4];
@@ -152,20 +160,54 @@ __device__ __forceinline__ void group_statistics(const float (&v)[4], int64_t b,
         const float dv = 256 * b + 64 * u + lane < total ? v[u] - mean : 0.f;
         s[u] = wave_sum(dv * dv);
     }
+    out[0] = cnt;
+    out[1] = mean;
+    out[2] = ((0.f + s[0]) + s[1]) + s[2] + s[3];
+}
+
+// The raw values of rows row0 .. row0 + rows - 1 are on their way: counts them into the groups they belong to, and forms
+// the statistics of those that are complete with them.  A tile's values are one piece (two with split heads) of at most 256,
+// so they touch two groups each: one per wavefront.
+__device__ void complete_groups(const RowsArgs &p, int64_t N, int64_t row0, int rows)
+{
+    unsigned tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));                               // (worked out here: not kept through the tile loop)
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");           // this wavefront's raw values have arrived
+    __syncthreads();
+    if (wave >= (p.split ? 4 : 2)) return;
+    const int64_t total = N * p.H;
+    const int width = p.split ? p.H / 2 : p.H;
+    const int64_t v0 = ((wave >> 1) * N + row0) * width, v1 = v0 + min((int64_t)rows, N - row0) * width;
+    const int64_t g = v0 / 256 + (wave & 1), first = 256 * g, last = min(first + 256, total);
+    if (first >= v1) return;
+    const unsigned mine = (unsigned)(min(v1, last) - max(v0, first));
+    unsigned before = 0;
+    if (lane == 0) before = atomicAdd(p.groups + g, mine);
+    before = __builtin_amdgcn_readfirstlane(before);
+    if (before + mine != (unsigned)(last - first)) return;
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    float v[4], out[3];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+        const int64_t t = first + 64 * u + lane;
+        v[u] = t < total ? get_raw(p.a + t) : 0.f;
+    }
+    group_statistics(v, g, total, lane, out);
     if (lane == 0) {
-        out[3 * b] = cnt;
-        out[3 * b + 1] = mean;
-        out[3 * b + 2] = ((0.f + s[0]) + s[1]) + s[2] + s[3];
+#pragma unroll
+        for (int i = 0; i < 3; i++) put_raw(p.part + 3 * g + i, out[i]);
+        __hip_atomic_store(p.groups + g, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 }
 
+template <bool SPREAD>
 __device__ void finish_exponents(const RowsArgs &p, int64_t total, float *red)
 {
-    constexpr int WAVES = RT / WAVE;
     __shared__ float stats[3 * KEPT * WAVES];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int64_t blocks = (total + 255) / 256;
-    const bool kept = blocks <= KEPT * WAVES;
+    const bool kept = blocks <= KEPT * WAVES, spread = SPREAD && spread_groups(total);
     float v[KEPT][4];
     auto fetch = [&](int64_t b0) {                              // this wavefront's groups b0 + wave, + 8, ...: 32 loads in flight
 #pragma unroll
@@ -176,18 +218,26 @@ __device__ void finish_exponents(const RowsArgs &p, int64_t total, float *red)
                 v[k][u] = t < total ? get_raw(p.a + t) : 0.f;
             }
     };
-    for (int64_t b0 = 0; b0 < blocks; b0 += KEPT * WAVES) {
+    for (int64_t b0 = 0; b0 < blocks && !spread; b0 += KEPT * WAVES) {
         fetch(b0);
 #pragma unroll
         for (int k = 0; k < KEPT; k++) {
             const int64_t b = b0 + wave + WAVES * k;
-            if (b < blocks) group_statistics(v[k], b, total, lane, kept ? stats : p.part);
+            float out[3];
+            if (b < blocks) group_statistics(v[k], b, total, lane, out);
+            if (b < blocks && lane == 0) {
+                float *to = (kept ? stats : p.part) + 3 * b;
+                to[0] = out[0];
+                to[1] = out[1];
+                to[2] = out[2];
+            }
         }
     }
     __syncthreads();
     if (wave == 0) {
         float n, mean, m2;
         if (kept) merge_statistics(stats, (int)blocks, lane, n, mean, m2);
+        else if (SPREAD) merge_statistics_of([&](int i) { return get_raw(p.part + i); }, (int)blocks, lane, n, mean, m2);
         else merge_statistics(p.part, (int)blocks, lane, n, mean, m2);
         if (lane == 0) {
             const float scale = 1.0f / sqrtf(m2 / (n - 1.0f));
@@ -228,6 +278,7 @@ __device__ void finish_exponents(const RowsArgs &p, int64_t total, float *red)
 }
 
 // A work-group that had rows (the first `tiles` of the grid) counts itself; the last one finishes the exponents of all.
+template <bool SPREAD>
 __device__ void finish_if_last(const RowsArgs &p, int64_t N, int64_t tiles, float *red)
 {
     const int64_t active = min((int64_t)gridDim.x, tiles);
@@ -240,7 +291,7 @@ __device__ void finish_if_last(const RowsArgs &p, int64_t N, int64_t tiles, floa
     __syncthreads();
     if (last) {
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-        finish_exponents(p, N * p.H, red);
+        finish_exponents<SPREAD>(p, N * p.H, red);
     }
 }
 
@@ -248,7 +299,7 @@ constexpr int FINISH_T = 256, FINISH_VALUES = 4 * FINISH_T;
 __global__ __launch_bounds__(FINISH_T) void finish_exponents_kernel(RowsArgs p)
 {
     if (*p.counter == 0) return;                                // stored statistics: mapped already
-    const int64_t total = p.N * p.H;
+    const int64_t total = live_count(p.live_N, p.N) * p.H;
     const float scale = p.part[0], shift = p.part[1];
 #pragma unroll
     for (int u = 0; u < 4; u++) {
@@ -272,7 +323,7 @@ __device__ __forceinline__ void pack_weights(const PackArgs &p, int x, int l, bo
 {
     const int u = x / (UNIT_FLOATS / 1024);
     if (p.zero && x == 0 && l == 0 && !transposed)
-        for (int t = threadIdx.x; t < p.words; t += 256) p.zero[t] = 0u;
+        for (int64_t t = threadIdx.x; t < p.words; t += 256) p.zero[t] = 0u;
     if (l == p.blocks && u > 0) return;
     const int at = 4 * (int)(x % (UNIT_FLOATS / 1024) * 256 + threadIdx.x);             // first of four floats of the unit
     const int wave = at / 2048, k = at / 256 % 8 * 16 + at / 64 % 4 * 4, col = 16 * wave + at / 4 % 16;
@@ -335,8 +386,8 @@ __global__ __launch_bounds__(256) void forward_prologue_kernel(PackArgs k, Prolo
     if (b < p.B) lattice_geometry_of(p.trans, b, p.vcell, p.recip, p.rvlen);
 }
 
-template <int R, int SRC, bool HEAD>
-__global__ __launch_bounds__(RT) void block_rows_kernel(RowsArgs p)
+template <int R, int SRC, bool HEAD, bool SPREAD>
+__global__ __launch_bounds__(RT, SPREAD && R == 2 ? 4 : 2) void block_rows_kernel(RowsArgs p)
 {
     constexpr int M = 4 * R;
     constexpr int FIRST = SRC == ROWS_TAIL ? 0 : SRC == ROWS_EMBED ? UNIT_EMBED : UNIT_QUERY;
@@ -498,9 +549,10 @@ __global__ __launch_bounds__(RT) void block_rows_kernel(RowsArgs p)
                 }
             }
         }
+        if (SPREAD && !stored && spread_groups(N * p.H)) complete_groups(p, N, row0, M);
         __syncthreads();                                        // the next tile overwrites the rows
     }
-    if (HEAD && !stored) finish_if_last(p, N, (N + M - 1) / M, red);
+    if (HEAD && !stored) finish_if_last<SPREAD>(p, N, (N + M - 1) / M, red);
 }
 
 // ---- training ------------------------------------------------------------------
@@ -669,7 +721,7 @@ __global__ __launch_bounds__(RT) void block_head_train_kernel(RowsArgs p)
             put_raw(p.a + at, alpha);
         }
     }
-    if (!stored) finish_if_last(p, N, (N + TM - 1) / TM, red);
+    if (!stored) finish_if_last<false>(p, N, (N + TM - 1) / TM, red);
 }
 
 // tail: from gy, the gradient behind the block,  gh = (gy W2) where h > 0,  gs = gh W1 + gy,  gatt = gs Wo
@@ -886,13 +938,13 @@ int rows_per_quad(int64_t N)
     return N <= 4 * cus ? 1 : N <= 8 * cus ? 2 : ceil(rounds) * 0.85 <= rounds ? 4 : 2;
 }
 
-template <int R>
+template <int R, bool SPREAD>
 void launch_rows(const RowsArgs &p, int source, bool head, unsigned grid, hipStream_t st)
 {
-    if (source == ROWS_TAIL && head) block_rows_kernel<R, ROWS_TAIL, true><<<grid, RT, 0, st>>>(p);
-    else if (source == ROWS_TAIL) block_rows_kernel<R, ROWS_TAIL, false><<<grid, RT, 0, st>>>(p);
-    else if (source == ROWS_EMBED) block_rows_kernel<R, ROWS_EMBED, true><<<grid, RT, 0, st>>>(p);
-    else block_rows_kernel<R, ROWS_PLAIN, true><<<grid, RT, 0, st>>>(p);
+    if (source == ROWS_TAIL && head) block_rows_kernel<R, ROWS_TAIL, true, SPREAD><<<grid, RT, 0, st>>>(p);
+    else if (source == ROWS_TAIL) block_rows_kernel<R, ROWS_TAIL, false, false><<<grid, RT, 0, st>>>(p);
+    else if (source == ROWS_EMBED) block_rows_kernel<R, ROWS_EMBED, true, SPREAD><<<grid, RT, 0, st>>>(p);
+    else block_rows_kernel<R, ROWS_PLAIN, true, SPREAD><<<grid, RT, 0, st>>>(p);
 }
 
 }  // namespace
@@ -932,10 +984,13 @@ int launch_block_rows(RowsArgs p, hipStream_t st)
     int64_t grid = (p.N + 4 * R - 1) / (4 * R);
     if (p.live_N && grid > 2 * cus) grid = 2 * cus;             // a capacity: stride over the tiles that exist
     CF_REQUIRE(grid < (1ll << 31), CF_ERR_UNSUPPORTED, "block rows: too many atoms");
-    p.apart = head && p.normalize && !p.live_N && p.N * p.H > 256 * KEPT * (RT / WAVE);
-    if (R == 1) launch_rows<1>(p, source, head, (unsigned)grid, st);
-    else if (R == 2) launch_rows<2>(p, source, head, (unsigned)grid, st);
-    else launch_rows<4>(p, source, head, (unsigned)grid, st);
+    const bool spread = head && p.normalize && p.groups && spread_groups(p.N * p.H);
+    p.apart = spread && (!p.live_N || spread_groups(p.N * p.H / 4));
+    if (spread && R == 4) launch_rows<4, true>(p, source, head, (unsigned)grid, st);
+    else if (spread) launch_rows<2, true>(p, source, head, (unsigned)grid, st);
+    else if (R == 1) launch_rows<1, false>(p, source, head, (unsigned)grid, st);
+    else if (R == 2) launch_rows<2, false>(p, source, head, (unsigned)grid, st);
+    else launch_rows<4, false>(p, source, head, (unsigned)grid, st);
     CF_CHECK_LAUNCH("block rows");
     if (p.apart) {
         finish_exponents_kernel<<<(unsigned)((p.N * p.H + FINISH_VALUES - 1) / FINISH_VALUES), FINISH_T, 0, st>>>(p);
@@ -977,7 +1032,7 @@ extern "C" int cf_pack_blocks(int64_t blocks, const float *const *weights, float
         a.packed_bwd = packed_bwd ? packed_bwd + first * cf::PACKED_BLOCK : nullptr;
         if (first == 0) {
             a.zero = (unsigned *)zero_words;
-            a.words = (int)words;
+            a.words = words;
         }
         const int rc = cf::launch_pack_weights(a, (hipStream_t)stream);
         if (rc) return rc;

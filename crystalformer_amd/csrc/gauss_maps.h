@@ -36,12 +36,13 @@ __device__ __forceinline__ void stat_merge(float &n, float &mean, float &m2, flo
     n = nt;
 }
 
-// (count, mean, M2) of all blocks, three floats each in `part`, by one wavefront in one fixed order; the same in
-// every lane.
-__device__ __forceinline__ void merge_statistics(const float *part, int blocks, int lane, float &n, float &mean, float &m2)
+// (count, mean, M2) of all blocks, three floats each (`part(i)` is the i-th), by one wavefront in one fixed order;
+// the same in every lane.
+template <class Part>
+__device__ __forceinline__ void merge_statistics_of(Part part, int blocks, int lane, float &n, float &mean, float &m2)
 {
     n = mean = m2 = 0.f;
-    for (int b = lane; b < blocks; b += WAVE) stat_merge(n, mean, m2, part[3 * b], part[3 * b + 1], part[3 * b + 2]);
+    for (int b = lane; b < blocks; b += WAVE) stat_merge(n, mean, m2, part(3 * b), part(3 * b + 1), part(3 * b + 2));
 #pragma unroll
     for (int off = 1; off < WAVE; off <<= 1) {
         const float nb = __shfl_xor(n, off, WAVE), mb = __shfl_xor(mean, off, WAVE),
@@ -52,6 +53,11 @@ __device__ __forceinline__ void merge_statistics(const float *part, int blocks, 
         stat_merge(n0, m0, q0, n1, m1, q1);
         n = n0; mean = m0; m2 = q0;
     }
+}
+
+__device__ __forceinline__ void merge_statistics(const float *part, int blocks, int lane, float &n, float &mean, float &m2)
+{
+    merge_statistics_of([=](int i) { return part[i]; }, blocks, lane, n, mean, m2);
 }
 
 }  // namespace cf

@@ -27,10 +27,10 @@ struct Carver {
 struct Buffers {
     float *rvlen, *rpos, *x[2], *h, *q, *k, *v, *qs, *a, *att, *z, *val, *prob, *rings, *pooled, *hidden;
     void *stats, *flags;
-    unsigned *counters;
+    unsigned *counters, *groups;
     float *packed;
     float *vcell, *recip, *kr, *sumexp;
-    int64_t stats_bytes, flag_bytes;
+    int64_t stats_bytes, flag_bytes, words;
 };
 
 // Whether the blocks with value bins start from staged rings, and the bytes these take.
@@ -62,6 +62,7 @@ void head_of(RowsArgs &r, const cf_forward_args &f, const cf_forward_block &p, c
     r.qs = b.qs; r.k = b.k; r.v = b.v; r.a = b.a;
     r.part = (float *)b.stats;
     r.counter = b.counters + l;
+    r.groups = b.groups;
 }
 
 int64_t carve(const cf_forward_args &f, const cf_forward_block *blocks, char *base, Buffers &b)
@@ -94,7 +95,9 @@ int64_t carve(const cf_forward_args &f, const cf_forward_block *blocks, char *ba
     b.stats_bytes = cf_gauss_exponents_workspace(N, f.H);
     b.stats = c.take<char>(b.stats_bytes);
     b.packed = rows ? c.take<float>(f.layers * PACKED_BLOCK + W * W) : nullptr;
-    b.counters = c.take<unsigned>(f.layers);
+    b.words = f.layers + (N * f.H + 255) / 256;
+    b.counters = c.take<unsigned>(b.words);
+    b.groups = b.counters + f.layers;
     b.flag_bytes = rings ? cf_real_enc_flag_bytes(U, f.H) : 0;
     b.flags = rings ? c.take<char>(b.flag_bytes) : nullptr;
     b.rings = rings ? c.take<float>(cf_real_enc_ring_bytes(U) / 4) : nullptr;
@@ -173,7 +176,7 @@ extern "C" int cf_forward(const cf_forward_args *f_, const cf_forward_block *blo
                 a.packed_embed = b.packed + f.layers * PACKED_BLOCK;
             }
             a.zero = b.counters;
-            a.words = (int)f.layers;
+            a.words = b.words;
             const PrologueArgs g{f.B, E, f.atom_start, f.edge_start, f.pos, f.tvecs, b.rpos, b.vcell, b.recip, b.rvlen, nullptr};
             if ((rc = launch_forward_prologue(a, g, (hipStream_t)stream))) return rc;
         }

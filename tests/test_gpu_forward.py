@@ -5,6 +5,7 @@ import pytest
 import torch
 
 from crystalformer_amd import executor, hip_funcs
+from crystalformer_amd.graphs import GraphedForward
 from crystalformer_amd.latticeformer import Latticeformer, default_params
 from crystalformer_amd.synthetic import CrystalBatch, make_batch
 from oracle import torch_model as om
@@ -139,6 +140,41 @@ def test_batch_statistics_of_many_atoms(dev, atoms, domain):
     b = batch_of(sizes).to(dev)
     native, modules = both_ways(model, b)
     assert_close(native, modules, "encoder", rtol=RTOL, atol=atol_rows(modules))
+
+
+# tiles of 4, 8 and 16 rows against groups of 256 values; the last group short; capacities below and above the one from
+# which the map is a launch of its own
+@pytest.mark.parametrize("heads,domain", [(4, "real"), (8, "real"), (16, "real"), (8, "multihead")])
+@pytest.mark.parametrize("atoms", [4095, 4096, 4098, 5601, 9001])
+def test_spread_statistics(dev, atoms, heads, domain):
+    """Statistics of groups formed by whichever work-group completes them: the module path's results, the same bits for
+    every pass over the same batch, and from a capacity graph those of the eager call."""
+    sizes = [8] * (atoms // 8) + ([atoms % 8] if atoms % 8 else [])
+    model = scaled(default_params(num_layers=3, value_pe_dist_real=0, domain=domain, head_num=heads,
+                                  adaptive_cutoff_sigma=0.0)).to(dev).eval()
+    b = batch_of(sizes).to(dev)
+    native, modules = both_ways(model, b)
+    assert_close(native, modules, "encoder", rtol=RTOL, atol=atol_rows(modules))
+    again, _ = both_ways(model, b)
+    assert torch.equal(native, again)
+    if domain == "real":
+        with torch.no_grad():
+            eager = model(b)
+        for capacity in (atoms + 8, 33000):
+            graph = GraphedForward(model, b, capacity=(len(sizes) + 4, capacity, 8 * capacity))
+            for _ in range(3):
+                assert torch.equal(graph(b), eager)
+    stored = []
+    for native_call in (True, False):
+        m = scaled(default_params(num_layers=1, value_pe_dist_real=0, domain=domain, head_num=heads,
+                                  adaptive_cutoff_sigma=0.0)).to(dev).train()
+        if not native_call:
+            m.encoder.layers[0].register_forward_hook(lambda *args: None)
+        with torch.no_grad():
+            m(b)
+        stored.append(m.encoder.layers[0].self_attn.gauss_scale.clone())
+    # (raw values summed in another order by the two paths' projections)
+    assert_close(stored[0], stored[1], "statistics", rtol=RTOL)
 
 
 def test_training_mode_without_gradients_stores_the_statistics(dev):

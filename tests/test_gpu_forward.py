@@ -104,10 +104,13 @@ def test_native_forward_with_its_head(dev, options):
 
 # rows: one work-group's tile of 4, 8 and 16 rows less one, exactly, plus one; either side of the row counts at
 # which the tile grows (four and eight rows per CU, one full round of sixteen)
-@pytest.mark.parametrize("atoms", [1, 3, 4, 5, 1023, 1025, 2047, 2049, 3480, 3490, 4097])
-def test_row_kernel_tiles_against_float64(dev, atoms):
-    """Embedding, tail and head of the 128-wide blocks on crystals of up to 16 atoms, encoder against the module
-    path and the last block's row-wise half against float64."""
+ROW_TILES = [1, 3, 4, 5, 1023, 1025, 2047, 2049, 3480, 3490, 4097]
+
+
+@pytest.mark.parametrize("atoms", ROW_TILES)
+def test_row_kernel_tiles_and_head(dev, atoms):
+    """Embedding, tail and head of the 128-wide blocks on crystals of up to 16 atoms against the module path, pooling and
+    the regression head on the encoder's output against float64."""
     torch.manual_seed(atoms)
     sizes = [16] * (atoms // 16) + ([atoms % 16] if atoms % 16 else [])
     model = scaled(default_params(num_layers=2, value_pe_dist_real=0)).to(dev).eval()
@@ -128,6 +131,33 @@ def test_row_kernel_tiles_against_float64(dev, atoms):
             ref = torch.nn.functional.linear(ref, m.weight.double(), m.bias.double()) if hasattr(m, "weight") else m(ref)
     assert_close(y, want, "model", rtol=RTOL)
     assert_close(y, ref.float(), "head", rtol=RTOL)
+
+
+@pytest.mark.parametrize("atoms", ROW_TILES)
+def test_row_kernel_tiles_against_float64(dev, atoms):
+    """Embedding, tail and head of the 128-wide blocks on crystals of up to 8 atoms: the encoder alone and the whole
+    model against the oracle in float64, under the batch's statistics (every exponent is in them) and stored ones."""
+    torch.manual_seed(atoms)
+    sizes = [8] * (atoms // 8) + ([atoms % 8] if atoms % 8 else [])
+    cfg = default_params(num_layers=2, value_pe_dist_real=0, adaptive_cutoff_sigma=0.0)
+    model = scaled(cfg).eval()
+    b = batch_of(sizes)
+    b64 = CrystalBatch(b.x.double(), b.pos.double(), b.batch, b.trans_vec.double(), b.sizes)
+    x = torch.nn.functional.linear(b.x, model.input_embeddings.weight.detach())
+    on_gpu = b.to(dev)
+    for stored in (False, True):
+        if stored:
+            for layer in model.encoder.layers:
+                layer.self_attn.gauss_scale.data.copy_(torch.tensor([0.7, -0.2]))
+        P = {k: v.detach().cpu().double() for k, v in model.state_dict().items()}
+        want_y = om.latticeformer_forward(P, cfg, b64)
+        want = om.encoder_forward(P, cfg, x.double(), b64.pos, b.batch, b64.trans_vec, b.sizes)
+        model.to(dev)
+        with torch.no_grad():
+            got = executor.encode(model.encoder, x.to(dev), on_gpu.pos, on_gpu.batch, on_gpu.trans_vec, on_gpu.sizes)
+            y = executor.forward(model, on_gpu)[0]
+        assert_close(got, want, "encoder", rtol=RTOL, atol=atol_rows(want))
+        assert_close(y, want_y, "model", rtol=RTOL)
 
 
 @pytest.mark.parametrize("domain", ["real", "multihead"])

@@ -10,8 +10,9 @@
 // A work-group of 8 wavefronts owns 4 R rows; the rows and all intermediates stay in LDS, the weights
 // (786 KB a block) stream from the L2, a 16-column tile per wavefront, two tiles ahead of their use.  At 64
 // bytes a clock a CU reads the weights in 5 us, and at 4 R = 8 rows the matrix cores (256 FLOP a clock and
-// CU) need as long; measured 14.2 us a launch with tail and head at 1774 rows (R 2), 10.1 at 12 rows (R 1), 20.3
-// at 4096 (R 4), against 35 us as six launches.  Variants: weights read from the matrices as they are 24 us (see
+// CU) need as long; measured back to back, with the weights in the L2, 14.2 us a launch with tail and head at 1774 rows
+// (R 2), 10.1 at 12 rows (R 1), 20.3 at 4096 (R 4), against 35 us as six launches; inside a forward, where other kernels
+// have run in between, 17.6, 13.7 and 25.8 us (kernel trace under profiles/).  Variants: weights read from the matrices as they are 24 us (see
 // pack_weights_kernel); every 16-column tile with its own read of the rows, its own epilogue and a barrier 16.5 us.
 //
 // v_mfma_f32_4x4x1_16b_f32: sixteen independent 4 x 4 blocks, here 4 column groups x 4 reduction slots.
@@ -316,8 +317,8 @@ constexpr int UNIT_FF1 = 1, UNIT_FF2 = 5, UNIT_EMBED = 8, UNIT_QUERY = 9, UNIT_E
 
 // The weights of up to PACK_BLOCKS blocks in the order the row kernel reads them: per unit and wavefront eight
 // 1 KB pieces, one per 16 reduction steps, in lane order.  Read from the matrices themselves every load
-// of a wavefront takes 64 bytes of 16 rows, 512 or 2048 bytes apart, which fall into a few of the L2's
-// channels: 24 us a launch.
+// of a wavefront takes 64 bytes of 16 rows, 512 or 2048 bytes apart: 24 us a launch (by the addresses these
+// fall into a few of the L2's channels; counters were not taken).
 constexpr int PACK_GRID = UNIT_END * UNIT_FLOATS / 1024;       // work-groups of 256 threads a block
 __device__ __forceinline__ void pack_weights(const PackArgs &p, int x, int l, bool transposed)
 {

@@ -45,7 +45,9 @@ bool use_rings(const cf_forward_args &f, int64_t U)
 // whatever the batch; the pair kernel, which stages for itself, is one.  Against that the rings' rounds are cheaper: 11.2
 // for 14.7 us at 4.1 thousand pairs in the fixed cube, 21.7 for 28.4 at 12.7 thousand, and at 29 thousand with nearly all
 // pairs in the cube 52 for 61 with everything counted.  So the rings from three rounds of the whole chip on (a unit per
-// wavefront, 16 a CU).  Where many pairs leave the cube the pair kernel stays ahead: 36.6 for 45.5 us at 12.7 thousand.
+// wavefront, 16 a CU).  The rule does not see how many pairs leave the cube, which only the device knows: where most do the
+// pair kernel would stay ahead above that line too, 36.6 for 45.5 us at 12.7 thousand pairs and 486 to 489 for 514 to 522
+// in the blocks of the seven-block model with r0 = 3, two thirds of whose pairs leave it.
 bool adaptive_rings_pay(int64_t U) { return U > 48 * (int64_t)device_cu_count(); }
 
 // Whether everything between two attentions runs as one launch.

@@ -2,10 +2,12 @@
 
 :func:`encode` and :func:`forward` run the encoder -- the latter with pooling and the regression
 head behind it -- through ``cf_forward``, which issues every launch from C++.  They serve the plain
-case (real domain, no norm layers, ReLU, softmax attention, exponents from the query, one value
-projection per head) without autograd and return ``None`` for everything else: other options,
-modules replaced by a user's own, forward hooks (which must see the intermediate outputs), kernel
-timing and counting.  The callers then run the modules one by one, with the same operators.
+case (real space, or for 128-wide blocks half of the heads in reciprocal space; no norm layers, ReLU,
+softmax attention, exponents from the query, one value projection per head) without autograd and
+return ``None`` for everything else: other options, modules or forwards replaced by a user's own,
+parameters worked out from others, blocks that do not agree on their mode, inputs of other shapes,
+forward hooks (which must see the intermediate outputs), kernel timing and counting.  The callers
+then run the modules one by one, with the same operators.
 """
 from __future__ import annotations
 
@@ -234,8 +236,9 @@ def _run(encoder: nn.Module, src: Tensor, pos: Tensor, batch: Tensor, trans: Ten
     args = _lib.ForwardArgs(
         N, layout.num_edges, sizes.numel(), len(blocks), H, width, ff, KM.LATTICE_RANGE, KM.MINIMUM_RANGE, 1,
         int(store), int(KM.STAGED_RINGS), int(KM.ADAPTIVE_RINGS), ops.STAGED_RINGS_MAX_BYTES, hidden,
-        targets, embed.in_features if embed else 0, src.data_ptr(), pos.data_ptr(), trans.data_ptr(), layout.batch.data_ptr(), layout.atom_start.data_ptr(),
-        layout.edge_start.data_ptr(), layout.edges.data_ptr(), layout.e_start.data_ptr(), layout.pairs.data_ptr(),
+        targets, embed.in_features if embed else 0, src.data_ptr(), pos.data_ptr(), trans.data_ptr(),
+        layout.batch.data_ptr(), layout.atom_start.data_ptr(), layout.edge_start.data_ptr(), layout.edges.data_ptr(),
+        layout.e_start.data_ptr(), layout.pairs.data_ptr(),
         _address(sched), *(_address(t) for t in tensors),
         *((_address(embed.weight), _address(embed.bias)) if embed else (None, None)), out.data_ptr())
     table = (_lib.ForwardBlock * len(blocks))(*(tuple(f) for f in blocks))

@@ -677,8 +677,8 @@ class BlockHeadHIP(torch.autograd.Function):
         got = _weight_gradients([(g, x, w, leaf, bias, i * W, need[1 + i], want_b)
                                  for i, (g, w, leaf) in enumerate(zip(gs, (wq, wk, wv), weights))])
         gb = torch.cat([b for _, b in got]) if want_b and got[0][1] is not None else None
-        return (gx if need[0] else None, *(w for w, _ in got), gb, gw_pos.view(w_pos.shape) if need[5] and gw_pos is not None else None,
-                *(None,) * 10)
+        gw_pos = gw_pos.view(w_pos.shape) if need[5] and gw_pos is not None else None
+        return (gx if need[0] else None, *(w for w, _ in got), gb, gw_pos, *(None,) * 10)
 
 
 class BlockTailHIP(torch.autograd.Function):

@@ -40,7 +40,8 @@ class ForwardArgs(ctypes.Structure):
                                      "adaptive", "update_stats", "staged_rings", "adaptive_rings", "ring_limit_bytes",
                                      "hidden", "targets", "embed_width")]
                 + [(n, _ptr) for n in ("x", "pos", "tvecs", "batch", "atom_start", "edge_start", "edges", "e_start",
-                                       "pairs", "sched", "w_head", "b_head", "w_last", "b_last", "w_embed", "b_embed", "out")])
+                                       "pairs", "sched", "w_head", "b_head", "w_last", "b_last", "w_embed", "b_embed",
+                                       "out")])
 
 
 # name -> (restype, argtypes); mirrors include/crystalformer_hip.h

@@ -1200,7 +1200,8 @@ def block_head_bwd(ga, gqs, gk, gv, carry, q: Tensor, w_pos: Tensor, alpha_n: Te
             or (ga is not None and ga.shape != alpha_n.shape) \
             or any(t is not None and t.shape != q.shape for t in (gqs, gk, gv, carry)) \
             or not (used is None or (_plain_f32(used, dev) and used.numel() == 2)):
-        raise _lib.CrystalformerHipError("block_head_bwd: operands of block_head and gradients of its outputs' shapes expected")
+        raise _lib.CrystalformerHipError("block_head_bwd: operands of block_head and gradients of its outputs' shapes "
+                                         "expected")
     _require_packed(packed_bwd, dev)
     lib = _lib.load()
     gq, gx = torch.empty((2, N, W), dtype=torch.float32, device=dev).unbind(0)

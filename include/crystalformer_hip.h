@@ -481,9 +481,9 @@ int cf_linear_weight_grad(const float *g, const float *x, int64_t N, int64_t C, 
  * Inference forward of the encoder -- and, with targets > 0, of mean pooling and the regression head --
  * in one call that issues every launch: what CrystalformerEncoderCUDA.forward
  * (models/indexed_latticeformer_encoder.py:872-890) and Latticeformer.forward
- * (models/latticeformer.py:291-302) do operator by operator, for blocks in the real domain without norm
- * layers (t-fixup), with ReLU, the plain softmax, one value projection per head and exponents from the
- * query.  The index structure of the batch (edges, row offsets, pair list) comes from cf_batch_layout.
+ * (models/latticeformer.py:291-302) do operator by operator, for blocks in real space, or with half of
+ * their heads in reciprocal space (coef_reci), without norm layers (t-fixup), with ReLU, the plain softmax,
+ * one value projection per head and exponents from the query.  The index structure of the batch (edges, row offsets, pair list) comes from cf_batch_layout.
  * With a size header set, N and E are the capacities (see cf_set_size_header).
  */
 typedef struct {

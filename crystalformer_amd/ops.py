@@ -1138,7 +1138,7 @@ class PackedBlocks:
                                                  "hidden units expected")
         lib = _lib.load()
         L = len(blocks)
-        self.floats = int(lib.cf_pack_blocks_floats(1))
+        self.floats = PACKED_BLOCK_FLOATS
         self.forward = torch.empty(L * self.floats, dtype=torch.float32, device=dev)
         self.backward = torch.empty(L * self.floats, dtype=torch.float32, device=dev)
         self.counters = torch.empty(L, dtype=torch.int32, device=dev)
@@ -1155,9 +1155,12 @@ class PackedBlocks:
                 self.counters[index:index + 1])
 
 
-def _require_packed(packed: Tensor, dev: torch.device) -> None:
-    if not _plain_f32(packed, dev) or packed.numel() != _lib.load().cf_pack_blocks_floats(1):
-        raise _lib.CrystalformerHipError("packed weights of one block expected (PackedBlocks.block)")
+PACKED_BLOCK_FLOATS = 12 * 128 * 128      # cf_pack_blocks_floats(1)
+
+
+def _rows_of(t: Optional[Tensor], numel: int) -> bool:
+    """Whether ``t`` is None or ``numel`` contiguous float32 values (its device is looked at by require_device)."""
+    return t is None or (t.numel() == numel and t.dtype is torch.float32 and t.is_contiguous())
 
 
 def block_head(x: Tensor, heads: int, packed: Tensor, counter: Tensor, b_in: Optional[Tensor], w_pos: Tensor,
@@ -1165,15 +1168,13 @@ def block_head(x: Tensor, heads: int, packed: Tensor, counter: Tensor, b_in: Opt
                lower_bound: float, coef: float, q_scale: float):
     """Query, key and value projections and the Gaussian exponents of a 128-wide block in one launch:
     ``(a, qs, k, v, q, alpha_n, used)`` as :func:`linear_rows` and :func:`gauss_exponents` give them."""
-    dev = require_device(x, packed, b_in, w_pos, gauss_scale)
+    dev = require_device(x, packed, counter, b_in, w_pos, gauss_scale)
     N, W = x.shape
-    if W != 128 or not _plain_f32(x, dev) or positive_func not in POSITIVE_FUNCS or w_pos.numel() != W \
-            or not _plain_f32(w_pos, dev) or not _plain_f32(gauss_scale, dev) or gauss_scale.numel() != 2 \
-            or not (b_in is None or (_plain_f32(b_in, dev) and b_in.numel() == 3 * W)) \
-            or counter.dtype is not torch.int32 or counter.get_device() != dev.index or counter.numel() < 1:
+    if W != 128 or not _rows_of(x, N * W) or positive_func not in POSITIVE_FUNCS or not _rows_of(w_pos, W) \
+            or not _rows_of(gauss_scale, 2) or not _rows_of(b_in, 3 * W) or not _rows_of(packed, PACKED_BLOCK_FLOATS) \
+            or counter.dtype is not torch.int32 or counter.numel() < 1:
         raise _lib.CrystalformerHipError("block_head: contiguous float32 rows of 128 and their block's parameters expected")
     lib = _lib.load()
-    _require_packed(packed, dev)
     q, qs, k, v = torch.empty((4, N, W), dtype=torch.float32, device=dev).unbind(0)
     a, alpha_n = torch.empty((2, N, heads), dtype=torch.float32, device=dev).unbind(0)
     used = torch.empty(2, dtype=torch.float32, device=dev) if normalize else None
@@ -1192,17 +1193,15 @@ def block_head_bwd(ga, gqs, gk, gv, carry, q: Tensor, w_pos: Tensor, alpha_n: Te
                    packed_bwd: Tensor, positive_func: str, beta: float, lower_bound: float, coef: float, q_scale: float):
     """(gq, gx, gw_pos) from the gradients of :func:`block_head`'s ``a``, ``qs``, ``k``, ``v`` and of the input's other
     uses (``carry``), None where there is none."""
-    dev = require_device(ga, gqs, gk, gv, carry, q, packed_bwd)
+    dev = require_device(ga, gqs, gk, gv, carry, q, w_pos, alpha_n, used, packed_bwd)
     ga, gqs, gk, gv, carry = (_f32(t, "gradient") for t in (ga, gqs, gk, gv, carry))
     N, W = q.shape
-    if W != 128 or not _plain_f32(q, dev) or not _plain_f32(w_pos, dev) or w_pos.numel() != W \
-            or not _plain_f32(alpha_n, dev) or alpha_n.dim() != 2 or alpha_n.shape[0] != N \
-            or (ga is not None and ga.shape != alpha_n.shape) \
-            or any(t is not None and t.shape != q.shape for t in (gqs, gk, gv, carry)) \
-            or not (used is None or (_plain_f32(used, dev) and used.numel() == 2)):
+    n, nh = N * W, N * alpha_n.shape[1]
+    if W != 128 or not (_rows_of(q, n) and _rows_of(gqs, n) and _rows_of(gk, n) and _rows_of(gv, n) and _rows_of(carry, n)
+                        and _rows_of(alpha_n, nh) and _rows_of(ga, nh) and _rows_of(w_pos, W) and _rows_of(used, 2)
+                        and _rows_of(packed_bwd, PACKED_BLOCK_FLOATS)):
         raise _lib.CrystalformerHipError("block_head_bwd: operands of block_head and gradients of its outputs' shapes "
                                          "expected")
-    _require_packed(packed_bwd, dev)
     lib = _lib.load()
     gq, gx = torch.empty((2, N, W), dtype=torch.float32, device=dev).unbind(0)
     gw = torch.empty(W, dtype=torch.float32, device=dev) if ga is not None else None
@@ -1224,10 +1223,10 @@ def block_tail(att: Tensor, x: Tensor, packed: Tensor, bo: Optional[Tensor], b1:
     128-wide block with 512 hidden units, in one launch."""
     dev = require_device(att, x, packed, bo, b1, b2)
     N, W = x.shape
-    if W != 128 or att.shape != x.shape or not _plain_f32(x, dev) or not _plain_f32(att, dev) or any(
-            b is not None and (not _plain_f32(b, dev) or b.numel() != n) for b, n in ((bo, W), (b1, 512), (b2, W))):
+    if W != 128 or att.shape != x.shape or not (_rows_of(x, N * W) and _rows_of(att, N * W) and _rows_of(bo, W)
+                                                and _rows_of(b1, 512) and _rows_of(b2, W)
+                                                and _rows_of(packed, PACKED_BLOCK_FLOATS)):
         raise _lib.CrystalformerHipError("block_tail: contiguous float32 rows of 128 and their block's biases expected")
-    _require_packed(packed, dev)
     s, y = torch.empty((2, N, W), dtype=torch.float32, device=dev).unbind(0)
     h = torch.empty((N, 512), dtype=torch.float32, device=dev)
     with device_guard(dev):
@@ -1242,9 +1241,8 @@ def block_tail_bwd(gy: Tensor, h: Tensor, packed_bwd: Tensor) -> Tuple[Tensor, T
     dev = require_device(gy, h, packed_bwd)
     gy = _f32(gy, "gy")
     N, W = gy.shape
-    if W != 128 or not _plain_f32(h, dev) or h.shape != (N, 512):
+    if W != 128 or not _rows_of(h, N * 512) or not _rows_of(packed_bwd, PACKED_BLOCK_FLOATS):
         raise _lib.CrystalformerHipError("block_tail_bwd: a gradient (N,128) and the hidden units (N,512) expected")
-    _require_packed(packed_bwd, dev)
     gs, gatt = torch.empty((2, N, W), dtype=torch.float32, device=dev).unbind(0)
     gh = torch.empty_like(h)
     with device_guard(dev):

@@ -23,7 +23,7 @@ struct RowsArgs {
     float *q, *alpha_n, *used;                //   the query, the normalised alpha, the (scale, shift) applied
     float *part;                              // statistics without stored ones: 3 floats per 256 values of a
     unsigned *counter;                        // zeroed word
-    unsigned *groups;                         // nullable: such a word per 256 values, left zero again
+    unsigned *groups;                         // inference: such a word per 256 values, left zero again
     int apart;                                // set by the launcher: such exponents are mapped by a launch of their own
     const int64_t *live_N;                    // set by the launcher
 };

@@ -138,10 +138,10 @@ __device__ __forceinline__ float get_raw(const float *p)
 // forms its statistics and the last one only merges: 10 us a block at 8192 atoms with the map, where the last work-group
 // took 33 for all of it (forwards of four blocks without value bins 712 for 797 us, 2617 for 2956 at 32768 atoms; 666 and
 // 2486 where statistics are stored).
-// The map beyond KEPT groups is a launch of its own (apart): it keeps one work-group busy for 39 us at 8192 atoms.  With
-// stored statistics that launch ends at once, 1.8 us a block.  A capacity, whose live rows are mostly fewer, takes it
-// from four times that size on (32768 atoms, all live, 2637 for 3299 us); training, which has stored statistics from its
-// second step on, does without it.
+// The map beyond KEPT groups is a launch of its own (apart): it keeps one work-group busy for 28 us at 8192 atoms (39 without
+// asking for the next values ahead).  With stored statistics that launch ends at once, 1.8 us a block.  A capacity, whose
+// live rows are mostly fewer, takes it from four times that size on (32768 atoms, all live, 2629 us; 3299 with one work-group);
+// training, which has stored statistics from its second step on, does without it.
 constexpr int KEPT = 8;                      // (all values of 2048 atoms with 8 heads)
 constexpr int WAVES = RT / WAVE;
 
@@ -208,7 +208,7 @@ __device__ void finish_exponents(const RowsArgs &p, int64_t total, float *red)
     __shared__ float stats[3 * KEPT * WAVES];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int64_t blocks = (total + 255) / 256;
-    const bool kept = blocks <= KEPT * WAVES, spread = SPREAD && spread_groups(total);
+    const bool kept = !spread_groups(total);
     float v[KEPT][4];
     auto fetch = [&](int64_t b0) {                              // this wavefront's groups b0 + wave, + 8, ...: 32 loads in flight
 #pragma unroll
@@ -219,7 +219,7 @@ __device__ void finish_exponents(const RowsArgs &p, int64_t total, float *red)
                 v[k][u] = t < total ? get_raw(p.a + t) : 0.f;
             }
     };
-    for (int64_t b0 = 0; b0 < blocks && !spread; b0 += KEPT * WAVES) {
+    for (int64_t b0 = 0; b0 < blocks && !(SPREAD && !kept); b0 += KEPT * WAVES) {
         fetch(b0);
 #pragma unroll
         for (int k = 0; k < KEPT; k++) {
@@ -266,14 +266,24 @@ __device__ void finish_exponents(const RowsArgs &p, int64_t total, float *red)
         if (p.alpha_n) p.alpha_n[t] = alpha;
         p.a[t] = positive_map(alpha, p.func, p.beta, p.lb) * (p.split && 2 * t >= total ? p.coef_second : p.coef);
     };
+    if (SPREAD && !kept) fetch(0);
     for (int64_t b0 = 0; b0 < blocks; b0 += KEPT * WAVES) {
-        if (!kept) fetch(b0);
+        float now[KEPT][4];
+        if (SPREAD) {                                           // the next values on their way while these are mapped
+#pragma unroll
+            for (int k = 0; k < KEPT; k++)
+#pragma unroll
+                for (int u = 0; u < 4; u++) now[k][u] = v[k][u];
+            if (b0 + KEPT * WAVES < blocks) fetch(b0 + KEPT * WAVES);
+        } else if (!kept) {
+            fetch(b0);
+        }
 #pragma unroll
         for (int k = 0; k < KEPT; k++)
 #pragma unroll
             for (int u = 0; u < 4; u++) {
                 const int64_t t = 256 * (b0 + wave + WAVES * k) + 64 * u + lane;
-                if (t < total) finish(t, v[k][u]);
+                if (t < total) finish(t, SPREAD ? now[k][u] : v[k][u]);
             }
     }
 }
@@ -985,7 +995,7 @@ int launch_block_rows(RowsArgs p, hipStream_t st)
     int64_t grid = (p.N + 4 * R - 1) / (4 * R);
     if (p.live_N && grid > 2 * cus) grid = 2 * cus;             // a capacity: stride over the tiles that exist
     CF_REQUIRE(grid < (1ll << 31), CF_ERR_UNSUPPORTED, "block rows: too many atoms");
-    const bool spread = head && p.normalize && p.groups && spread_groups(p.N * p.H);
+    const bool spread = head && p.normalize && spread_groups(p.N * p.H);
     p.apart = spread && (!p.live_N || spread_groups(p.N * p.H / 4));
     if (spread && R == 4) launch_rows<4, true>(p, source, head, (unsigned)grid, st);
     else if (spread) launch_rows<2, true>(p, source, head, (unsigned)grid, st);

@@ -6,6 +6,7 @@
 // one crystal of 12 atoms whose kernels take 0.20 ms); from here a launch costs 2-3 us.
 #include "cf_common.h"
 #include "block_rows.h"
+#include "real_enc_infer.h"
 
 namespace {
 
@@ -26,14 +27,28 @@ struct Carver {
 
 struct Buffers {
     float *rvlen, *rpos, *x[2], *h, *q, *k, *v, *qs, *a, *att, *z, *val, *prob, *rings, *pooled, *hidden;
-    void *stats, *flags;
+    void *stats, *flags, *units;
+    char *weights;
     unsigned *counters, *groups;
     float *packed;
     float *vcell, *recip, *kr, *sumexp;
-    int64_t stats_bytes, flag_bytes, words;
+    int64_t stats_bytes, flag_bytes, words, weight_bytes;
 };
 
-// Whether the blocks with value bins start from staged rings, and the bytes these take.
+// How a block with value bins is encoded: from units staged by real_enc_infer.hip wherever that is served.  Adaptive boxes are
+// staged in the box of the weakest exponent the positive map allows: with a lower bound below a quarter it has more than
+// eight times the translations of an exponent around one, and staging would cost more than it saves.
+bool boxes_of(const cf_forward_args &f, const cf_forward_block &p) { return f.adaptive != 0 && p.cutoff != 0.0; }
+int64_t real_heads(const cf_forward_args &f, const cf_forward_block &p) { return p.coef_reci != 0.0 ? f.H / 2 : f.H; }
+bool staged_block(const cf_forward_args &f, const cf_forward_block &p)
+{
+    const bool boxes = boxes_of(f, p);
+    return p.bins > 0 && f.staged_rings && (!boxes || (f.adaptive_rings && (p.cutoff > 0.0 || p.lower_bound >= 0.25))) &&
+           infer_served(f.N, f.E, real_heads(f, p), p.bins, f.width / f.H, boxes, (int)f.lattice_range, p.weakest,
+                        f.ring_limit_bytes);
+}
+
+// Whether the other blocks with value bins start from staged rings, and the bytes these take.
 bool use_rings(const cf_forward_args &f, int64_t U)
 {
     if (!f.staged_rings || U < 1) return false;
@@ -72,8 +87,21 @@ int64_t carve(const cf_forward_args &f, const cf_forward_block *blocks, char *ba
     Carver c{base, 0};
     const int64_t N = f.N, E = f.E, U = (N + E) / 2, W = f.width;
     bool rings = false, bins = false;
-    for (int64_t l = 0; l < f.layers; l++) bins = bins || blocks[l].bins > 0;
-    rings = bins && use_rings(f, U);
+    int64_t units = 0;
+    b.weight_bytes = 0;
+    for (int64_t l = 0; l < f.layers; l++) {
+        const cf_forward_block &p = blocks[l];
+        bins = bins || p.bins > 0;
+        if (!staged_block(f, p)) {
+            rings = rings || p.bins > 0;
+            continue;
+        }
+        const int64_t one = infer_units_bytes(U, boxes_of(f, p), f.ring_limit_bytes),
+                      w = infer_weights_bytes(real_heads(f, p), p.bins, W / f.H);
+        units = one > units ? one : units;
+        b.weight_bytes = w > b.weight_bytes ? w : b.weight_bytes;
+    }
+    rings = rings && use_rings(f, U);
     const bool rows = use_rows(f);
     b.rvlen = c.take<float>(3 * f.B);
     b.rpos = c.take<float>(3 * E);
@@ -103,6 +131,8 @@ int64_t carve(const cf_forward_args &f, const cf_forward_block *blocks, char *ba
     b.flag_bytes = rings ? cf_real_enc_flag_bytes(U, f.H) : 0;
     b.flags = rings ? c.take<char>(b.flag_bytes) : nullptr;
     b.rings = rings ? c.take<float>(cf_real_enc_ring_bytes(U) / 4) : nullptr;
+    b.units = units ? c.take<char>(units) : nullptr;
+    b.weights = units ? c.take<char>(f.layers * b.weight_bytes) : nullptr;
     b.pooled = c.take<float>(f.B * W);
     b.hidden = c.take<float>(f.B * (f.hidden > 0 ? f.hidden : 1));
     return c.used;
@@ -188,6 +218,7 @@ extern "C" int cf_forward(const cf_forward_args *f_, const cf_forward_block *blo
     }
     if (b.kr && (rc = cf_kr_base(b.rpos, b.recip, f.batch, f.edges, E, b.kr, stream))) return rc;
     const cf_forward_block *staged = nullptr;      // the block whose grid the rings in b.rings hold
+    int64_t units_until = 0;                       // blocks whose units are in b.units and whose projections are packed
     const float *x = f.x;
     int side = 0;
     if (rows) {
@@ -213,7 +244,30 @@ extern "C" int cf_forward(const cf_forward_args *f_, const cf_forward_block *blo
         const bool adaptive = rvlen != nullptr;
         const bool split = p.coef_reci != 0.0;                  // real space: the first half of the heads
         const int64_t HR = split ? H / 2 : H;
-        if (p.bins > 0 && b.rings && (!adaptive || (f.adaptive_rings && HR <= 8 && adaptive_rings_pay(U)))) {
+        if (staged_block(f, p)) {
+            const float cutoff = adaptive ? (float)p.cutoff : 0.0f;
+            if (l >= units_until) {
+                // units for this block and those behind it that share them, their projections packed alongside
+                const float *w[INFER_WEIGHT_BLOCKS];
+                int bins[INFER_WEIGHT_BLOCKS], count = 0;
+                for (units_until = l; units_until < f.layers && count < INFER_WEIGHT_BLOCKS; units_until++, count++) {
+                    const cf_forward_block &o = blocks[units_until];
+                    if (!staged_block(f, o) || o.weakest != p.weakest || boxes_of(f, o) != adaptive ||
+                        (adaptive && o.cutoff != p.cutoff) || real_heads(f, o) != HR)
+                        break;
+                    w[count] = o.w_pe;
+                    bins[count] = (int)o.bins;
+                }
+                if ((rc = launch_infer_stage(b.rpos, f.tvecs, rvlen, f.pairs, U, p.weakest, cutoff, (int)f.lattice_range,
+                                             (int)f.minimum_range, f.ring_limit_bytes, b.units, count, w, bins, HR, D,
+                                             b.weights + l * b.weight_bytes, b.weight_bytes, (hipStream_t)stream)))
+                    return rc;
+            }
+            rc = launch_real_enc_infer(b.a, b.rpos, f.tvecs, f.pairs, U, HR, p.bins, D, p.dist_max, p.wscale,
+                                       b.weights + l * b.weight_bytes, rvlen, cutoff, (int)f.lattice_range,
+                                       (int)f.minimum_range, p.weakest, f.ring_limit_bytes, b.units, b.z, b.val,
+                                       (hipStream_t)stream);
+        } else if (p.bins > 0 && b.rings && (!adaptive || (f.adaptive_rings && HR <= 8 && adaptive_rings_pay(U)))) {
             if (!staged || staged->bins != p.bins || staged->dist_max != p.dist_max || staged->wscale != p.wscale ||
                 staged->weakest != p.weakest) {
                 if ((rc = cf_real_enc_ring_stage(b.rpos, f.tvecs, f.pairs, U, p.bins, p.dist_max, p.wscale,

@@ -8,7 +8,7 @@ struct RowsArgs {
     int64_t N;
     int H, embed_width;
     const float *att, *x;                     // attention output; block input (or the rows to embed)
-    const float *packed_tail, *packed_head;   // packed weights of the block each belongs to, null: no such part
+    const float *packed_tail, *packed_head;   // packed weights of the block each belongs to (inference: split), null: no such part
     const float *bo, *b1, *b2;                // tail
     const float *packed_embed, *b_embed;      // null: x is the block input itself
     float *y;                                 // tail or embedding: the rows behind it
@@ -30,6 +30,7 @@ struct RowsArgs {
 
 constexpr int PACK_BLOCKS = 32;               // blocks per packing launch (48 bytes of kernel arguments each)
 constexpr int64_t PACKED_BLOCK = 12 * 128 * 128;   // floats a block
+constexpr int64_t SPLIT_BLOCK = PACKED_BLOCK + 12 * 128;   // with its columns' exponents, for cf_forward's row kernel
 struct PackSource {
     const float *wo, *w1, *w2, *wq, *wk, *wv;
 };
@@ -51,7 +52,8 @@ struct PrologueArgs {
     float *rpos, *vcell, *recip, *rvlen;      // vcell, recip nullable
     const int64_t *live_E;                    // set by the launcher
 };
-// packing, edge offsets (cf_edge_index) and lattice geometry (cf_lattice_geometry) at once
+// split packing (packed: blocks x SPLIT_BLOCK floats, packed_embed: 128 x 129), edge offsets (cf_edge_index) and lattice
+// geometry (cf_lattice_geometry) at once
 int launch_forward_prologue(const PackArgs &k, PrologueArgs p, hipStream_t st);
 
 struct TailBwdArgs {

@@ -7,26 +7,24 @@
 // first head.  As four linear launches and two for the exponents this was 6.6 and 4.5 us each at the 1.8
 // thousand rows of a batch, most of it not arithmetic: 0.7 GFLOP a block take 4.8 us at the fp32 matrix rate.
 //
-// A work-group of 8 wavefronts owns 4 R rows; the rows and all intermediates stay in LDS, the weights
-// (786 KB a block) stream from the L2, a 16-column tile per wavefront, two tiles ahead of their use.  At 64
-// bytes a clock a CU reads the weights in 5 us, and at 4 R = 8 rows the matrix cores (256 FLOP a clock and
-// CU) need as long; measured back to back, with the weights in the L2, 14.2 us a launch with tail and head at 1774 rows
-// (R 2), 10.1 at 12 rows (R 1), 20.3 at 4096 (R 4), against 35 us as six launches; inside a forward, where other kernels
-// have run in between, 17.6, 13.7 and 25.8 us (kernel trace under profiles/).  Variants: weights read from the matrices as they are 24 us (see
-// pack_weights_kernel); every 16-column tile with its own read of the rows, its own epilogue and a barrier 16.5 us.
-//
-// v_mfma_f32_4x4x1_16b_f32: sixteen independent 4 x 4 blocks, here 4 column groups x 4 reduction slots.
-//   B: lane (kq, c) = (lane / 16, lane % 16) holds W[col c][k0 + 4 kq + s], one component of a 16-byte load
-//      (16 rows of W, 64 consecutive bytes of each);
-//   A: lane l holds x[row l % 4][k0 + l / 4], one 4-byte LDS read for four steps: step s broadcasts block
-//      4 kq + s of each group of four (CBSZ 2, ABID s) to the group;
-//   D: lane (kq, c), register r: row r, column c, summed over the reduction slots 4 kq .. 4 kq + 3 of every
-//      16; two lane swaps at the end add the four slots and leave row kq, column c in each lane.
-// A row's sums do not depend on R or on the tile it falls in.
+// A work-group of 8 wavefronts owns 16 T rows; the rows and all intermediates stay in LDS, the weights
+// (786 KB a block) stream from the L2, a 16-column tile per wavefront, two tiles ahead of their use.  The products
+// are split f16 ones (split_f16.h): a column's weights are scaled and split once per forward (forward_prologue_kernel), a
+// row's values in LDS in front of each layer, in place.  So the matrix cores need 2.7 us for 16 rows, where fp32 ones
+// needed 10 and bound the launch at 4096 rows, and 16 rows are the least tile: half the work-groups, and half the weights
+// asked of the L2, that eight fp32 rows had at 1774 rows.  What bounds a launch now is the chain of one tile: 16 rows are
+// staged in 2.5 us, each of the twelve units of 128 columns takes 0.5, each of the four splits 0.3, output and exponents 0.9.
+// Without the weights' loads it would be 10.4 us at 12 rows; five buffers of weights instead of three: 0.9 us slower.
+// Measured, tail and head in a forward, fp32 products -> these: 12 rows 13.6 -> 12.5 us, 290 rows 13.9 -> 13.4,
+// 1774 rows 18.2 -> 13.9 (0.70 GFLOP: 50 TFLOP/s), 5.2 thousand rows 40 -> 21.4 (95 TFLOP/s).
+// Operands of v_mfma_f32_16x16x32_f16, lane (q, c) = (lane / 16, lane % 16), reduction step s of 32:
+//   A: 16 bytes of row c at k = 32 s + 8 q, hi or lo;  B: the same of column c's weights;  D: row 4 q + r, column c.
+// A row's sums do not depend on T or on the tile it falls in.
 #include "cf_common.h"
 #include "block_rows.h"
 #include "gauss_maps.h"
 #include "lattice_geometry.h"
+#include "split_f16.h"
 
 #include <math.h>
 
@@ -34,11 +32,8 @@ namespace {
 
 using namespace cf;
 
-typedef float float4_t __attribute__((ext_vector_type(4)));
-
 constexpr int RW = 128, RF = 512;            // block width, hidden units
-constexpr int LDX = RW + 16, LDH = RF + 16;  // LDS row strides: 16 mod 64, so the four rows of an A read and
-                                             // the four rows of a D write fall into disjoint banks
+constexpr int LDX = RW + 4, LDH = RF + 4;    // LDS row strides: 4 mod 64, so 16 rows' 16-byte reads cover all banks
 constexpr int RT = 512;                      // threads
 
 enum Source { ROWS_PLAIN = 0, ROWS_EMBED = 1, ROWS_TAIL = 2 };
@@ -56,67 +51,96 @@ __device__ __forceinline__ void load_weights(Weights &b, const float *__restrict
 }
 
 // The rows' values of 128 reduction steps as A operands.
-template <int R>
+template <int T>
 struct Rows {
-    float x[8][R];
+    int4_t hi[T][4], lo[T][4];
 };
 
-template <int R>
-__device__ __forceinline__ void read_rows(Rows<R> &a, const float *xs, int ld, int lane)
+template <int T>
+__device__ __forceinline__ void read_rows(Rows<T> &a, const float *xs, int ld, int lane)
 {
-    const float *xr = xs + (lane & 3) * ld + (lane >> 2);
+    const float *xr = xs + (lane & 15) * ld + 8 * (lane >> 4);
 #pragma unroll
-    for (int c = 0; c < 8; c++)
+    for (int t = 0; t < T; t++)
 #pragma unroll
-        for (int r = 0; r < R; r++) a.x[c][r] = xr[4 * r * ld + 16 * c];
+        for (int s = 0; s < 4; s++) {
+            a.hi[t][s] = *reinterpret_cast<const int4_t *>(xr + 16 * t * ld + 32 * s);
+            a.lo[t][s] = *reinterpret_cast<const int4_t *>(xr + 16 * t * ld + 32 * s + 4);
+        }
 }
 
-template <int R>
-__device__ __forceinline__ void multiply(float4_t (&acc)[R], const Weights &b, const Rows<R> &a)
+// acc = the 128 steps' products.  (Each kind is summed apart: every addition to the large sum rounds it, and four chains of
+// four keep the matrix cores busier than one of sixteen.)
+template <int T>
+__device__ __forceinline__ void multiply(float4_t (&acc)[T], const Weights &b, const Rows<T> &a)
 {
+    const float4_t zero = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int c = 0; c < 8; c++) {
+    for (int t = 0; t < T; t++) {
+        float4_t hh = zero, hl = zero, lh = zero, ll = zero;
 #pragma unroll
-        for (int r = 0; r < R; r++) acc[r] = __builtin_amdgcn_mfma_f32_4x4x1f32(a.x[c][r], b.w[c][0], acc[r], 2, 0, 0);
-#pragma unroll
-        for (int r = 0; r < R; r++) acc[r] = __builtin_amdgcn_mfma_f32_4x4x1f32(a.x[c][r], b.w[c][1], acc[r], 2, 1, 0);
-#pragma unroll
-        for (int r = 0; r < R; r++) acc[r] = __builtin_amdgcn_mfma_f32_4x4x1f32(a.x[c][r], b.w[c][2], acc[r], 2, 2, 0);
-#pragma unroll
-        for (int r = 0; r < R; r++) acc[r] = __builtin_amdgcn_mfma_f32_4x4x1f32(a.x[c][r], b.w[c][3], acc[r], 2, 3, 0);
+        for (int s = 0; s < 4; s++) {
+            const int4_t hi = __builtin_bit_cast(int4_t, b.w[2 * s]), lo = __builtin_bit_cast(int4_t, b.w[2 * s + 1]);
+            hh = mfma32(a.hi[t][s], hi, hh);
+            hl = mfma32(a.hi[t][s], lo, hl);
+            lh = mfma32(a.lo[t][s], hi, lh);
+            ll = mfma32(a.lo[t][s], lo, ll);
+        }
+        acc[t] = hh + ((hl + lh) + ll);
+        // (the products belong here: left to itself the compiler moves them to where the sums are used, and keeps
+        // every weight until then)
+        asm volatile("" : "+v"(acc[t]));
     }
-    // (the products belong here: left to itself the compiler moves them to where the sums are used, and keeps
-    // every weight until then)
+}
+
+// The largest magnitude of 32 adjacent lanes, in each of them.
+__device__ __forceinline__ float half_wave_max(float v)
+{
+    v = fmaxf(v, dpp_f<DPP_QUAD_1032, 0xF>(v, v));
+    v = fmaxf(v, dpp_f<DPP_QUAD_2301, 0xF>(v, v));
+    v = fmaxf(v, dpp_f<DPP_ROW_ROR4, 0xF>(v, v));
+    v = fmaxf(v, dpp_f<DPP_ROW_ROR8, 0xF>(v, v));
+    const unsigned x = (unsigned)__float_as_int(v);
+    const uint2_cf r = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+    return fmaxf(__int_as_float((int)r[0]), __int_as_float((int)r[1]));
+}
+
+// Four values of each of L pieces of 128 columns of a row, scaled to [2^14, 2^15) of the row's largest and split: of every
+// eight values (32 bytes) the eight his, then the eight los.  32 threads a row, thread j has columns 4 j .. 4 j + 3.
+template <int L>
+__device__ __forceinline__ void split_row(float4_t (&v)[L], float *row, int j, int *exp)
+{
+    float zero = 0.f, top = 0.f;
+    asm volatile("" : "+v"(zero));
 #pragma unroll
-    for (int r = 0; r < R; r++) asm volatile("" : "+v"(acc[r]));
-}
-
-__device__ __forceinline__ float lo_f(uint2_cf r) { return __int_as_float((int)r[0]) + __int_as_float((int)r[1]); }
-
-// Sum over the four reduction slots: lane (g, c) gets row g of the tile.
-__device__ __forceinline__ float slot_sum(float4_t a)
-{
-    const float u = lo_f(__builtin_amdgcn_permlane32_swap(__float_as_int(a[0]), __float_as_int(a[2]), false, false));
-    const float v = lo_f(__builtin_amdgcn_permlane32_swap(__float_as_int(a[1]), __float_as_int(a[3]), false, false));
-    return lo_f(__builtin_amdgcn_permlane16_swap(__float_as_int(u), __float_as_int(v), false, false));
-}
-
-template <int R>
-__device__ __forceinline__ void clear(float4_t (&acc)[R])
-{
+    for (int l = 0; l < L; l++)
 #pragma unroll
-    for (int r = 0; r < R; r++) acc[r] = float4_t{0.f, 0.f, 0.f, 0.f};
+        for (int i = 0; i < 4; i++) top = fmaxf(top, fabsf(v[l][i]));
+    const int e = __builtin_amdgcn_frexp_expf(half_wave_max(top));               // (0 for 0, infinity and NaN)
+    if (j == 0) *exp = e;
+    float *hi = row + 8 * (j / 2) + 2 * (j % 2);
+#pragma unroll
+    for (int l = 0; l < L; l++) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) v[l][i] = ldexpf(v[l][i], 15 - e);
+        const Split2 a = split2(v[l][0], v[l][1], 1.0f, zero), b = split2(v[l][2], v[l][3], 1.0f, zero);
+        *reinterpret_cast<int2_t *>(hi + RW * l) = int2_t{a.hi, b.hi};
+        *reinterpret_cast<int2_t *>(hi + RW * l + 4) = int2_t{a.lo, b.lo};
+    }
 }
 
-// Rows row0 .. of a (N, 128) matrix into LDS (rows past the end repeat the last one).
-template <int R>
-__device__ __forceinline__ void stage_rows(float *dst, const float *__restrict__ src, int64_t row0, int64_t N)
+// The rows of an LDS buffer split in place (a group's two lanes have read both before either writes).
+template <int M, int L>
+__device__ __forceinline__ void split_rows(float *xs, int ld, int *exps)
 {
-    for (int t = threadIdx.x; t < 4 * R * (RW / 4); t += RT) {
-        const int r = t / (RW / 4), c = t % (RW / 4);
-        const int64_t row = min(row0 + r, N - 1);
-        *reinterpret_cast<float4_t *>(dst + r * LDX + 4 * c) =
-            *reinterpret_cast<const float4_t *>(src + row * RW + 4 * c);
+    const int j = threadIdx.x % 32;
+#pragma unroll
+    for (int r0 = 0; r0 < M; r0 += RT / 32) {
+        const int r = r0 + threadIdx.x / 32;
+        float4_t v[L];
+#pragma unroll
+        for (int l = 0; l < L; l++) v[l] = *reinterpret_cast<const float4_t *>(xs + r * ld + 4 * j + RW * l);
+        split_row<L>(v, xs + r * ld, j, exps + r);
     }
 }
 
@@ -167,8 +191,8 @@ __device__ __forceinline__ void group_statistics(const float (&v)[4], int64_t b,
 }
 
 // The raw values of rows row0 .. row0 + rows - 1 are on their way: counts them into the groups they belong to, and forms
-// the statistics of those that are complete with them.  A tile's values are one piece (two with split heads) of at most 256,
-// so they touch two groups each: one per wavefront.
+// the statistics of those that are complete with them.  A tile's values are one piece (two with split heads) of at most 256
+// (launch_block_rows sees to it), so they touch two groups each: one per wavefront.
 __device__ void complete_groups(const RowsArgs &p, int64_t N, int64_t row0, int rows)
 {
     unsigned tid = threadIdx.x;
@@ -368,6 +392,65 @@ __device__ __forceinline__ void pack_weights(const PackArgs &p, int x, int l, bo
         *reinterpret_cast<const float4_t *>(src);
 }
 
+// The same weights for the inference kernel: per unit and wavefront four reduction steps of 32, hi and lo, 1 KB each in lane
+// order, a column scaled by its largest magnitude in the unit; behind the units the columns' exponents.
+constexpr int SPLIT_TILES = UNIT_END * 8, SPLIT_WAVES = 4;      // wavefronts a block, a work-group
+__device__ __forceinline__ void pack_split(const PackArgs &p, int x, int l)
+{
+    const int lane = threadIdx.x & 63, q = lane >> 4, c = lane & 15;
+    const int tile = x * SPLIT_WAVES + (int)(threadIdx.x >> 6), u = tile / 8, wave = tile % 8, col = 16 * wave + c;
+    if (l == p.blocks && u > 0) return;
+    const float *row;
+    if (l == p.blocks) {
+        row = p.w_embed + col * p.embed_width;
+    } else {
+        const PackSource &w = p.block[l];
+        if (u == 0) row = w.wo + col * RW;
+        else if (u < UNIT_FF2) row = w.w1 + ((u - UNIT_FF1) * RW + col) * RW;
+        else if (u < UNIT_QUERY) row = w.w2 + col * RF + (u - UNIT_FF2) * RW;
+        else row = (u == UNIT_QUERY ? w.wq : u == UNIT_QUERY + 1 ? w.wk : w.wv) + col * RW;
+    }
+    float4_t w[4][2];
+    if (l == p.blocks) {                                        // (an embedding's rows: any width, not aligned)
+#pragma unroll
+        for (int s = 0; s < 4; s++)
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                const int k = 32 * s + 8 * q + i;
+                w[s][i / 4][i % 4] = k < p.embed_width ? row[k] : 0.f;
+            }
+    } else {
+#pragma unroll
+        for (int s = 0; s < 4; s++)
+#pragma unroll
+            for (int i = 0; i < 2; i++) w[s][i] = *reinterpret_cast<const float4_t *>(row + 32 * s + 8 * q + 4 * i);
+    }
+    float top = 0.f;
+#pragma unroll
+    for (int s = 0; s < 4; s++)
+#pragma unroll
+        for (int i = 0; i < 8; i++) top = fmaxf(top, fabsf(w[s][i / 4][i % 4]));
+    const int e = __builtin_amdgcn_frexp_expf(rows_max(top));
+    float zero = 0.f;
+    asm volatile("" : "+v"(zero));
+    float *units = l == p.blocks ? p.packed_embed : p.packed + (int64_t)l * SPLIT_BLOCK;
+    int4_t *out = reinterpret_cast<int4_t *>(units + u * UNIT_FLOATS) + wave * 8 * WAVE + lane;
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+        int4_t hi, lo;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const Split2 y = split2(ldexpf(w[s][i / 2][2 * i % 4], 15 - e), ldexpf(w[s][i / 2][2 * i % 4 + 1], 15 - e), 1.0f, zero);
+            hi[i] = y.hi;
+            lo[i] = y.lo;
+        }
+        out[2 * s * WAVE] = hi;
+        out[(2 * s + 1) * WAVE] = lo;
+    }
+    int *exps = reinterpret_cast<int *>(units + (l == p.blocks ? UNIT_FLOATS : PACKED_BLOCK)) + u * RW;
+    if (lane < 16) exps[col] = e - 30;                          // (a row's and a column's 2^15)
+}
+
 __global__ __launch_bounds__(256) void pack_weights_kernel(PackArgs p)
 {
     pack_weights(p, blockIdx.x, blockIdx.y, blockIdx.z == 1);
@@ -377,13 +460,16 @@ __global__ __launch_bounds__(256) void pack_weights_kernel(PackArgs p)
 // 2 to 4 us: the packed weights, the offsets p_j - p_i of the edges and the lattices' geometry.
 __global__ __launch_bounds__(256) void forward_prologue_kernel(PackArgs k, PrologueArgs p)
 {
+    constexpr int GROUPS = SPLIT_TILES / SPLIT_WAVES;
     const int layers = k.blocks + (k.w_embed ? 1 : 0);
     int64_t x = blockIdx.x;
-    if (x < (int64_t)layers * PACK_GRID) {
-        pack_weights(k, (int)(x % PACK_GRID), (int)(x / PACK_GRID), false);
+    if (x < (int64_t)layers * GROUPS) {
+        if (x == 0)
+            for (int64_t t = threadIdx.x; t < k.words; t += 256) k.zero[t] = 0u;
+        pack_split(k, (int)(x % GROUPS), (int)(x / GROUPS));
         return;
     }
-    x -= (int64_t)layers * PACK_GRID;
+    x -= (int64_t)layers * GROUPS;
     const int64_t edge_groups = (p.E + 255) / 256;
     if (x < edge_groups) {
         const int64_t e = x * 256 + threadIdx.x;
@@ -397,19 +483,22 @@ __global__ __launch_bounds__(256) void forward_prologue_kernel(PackArgs k, Prolo
     if (b < p.B) lattice_geometry_of(p.trans, b, p.vcell, p.recip, p.rvlen);
 }
 
-template <int R, int SRC, bool HEAD, bool SPREAD>
-__global__ __launch_bounds__(RT, SPREAD && R == 2 ? 4 : 2) void block_rows_kernel(RowsArgs p)
+template <int T, int SRC, bool HEAD, bool SPREAD>
+__global__ __launch_bounds__(RT, 2) void block_rows_kernel(RowsArgs p)
 {
-    constexpr int M = 4 * R;
+    constexpr int M = 16 * T;
     constexpr int FIRST = SRC == ROWS_TAIL ? 0 : SRC == ROWS_EMBED ? UNIT_EMBED : UNIT_QUERY;
     constexpr int END = HEAD ? UNIT_END : UNIT_QUERY;
-    __shared__ __align__(16) float b0[M * LDX];
-    __shared__ __align__(16) float b1[M * LDX];
+    __shared__ __align__(16) float b0[M * LDX];                 // tail: attention output; then the rows behind it
+    __shared__ __align__(16) float b1[M * LDX];                 // tail: block input, then s
+    __shared__ __align__(16) float b2[M * LDX];                 // what the coming layer takes, split
     __shared__ __align__(16) float hs[M * LDH];                 // hidden units, then query, key, value
     __shared__ float biases[UNIT_END * RW], w_pos[RW];
+    __shared__ int w_exp[UNIT_END * RW];
+    __shared__ __align__(16) int x_exp[M];
     __shared__ float red[2];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int kq = lane >> 4, c = lane & 15;
+    const int q = lane >> 4, c = lane & 15;
     const int col = 16 * wave + c;
     const int64_t N = live_count(p.live_N, p.N);
     bool stored = true;
@@ -423,106 +512,167 @@ __global__ __launch_bounds__(RT, SPREAD && R == 2 ? 4 : 2) void block_rows_kerne
         if (SRC == ROWS_EMBED && u == UNIT_EMBED) return p.packed_embed;
         return (u < UNIT_QUERY ? p.packed_tail : p.packed_head) + u * UNIT_FLOATS;
     };
+    // this lane's value of row 16 t + 4 q + r in unit u
+    auto value = [&](const float4_t (&acc)[T], int t, int r, int u) -> float {
+        const int4_t e = *reinterpret_cast<const int4_t *>(x_exp + 16 * t + 4 * q);
+        return ldexpf(acc[t][r], e[r] + w_exp[u * RW + col]) + biases[u * RW + col];
+    };
     // (one tile per work-group unless the grid was cut short: with a live row count it covers a capacity)
     bool first = true;
     for (int64_t row0 = (int64_t)blockIdx.x * M; row0 < N; row0 += (int64_t)gridDim.x * M) {
-        float4_t acc[R];
-        Weights wa, wb, wc;
+        float4_t acc[T];
+        // AHEAD + 1 buffers in turn: unit u lies in buffer (u - FIRST) % BUFFERS
+        constexpr int BUFFERS = 3;
+        Weights w[BUFFERS];
         unsigned woff = (unsigned)(wave * 2048 + lane * 4) * 4u;
         asm volatile("" : "+v"(woff));       // (not a constant of this loop: else a hundred registers hold addresses)
-        load_weights(wa, unit_weights(FIRST), woff);
-        if (SRC == ROWS_TAIL) {
-            stage_rows<R>(b0, p.att, row0, N);
-            stage_rows<R>(b1, p.x, row0, N);
-        } else if (SRC == ROWS_PLAIN) {
-            stage_rows<R>(b0, p.x, row0, N);
-        } else {
-            const int K = p.embed_width;
-            for (int t = threadIdx.x; t < M * RW; t += RT) {
-                const int r = t / RW, k = t % RW;
-                b1[r * LDX + k] = k < K ? p.x[min(row0 + r, N - 1) * K + k] : 0.f;
+        auto fetch = [&](int u) {
+            if (u < END) load_weights(w[(u - FIRST) % BUFFERS], unit_weights(u), woff);
+        };
+        auto unit = [&](int u) -> Weights & {
+            fetch(u + BUFFERS - 1);
+            return w[(u - FIRST) % BUFFERS];
+        };
+        fetch(FIRST);
+        // everything the tile needs is asked for before any of it is used
+        constexpr int PASSES = M / (RT / 32), EACH = (END - FIRST) * RW / RT;
+        const int j = threadIdx.x % 32, k = threadIdx.x % RW;
+        float4_t in[PASSES][1], residual[PASSES];
+#pragma unroll
+        for (int t = 0; t < PASSES; t++) {
+            const int64_t row = min(row0 + 16 * t + threadIdx.x / 32, N - 1);
+            if (SRC == ROWS_EMBED) {
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    in[t][0][i] = 4 * j + i < p.embed_width ? p.x[row * p.embed_width + 4 * j + i] : 0.f;
+            } else {
+                in[t][0] = *reinterpret_cast<const float4_t *>((SRC == ROWS_TAIL ? p.att : p.x) + row * RW + 4 * j);
             }
+            if (SRC == ROWS_TAIL) residual[t] = *reinterpret_cast<const float4_t *>(p.x + row * RW + 4 * j);
         }
         if (first) {
-            first = false;
-            for (int t = threadIdx.x; t < (END - FIRST) * RW; t += RT) {
-                const int u = FIRST + t / RW, k = t % RW;
-                const float *src = u >= UNIT_QUERY ? p.b_in : SRC == ROWS_EMBED ? p.b_embed : u == 0 ? p.bo
-                                   : u < UNIT_FF2 ? p.b1 : p.b2;
-                const int at = u >= UNIT_QUERY ? u - UNIT_QUERY : u >= UNIT_FF1 && u < UNIT_FF2 ? u - UNIT_FF1 : 0;
-                biases[u * RW + k] = src ? src[at * RW + k] : 0.f;
+            // unit by unit, four at a time (the reduction's four units share one bias)
+            float bias[EACH + 1], wp = 0.f;
+            int exps[EACH + 1];
+#pragma unroll
+            for (int i = 0; i <= EACH; i++) {
+                const int u = FIRST + 4 * i + threadIdx.x / RW;
+                if (u >= END) break;
+                const bool embed = SRC == ROWS_EMBED && u == UNIT_EMBED;
+                const float *src = u >= UNIT_QUERY ? p.b_in : embed ? p.b_embed : u == 0 ? p.bo : u < UNIT_FF2 ? p.b1 : p.b2;
+                const int from = u >= UNIT_QUERY ? u - UNIT_QUERY : u >= UNIT_FF1 && u < UNIT_FF2 ? u - UNIT_FF1 : 0;
+                bias[i] = src && (embed || u <= UNIT_FF2 || u >= UNIT_QUERY) ? src[from * RW + k] : 0.f;
+                exps[i] = embed ? reinterpret_cast<const int *>(p.packed_embed + UNIT_FLOATS)[k]
+                                : reinterpret_cast<const int *>((u < UNIT_QUERY ? p.packed_tail : p.packed_head) + PACKED_BLOCK)[u * RW + k];
             }
-            if (HEAD && threadIdx.x < RW) w_pos[threadIdx.x] = p.w_pos[threadIdx.x];
+            if (HEAD) wp = p.w_pos[k];
+            first = false;
+#pragma unroll
+            for (int i = 0; i <= EACH; i++) {
+                const int u = FIRST + 4 * i + threadIdx.x / RW;
+                if (u >= END) break;
+                biases[u * RW + k] = bias[i];
+                w_exp[u * RW + k] = exps[i];
+            }
+            if (HEAD && threadIdx.x < RW) w_pos[k] = wp;
         }
-        load_weights(wb, unit_weights(FIRST + 1), woff);
+#pragma unroll
+        for (int u = 1; u < BUFFERS - 1; u++) fetch(FIRST + u);
+#pragma unroll
+        for (int t = 0; t < PASSES; t++) {
+            const int r = 16 * t + threadIdx.x / 32;
+            split_row<1>(in[t], b2 + r * LDX, j, x_exp + r);
+            if (SRC == ROWS_TAIL) *reinterpret_cast<float4_t *>(b1 + r * LDX + 4 * j) = residual[t];
+        }
         __syncthreads();
-        const int at = kq * LDX + col, at_h = kq * LDH + col;   // this lane's results: rows 4 r + kq
-        Rows<R> x;
+        const int at = 4 * q * LDX + col, at_h = 4 * q * LDH + col;          // this lane's results: rows 16 t + 4 q + r
+        Rows<T> x;
         if (SRC == ROWS_TAIL) {
             // output projection and residual: s replaces x in place
-            load_weights(wc, unit_weights(2), woff);
-            read_rows(x, b0, LDX, lane);
-            clear(acc);
-            multiply(acc, wa, x);
+            read_rows(x, b2, LDX, lane);
+            multiply(acc, unit(0), x);
 #pragma unroll
-            for (int r = 0; r < R; r++) b1[at + 4 * r * LDX] += slot_sum(acc[r]) + biases[col];
-            __syncthreads();
-            // hidden units, four tiles on one read of the rows
-            read_rows(x, b1, LDX, lane);
-            float4_t hid[4][R];
+            for (int t = 0; t < T; t++)
 #pragma unroll
-            for (int u = 0; u < 4; u++) {
-                Weights &cur = u % 3 == 0 ? wb : u % 3 == 1 ? wc : wa, &nxt = u % 3 == 0 ? wa : u % 3 == 1 ? wb : wc;
-                load_weights(nxt, unit_weights(UNIT_FF1 + 2 + u), woff);
-                clear(hid[u]);
-                multiply(hid[u], cur, x);
-            }
-#pragma unroll
-            for (int u = 0; u < 4; u++)
-#pragma unroll
-                for (int r = 0; r < R; r++) {
-                    const float v = slot_sum(hid[u][r]) + biases[(UNIT_FF1 + u) * RW + col];
-                    hs[at_h + 4 * r * LDH + u * RW] = v < 0.f ? 0.f : v;          // (a NaN stays one, as in torch.relu)
+                for (int r = 0; r < 4; r++) {
+                    float *s = b1 + at + (16 * t + r) * LDX;
+                    const float v = *s + value(acc, t, r, 0);
+                    *s = v;
+                    b0[at + (16 * t + r) * LDX] = v;
                 }
             __syncthreads();
-            clear(acc);
+            split_rows<M, 1>(b0, LDX, x_exp);
+            __syncthreads();
+            // hidden units, four tiles on one read of the rows
+            read_rows(x, b0, LDX, lane);
 #pragma unroll
             for (int u = 0; u < 4; u++) {
-                Weights &cur = u % 3 == 0 ? wc : u % 3 == 1 ? wa : wb, &nxt = u % 3 == 0 ? wb : u % 3 == 1 ? wc : wa;
-                if (UNIT_FF2 + 2 + u < END) load_weights(nxt, unit_weights(UNIT_FF2 + 2 + u), woff);
-                read_rows(x, hs + u * RW, LDH, lane);
-                multiply(acc, cur, x);
+                multiply(acc, unit(UNIT_FF1 + u), x);
+#pragma unroll
+                for (int t = 0; t < T; t++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) {
+                        const float v = value(acc, t, r, UNIT_FF1 + u);
+                        hs[at_h + (16 * t + r) * LDH + u * RW] = v < 0.f ? 0.f : v;   // (a NaN stays one, as in torch.relu)
+                    }
+            }
+            __syncthreads();
+            split_rows<M, 4>(hs, LDH, x_exp);
+            __syncthreads();
+            float y[T][4];
+            Rows<T> ahead;                                      // (read a unit before it is multiplied)
+            read_rows(x, hs, LDH, lane);
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                Rows<T> &now = u % 2 ? ahead : x;
+                if (u < 3) read_rows(u % 2 ? x : ahead, hs + (u + 1) * RW, LDH, lane);
+                multiply(acc, unit(UNIT_FF2 + u), now);
+                // (a unit's columns have exponents of their own)
+#pragma unroll
+                for (int t = 0; t < T; t++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) y[t][r] = (u == 0 ? 0.f : y[t][r]) + value(acc, t, r, UNIT_FF2 + u);
             }
 #pragma unroll
-            for (int r = 0; r < R; r++)
-                b0[at + 4 * r * LDX] = slot_sum(acc[r]) + biases[UNIT_FF2 * RW + col] + b1[at + 4 * r * LDX];
+            for (int t = 0; t < T; t++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const int i = at + (16 * t + r) * LDX;
+                    const float v = y[t][r] + b1[i];
+                    b0[i] = v;
+                    if (HEAD) b2[i] = v;
+                }
             __syncthreads();
         } else if (SRC == ROWS_EMBED) {
-            load_weights(wc, unit_weights(UNIT_QUERY + 1), woff);
-            read_rows(x, b1, LDX, lane);
-            clear(acc);
-            multiply(acc, wa, x);
+            read_rows(x, b2, LDX, lane);
+            multiply(acc, unit(UNIT_EMBED), x);
+            float v[T][4];
 #pragma unroll
-            for (int r = 0; r < R; r++) b0[at + 4 * r * LDX] = slot_sum(acc[r]) + biases[UNIT_EMBED * RW + col];
+            for (int t = 0; t < T; t++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) v[t][r] = value(acc, t, r, UNIT_EMBED);
+            __syncthreads();                                    // (the rows to embed have been read)
+#pragma unroll
+            for (int t = 0; t < T; t++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) b0[at + (16 * t + r) * LDX] = b2[at + (16 * t + r) * LDX] = v[t][r];
             __syncthreads();
         }
         if (HEAD) {
-            float4_t proj[3][R];
-            read_rows(x, b0, LDX, lane);
-            constexpr int S = SRC == ROWS_EMBED ? 1 : 0;         // (the buffer that holds the query weights)
+            if (SRC != ROWS_PLAIN) {
+                split_rows<M, 1>(b2, LDX, x_exp);
+                __syncthreads();
+            }
+            read_rows(x, b2, LDX, lane);
 #pragma unroll
             for (int u = 0; u < 3; u++) {
-                Weights &cur = (u + S) % 3 == 0 ? wa : (u + S) % 3 == 1 ? wb : wc;
-                Weights &nxt = (u + S) % 3 == 0 ? wc : (u + S) % 3 == 1 ? wa : wb;
-                if (u == 0) load_weights(nxt, unit_weights(UNIT_QUERY + 2), woff);
-                clear(proj[u]);
-                multiply(proj[u], cur, x);
+                multiply(acc, unit(UNIT_QUERY + u), x);
+#pragma unroll
+                for (int t = 0; t < T; t++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++)
+                        hs[at_h + (16 * t + r) * LDH + u * RW] = value(acc, t, r, UNIT_QUERY + u);
             }
-#pragma unroll
-            for (int u = 0; u < 3; u++)
-#pragma unroll
-                for (int r = 0; r < R; r++)
-                    hs[at_h + 4 * r * LDH + u * RW] = slot_sum(proj[u][r]) + biases[(UNIT_QUERY + u) * RW + col];
         }
         if (HEAD) __syncthreads();
         // results leave LDS in whole rows once the loop has no more loads to wait for
@@ -939,23 +1089,13 @@ __global__ __launch_bounds__(PH_T) void pool_head_kernel(PoolHeadArgs p)
     }
 }
 
-// Rows per work-group over four.  One while that gives a CU at most one tile, two while that does.  Beyond, sixteen
-// rows cost 20 us a round of tiles (one per CU), eight rows 23.5 us per two tiles and CU, side by side: sixteen
-// where the last round is full enough (4096 rows 20.3 against 23.3 us, 5600 rows 37.8 against 32.5).
-int rows_per_quad(int64_t N)
-{
-    const int64_t cus = device_cu_count();
-    const double rounds = (double)N / (double)(16 * cus);
-    return N <= 4 * cus ? 1 : N <= 8 * cus ? 2 : ceil(rounds) * 0.85 <= rounds ? 4 : 2;
-}
-
-template <int R, bool SPREAD>
+template <int T, bool SPREAD>
 void launch_rows(const RowsArgs &p, int source, bool head, unsigned grid, hipStream_t st)
 {
-    if (source == ROWS_TAIL && head) block_rows_kernel<R, ROWS_TAIL, true, SPREAD><<<grid, RT, 0, st>>>(p);
-    else if (source == ROWS_TAIL) block_rows_kernel<R, ROWS_TAIL, false, false><<<grid, RT, 0, st>>>(p);
-    else if (source == ROWS_EMBED) block_rows_kernel<R, ROWS_EMBED, true, SPREAD><<<grid, RT, 0, st>>>(p);
-    else block_rows_kernel<R, ROWS_PLAIN, true, SPREAD><<<grid, RT, 0, st>>>(p);
+    if (source == ROWS_TAIL && head) block_rows_kernel<T, ROWS_TAIL, true, SPREAD><<<grid, RT, 0, st>>>(p);
+    else if (source == ROWS_TAIL) block_rows_kernel<T, ROWS_TAIL, false, false><<<grid, RT, 0, st>>>(p);
+    else if (source == ROWS_EMBED) block_rows_kernel<T, ROWS_EMBED, true, SPREAD><<<grid, RT, 0, st>>>(p);
+    else block_rows_kernel<T, ROWS_PLAIN, true, SPREAD><<<grid, RT, 0, st>>>(p);
 }
 
 }  // namespace
@@ -978,7 +1118,7 @@ int launch_pack_weights(const PackArgs &p, hipStream_t st)
 int launch_forward_prologue(const PackArgs &k, PrologueArgs p, hipStream_t st)
 {
     p.live_E = live_edges(p.E);
-    const int64_t grid = (int64_t)(k.blocks + (k.w_embed ? 1 : 0)) * PACK_GRID + (p.E + 255) / 256 + (p.B + 255) / 256;
+    const int64_t grid = (int64_t)(k.blocks + (k.w_embed ? 1 : 0)) * (SPLIT_TILES / SPLIT_WAVES) + (p.E + 255) / 256 + (p.B + 255) / 256;
     CF_REQUIRE(grid < (1ll << 31), CF_ERR_UNSUPPORTED, "forward: too many edges");
     forward_prologue_kernel<<<(unsigned)grid, 256, 0, st>>>(k, p);
     CF_CHECK_LAUNCH("forward: prologue");
@@ -991,17 +1131,20 @@ int launch_block_rows(RowsArgs p, hipStream_t st)
     const bool head = p.packed_head != nullptr;
     p.live_N = live_atoms(p.N);
     const int64_t cus = device_cu_count();
-    const int R = p.live_N ? 2 : rows_per_quad(p.N);            // (live rows are somewhere below the capacity)
-    int64_t grid = (p.N + 4 * R - 1) / (4 * R);
+    // 32 rows a tile beyond one round of 16 (a tile a CU): 257 to 512 tiles of 16 are two rounds, the second short of
+    // work, and ask for the weights twice as often.  At 5.2 thousand rows 21.4 us a launch against 28.6; up to one round 16 are
+    // better, with all CUs at work (1774 rows: 13.9 us, on 111 of them, and a tile of 32 is the 21.4).
+    // (Live rows are somewhere below the capacity; a tile has at most 256 exponents, see complete_groups.)
+    const int T = !p.live_N && p.N > 16 * cus && p.H <= 8 ? 2 : 1;
+    int64_t grid = (p.N + 16 * T - 1) / (16 * T);
     if (p.live_N && grid > 2 * cus) grid = 2 * cus;             // a capacity: stride over the tiles that exist
     CF_REQUIRE(grid < (1ll << 31), CF_ERR_UNSUPPORTED, "block rows: too many atoms");
     const bool spread = head && p.normalize && spread_groups(p.N * p.H);
     p.apart = spread && (!p.live_N || spread_groups(p.N * p.H / 4));
-    if (spread && R == 4) launch_rows<4, true>(p, source, head, (unsigned)grid, st);
-    else if (spread) launch_rows<2, true>(p, source, head, (unsigned)grid, st);
-    else if (R == 1) launch_rows<1, false>(p, source, head, (unsigned)grid, st);
-    else if (R == 2) launch_rows<2, false>(p, source, head, (unsigned)grid, st);
-    else launch_rows<4, false>(p, source, head, (unsigned)grid, st);
+    if (spread && T == 2) launch_rows<2, true>(p, source, head, (unsigned)grid, st);
+    else if (spread) launch_rows<1, true>(p, source, head, (unsigned)grid, st);
+    else if (T == 2) launch_rows<2, false>(p, source, head, (unsigned)grid, st);
+    else launch_rows<1, false>(p, source, head, (unsigned)grid, st);
     CF_CHECK_LAUNCH("block rows");
     if (p.apart) {
         finish_exponents_kernel<<<(unsigned)((p.N * p.H + FINISH_VALUES - 1) / FINISH_VALUES), FINISH_T, 0, st>>>(p);

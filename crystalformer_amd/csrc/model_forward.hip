@@ -71,7 +71,7 @@ bool use_rows(const cf_forward_args &f) { return block_rows_served(f.width, f.ff
 // The head of block l: projections and exponents.
 void head_of(RowsArgs &r, const cf_forward_args &f, const cf_forward_block &p, const Buffers &b, int64_t l)
 {
-    r.packed_head = b.packed + l * PACKED_BLOCK; r.b_in = p.b_in; r.w_pos = p.w_pos;
+    r.packed_head = b.packed + l * SPLIT_BLOCK; r.b_in = p.b_in; r.w_pos = p.w_pos;
     r.gauss_scale = p.gauss_scale;
     r.normalize = (int)p.normalize; r.update_stats = (int)f.update_stats; r.func = (int)p.positive_func;
     r.beta = (float)p.beta; r.lb = (float)p.lower_bound; r.coef = (float)p.coef; r.q_scale = (float)p.q_scale;
@@ -124,7 +124,7 @@ int64_t carve(const cf_forward_args &f, const cf_forward_block *blocks, char *ba
     b.val = bins ? c.take<float>(E * W) : nullptr;
     b.stats_bytes = cf_gauss_exponents_workspace(N, f.H);
     b.stats = c.take<char>(b.stats_bytes);
-    b.packed = rows ? c.take<float>(f.layers * PACKED_BLOCK + W * W) : nullptr;
+    b.packed = rows ? c.take<float>(f.layers * SPLIT_BLOCK + W * (W + 1)) : nullptr;
     b.words = f.layers + (N * f.H + 255) / 256;
     b.counters = c.take<unsigned>(b.words);
     b.groups = b.counters + f.layers;
@@ -197,15 +197,15 @@ extern "C" int cf_forward(const cf_forward_args *f_, const cf_forward_block *blo
                 const cf_forward_block &p = blocks[first + i];
                 a.block[i] = PackSource{p.wo, p.w1, p.w2, p.wq, p.wk, p.wv};
             }
-            a.packed = b.packed + first * PACKED_BLOCK;
+            a.packed = b.packed + first * SPLIT_BLOCK;
             if (first > 0) {
-                if ((rc = launch_pack_weights(a, (hipStream_t)stream))) return rc;
+                if ((rc = launch_forward_prologue(a, PrologueArgs{}, (hipStream_t)stream))) return rc;
                 continue;
             }
             if (f.w_embed) {
                 a.w_embed = f.w_embed;
                 a.embed_width = (int)f.embed_width;
-                a.packed_embed = b.packed + f.layers * PACKED_BLOCK;
+                a.packed_embed = b.packed + f.layers * SPLIT_BLOCK;
             }
             a.zero = b.counters;
             a.words = b.words;
@@ -226,7 +226,7 @@ extern "C" int cf_forward(const cf_forward_args *f_, const cf_forward_block *blo
         r.N = N; r.H = (int)H; r.x = f.x;
         head_of(r, f, blocks[0], b, 0);
         if (f.w_embed) {
-            r.packed_embed = b.packed + f.layers * PACKED_BLOCK; r.b_embed = f.b_embed; r.embed_width = (int)f.embed_width;
+            r.packed_embed = b.packed + f.layers * SPLIT_BLOCK; r.b_embed = f.b_embed; r.embed_width = (int)f.embed_width;
             r.y = b.x[1];
             x = b.x[1];
         }
@@ -298,7 +298,7 @@ extern "C" int cf_forward(const cf_forward_args *f_, const cf_forward_block *blo
         if (rows) {
             RowsArgs r{};
             r.N = N; r.H = (int)H; r.att = b.att; r.x = x; r.y = y;
-            r.packed_tail = b.packed + l * PACKED_BLOCK; r.bo = p.bo; r.b1 = p.b1; r.b2 = p.b2;
+            r.packed_tail = b.packed + l * SPLIT_BLOCK; r.bo = p.bo; r.b1 = p.b1; r.b2 = p.b2;
             if (l + 1 < f.layers) head_of(r, f, blocks[l + 1], b, l + 1);
             if ((rc = launch_block_rows(r, (hipStream_t)stream))) return rc;
             x = y;

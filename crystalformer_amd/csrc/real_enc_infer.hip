@@ -23,58 +23,18 @@
 // (split, scaled by a power of two per row, in registers) with that head's 16 columns.
 #include "real_enc_infer.h"
 #include "real_enc_pair.h"
+#include "split_f16.h"
 
 namespace {
 
 using namespace cf;
 using namespace cfpair;
 
-typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
-typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
-typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
-typedef int int4_t __attribute__((ext_vector_type(4)));
-typedef int int2_t __attribute__((ext_vector_type(2)));
-
 constexpr float SPLIT = 32768.0f;           // values up to 1 are split scaled by it: 22 bits down to 2^-18, absolute 2^-40 below
 constexpr float PAD_D2 = 1e30f;             // d^2 of a slot without a translation: weight 0 and Gaussian 0
 constexpr float LEAST_A2 = -1e-25f;         // no decay slower: 1 for every real distance, 0 for PAD_D2
 constexpr int CLASSES = 8;                  // of d^2: seven of equal width and one for what lies beyond
 constexpr float CLASSED = 0.55f;            // share of the staged range that the seven cover
-
-// x0, x1 times `scale` as two halves each, packed in pairs.
-struct Split2 {
-    int hi, lo;
-};
-__device__ __forceinline__ Split2 split2(float x0, float x1, float scale, float zero)
-{
-    half2_t h = {(_Float16)__builtin_fmaf(x0, scale, zero), (_Float16)__builtin_fmaf(x1, scale, zero)};
-    Split2 s;
-    s.hi = __builtin_bit_cast(int, h);
-    asm("" : "+v"(s.hi));                   // (one packed register: else the second half is worked out twice)
-    h = __builtin_bit_cast(half2_t, s.hi);
-    const half2_t l = {(_Float16)__builtin_fmaf(x0, scale, -(float)h[0]), (_Float16)__builtin_fmaf(x1, scale, -(float)h[1])};
-    s.lo = __builtin_bit_cast(int, l);
-    return s;
-}
-
-__device__ __forceinline__ float4_t mfma16(int2_t a, int2_t b, float4_t c)
-{
-    return __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(half4_t, a), __builtin_bit_cast(half4_t, b), c, 0, 0, 0);
-}
-__device__ __forceinline__ float4_t mfma32(int4_t a, int4_t b, float4_t c)
-{
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, a), __builtin_bit_cast(half8_t, b), c, 0, 0, 0);
-}
-
-__device__ __forceinline__ float rows_max(float v)
-{
-    unsigned x = (unsigned)__float_as_int(v);
-    uint2_cf r = __builtin_amdgcn_permlane16_swap(x, x, false, false);
-    v = fmaxf(__int_as_float((int)r[0]), __int_as_float((int)r[1]));
-    x = (unsigned)__float_as_int(v);
-    r = __builtin_amdgcn_permlane32_swap(x, x, false, false);
-    return fmaxf(__int_as_float((int)r[0]), __int_as_float((int)r[1]));
-}
 
 // Smallest and largest by the bits: of floats >= 0 the signed order is theirs, of floats < 0 it is turned round.  (As
 // floats every step costs a canonicalising instruction and a move beside the one on the DPP path.  A NaN has the largest

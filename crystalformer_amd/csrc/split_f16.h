@@ -1,0 +1,52 @@
+// fp32 products on the f16 matrix instructions: both factors as two halves of 11 bits, x 2^k = hi + lo, and all four
+// products summed in fp32.  Scaled so that the largest value lies in [2^14, 2^15) a value keeps 22 bits and a sign down to
+// 2^-17 of it and 2^-40 of it absolutely below.  v_mfma_f32_16x16x32_f16 runs beside vector instructions (17 cycles; eight
+// v_fma beside it 36, 22 without it) where v_mfma_f32_16x16x4_f32 holds them up (32 cycles; 57 with the same eight).
+#pragma once
+#include "cf_common.h"
+
+namespace cf {
+
+typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
+typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
+typedef int int4_t __attribute__((ext_vector_type(4)));
+typedef int int2_t __attribute__((ext_vector_type(2)));
+typedef float float4_t __attribute__((ext_vector_type(4)));
+
+// x0, x1 times `scale` as two halves each, packed in pairs.
+struct Split2 {
+    int hi, lo;
+};
+__device__ __forceinline__ Split2 split2(float x0, float x1, float scale, float zero)
+{
+    half2_t h = {(_Float16)__builtin_fmaf(x0, scale, zero), (_Float16)__builtin_fmaf(x1, scale, zero)};
+    Split2 s;
+    s.hi = __builtin_bit_cast(int, h);
+    asm("" : "+v"(s.hi));                   // (one packed register: else the second half is worked out twice)
+    h = __builtin_bit_cast(half2_t, s.hi);
+    const half2_t l = {(_Float16)__builtin_fmaf(x0, scale, -(float)h[0]), (_Float16)__builtin_fmaf(x1, scale, -(float)h[1])};
+    s.lo = __builtin_bit_cast(int, l);
+    return s;
+}
+
+__device__ __forceinline__ float4_t mfma16(int2_t a, int2_t b, float4_t c)
+{
+    return __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(half4_t, a), __builtin_bit_cast(half4_t, b), c, 0, 0, 0);
+}
+__device__ __forceinline__ float4_t mfma32(int4_t a, int4_t b, float4_t c)
+{
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, a), __builtin_bit_cast(half8_t, b), c, 0, 0, 0);
+}
+
+__device__ __forceinline__ float rows_max(float v)
+{
+    unsigned x = (unsigned)__float_as_int(v);
+    uint2_cf r = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+    v = fmaxf(__int_as_float((int)r[0]), __int_as_float((int)r[1]));
+    x = (unsigned)__float_as_int(v);
+    r = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+    return fmaxf(__int_as_float((int)r[0]), __int_as_float((int)r[1]));
+}
+
+}  // namespace cf

@@ -119,13 +119,15 @@ class CrystalformerEncoderLayerCUDA(Module):
     def forward(self, src: Tensor, batch: Tensor, edges: Tensor, pos_ij: Tensor = None,
                 dist2_min: Tensor = None, trans: Tensor = None, kr_base: Tensor = None,
                 rvecs: Tensor = None, vcell: Tensor = None, onehot: Tensor = None, packed=None) -> Tensor:
-        """``packed`` (an extension): this block's weights as the one-launch row kernels read them, from the
-        encoder in a fused training step."""
+        """``packed`` (an extension): this block's weights as the one-launch row kernels read them, or the block as one
+        call, from the encoder in a fused training step."""
         if self.domain in ("real", "multihead"):
             assert pos_ij is not None and trans is not None
         if self.domain in ("reci", "multihead", "RECI"):
             assert kr_base is not None and rvecs is not None and rvecs.dim() == 3 and vcell is not None
         x = src
+        if type(packed) is hip_funcs.TrainBlock:
+            return packed(self, x)
         if packed is not None:
             attn, W = self.self_attn, self.linear1.in_features
             a, qs, k, v, x = hip_funcs.BlockHeadHIP.apply(
@@ -235,10 +237,12 @@ class CrystalformerEncoderCUDA(Module):
             kr_base = ops.kr_base(pos_ij, recip, batch, edges)
         output = src
         pack = executor.pack_for_training(self, src)
+        native = executor.native_training(self, pack, layout, pos_ij, trans, rvlen) if pack is not None else None
         for i, layer in enumerate(self.layers):
             if pack is not None:
                 output = layer(output, batch, edges, pos_ij, dist2_min, trans, kr_base, rvecs, vcell, onehot,
-                               packed=pack.block(i))
+                               packed=native[i] if native is not None and native[i].differentiates(layer, output)
+                               else pack.block(i))
                 continue
             output = layer(output, batch, edges, pos_ij, dist2_min, trans, kr_base, rvecs, vcell, onehot)
         if self.norm is not None:

@@ -140,7 +140,7 @@ def pack_for_training(encoder: nn.Module, src: Tensor) -> Optional["ops.PackedBl
             or _torch_module._global_forward_hooks or _torch_module._global_forward_pre_hooks \
             or _torch_module._global_backward_hooks or _torch_module._global_backward_pre_hooks:
         return None
-    blocks = []
+    blocks, settings = [], []
     for layer in encoder._modules["layers"]._modules.values():
         mods = layer._modules
         if _touched(layer, backward=True):
@@ -151,7 +151,32 @@ def pack_for_training(encoder: nn.Module, src: Tensor) -> Optional["ops.PackedBl
         attn = mods["self_attn"]
         blocks.append((attn.out_proj.weight, mods["linear1"].weight, mods["linear2"].weight, attn.q_proj_weight,
                        attn.k_proj_weight, attn.v_proj_weight))
-    return ops.PackedBlocks(blocks) if blocks else None
+        settings.append((got[0], got[1], attn.training))
+    if not blocks:
+        return None
+    pack = ops.PackedBlocks(blocks)
+    pack.settings = settings
+    return pack
+
+
+def native_training(encoder: nn.Module, pack: "ops.PackedBlocks", layout, rpos: Tensor, tvecs: Tensor, rvlen: Tensor):
+    """The blocks of a fused training step as one call each way (:class:`hip_funcs.BlockTrainHIP`), in the order of the
+    layers, or None where the operators run one by one: under instrumentation, without a pair list, with operands that the
+    operators convert or refuse, or with an encoding other than the one the call has."""
+    if ops.instrumented() or layout.pairs is None or layout.num_edges == 0 or not hip_funcs.KernelManager.DENSE_EDGE_BLOCKS:
+        return None
+    index, B = layout.batch.get_device(), tvecs.shape[0]
+    if not _ready(rpos, 3 * layout.num_edges, index) or not _ready(tvecs, 9 * B, index) or not _ready(rvlen, 3 * B, index) \
+            or tvecs.dim() != 3 or layout.atom_start.numel() != B + 1:
+        return None
+    shared = hip_funcs.TrainGeometry(pack, layout, rpos, tvecs, rvlen)
+    blocks = []
+    for i, (layer, (fields, heads, training)) in enumerate(zip(encoder.layers, pack.settings)):
+        attn = layer.self_attn
+        if not attn.params.use_low_memory or "encode_and_attend" in attn.__dict__ or "exponent_settings" in attn.__dict__:
+            return None
+        blocks.append(hip_funcs.TrainBlock(shared, i, fields, heads, training))
+    return blocks
 
 
 def _head(mlp: nn.Module, width: int, device_index: int) -> Optional[Tuple[tuple, int, int]]:

@@ -706,6 +706,151 @@ class BlockTailHIP(torch.autograd.Function):
         return (gatt if need[0] else None, gs if need[1] else None, *(t for pair in got for t in pair), None)
 
 
+class TrainBlock:
+    """What the blocks of one fused training step have in common, and one block's own settings: made by
+    :func:`executor.native_training` for every forward pass."""
+
+    __slots__ = ("shared", "index", "fields", "heads", "update_stats")
+
+    def __init__(self, shared, index, fields, heads, update_stats):
+        self.shared, self.index, self.fields, self.heads, self.update_stats = shared, index, fields, heads, update_stats
+
+    @staticmethod
+    def differentiates(layer, x: Tensor) -> bool:
+        """Whether the gradient goes through all of the block (else the operators one by one leave out what nobody wants)."""
+        own = layer.self_attn._parameters
+        return x.requires_grad or any(t is not None and t.requires_grad for t in (
+            own["q_proj_weight"], own["k_proj_weight"], own["v_proj_weight"], own["in_proj_bias"], own["lattice_pos_weights"]))
+
+    def __call__(self, layer, x: Tensor) -> Tensor:
+        own, out, one, two = (m._parameters for m in (layer.self_attn, layer.self_attn.out_proj, layer.linear1, layer.linear2))
+        return BlockTrainHIP.apply(
+            x, own["q_proj_weight"], own["k_proj_weight"], own["v_proj_weight"], own["in_proj_bias"],
+            own["lattice_pos_weights"], own["pe_dist_proj"] if self.fields[13] else None, out["weight"], out["bias"],
+            one["weight"], one["bias"], two["weight"], two["bias"], own["gauss_scale"], self)
+
+
+class TrainGeometry:
+    """Index structure and geometry of a fused training step's batch, and the rings its blocks share."""
+
+    __slots__ = ("pack", "layout", "rpos", "tvecs", "rvlen", "rings")
+
+    def __init__(self, pack, layout, rpos, tvecs, rvlen):
+        self.pack, self.layout, self.rpos, self.tvecs, self.rvlen, self.rings = pack, layout, rpos, tvecs, rvlen, {}
+
+
+class BlockTrainHIP(torch.autograd.Function):
+    """A 128-wide real-space block with 512 hidden units: what :class:`BlockHeadHIP`,
+    :class:`RealPeriodicEncodingWithProjFuncCUDA`, :class:`FusedDotProductAttentionCUDA` and :class:`BlockTailHIP` do one
+    after the other, as one node and one native call each way.  Same launches, same bits; weight gradients from the
+    grouped kernel (deferred inside :class:`deferred_weight_grads`)."""
+
+    @staticmethod
+    def forward(ctx, x, wq, wk, wv, b_in, w_pos, w_pe, wo, bo, w1, b1, w2, b2, gauss_scale, block):
+        from ctypes import byref, c_int64
+        shared, f, H = block.shared, block.fields, block.heads
+        lay, pack = shared.layout, shared.pack
+        bins, normalize, func, dist_max, wscale, cutoff, weakest, coef, lower, beta, q_scale = f[13:24]
+        dev, N, E = x.device, x.shape[0], lay.num_edges
+        U, B = lay.pairs.shape[0], shared.tvecs.shape[0]
+        KM = KernelManager
+        ranges = (KM.LATTICE_RANGE, KM.MINIMUM_RANGE)
+        rings = None
+        # (as RealPeriodicEncodingWithProjFuncCUDA decides)
+        if KM.STAGED_RINGS and bins > 0 and (cutoff == 0.0 or (KM.ADAPTIVE_RINGS and H <= 8)):
+            key = (bins, dist_max, wscale, weakest)
+            if key not in shared.rings:
+                shared.rings[key] = ops.staged_rings(shared.rpos, shared.tvecs, lay.pairs, bins, dist_max, wscale, ranges[0],
+                                                     weakest)
+            rings = shared.rings[key]
+        sched = ops._scheduling_words(dev) if rings is None and ops.DYNAMIC_ROUNDS else None
+        floats, i = pack.floats, block.index
+        y = torch.empty_like(x)
+        conf = (N, E, B, U, H, bins, *ranges, normalize, int(block.update_stats), func)
+        reals = (dist_max, wscale, cutoff, beta, lower, coef, q_scale)
+        args = _lib.BlockTrain(
+            *conf, 0, *reals, x.data_ptr(), pack.forward.data_ptr() + 4 * floats * i, None, f[3], f[4], f[5], f[6], f[8],
+            f[10], f[12], shared.rpos.data_ptr(), shared.tvecs.data_ptr(), shared.rvlen.data_ptr(), lay.batch.data_ptr(),
+            lay.edges.data_ptr(), lay.e_start.data_ptr(), lay.atom_start.data_ptr(), lay.edge_start.data_ptr(),
+            lay.pairs.data_ptr(), _lib.ptr(rings), _lib.ptr(sched), pack.counters.data_ptr() + 4 * i, y.data_ptr())
+        need = (c_int64 * 4)()
+        L = _lib.load()
+        _lib.check(L.cf_block_train_bytes(byref(args), need), "cf_block_train_bytes")
+        saved = torch.empty(need[0] // 4, dtype=torch.float32, device=dev)
+        scratch = torch.empty(max(need[1], 1), dtype=torch.uint8, device=dev)
+        args.saved, args.scratch = saved.data_ptr(), scratch.data_ptr()
+        with _lib.device_guard(dev):
+            rc = L.cf_block_train_fwd(byref(args), _lib.stream_handle(dev))
+        _lib.check(rc, "cf_block_train_fwd")
+        ctx.save_for_backward(x, wq, wk, wv, w_pos, w_pe, wo, w1, w2, saved, pack.backward[floats * i:floats * (i + 1)],
+                              shared.rpos, shared.tvecs, shared.rvlen, lay.batch, lay.edges)
+        # (what the backward call starts from, as above)
+        ctx.conf, ctx.layout = (conf, reals), lay
+        ctx.rings = rings if cutoff == 0.0 and bins <= 64 and x.shape[1] // H <= 16 else None
+        ctx.leaves = tuple(_leaf(t) for t in (wq, wk, wv, b_in, wo, bo, w1, b1, w2, b2))
+        ctx.has_bias = tuple(t is not None for t in (b_in, bo, b1, b2))
+        return y
+
+    @staticmethod
+    def backward(ctx, gy):
+        from ctypes import byref, c_int64
+        (x, wq, wk, wv, w_pos, w_pe, wo, w1, w2, saved, packed_bwd, rpos, tvecs, rvlen, batch, edges) = ctx.saved_tensors
+        ops._refuse_live_sizes("a training block's backward pass")
+        # (whatever a saved-tensor hook brought back: the same values, in the same place and type)
+        dev = ops.require_device(gy, x, w_pos, w_pe, saved, packed_bwd, rpos, tvecs, rvlen, batch, edges)
+        gy, x, w_pos, w_pe, saved, packed_bwd, rpos, tvecs, rvlen = (
+            ops._f32(t, "saved operand") for t in (gy, x, w_pos, w_pe, saved, packed_bwd, rpos, tvecs, rvlen))
+        batch, edges = ops._i64(batch, "batch"), ops._i64(edges, "edges")
+        conf, reals = ctx.conf
+        lay, rings = ctx.layout, ctx.rings
+        N, E, B, _, H, bins = conf[:6]
+        W = gy.shape[1]
+        if any(t.numel() != n for t, n in ((gy, N * W), (x, N * W), (w_pos, W), (packed_bwd, ops.PACKED_BLOCK_FLOATS),
+                                           (rpos, 3 * E), (tvecs, 9 * B), (rvlen, 3 * B), (batch, N), (edges, 2 * E))) \
+                or (bins > 0 and w_pe.numel() != W * bins):
+            raise _lib.CrystalformerHipError("a training block's saved operands have other shapes than its forward pass's")
+        need = ctx.needs_input_grad
+        gw_pe = torch.empty_like(w_pe) if w_pe is not None and need[6] else None
+        args = _lib.BlockTrain(
+            *conf, int(gw_pe is not None), *reals, x.data_ptr(), None, packed_bwd.data_ptr(), None, w_pos.data_ptr(), None,
+            _lib.ptr(w_pe), None, None, None, rpos.data_ptr(), tvecs.data_ptr(), rvlen.data_ptr(), batch.data_ptr(),
+            edges.data_ptr(), lay.e_start.data_ptr(), lay.atom_start.data_ptr(), lay.edge_start.data_ptr(),
+            lay.pairs.data_ptr(), _lib.ptr(rings), None, None, None, saved.data_ptr(), None, gy.data_ptr(), None,
+            _lib.ptr(gw_pe))
+        bytes_ = (c_int64 * 4)()
+        L = _lib.load()
+        _lib.check(L.cf_block_train_bytes(byref(args), bytes_), "cf_block_train_bytes")
+        if saved.numel() * 4 != bytes_[0]:
+            raise _lib.CrystalformerHipError("a training block's saved operands have other shapes than its forward pass's")
+        kept = torch.empty(bytes_[2] // 4, dtype=torch.float32, device=dev)
+        scratch = torch.empty(bytes_[3], dtype=torch.uint8, device=dev)
+        args.kept, args.scratch = kept.data_ptr(), scratch.data_ptr()
+        with _lib.device_guard(dev):
+            rc = L.cf_block_train_bwd(byref(args), _lib.stream_handle(dev))
+        _lib.check(rc, "cf_block_train_bwd")
+        n = N * W
+        gq, gk, gv, gs, gx = (kept.as_strided((N, W), (W, 1), k * n) for k in range(5))
+        gh, gw_pos = kept.as_strided((N, 4 * W), (4 * W, 1), 5 * n), kept.as_strided((W,), (1,), 9 * n)
+        att, s, h = (saved.as_strided((N, c), (c, 1), at) for c, at in ((W, 0), (W, n), (4 * W, 2 * n)))
+        lq, lk, lv, b_in, lo, bo, l1, b1, l2, b2 = ctx.leaves
+        has_in, has_o, has_1, has_2 = ctx.has_bias
+        tail = _weight_gradients([
+            (g, a, w, leaf if not has or bias is not None else None, bias, 0, need[k], has and need[k + 1])
+            for g, a, w, leaf, bias, has, k in ((gs, att, wo, lo, bo, has_o, 7), (gh, s, w1, l1, b1, has_1, 9),
+                                                (gy, h, w2, l2, b2, has_2, 11))])
+        want_b = has_in and need[4]
+        head = (lq, lk, lv)
+        # (one bias vector for the three layers: all of them deferred, or none)
+        if not ((not has_in or (b_in is not None and b_in.grad is None and want_b)) and all(need[1:4])
+                and all(w is not None and w.grad is None for w in head)):
+            head = (None, None, None)
+        got = _weight_gradients([(g, x, w, leaf, b_in, i * W, need[1 + i], want_b)
+                                 for i, (g, w, leaf) in enumerate(zip((gq, gk, gv), (wq, wk, wv), head))])
+        gb = torch.cat([b for _, b in got]) if want_b and got[0][1] is not None else None
+        return (gx if need[0] else None, *(w for w, _ in got), gb, gw_pos.view(w_pos.shape) if need[5] else None, gw_pe,
+                *(t for pair in tail for t in pair), None, None)
+
+
 # A list while a training step defers its linear layers' weight gradients (see
 # :func:`deferred_weight_grads`), else None.
 _deferred = None

@@ -44,6 +44,16 @@ class ForwardArgs(ctypes.Structure):
                                        "out")])
 
 
+class BlockTrain(ctypes.Structure):
+    """``cf_block_train`` of include/crystalformer_hip.h."""
+    _fields_ = ([(n, _i64) for n in ("N", "E", "B", "U", "H", "bins", "lattice_range", "minimum_range", "normalize",
+                                     "update_stats", "positive_func", "want_gw_pe")]
+                + [(n, _dbl) for n in ("dist_max", "wscale", "cutoff", "beta", "lower_bound", "coef", "q_scale")]
+                + [(n, _ptr) for n in ("x", "packed", "packed_bwd", "b_in", "w_pos", "gauss_scale", "w_pe", "bo", "b1", "b2",
+                                       "rpos", "tvecs", "rvlen", "batch", "edges", "e_start", "atom_start", "edge_start",
+                                       "pairs", "rings", "sched", "counter", "y", "saved", "scratch", "gy", "kept", "gw_pe")])
+
+
 # name -> (restype, argtypes); mirrors include/crystalformer_hip.h
 SIGNATURES = {
     "cf_version": (_int, []),
@@ -101,6 +111,9 @@ SIGNATURES = {
     "cf_block_head_bwd": (_int, [_ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _i64, _i64, _ptr, _int, _f32, _f32,
                                  _f32, _f32, _ptr, _ptr, _ptr, _ptr, _ptr]),
     "cf_forward": (_int, [_ptr, _ptr, _ptr, _i64, _ptr]),
+    "cf_block_train_bytes": (_int, [_ptr, _ptr]),
+    "cf_block_train_fwd": (_int, [_ptr, _ptr]),
+    "cf_block_train_bwd": (_int, [_ptr, _ptr]),
     "cf_kr_base": (_int, [_ptr, _ptr, _ptr, _ptr, _i64, _ptr, _ptr]),
     "cf_reci_enc_fwd": (_int, [_ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _i64, _i64, _i64, _int, _ptr, _ptr, _ptr]),
     "cf_reci_enc_bwd": (_int, [_ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _i64, _i64, _i64, _int, _int, _ptr, _ptr]),

@@ -1125,7 +1125,7 @@ class PackedBlocks:
     """Weights of a stack of blocks in the order the one-launch row kernels read them, forward and backward
     form, and a zeroed counter per block; made anew for every forward pass."""
 
-    __slots__ = ("forward", "backward", "counters", "floats")
+    __slots__ = ("forward", "backward", "counters", "floats", "settings")
 
     def __init__(self, blocks):
         """``blocks``: (Wo, W1, W2, Wq, Wk, Wv) per block, contiguous float32 on one GPU."""

@@ -577,6 +577,37 @@ int cf_block_head_bwd(const float *ga, const float *gqs, const float *gk, const 
                       float *g_alpha, float *gq, float *gx, float *gw_pos, void *stream);
 
 /*
+ * A 128-wide real-space block with 512 hidden units of a training step (the row kernels above around the encoding and the
+ * attention, models/indexed_lattice_multi_head_attention_cuda.py:636-790 and the encoder layer around it) as one call
+ * forward and one backward: the launches of cf_block_head, cf_real_enc_fwd(_rings), cf_fused_dpa_fwd, cf_block_tail and of
+ * their backward calls, on dense edge lists, results the same to the bit.  Not under a size header.
+ *   saved    written forward, read backward: att (N,128), s (N,128), h (N,512) at its start, rows of whole 256 bytes
+ *   kept     written backward: gq, gk, gv, gs, gx (N,128), gh (N,512), gw_pos (128), in this order
+ *   bytes_4  sizes of saved, forward scratch, kept, backward scratch (256-byte aligned memory; by sizes, bins, normalize,
+ *            cutoff, rings and want_gw_pe)
+ */
+typedef struct {
+    int64_t N, E, B, U, H, bins, lattice_range, minimum_range, normalize, update_stats, positive_func, want_gw_pe;
+    double dist_max, wscale, cutoff, beta, lower_bound, coef, q_scale;    /* cutoff 0: fixed cube */
+    const float *x, *packed, *packed_bwd, *b_in, *w_pos;                  /* packed(_bwd): the block's part of cf_pack_blocks */
+    float *gauss_scale;
+    const float *w_pe, *bo, *b1, *b2;                                     /* (H, D, bins) or NULL; biases nullable */
+    const float *rpos, *tvecs, *rvlen;
+    const int64_t *batch, *edges, *e_start, *atom_start, *edge_start, *pairs;
+    const void *rings;                                                    /* cf_real_enc_ring_stage, nullable */
+    int32_t *sched, *counter;
+    float *y;
+    void *saved, *scratch;
+    const float *gy;                                                      /* backward: from here */
+    void *kept;
+    float *gw_pe;
+} cf_block_train;
+
+int cf_block_train_bytes(const cf_block_train *args, int64_t *bytes_4);
+int cf_block_train_fwd(const cf_block_train *args, void *stream);
+int cf_block_train_bwd(const cf_block_train *args, void *stream);
+
+/*
  * Reciprocal-space periodic encoding (ReciPeriodicEncodingFuncCUDA, models/cuda_funcs/reci_space_enc.py:17-99;
  * kernels models/kernels/reci_enc_fwd.cu:3-68, reci_enc_bwd.cu:3-71), LATTICE_RANGE passed at run time:
  *   S[e,h] = sum over n1 in [0,R] (weight 2 for n1 != 0), n2, n3 in [-R,R] of

@@ -34,6 +34,7 @@ constexpr float SPLIT = 32768.0f;           // values up to 1 are split scaled b
 constexpr float PAD_D2 = 1e30f;             // d^2 of a slot without a translation: weight 0 and Gaussian 0
 constexpr float LEAST_A2 = -1e-25f;         // no decay slower: 1 for every real distance, 0 for PAD_D2
 constexpr int CLASSES = 8;                  // of d^2: seven of equal width and one for what lies beyond
+constexpr int MOST_STAGED = 832;            // of a pair (fewer than 16 x 64: a lane's share of a class is counted in four bits)
 constexpr float CLASSED = 0.55f;            // share of the staged range that the seven cover
 
 // Smallest and largest by the bits: of floats >= 0 the signed order is theirs, of floats < 0 it is turned round.  (As
@@ -149,7 +150,7 @@ __device__ __forceinline__ void pack_projection(const WeightArgs &p, int l, int 
 
 constexpr int STAGE_WAVES = 4;
 
-// A wavefront per unit, the next unit's cell requested ahead.  LDS per wavefront: capacity + 64 distances and packed n.
+// A wavefront per unit, the next unit's cell requested ahead.  LDS per wavefront: capacity + 64 distances and packed n, and 1 KB of places.
 // The first work-groups pack the blocks' projections instead.
 __global__ __launch_bounds__(STAGE_WAVES * 64) void infer_stage_kernel(StageArgs p, WeightArgs w)
 {
@@ -176,6 +177,9 @@ __global__ __launch_bounds__(STAGE_WAVES * 64) void infer_stage_kernel(StageArgs
     const int cap = p.capacity;
     float *cand_d2 = lds + wave * (p.n ? 3 : 2) * (cap + WAVE) / 2;
     unsigned short *cand_n = reinterpret_cast<unsigned short *>(cand_d2 + cap + WAVE);
+    // (places of a class's next, a column a lane: behind all wavefronts' candidates)
+    unsigned short *places = reinterpret_cast<unsigned short *>(lds + STAGE_WAVES * (p.n ? 3 : 2) * (cap + WAVE) / 2) +
+                             wave * CLASSES * WAVE;
     struct Ids { int64_t e_ij, e_ji, i, j, n; };
     auto ids_of = [&](int64_t u_) -> Ids {
         const ConstLong d = (ConstLong)p.pairs + (u_ < U ? u_ : U - 1) * PAIR_FIELDS;
@@ -274,79 +278,121 @@ __global__ __launch_bounds__(STAGE_WAVES * 64) void infer_stage_kernel(StageArgs
                     keep(d2c[ch], ch * WAVE + lane < bx.T, pre[ch][0], pre[ch][1], pre[ch][2]);
             if (!hold_cube) least = wave_min_positive(fminf(d2c[0], d2c[1]));
         } else {
-            // 64 translations on: the digits of 64 in the box's mixed radix, with carries
-            int i1, i2, i3;
-            decode(bx, min(lane, bx.T - 1), i1, i2, i3);
-            int s1 = __builtin_amdgcn_readlane(i1, 63) + bx.U1, s2 = __builtin_amdgcn_readlane(i2, 63) + bx.U2,
-                s3 = __builtin_amdgcn_readlane(i3, 63) + bx.U3 + 1;               // (63 and one)
-            if (s3 == bx.S3) s3 = 0, s2++;
-            if (s2 == bx.S2) s2 = 0, s1++;
-            const float f1 = (float)s1, f2 = (float)s2, f3 = (float)s3, S2 = (float)bx.S2, S3 = (float)bx.S3,
-                        U2 = (float)bx.U2, U3 = (float)bx.U3;
-            float n1 = (float)i1, n2 = (float)i2, n3 = (float)i3, closest = PAD_D2;
-            for (int c0 = 0; c0 < bx.T; c0 += WAVE) {
-                const bool valid = c0 + lane < bx.T;
-                const float d2 = dist2(cell, n1, n2, n3);
-                closest = fminf(closest, valid ? d2 : PAD_D2);
-                keep(d2, valid, n1, n2, n3);
-                n3 += f3;
-                const bool c3 = n3 > U3;
-                n3 -= c3 ? S3 : 0.f;
-                n2 += c3 ? f2 + 1.0f : f2;
-                const bool c2 = n2 > U2;
-                n2 -= c2 ? S2 : 0.f;
-                n1 += c2 ? f1 + 1.0f : f1;
+            // A lane has a place (two of the three numbers) and walks along the third axis, the one that leaves the fewest
+            // steps of 64 places: 15 instructions a step.  (All three numbers of 64 consecutive translations, carried from
+            // step to step, took 45: 958 thousand pairs with 232 of them staged 1030 us, so 915, with the ranking below 770.)
+            const int S1 = 2 * bx.U1 + 1;
+            const int s1 = ((bx.S2 * bx.S3 + 63) >> 6) * S1, s2 = ((S1 * bx.S3 + 63) >> 6) * bx.S2,
+                      s3 = ((S1 * bx.S2 + 63) >> 6) * bx.S3;
+            const int along = s1 <= s2 && s1 <= s3 ? 0 : s2 <= s3 ? 1 : 2;
+            const bool x1 = along == 0, x2 = along == 1;         // the lanes' axes: (2, 3), (1, 3), (1, 2)
+            const int Ua = x1 ? bx.U2 : bx.U1, Ub = x1 || x2 ? bx.U3 : bx.U2, Uc = x1 ? bx.U1 : x2 ? bx.U2 : bx.U3;
+            const int Sb = 2 * Ub + 1, plane = (2 * Ua + 1) * Sb;
+            const int code_a = x1 ? 32 : 1, code_b = x1 || x2 ? 1024 : 32, code_c = x1 ? 1 : x2 ? 32 : 1024;
+            float ta[3], tb[3], tc[3];
+#pragma unroll
+            for (int i = 0; i < 3; i++) {
+                ta[i] = x1 ? cell.t[3 + i] : cell.t[i];
+                tb[i] = x1 || x2 ? cell.t[6 + i] : cell.t[3 + i];
+                tc[i] = x1 ? cell.t[i] : x2 ? cell.t[3 + i] : cell.t[6 + i];
+            }
+            const float inv_Sb = __builtin_amdgcn_rcpf((float)Sb);
+            float closest = PAD_D2;
+            for (int p0 = 0; p0 < plane; p0 += WAVE) {
+                const bool valid = p0 + lane < plane;
+                const unsigned long long there = __ballot(valid);
+                const int at_place = min(p0 + lane, plane - 1);
+                const int ia = (int)(((float)at_place + 0.5f) * inv_Sb), ib = at_place - ia * Sb;
+                const float na = (float)(ia - Ua), nb = (float)(ib - Ub);
+                const float bx_ = __builtin_fmaf(na, ta[0], __builtin_fmaf(nb, tb[0], cell.rx));
+                const float by_ = __builtin_fmaf(na, ta[1], __builtin_fmaf(nb, tb[1], cell.ry));
+                const float bz_ = __builtin_fmaf(na, ta[2], __builtin_fmaf(nb, tb[2], cell.rz));
+                int code = (ia - Ua) * code_a + (ib - Ub) * code_b - Uc * code_c + 16 * (1 + 32 + 1024);
+                float nc = (float)-Uc;
+                int here = __float_as_int(PAD_D2);               // (see dpp_min)
+                for (int c_ = -Uc; c_ <= Uc; c_++) {
+                    const float vx = __builtin_fmaf(nc, tc[0], bx_), vy = __builtin_fmaf(nc, tc[1], by_),
+                                vz = __builtin_fmaf(nc, tc[2], bz_);
+                    const float d2 = __builtin_fmaf(vx, vx, __builtin_fmaf(vy, vy, vz * vz));
+                    here = min(here, __float_as_int(d2));
+                    const bool alive = !(d2 >= limit);           // (NaN is never beyond)
+                    const unsigned long long mask = __ballot(alive) & there;
+                    if (count <= cap) {                          // (more: the unit isn't staged)
+                        const int at = lanes_below(mask, count);
+                        if (alive && valid) {
+                            cand_d2[at] = d2;
+                            cand_n[at] = (unsigned short)code;
+                        }
+                    }
+                    count += __popcll(mask);
+                    nc += 1.0f;
+                    code += code_c;
+                }
+                closest = fminf(closest, valid ? __int_as_float(here) : PAD_D2);
             }
             least = fminf(bound, wave_min_positive(closest));
         }
         const bool fits = count <= cap && max(bx.U1, max(bx.U2, bx.U3)) <= 15;
         wave_mem_sync();
         if (fits) {
-            // ranked in classes, within a chunk of 64 by two packed prefix sums (a byte a class)
             const float scale = __builtin_amdgcn_rcpf(class_width(limit, least));
             auto class_of = [&](float d2) -> int { return min(max((int)((d2 - least) * scale), 0), CLASSES - 1); };
-            int base = 0;                                        // lane k: where class k goes on
-            if (count > WAVE) {
-                int total[CLASSES];
-#pragma unroll
-                for (int k = 0; k < CLASSES; k++) total[k] = 0;
-                for (int b = 0; b < count; b += WAVE) {
-                    const int cls = b + lane < count ? class_of(cand_d2[b + lane]) : CLASSES;
-#pragma unroll
-                    for (int k = 0; k < CLASSES; k++) total[k] += __popcll(__ballot(cls == k));
-                }
-                int before = 0;
-#pragma unroll
-                for (int k = 0; k < CLASSES; k++) {
-                    base = lane == k ? before : base;
-                    before += total[k];
-                }
-            }
-            for (int b = 0; b < count; b += WAVE) {
-                const bool held = b + lane < count;
-                const float d2 = held ? cand_d2[b + lane] : 0.f;
-                int at = b + lane;
+            if (count <= WAVE) {
+                const bool held = lane < count;
+                const float d2 = held ? cand_d2[lane] : 0.f;
+                int at = lane;
                 if (count > 16) {
+                    // ranked in classes by two packed prefix sums over the lanes (a byte a class)
                     const int cls = class_of(d2), shift = 8 * (cls & 3);
                     const int one = held ? 1 << shift : 0;
                     const int low = cls < 4 ? one : 0, high = cls < 4 ? 0 : one;
                     const int upto0 = wave_inclusive_scan_i(low), upto1 = wave_inclusive_scan_i(high);
                     const unsigned t0 = (unsigned)__builtin_amdgcn_readlane(upto0, 63),
                                    t1 = (unsigned)__builtin_amdgcn_readlane(upto1, 63);
-                    unsigned r = cls < 4 ? (unsigned)(upto0 - low) : (unsigned)(upto1 - high);
-                    if (count <= WAVE) {                         // (the classes below are all in this chunk)
-                        const unsigned b0 = (t0 << 8) + (t0 << 16) + (t0 << 24), all0 = (t0 * 0x01010101u) >> 24;
-                        const unsigned b1 = (t1 << 8) + (t1 << 16) + (t1 << 24) + all0 * 0x01010101u;
-                        r += cls < 4 ? b0 : b1;
-                        at = (int)(r >> shift) & 0xFF;
-                    } else {
-                        at = ((int)(r >> shift) & 0xFF) + __shfl(base, cls, WAVE);
-                        base += (int)((lane < 4 ? t0 : t1) >> (8 * (lane & 3))) & 0xFF;
-                    }
+                    const unsigned b0 = (t0 << 8) + (t0 << 16) + (t0 << 24), all0 = (t0 * 0x01010101u) >> 24;
+                    const unsigned b1 = (t1 << 8) + (t1 << 16) + (t1 << 24) + all0 * 0x01010101u;
+                    const unsigned r = (cls < 4 ? (unsigned)(upto0 - low) : (unsigned)(upto1 - high)) + (cls < 4 ? b0 : b1);
+                    at = (int)(r >> shift) & 0xFF;
                 }
                 if (held) {
                     p.d2[u * cap + at] = d2;
-                    if (p.n) p.n[u * cap + at] = cand_n[b + lane];
+                    if (p.n) p.n[u * cap + at] = cand_n[lane];
+                }
+            } else {
+                // More: each lane counts its own (lane, lane + 64, ..) in four bits a class, one prefix sum over the lanes
+                // in 16 bits a class says where its first of every class goes, and it counts on from there in LDS.  (A prefix
+                // sum for every 64: 60 instructions each where this takes 25.)
+                unsigned mine = 0;
+                for (int b = lane; b < count; b += WAVE) mine += 1u << (4 * class_of(cand_d2[b]));
+                int own[4], upto[4];                             // classes k and k + 4
+                unsigned total[CLASSES], start = 0;
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    own[k] = (int)((mine >> (4 * k)) & 0x000F000Fu);
+                    upto[k] = wave_inclusive_scan_i(own[k]);
+                    const unsigned t = (unsigned)__builtin_amdgcn_readlane(upto[k], 63);
+                    total[k] = t & 0xFFFFu;
+                    total[k + 4] = t >> 16;
+                }
+                unsigned first_[CLASSES];
+#pragma unroll
+                for (int k = 0; k < CLASSES; k++) {
+                    first_[k] = start;
+                    start += total[k];
+                }
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    const unsigned from = (unsigned)(upto[k] - own[k]) + (first_[k] | first_[k + 4] << 16);
+                    places[k * WAVE + lane] = (unsigned short)from;
+                    places[(k + 4) * WAVE + lane] = (unsigned short)(from >> 16);
+                }
+                for (int b = lane; b < count; b += WAVE) {
+                    const float d2 = cand_d2[b];
+                    unsigned short *next = places + class_of(d2) * WAVE + lane;
+                    const int at = *next;
+                    *next = (unsigned short)(at + 1);
+                    p.d2[u * cap + at] = d2;
+                    if (p.n) p.n[u * cap + at] = cand_n[b];
                 }
             }
         }
@@ -696,12 +742,14 @@ __global__ __launch_bounds__(512, DT > 1 || NT > 4 ? 6 : 8) void real_enc_infer_
     }
 }
 
-// Entries a unit may have: all of a small fixed cube, else what `limit` bytes hold of 6-byte entries, in powers of two from
-// 128 to 1024 (seven blocks on 256 crystals, r0 = 3 A: 232 in the mean, one unit in a hundred above 700).
+// Entries a unit may have: all of a small fixed cube, else 832 (what leaves six staging work-groups a CU: seven blocks on 256
+// crystals, r0 = 3 A, have 232 in the mean and one unit in a hundred above 700), or the power of two from 128 to 512 whose
+// 6-byte entries `limit` bytes hold.
 int capacity_of(int64_t U, bool boxes, int64_t limit)
 {
     if (!boxes) return 128;
-    int cap = 1024;
+    if (U * MOST_STAGED * 6 <= limit) return MOST_STAGED;
+    int cap = 512;
     while (cap > 128 && U * cap * 6 > limit) cap >>= 1;
     return cap;
 }
@@ -782,7 +830,7 @@ int launch_infer_stage(const float *rpos, const float *tvecs, const float *rvlen
         w.bins[l] = bins[l];
     }
     const int packs = w.blocks * w.heads * w.DT, pack_groups = (packs + STAGE_WAVES - 1) / STAGE_WAVES;
-    const size_t lds = (size_t)STAGE_WAVES * (boxes ? 3 : 2) * (m.capacity + WAVE) * 2;
+    const size_t lds = (size_t)STAGE_WAVES * ((boxes ? 3 : 2) * (m.capacity + WAVE) * 2 + CLASSES * WAVE * 2);
     const int64_t want = (U + STAGE_WAVES - 1) / STAGE_WAVES, cap = persistent_grid_cap(lds > 20000 ? 6 : 8);
     infer_stage_kernel<<<pack_groups + (int)(want < cap ? want : cap), STAGE_WAVES * WAVE, lds, st>>>(p, w);
     CF_CHECK_LAUNCH("infer_stage");

@@ -30,7 +30,7 @@ from .lib import device_guard, stream_handle
 
 
 # What the staged translations of a forward may take: 700 MB for 890 thousand atom pairs in the fixed cube; with adaptive boxes
-# the capacity of a pair follows from it (256 translations there, 1024 below 250 thousand pairs).
+# the capacity of a pair follows from it (256 translations there, 832 below 320 thousand pairs).
 STAGED_UNITS_MAX_BYTES = 3 << 29
 
 

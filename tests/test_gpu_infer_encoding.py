@@ -1,6 +1,6 @@
 """The encoding of an inference forward (``csrc/real_enc_infer.hip``: units staged once, split matrix products) against the
 operators' kernels, which have the reference's sums in fp32, and against the oracle in float64: the edges of its groups
-(16), chunks (64) and images (1024), of its bin and row tiles, and the units its staging leaves to the blocks."""
+(16), chunks (64) and images (832), of its bin and row tiles, and the units its staging leaves to the blocks."""
 import dataclasses
 
 import pytest
@@ -59,6 +59,14 @@ def test_heads_and_row_tiles(dev, width, heads, adaptive):
 def test_translations_a_unit(dev, length, r0, options):
     cell = list(length) if isinstance(length, tuple) else [length, 1.1 * length, 0.9 * length]
     compare(dev, crystals([cell, [8.0, 7.0, 9.0]], [6, 9]), scale_real=[r0], **options)
+
+
+# boxes longest along each axis, whose translations are walked along one of the three; more than 64 staged, and counts on both
+# sides of what an image holds
+@pytest.mark.parametrize("length", [(20.0, 3.0, 4.0), (3.0, 20.0, 4.0), (4.0, 3.0, 20.0), (2.5, 2.5, 9.0), (9.0, 2.5, 2.5),
+                                    (2.5, 9.0, 2.5), (2.7,) * 3, (2.9,) * 3, (3.1,) * 3, (3.3,) * 3])
+def test_boxes_along_each_axis(dev, length):
+    compare(dev, crystals([list(length)] * 3, [4, 9, 1], angles=[[80.0, 95.0, 110.0]] * 3), scale_real=[3.0])
 
 
 def test_less_room_than_units_need(dev, monkeypatch):

@@ -604,7 +604,8 @@ def main() -> int:
     ms_per_step = elapsed / args.steps * 1e3
     value = B * args.steps / elapsed
 
-    # ---- roofline of the dominant kernel (periodic encoding, forward)
+    # ---- roofline of the operators' encoding kernel, forward (the timed steps' native call has an encoding of its own, whose
+    # products are split f16 ones; training and callers of the operators run this one)
     enc_ms = [s.elapsed_time(e) for (name, s, e, info) in log if name == "real_enc_fwd"]
     dpa_ms = [s.elapsed_time(e) for (name, s, e, info) in log if name == "fused_dpa_fwd"]
     stage_ms = [s.elapsed_time(e) for (name, s, e, info) in log if name == "real_enc_ring_stage"]

@@ -16,6 +16,9 @@
 //     4.5 tiles of 16 a pair with r0 = 1.4 A where the others evaluate 32 and 16 of 4, 64 and 10 where 98 and 47 with 3 A;
 //   * square roots, column lookups and tile tests are made for these only, lane = translation;
 //   * nothing about the pair passes through vector registers: its 32 bytes are scalar loads.
+// What bounds a block now is the issue of vector instructions, 843 a pair at the largest, slots 84 % busy.  Measured, pair and
+// ring kernels -> this, a block: 28 thousand pairs in the fixed cube 43.5 -> 33.8 us, in boxes 45.4 and 9.4 for the lists ->
+// 38.1, 294 thousand (mean of seven blocks) 440 and 15 -> 276, 958 thousand 3060 -> 1570.
 //
 // Lane roles of the accumulation (q = lane / 16, c = lane % 16): lane (q, c) holds translations 4 q .. 4 q + 3 of a group of
 // 16: column c's weights (B operand) and the Gaussians of bin 16 m + c of every tile m in reach (A operand).  Projection

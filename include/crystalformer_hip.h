@@ -509,7 +509,8 @@ typedef struct {
     int64_t lattice_range, minimum_range;
     int64_t adaptive;                 /* 0: cutoffs are ignored, every box is the fixed cube */
     int64_t update_stats;             /* training mode without gradients: store the exponent statistics */
-    int64_t staged_rings, adaptive_rings, ring_limit_bytes;   /* whether and up to what size blocks share staged rings */
+    int64_t staged_rings, adaptive_rings, ring_limit_bytes;   /* whether blocks (with adaptive boxes too) share staged
+                                         translations, and how many bytes these may take */
     int64_t hidden, targets;          /* head: width -> hidden (ReLU) -> targets; hidden 0: width -> targets;
                                          targets 0: out takes the encoder's output (N, width) */
     int64_t embed_width;

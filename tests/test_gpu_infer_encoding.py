@@ -97,7 +97,7 @@ def test_skewed_cells_with_and_without_a_floor(dev, floor, monkeypatch):
     assert_close(native, modules, "encoder", atol=atol_rows(modules))
 
 
-@pytest.mark.parametrize("bound", [0.0, 0.1, 0.25, 0.9])
+@pytest.mark.parametrize("bound", [0.0, 0.04, 0.05, 0.1, 0.25, 0.9])
 @pytest.mark.parametrize("adaptive", [-3.5, 0.0])
 def test_bounds_of_the_exponents(dev, bound, adaptive):
     compare(dev, batch_of([5, 14]), gauss_lb_real=bound, positive_func="abs", adaptive_cutoff_sigma=adaptive)

@@ -114,6 +114,9 @@ int check_block(const cf_block_train *args, const char *who)
     const cf_block_train &f = *args;
     CF_REQUIRE(f.N >= 1 && f.E >= 1 && f.B >= 1 && f.U >= 1 && f.H >= 1 && f.H <= 32 && W % f.H == 0 && W / f.H % 4 == 0 &&
                    f.bins >= 0 && f.bins <= 128, CF_ERR_INVALID_ARGUMENT, "%s: bad sizes", who);
+    CF_REQUIRE(2 * f.U == f.E + f.N, CF_ERR_INVALID_ARGUMENT,
+               "%s: a pair list over dense crystal blocks has (E+N)/2 = %lld entries, got %lld", who,
+               (long long)((f.E + f.N) / 2), (long long)f.U);
     return CF_OK;
 }
 

@@ -237,7 +237,7 @@ class CrystalformerEncoderCUDA(Module):
             kr_base = ops.kr_base(pos_ij, recip, batch, edges)
         output = src
         pack = executor.pack_for_training(self, src)
-        native = executor.native_training(self, pack, layout, pos_ij, trans, rvlen) if pack is not None else None
+        native = executor.native_training(self, src, pack, layout, pos_ij, trans, rvlen) if pack is not None else None
         for i, layer in enumerate(self.layers):
             if pack is not None:
                 output = layer(output, batch, edges, pos_ij, dist2_min, trans, kr_base, rvecs, vcell, onehot,

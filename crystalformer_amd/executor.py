@@ -159,11 +159,14 @@ def pack_for_training(encoder: nn.Module, src: Tensor) -> Optional["ops.PackedBl
     return pack
 
 
-def native_training(encoder: nn.Module, pack: "ops.PackedBlocks", layout, rpos: Tensor, tvecs: Tensor, rvlen: Tensor):
+def native_training(encoder: nn.Module, src: Tensor, pack: "ops.PackedBlocks", layout, rpos: Tensor, tvecs: Tensor,
+                    rvlen: Tensor):
     """The blocks of a fused training step as one call each way (:class:`hip_funcs.BlockTrainHIP`), in the order of the
     layers, or None where the operators run one by one: under instrumentation, without a pair list, with operands that the
-    operators convert or refuse, or with an encoding other than the one the call has."""
-    if ops.instrumented() or layout.pairs is None or layout.num_edges == 0 or not hip_funcs.KernelManager.DENSE_EDGE_BLOCKS:
+    operators convert or refuse (a row too many or too few among them), or with an encoding other than the one the call
+    has."""
+    if ops.instrumented() or layout.pairs is None or layout.num_edges == 0 or src.shape[0] != layout.num_atoms \
+            or not hip_funcs.KernelManager.DENSE_EDGE_BLOCKS:
         return None
     index, B = layout.batch.get_device(), tvecs.shape[0]
     if not _ready(rpos, 3 * layout.num_edges, index) or not _ready(tvecs, 9 * B, index) or not _ready(rvlen, 3 * B, index) \

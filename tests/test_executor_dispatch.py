@@ -1,12 +1,14 @@
 """Which models, batches and settings the native inference call is chosen for, on the CPU (the call itself is
 replaced by a marker), and on the GPU that everything it leaves alone computes what its modules say."""
+import ctypes
 import dataclasses
+import types
 
 import pytest
 import torch
 from torch import nn
 
-from crystalformer_amd import executor
+from crystalformer_amd import executor, lib, ops
 from crystalformer_amd.encoder import CrystalformerEncoderCUDA
 from crystalformer_amd.lib import CrystalformerHipError
 from crystalformer_amd.latticeformer import Latticeformer, default_params
@@ -378,3 +380,21 @@ def test_declined_models_are_hardly_looked_at(monkeypatch):
             assert executor.forward(model, b) == (None, None)
             assert executor.encode(model.encoder, b.x, b.pos, b.batch, b.trans_vec, b.sizes) is None
         assert not looked, options
+
+
+@pytest.mark.parametrize("rows, served", [(0, True), (1, False), (-1, False)])
+def test_a_training_block_has_a_row_an_atom(rows, served):
+    """A row too many or too few is left to the operators, which say what is wrong, before anything is launched: the
+    native call has the batch's index structure and takes the row count from the features."""
+    model, b = small_model().train(), small_batch()
+    N, E, B = len(b.batch), int((b.sizes ** 2).sum()), len(b.sizes)
+    layout = ops.BatchLayout()
+    layout.batch, layout.pairs, layout.num_atoms, layout.num_edges = b.batch, torch.zeros((E + N) // 2, 5), N, E
+    layout.atom_start = torch.zeros(B + 1, dtype=torch.int64)
+    pack = types.SimpleNamespace(settings=[([0] * 26, 8, True)] * 2)
+    got = executor.native_training(model.encoder, torch.zeros(N + rows, 128), pack, layout, torch.zeros(E, 3),
+                                   b.trans_vec, torch.zeros(B, 3))
+    assert (got is not None) == served
+    need = (ctypes.c_int64 * 4)()
+    args = lib.BlockTrain(N + rows, E, B, (E + N) // 2, 8, 64)
+    assert (lib.load().cf_block_train_bytes(ctypes.byref(args), need) == 0) == served

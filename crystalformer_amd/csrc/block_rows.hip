@@ -10,7 +10,9 @@
 // A work-group of 8 wavefronts owns 16 T rows; the rows and all intermediates stay in LDS, the weights
 // (786 KB a block) stream from the L2, a 16-column tile per wavefront, two tiles ahead of their use.  The products
 // are split f16 ones (split_f16.h): a column's weights are scaled and split once per forward (forward_prologue_kernel), a
-// row's values in LDS in front of each layer, in place.  So the matrix cores need 2.7 us for 16 rows, where fp32 ones
+// row's values in LDS in front of each layer, in place, each in pieces of 128 with a scale of their own.  A value 2^-27 of the
+// largest of its piece keeps its 22 bits: hidden units 2^26 apart that meet weights as far apart are as close to float64 as any
+// (rms 8.3e-8 of an encoder's output; fp32 products, whose sums round oftener, 1.5e-7).  So the matrix cores need 2.7 us for 16 rows, where fp32 ones
 // needed 10 and bound the launch at 4096 rows, and 16 rows are the least tile: half the work-groups, and half the weights
 // asked of the L2, that eight fp32 rows had at 1774 rows.  What bounds a launch now is the chain of one tile: 16 rows are
 // staged in 2.5 us, each of the twelve units of 128 columns takes 0.5, each of the four splits 0.3, output and exponents 0.9.
@@ -86,7 +88,7 @@ __device__ __forceinline__ void multiply(float4_t (&acc)[T], const Weights &b, c
             lh = mfma32(a.lo[t][s], hi, lh);
             ll = mfma32(a.lo[t][s], lo, ll);
         }
-        acc[t] = hh + ((hl + lh) + ll);
+        acc[t] = sum_of_kinds(hh, hl, lh, ll);
         // (the products belong here: left to itself the compiler moves them to where the sums are used, and keeps
         // every weight until then)
         asm volatile("" : "+v"(acc[t]));
@@ -105,31 +107,35 @@ __device__ __forceinline__ float half_wave_max(float v)
     return fmaxf(__int_as_float((int)r[0]), __int_as_float((int)r[1]));
 }
 
-// Four values of each of L pieces of 128 columns of a row, scaled to [2^14, 2^15) of the row's largest and split: of every
-// eight values (32 bytes) the eight his, then the eight los.  32 threads a row, thread j has columns 4 j .. 4 j + 3.
+// Four values of each of L pieces of 128 columns of a row, scaled by the largest magnitude of the row's piece and split
+// (split2_far): of every eight values (32 bytes) the eight his, then the eight los.  32 threads a row, thread j has columns
+// 4 j .. 4 j + 3; the exponent of piece l goes to exp[l * stride].
 template <int L>
-__device__ __forceinline__ void split_row(float4_t (&v)[L], float *row, int j, int *exp)
+__device__ __forceinline__ void split_row(float4_t (&v)[L], float *row, int j, int *exp, int stride)
 {
-    float zero = 0.f, top = 0.f;
+    float zero = 0.f;
     asm volatile("" : "+v"(zero));
+    float *hi = row + 8 * (j / 2) + 2 * (j % 2);
+    int e[L];
 #pragma unroll
-    for (int l = 0; l < L; l++)
+    for (int l = 0; l < L; l++) {
+        float top = 0.f;
 #pragma unroll
         for (int i = 0; i < 4; i++) top = fmaxf(top, fabsf(v[l][i]));
-    const int e = __builtin_amdgcn_frexp_expf(half_wave_max(top));               // (0 for 0, infinity and NaN)
-    if (j == 0) *exp = e;
-    float *hi = row + 8 * (j / 2) + 2 * (j % 2);
+        e[l] = __builtin_amdgcn_frexp_expf(half_wave_max(top));                  // (0 for 0, infinity and NaN)
+        if (j == 0) exp[l * stride] = e[l];
+    }
 #pragma unroll
     for (int l = 0; l < L; l++) {
 #pragma unroll
-        for (int i = 0; i < 4; i++) v[l][i] = ldexpf(v[l][i], 15 - e);
-        const Split2 a = split2(v[l][0], v[l][1], 1.0f, zero), b = split2(v[l][2], v[l][3], 1.0f, zero);
+        for (int i = 0; i < 4; i++) v[l][i] = ldexpf(v[l][i], 26 - e[l]);
+        const Split2 a = split2_far(v[l][0], v[l][1], zero), b = split2_far(v[l][2], v[l][3], zero);
         *reinterpret_cast<int2_t *>(hi + RW * l) = int2_t{a.hi, b.hi};
         *reinterpret_cast<int2_t *>(hi + RW * l + 4) = int2_t{a.lo, b.lo};
     }
 }
 
-// The rows of an LDS buffer split in place (a group's two lanes have read both before either writes).
+// The rows of an LDS buffer split in place (a group's two lanes have read both before either writes); exps: M a piece.
 template <int M, int L>
 __device__ __forceinline__ void split_rows(float *xs, int ld, int *exps)
 {
@@ -140,7 +146,7 @@ __device__ __forceinline__ void split_rows(float *xs, int ld, int *exps)
         float4_t v[L];
 #pragma unroll
         for (int l = 0; l < L; l++) v[l] = *reinterpret_cast<const float4_t *>(xs + r * ld + 4 * j + RW * l);
-        split_row<L>(v, xs + r * ld, j, exps + r);
+        split_row<L>(v, xs + r * ld, j, exps + r, M);
     }
 }
 
@@ -440,7 +446,7 @@ __device__ __forceinline__ void pack_split(const PackArgs &p, int x, int l)
         int4_t hi, lo;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            const Split2 y = split2(ldexpf(w[s][i / 2][2 * i % 4], 15 - e), ldexpf(w[s][i / 2][2 * i % 4 + 1], 15 - e), 1.0f, zero);
+            const Split2 y = split2_far(ldexpf(w[s][i / 2][2 * i % 4], 26 - e), ldexpf(w[s][i / 2][2 * i % 4 + 1], 26 - e), zero);
             hi[i] = y.hi;
             lo[i] = y.lo;
         }
@@ -495,7 +501,7 @@ __global__ __launch_bounds__(RT, 2) void block_rows_kernel(RowsArgs p)
     __shared__ __align__(16) float hs[M * LDH];                 // hidden units, then query, key, value
     __shared__ float biases[UNIT_END * RW], w_pos[RW];
     __shared__ int w_exp[UNIT_END * RW];
-    __shared__ __align__(16) int x_exp[M];
+    __shared__ __align__(16) int x_exp[4 * M];                  // (the reduction's four pieces of a row have their own)
     __shared__ float red[2];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int q = lane >> 4, c = lane & 15;
@@ -514,7 +520,8 @@ __global__ __launch_bounds__(RT, 2) void block_rows_kernel(RowsArgs p)
     };
     // this lane's value of row 16 t + 4 q + r in unit u
     auto value = [&](const float4_t (&acc)[T], int t, int r, int u) -> float {
-        const int4_t e = *reinterpret_cast<const int4_t *>(x_exp + 16 * t + 4 * q);
+        const int piece = u >= UNIT_FF2 && u < UNIT_FF2 + 4 && SRC == ROWS_TAIL ? u - UNIT_FF2 : 0;
+        const int4_t e = *reinterpret_cast<const int4_t *>(x_exp + piece * M + 16 * t + 4 * q);
         return ldexpf(acc[t][r], e[r] + w_exp[u * RW + col]) + biases[u * RW + col];
     };
     // (one tile per work-group unless the grid was cut short: with a live row count it covers a capacity)
@@ -581,7 +588,7 @@ __global__ __launch_bounds__(RT, 2) void block_rows_kernel(RowsArgs p)
 #pragma unroll
         for (int t = 0; t < PASSES; t++) {
             const int r = 16 * t + threadIdx.x / 32;
-            split_row<1>(in[t], b2 + r * LDX, j, x_exp + r);
+            split_row<1>(in[t], b2 + r * LDX, j, x_exp + r, M);
             if (SRC == ROWS_TAIL) *reinterpret_cast<float4_t *>(b1 + r * LDX + 4 * j) = residual[t];
         }
         __syncthreads();

@@ -33,7 +33,7 @@ namespace {
 using namespace cf;
 using namespace cfpair;
 
-constexpr float SPLIT = 32768.0f;           // values up to 1 are split scaled by it: 22 bits down to 2^-18, absolute 2^-40 below
+constexpr float SPLIT = 32768.0f;           // values up to 1 are split scaled by it: 22 bits down to 2^-17, off by up to 2^-40 below
 constexpr float PAD_D2 = 1e30f;             // d^2 of a slot without a translation: weight 0 and Gaussian 0
 constexpr float LEAST_A2 = -1e-25f;         // no decay slower: 1 for every real distance, 0 for PAD_D2
 constexpr int CLASSES = 8;                  // of d^2: seven of equal width and one for what lies beyond

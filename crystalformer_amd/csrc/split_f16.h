@@ -1,6 +1,6 @@
 // fp32 products on the f16 matrix instructions: both factors as two halves of 11 bits, x 2^k = hi + lo, and all four
 // products summed in fp32.  Scaled so that the largest value lies in [2^14, 2^15) a value keeps 22 bits and a sign down to
-// 2^-17 of it and 2^-40 of it absolutely below.  v_mfma_f32_16x16x32_f16 runs beside vector instructions (17 cycles; eight
+// 2^-16 of it and is off by up to 2^-39 of it below (a half's last bit is 2^-24).  v_mfma_f32_16x16x32_f16 runs beside vector instructions (17 cycles; eight
 // v_fma beside it 36, 22 without it) where v_mfma_f32_16x16x4_f32 holds them up (32 cycles; 57 with the same eight).
 #pragma once
 #include "cf_common.h"
@@ -28,6 +28,31 @@ __device__ __forceinline__ Split2 split2(float x0, float x1, float scale, float 
     const half2_t l = {(_Float16)__builtin_fmaf(x0, scale, -(float)h[0]), (_Float16)__builtin_fmaf(x1, scale, -(float)h[1])};
     s.lo = __builtin_bit_cast(int, l);
     return s;
+}
+
+// The same with the second halves scaled by 2^11 beyond the first, for values that share a scale with others of any size: of
+// values scaled by 2^26 (the largest in [2^25, 2^26)) one keeps 22 bits and a sign down to 2^-27 of the largest and is off by up
+// to 2^-50 of it below.  The products of each kind of halves are summed apart (sum_of_kinds), which a long sum wants anyway:
+// every addition to the large sum rounds it.
+constexpr float LO_SCALE = 2048.0f;
+__device__ __forceinline__ Split2 split2_far(float y0, float y1, float zero)
+{
+    half2_t h = {(_Float16)__builtin_fmaf(y0, 1.0f / LO_SCALE, zero), (_Float16)__builtin_fmaf(y1, 1.0f / LO_SCALE, zero)};
+    Split2 s;
+    s.hi = __builtin_bit_cast(int, h);
+    asm("" : "+v"(s.hi));                   // (as above)
+    h = __builtin_bit_cast(half2_t, s.hi);
+    const half2_t l = {(_Float16)__builtin_fmaf((float)h[0], -LO_SCALE, y0), (_Float16)__builtin_fmaf((float)h[1], -LO_SCALE, y1)};
+    s.lo = __builtin_bit_cast(int, l);
+    return s;
+}
+__device__ __forceinline__ float4_t sum_of_kinds(float4_t hh, float4_t hl, float4_t lh, float4_t ll)
+{
+    float4_t r;
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+        r[i] = __builtin_fmaf(__builtin_fmaf(ll[i], 1.0f / LO_SCALE, hl[i] + lh[i]), 1.0f / LO_SCALE, hh[i]);
+    return r;
 }
 
 __device__ __forceinline__ float4_t mfma16(int2_t a, int2_t b, float4_t c)

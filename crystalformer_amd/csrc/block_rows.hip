@@ -12,13 +12,15 @@
 // are split f16 ones (split_f16.h): a column's weights are scaled and split once per forward (forward_prologue_kernel), a
 // row's values in LDS in front of each layer, in place, each in pieces of 128 with a scale of their own.  A value 2^-27 of the
 // largest of its piece keeps its 22 bits: hidden units 2^26 apart that meet weights as far apart are as close to float64 as any
-// (rms 8.3e-8 of an encoder's output; fp32 products, whose sums round oftener, 1.5e-7).  So the matrix cores need 2.7 us for 16 rows, where fp32 ones
-// needed 10 and bound the launch at 4096 rows, and 16 rows are the least tile: half the work-groups, and half the weights
-// asked of the L2, that eight fp32 rows had at 1774 rows.  What bounds a launch now is the chain of one tile: 16 rows are
-// staged in 2.5 us, each of the twelve units of 128 columns takes 0.5, each of the four splits 0.3, output and exponents 0.9.
-// Without the weights' loads it would be 10.4 us at 12 rows; five buffers of weights instead of three: 0.9 us slower.
-// Measured, tail and head in a forward, fp32 products -> these: 12 rows 13.6 -> 12.5 us, 290 rows 13.9 -> 13.4,
-// 1774 rows 18.2 -> 13.9 (0.70 GFLOP: 50 TFLOP/s), 5.2 thousand rows 40 -> 21.4 (95 TFLOP/s).
+// (rms 8.3e-8 of an encoder's output, up to 2^28; fp32 products, whose sums round oftener, 1.5e-7), 2^32 apart 2.2e-7, 2^36
+// 3.1e-6.  So the matrix cores need 2.7 us for 16 rows, where fp32 ones needed 10 and bound the launch at 4096 rows, and 16 rows
+// are the least tile: half the work-groups, and half the weights asked of the L2, that eight fp32 rows had at 1774 rows.  What
+// bounds a launch now is the chain of one tile: 16 rows are staged in 2.5 us, each of the twelve units of 128 columns takes
+// 0.5, each of the four splits 0.3, output and exponents 0.9.  Without the weights' loads it would be 10.4 us at 12 rows; five
+// buffers of weights instead of three: 0.9 us slower.
+// Measured, tail and head in a forward, fp32 products -> these: 12 rows 13.7 -> 12.7 us, 1774 rows 17.6 -> 13.6 (0.70 GFLOP: 51
+// TFLOP/s), 4096 rows 25.8 -> 17.1, 5.2 thousand rows 40 -> 21.5 (95 TFLOP/s).  One scale a row instead of one a piece, and first
+// and second halves scaled alike, made it 12.2, 13.4, 16.8 and 20.0, and lost what lies below 2^-16 of a row's largest.
 // Operands of v_mfma_f32_16x16x32_f16, lane (q, c) = (lane / 16, lane % 16), reduction step s of 32:
 //   A: 16 bytes of row c at k = 32 s + 8 q, hi or lo;  B: the same of column c's weights;  D: row 4 q + r, column c.
 // A row's sums do not depend on T or on the tile it falls in.
@@ -95,16 +97,22 @@ __device__ __forceinline__ void multiply(float4_t (&acc)[T], const Weights &b, c
     }
 }
 
-// The largest magnitude of 32 adjacent lanes, in each of them.
-__device__ __forceinline__ float half_wave_max(float v)
+// The largest of 32 adjacent lanes' magnitudes, in each of them.  By the bits: of floats >= 0 the order of the integers is
+// theirs (as floats every step costs a canonicalising instruction beside the one on the DPP path).
+template <int CTRL>
+__device__ __forceinline__ int dpp_max(int v)
 {
-    v = fmaxf(v, dpp_f<DPP_QUAD_1032, 0xF>(v, v));
-    v = fmaxf(v, dpp_f<DPP_QUAD_2301, 0xF>(v, v));
-    v = fmaxf(v, dpp_f<DPP_ROW_ROR4, 0xF>(v, v));
-    v = fmaxf(v, dpp_f<DPP_ROW_ROR8, 0xF>(v, v));
-    const unsigned x = (unsigned)__float_as_int(v);
-    const uint2_cf r = __builtin_amdgcn_permlane16_swap(x, x, false, false);
-    return fmaxf(__int_as_float((int)r[0]), __int_as_float((int)r[1]));
+    return max(v, __builtin_amdgcn_update_dpp(v, v, CTRL, 0xF, 0xF, false));
+}
+__device__ __forceinline__ int magnitude_bits(float x) { return __float_as_int(x) & 0x7FFFFFFF; }
+__device__ __forceinline__ int half_wave_max(int v)
+{
+    v = dpp_max<DPP_QUAD_1032>(v);
+    v = dpp_max<DPP_QUAD_2301>(v);
+    v = dpp_max<DPP_ROW_ROR4>(v);
+    v = dpp_max<DPP_ROW_ROR8>(v);
+    const uint2_cf r = __builtin_amdgcn_permlane16_swap((unsigned)v, (unsigned)v, false, false);
+    return max((int)r[0], (int)r[1]);
 }
 
 // Four values of each of L pieces of 128 columns of a row, scaled by the largest magnitude of the row's piece and split
@@ -116,13 +124,26 @@ __device__ __forceinline__ void split_row(float4_t (&v)[L], float *row, int j, i
     float zero = 0.f;
     asm volatile("" : "+v"(zero));
     float *hi = row + 8 * (j / 2) + 2 * (j % 2);
+    int top[L], all = 0;
+#pragma unroll
+    for (int l = 0; l < L; l++) {
+        top[l] = max(max(magnitude_bits(v[l][0]), magnitude_bits(v[l][1])), max(magnitude_bits(v[l][2]), magnitude_bits(v[l][3])));
+        top[l] = half_wave_max(top[l]);
+        all = max(all, top[l]);
+    }
+    if (__builtin_expect(__ballot(all >= 0x7F800000) != 0ull, 0)) {              // infinities, or not a number
+#pragma unroll
+        for (int l = 0; l < L; l++) {
+            float t = 0.f;
+#pragma unroll
+            for (int i = 0; i < 4; i++) t = fmaxf(t, finite_magnitude(v[l][i]));
+            top[l] = half_wave_max(__float_as_int(t));
+        }
+    }
     int e[L];
 #pragma unroll
     for (int l = 0; l < L; l++) {
-        float top = 0.f;
-#pragma unroll
-        for (int i = 0; i < 4; i++) top = fmaxf(top, fabsf(v[l][i]));
-        e[l] = __builtin_amdgcn_frexp_expf(half_wave_max(top));                  // (0 for 0, infinity and NaN)
+        e[l] = __builtin_amdgcn_frexp_expf(__int_as_float(top[l]));              // (0 for 0)
         if (j == 0) exp[l * stride] = e[l];
     }
 #pragma unroll
@@ -436,7 +457,16 @@ __device__ __forceinline__ void pack_split(const PackArgs &p, int x, int l)
     for (int s = 0; s < 4; s++)
 #pragma unroll
         for (int i = 0; i < 8; i++) top = fmaxf(top, fabsf(w[s][i / 4][i % 4]));
-    const int e = __builtin_amdgcn_frexp_expf(rows_max(top));
+    top = rows_max(top);
+    if (__ballot(top == __builtin_inff()) != 0ull) {
+        top = 0.f;
+#pragma unroll
+        for (int s = 0; s < 4; s++)
+#pragma unroll
+            for (int i = 0; i < 8; i++) top = fmaxf(top, finite_magnitude(w[s][i / 4][i % 4]));
+        top = rows_max(top);
+    }
+    const int e = __builtin_amdgcn_frexp_expf(top);
     float zero = 0.f;
     asm volatile("" : "+v"(zero));
     float *units = l == p.blocks ? p.packed_embed : p.packed + (int64_t)l * SPLIT_BLOCK;
@@ -634,7 +664,7 @@ __global__ __launch_bounds__(RT, 2) void block_rows_kernel(RowsArgs p)
                 Rows<T> &now = u % 2 ? ahead : x;
                 if (u < 3) read_rows(u % 2 ? x : ahead, hs + (u + 1) * RW, LDH, lane);
                 multiply(acc, unit(UNIT_FF2 + u), now);
-                // (a unit's columns have exponents of their own)
+                // (a unit's columns have exponents of their own, and a row's pieces)
 #pragma unroll
                 for (int t = 0; t < T; t++)
 #pragma unroll
@@ -1139,8 +1169,8 @@ int launch_block_rows(RowsArgs p, hipStream_t st)
     p.live_N = live_atoms(p.N);
     const int64_t cus = device_cu_count();
     // 32 rows a tile beyond one round of 16 (a tile a CU): 257 to 512 tiles of 16 are two rounds, the second short of
-    // work, and ask for the weights twice as often.  At 5.2 thousand rows 21.4 us a launch against 28.6; up to one round 16 are
-    // better, with all CUs at work (1774 rows: 13.9 us, on 111 of them, and a tile of 32 is the 21.4).
+    // work, and ask for the weights twice as often.  At 5.2 thousand rows 21.5 us a launch against 28.6; up to one round 16 are
+    // better, with all CUs at work (1774 rows: 13.6 us, on 111 of them, and a tile of 32 is the 21.5).
     // (Live rows are somewhere below the capacity; a tile has at most 256 exponents, see complete_groups.)
     const int T = !p.live_N && p.N > 16 * cus && p.H <= 8 ? 2 : 1;
     int64_t grid = (p.N + 16 * T - 1) / (16 * T);

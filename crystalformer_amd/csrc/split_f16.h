@@ -46,14 +46,22 @@ __device__ __forceinline__ Split2 split2_far(float y0, float y1, float zero)
     s.lo = __builtin_bit_cast(int, l);
     return s;
 }
+// (An infinite value's second half is not a number, and an infinity times a second half has any sign: the first halves' product
+// is fp32's answer then, the rest is kept finite.  Of finite values the rest is below 2^60.)
 __device__ __forceinline__ float4_t sum_of_kinds(float4_t hh, float4_t hl, float4_t lh, float4_t ll)
 {
     float4_t r;
 #pragma unroll
-    for (int i = 0; i < 4; i++)
-        r[i] = __builtin_fmaf(__builtin_fmaf(ll[i], 1.0f / LO_SCALE, hl[i] + lh[i]), 1.0f / LO_SCALE, hh[i]);
+    for (int i = 0; i < 4; i++) {
+        const float rest = __builtin_fmaf(ll[i], 1.0f / LO_SCALE, hl[i] + lh[i]);
+        r[i] = __builtin_fmaf(__builtin_amdgcn_fmed3f(rest, -0x1p100f, 0x1p100f), 1.0f / LO_SCALE, hh[i]);
+    }
     return r;
 }
+
+// (The exponent of a group of values is that of its largest finite one: beside an infinity's own the others would leave a
+// half's range.)
+__device__ __forceinline__ float finite_magnitude(float x) { return fabsf(x) < __builtin_inff() ? fabsf(x) : 0.f; }
 
 __device__ __forceinline__ float4_t mfma16(int2_t a, int2_t b, float4_t c)
 {

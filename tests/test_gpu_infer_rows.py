@@ -104,3 +104,32 @@ def test_features_at_the_ends_of_the_range(dev, value):
         assert torch.isfinite(native).all()
     else:
         assert torch.equal(torch.isfinite(native).all(1), torch.isfinite(modules).all(1))
+
+
+# One infinite weight, behind which a product is infinite with the other factor's sign (and not a number where that is zero)
+@pytest.mark.parametrize("where", ["linear2.weight", "linear1.weight", "self_attn.out_proj.weight", "self_attn.v_proj_weight"])
+@pytest.mark.parametrize("value", [float("inf"), float("-inf")])
+def test_infinite_weights(dev, where, value):
+    model = prepared(dev, num_layers=1)
+    b = batch_of([1, 5, 40]).to(dev)
+    with torch.no_grad():
+        dict(model.encoder.layers[0].named_parameters())[where][37, 50] = value
+        model.encoder.layers[0].linear2.weight[5, 3] = 0.0
+    native, modules = both_ways(model, b)
+    assert torch.isinf(modules).any() or where != "linear2.weight"
+    for same in (torch.isposinf, torch.isneginf, torch.isnan):
+        assert torch.equal(same(native), same(modules))
+    finite = torch.isfinite(modules)
+    if finite.any():
+        assert_close(native[finite], modules[finite], "finite values", rtol=RTOL, atol=RTOL * float(modules[finite].abs().max()))
+
+
+def test_infinite_rows(dev):
+    """A row with an infinity in front of the head whose products nobody adds up again: the values behind the embedding."""
+    model = prepared(dev, num_layers=1)
+    for sign in (1.0, -1.0):
+        b = batch_of([3, 4])
+        b.x[1, 7] = sign * float("inf")
+        native, modules = both_ways(model, b.to(dev))
+        for same in (torch.isposinf, torch.isneginf, torch.isnan):
+            assert torch.equal(same(native), same(modules))

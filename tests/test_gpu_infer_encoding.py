@@ -127,3 +127,38 @@ def test_no_further_from_float64_than_the_operators(dev, r0):
     err = [float((t.cpu().double() - want).square().mean().sqrt()) for t in (native, modules)]
     print("\nrms from float64: staged %.3e, operators %.3e" % tuple(err), flush=True)
     assert err[0] <= 1.1 * err[1], err
+
+
+def distances_from_float64(dev, cfg, change, b):
+    """Root mean squares of the distance to the oracle in float64: (native call, operators), one block after ``change``."""
+    model = scaled(cfg)
+    with torch.no_grad():
+        change(model)
+    P = {k: v.detach().double() for k, v in model.state_dict().items()}
+    with torch.no_grad():
+        x = torch.nn.functional.linear(b.x.double(), P["input_embeddings.weight"])
+        want = om.encoder_forward(P, cfg, x, b.pos.double(), b.batch, b.trans_vec.double(), b.sizes)
+    want = want[0] if isinstance(want, tuple) else want
+    return [float((t.cpu().double() - want).square().mean().sqrt()) for t in both_ways(model.to(dev).eval(), b.to(dev))]
+
+
+# Bins whose weights are up to 2^24 apart: within a tenth of the fp32 products' own distance.
+@pytest.mark.parametrize("bins", [16, 64])
+def test_projections_of_any_magnitude(dev, bins):
+    def change(model):
+        g = torch.Generator().manual_seed(12)
+        model.encoder.layers[0].self_attn.pe_dist_proj.mul_(torch.exp2(torch.randint(-24, 1, (bins,), generator=g).float()))
+    cfg = default_params(num_layers=1, adaptive_cutoff_sigma=0.0, value_pe_dist_real=bins)
+    err = distances_from_float64(dev, cfg, change, batch_of([40, 17, 25, 8]))
+    assert err[0] <= 1.1 * err[1], err
+
+
+def test_infinite_projection_weights(dev):
+    model = scaled(default_params(num_layers=1)).to(dev).eval()
+    with torch.no_grad():
+        model.encoder.layers[0].self_attn.pe_dist_proj[0, 3, 5, 20] = float("inf")
+        model.encoder.layers[0].self_attn.out_proj.weight[:, 3 * 16 + 5] = 0.0
+        model.encoder.layers[0].self_attn.out_proj.weight[7, 3 * 16 + 5] = 1.0
+    native, modules = both_ways(model, batch_of([1, 7, 20]).to(dev))
+    for same in (torch.isposinf, torch.isneginf, torch.isnan):
+        assert torch.equal(same(native), same(modules))

@@ -46,7 +46,7 @@ bool staged_block(const cf_forward_args &f, const cf_forward_block &p)
     const bool boxes = boxes_of(f, p);
     return p.bins > 0 && f.staged_rings && (!boxes || (f.adaptive_rings && (p.cutoff > 0.0 || p.lower_bound >= 0.05))) &&
            infer_served(f.N, f.E, real_heads(f, p), p.bins, f.width / f.H, boxes, (int)f.lattice_range, p.weakest,
-                        f.ring_limit_bytes);
+                        f.unit_limit_bytes);
 }
 
 // Whether the other blocks with value bins start from staged rings, and the bytes these take.
@@ -97,7 +97,7 @@ int64_t carve(const cf_forward_args &f, const cf_forward_block *blocks, char *ba
             rings = rings || p.bins > 0;
             continue;
         }
-        const int64_t one = infer_units_bytes(U, boxes_of(f, p), f.ring_limit_bytes),
+        const int64_t one = infer_units_bytes(U, boxes_of(f, p), f.unit_limit_bytes),
                       w = infer_weights_bytes(real_heads(f, p), p.bins, W / f.H);
         units = one > units ? one : units;
         b.weight_bytes = w > b.weight_bytes ? w : b.weight_bytes;
@@ -247,10 +247,14 @@ extern "C" int cf_forward(const cf_forward_args *f_, const cf_forward_block *blo
         const int64_t HR = split ? H / 2 : H;
         if (staged_block(f, p)) {
             const float cutoff = adaptive ? (float)p.cutoff : 0.0f;
+            // (blocks of more pairs than fit at once stage slice by slice, each for itself)
+            const int64_t slice = infer_slice(U, adaptive, f.unit_limit_bytes);
+            const float *w[INFER_WEIGHT_BLOCKS];
+            int bins[INFER_WEIGHT_BLOCKS], count = 0;
+            bool stage = slice < U;
             if (l >= units_until) {
                 // units for this block and those behind it that share them, their projections packed alongside
-                const float *w[INFER_WEIGHT_BLOCKS];
-                int bins[INFER_WEIGHT_BLOCKS], count = 0;
+                stage = true;
                 for (units_until = l; units_until < f.layers && count < INFER_WEIGHT_BLOCKS; units_until++, count++) {
                     const cf_forward_block &o = blocks[units_until];
                     if (!staged_block(f, o) || o.weakest != p.weakest || boxes_of(f, o) != adaptive ||
@@ -259,15 +263,17 @@ extern "C" int cf_forward(const cf_forward_args *f_, const cf_forward_block *blo
                     w[count] = o.w_pe;
                     bins[count] = (int)o.bins;
                 }
-                if ((rc = launch_infer_stage(b.rpos, f.tvecs, rvlen, f.pairs, U, p.weakest, cutoff, (int)f.lattice_range,
-                                             (int)f.minimum_range, f.ring_limit_bytes, b.units, count, w, bins, HR, D,
-                                             b.weights + l * b.weight_bytes, b.weight_bytes, (hipStream_t)stream)))
-                    return rc;
             }
-            rc = launch_real_enc_infer(b.a, b.rpos, f.tvecs, f.pairs, U, HR, p.bins, D, p.dist_max, p.wscale,
-                                       b.weights + l * b.weight_bytes, rvlen, cutoff, (int)f.lattice_range,
-                                       (int)f.minimum_range, p.weakest, f.ring_limit_bytes, b.units, b.z, b.val,
-                                       (hipStream_t)stream);
+            for (int64_t before = 0; before < U && !rc; before += slice, count = 0) {
+                const int64_t here = before + slice < U ? slice : U - before;
+                if (stage && (rc = launch_infer_stage(b.rpos, f.tvecs, rvlen, f.pairs, U, before, here, p.weakest, cutoff,
+                                                      (int)f.lattice_range, (int)f.minimum_range, b.units, count, w, bins, HR,
+                                                      D, b.weights + l * b.weight_bytes, b.weight_bytes, (hipStream_t)stream)))
+                    return rc;
+                rc = launch_real_enc_infer(b.a, b.rpos, f.tvecs, f.pairs, U, before, here, HR, p.bins, D, p.dist_max, p.wscale,
+                                           b.weights + l * b.weight_bytes, rvlen, cutoff, (int)f.lattice_range,
+                                           (int)f.minimum_range, p.weakest, b.units, b.z, b.val, (hipStream_t)stream);
+            }
         } else if (p.bins > 0 && b.rings && (!adaptive || (f.adaptive_rings && HR <= 8 && adaptive_rings_pay(U)))) {
             if (!staged || staged->bins != p.bins || staged->dist_max != p.dist_max || staged->wscale != p.wscale ||
                 staged->weakest != p.weakest) {

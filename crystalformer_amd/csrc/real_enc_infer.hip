@@ -95,10 +95,16 @@ typedef const InferUnit __attribute__((address_space(4))) *InferUnitPtr;
 typedef const float __attribute__((address_space(4))) *ConstFloat;
 typedef const int64_t __attribute__((address_space(4))) *ConstLong;
 
+// Pairs of a slice that exist.
+__device__ __forceinline__ int64_t live_in_slice(const int64_t *live_U, int64_t before, int64_t U)
+{
+    return min(live_count(live_U, before + U) - before, U);
+}
+
 struct StageArgs {
     const float *rpos, *tvecs, *rvlen;
-    const int64_t *pairs;
-    int64_t U;
+    const int64_t *pairs;                   // this slice's, as units, d2 and n
+    int64_t U, before;                      // pairs of the slice, of the slices before it
     const int64_t *live_U;
     float weak_a, cutoff;
     int lattice_range, min_range, capacity;
@@ -173,7 +179,7 @@ __global__ __launch_bounds__(STAGE_WAVES * 64) void infer_stage_kernel(StageArgs
         }
         return;
     }
-    const int64_t U = live_count(p.live_U, p.U);
+    const int64_t U = live_in_slice(p.live_U, p.before, p.U);
     const int64_t waves = (int64_t)(gridDim.x - pack_groups) * STAGE_WAVES;
     const int64_t first = (int64_t)(blockIdx.x - pack_groups) * STAGE_WAVES + wave;
     if (first >= U) return;
@@ -426,7 +432,7 @@ struct InferArgs {
     const unsigned short *n;
     const int4_t *weights;                  // this block's, see WeightArgs
     float *z, *v;
-    int64_t U;
+    int64_t U, before;                      // as in StageArgs
     const int64_t *live_U;
     int H, D, heads, capacity, lattice_range, min_range, rounds_per_group;
     float cutoff, bin_step, s_scale, inv_bin_step;
@@ -449,7 +455,7 @@ __global__ __launch_bounds__(512, DT > 1 || NT > 4 ? 6 : 8) void real_enc_infer_
     const int q = lane >> 4, c = lane & 15;
     const int H = x.H, cap = x.capacity;
     const int hg = x.heads == 8 ? 0 : (int)blockIdx.x / x.rounds_per_group;
-    const int64_t U = live_count(x.live_U, x.U);
+    const int64_t U = live_in_slice(x.live_U, x.before, x.U);
     const int64_t first = (int64_t)((int)blockIdx.x - hg * x.rounds_per_group) * WPB;
     if (first >= U) return;
     const int64_t u = first + wave < U ? first + wave : first;
@@ -746,16 +752,11 @@ __global__ __launch_bounds__(512, DT > 1 || NT > 4 ? 6 : 8) void real_enc_infer_
 }
 
 // Entries a unit may have: all of a small fixed cube, else 832 (what leaves six staging work-groups a CU: seven blocks on 256
-// crystals, r0 = 3 A, have 232 in the mean and one unit in a hundred above 700), or the power of two from 128 to 512 whose
-// 6-byte entries `limit` bytes hold.
-int capacity_of(int64_t U, bool boxes, int64_t limit)
-{
-    if (!boxes) return 128;
-    if (U * MOST_STAGED * 6 <= limit) return MOST_STAGED;
-    int cap = 512;
-    while (cap > 128 && U * cap * 6 > limit) cap >>= 1;
-    return cap;
-}
+// crystals, r0 = 3 A, have 232 in the mean and one unit in a hundred above 700).  The same whatever the batch: a unit that has
+// more is formed by the blocks, in another order, and its bits must not depend on what else is in the batch, nor on the capacity
+// of a graph that serves it.
+constexpr int capacity_of(bool boxes) { return boxes ? MOST_STAGED : 128; }
+constexpr int64_t bytes_a_unit(bool boxes) { return (int64_t)sizeof(InferUnit) + capacity_of(boxes) * (boxes ? 6 : 4); }
 
 int64_t align256(int64_t x) { return (x + 255) & ~(int64_t)255; }
 
@@ -763,21 +764,19 @@ struct Carved {
     InferUnit *units;
     float *d2;
     unsigned short *n;
-    int capacity;
     int64_t bytes;
 };
-Carved carve_units(void *base, int64_t U, bool boxes, int64_t limit)
+Carved carve_units(void *base, int64_t U, bool boxes)
 {
     Carved r;
-    r.capacity = capacity_of(U, boxes, limit);
     char *b = (char *)base;
     int64_t at = 0;
     r.units = (InferUnit *)(b + at);
     at += align256(U * (int64_t)sizeof(InferUnit));
     r.d2 = (float *)(b + at);
-    at += align256(U * r.capacity * 4);
+    at += align256(U * capacity_of(boxes) * 4);
     r.n = boxes ? (unsigned short *)(b + at) : nullptr;
-    if (boxes) at += align256(U * r.capacity * 2);
+    if (boxes) at += align256(U * capacity_of(boxes) * 2);
     r.bytes = at;
     return r;
 }
@@ -789,19 +788,30 @@ int row_tiles_of(int64_t D) { return D > 16 ? 2 : 1; }
 
 namespace cf {
 
-// Whether a block's units can be staged: boxes that are the fixed cube of up to 128 translations or adaptive, images of no
-// more than `limit` bytes at the least capacity, a shape the kernel has.  `weakest` <= 0 bounds the exponents from above.
+// Whether a block's units can be staged: boxes that are the fixed cube of up to 128 translations or adaptive, room for a slice
+// worth a launch, a shape the kernel has.  The batch's size decides only at 2^30 values of v (8.4 million edges of 128 wide
+// blocks), where offsets leave 32 bits and the attention changes its kernel too: below it a graph of any capacity and an eager
+// forward agree to the bit.  `weakest` <= 0 bounds the exponents from above.
 bool infer_served(int64_t N, int64_t E, int64_t H, int64_t K, int64_t D, bool boxes, int lattice_range, double weakest,
                   int64_t limit)
 {
     const int64_t cube = (int64_t)(2 * lattice_range + 1) * (2 * lattice_range + 1) * (2 * lattice_range + 1);
-    const int64_t U = (N + E) / 2;
-    return U >= 1 && K >= 1 && K <= 128 && D >= 1 && D <= 32 && weakest <= 0 && lattice_range >= 0 &&
-           lattice_range <= MAX_RANGE && (boxes || cube <= 128) && U * (boxes ? 128 * 6 : 128 * 4) <= limit &&
-           E * H * D < (1ll << 30) && N * H < (1ll << 32);       // (32-bit offsets in the kernel)
+    return N + E >= 2 && K >= 1 && K <= 128 && D >= 1 && D <= 32 && weakest <= 0 && lattice_range >= 0 &&
+           lattice_range <= MAX_RANGE && (boxes || cube <= 128) && limit >= INFER_LEAST_SLICE * bytes_a_unit(boxes) &&
+           E * H * D < (1ll << 30) && N * H < (1ll << 32);
 }
 
-int64_t infer_units_bytes(int64_t U, bool boxes, int64_t limit) { return U < 1 ? 0 : carve_units(nullptr, U, boxes, limit).bytes; }
+// Units staged at a time: all, or as many whole rounds as `limit` bytes hold.
+int64_t infer_slice(int64_t U, bool boxes, int64_t limit)
+{
+    const int64_t most = limit / bytes_a_unit(boxes) / WPB * WPB;
+    return U < most ? U : most;
+}
+
+int64_t infer_units_bytes(int64_t U, bool boxes, int64_t limit)
+{
+    return U < 1 ? 0 : carve_units(nullptr, infer_slice(U, boxes, limit), boxes).bytes;
+}
 
 // Packed projection of a block with up to K bins.
 int64_t infer_weights_bytes(int64_t H, int64_t K, int64_t D)
@@ -810,20 +820,20 @@ int64_t infer_weights_bytes(int64_t H, int64_t K, int64_t D)
     return align256(tiles * (pieces_of(tiles_of(K)) * WAVE * 16 + 64));
 }
 
-// Stages the units, and packs the projections of `blocks` blocks (weights: (H, D, bins[l]) each, null: none) into `packed`,
-// infer_weights_bytes apart.
+// Stages the units of pairs `before` .. `before` + `slice` - 1 of U, and packs the projections of `blocks` blocks (weights:
+// (H, D, bins[l]) each) into `packed`, infer_weights_bytes apart.
 int launch_infer_stage(const float *rpos, const float *tvecs, const float *rvlen, const int64_t *pairs, int64_t U,
-                       double weakest, float cutoff, int lattice_range, int min_range, int64_t limit, void *staged, int blocks,
-                       const float *const *weights, const int *bins, int64_t H, int64_t D, void *packed, int64_t packed_bytes,
-                       hipStream_t st)
+                       int64_t before, int64_t slice, double weakest, float cutoff, int lattice_range, int min_range,
+                       void *staged, int blocks, const float *const *weights, const int *bins, int64_t H, int64_t D,
+                       void *packed, int64_t packed_bytes, hipStream_t st)
 {
     const bool boxes = rvlen && cutoff != 0.0f;
-    const Carved m = carve_units(staged, U, boxes, limit);
+    const Carved m = carve_units(staged, slice, boxes);
     StageArgs p{};
-    p.rpos = rpos; p.tvecs = tvecs; p.rvlen = boxes ? rvlen : nullptr; p.pairs = pairs;
-    p.U = U; p.live_U = live_units(U);
+    p.rpos = rpos; p.tvecs = tvecs; p.rvlen = boxes ? rvlen : nullptr; p.pairs = pairs + before * PAIR_FIELDS;
+    p.U = slice; p.before = before; p.live_U = live_units(U);
     p.weak_a = (float)weakest; p.cutoff = boxes ? cutoff : 0.0f;
-    p.lattice_range = lattice_range; p.min_range = min_range; p.capacity = m.capacity;
+    p.lattice_range = lattice_range; p.min_range = min_range; p.capacity = capacity_of(boxes);
     p.units = m.units; p.d2 = m.d2; p.n = m.n;
     WeightArgs w{};
     w.blocks = blocks; w.H = (int)H; w.D = (int)D; w.heads = heads_of(H); w.DT = row_tiles_of(D);
@@ -833,33 +843,34 @@ int launch_infer_stage(const float *rpos, const float *tvecs, const float *rvlen
         w.bins[l] = bins[l];
     }
     const int packs = w.blocks * w.heads * w.DT, pack_groups = (packs + STAGE_WAVES - 1) / STAGE_WAVES;
-    const size_t lds = (size_t)STAGE_WAVES * ((boxes ? 3 : 2) * (m.capacity + WAVE) * 2 + CLASSES * WAVE * 2);
-    const int64_t want = (U + STAGE_WAVES - 1) / STAGE_WAVES, cap = persistent_grid_cap(lds > 20000 ? 6 : 8);
+    const size_t lds = (size_t)STAGE_WAVES * ((boxes ? 3 : 2) * (p.capacity + WAVE) * 2 + CLASSES * WAVE * 2);
+    const int64_t want = (slice + STAGE_WAVES - 1) / STAGE_WAVES, cap = persistent_grid_cap(lds > 20000 ? 6 : 8);
     infer_stage_kernel<<<pack_groups + (int)(want < cap ? want : cap), STAGE_WAVES * WAVE, lds, st>>>(p, w);
     CF_CHECK_LAUNCH("infer_stage");
     return CF_OK;
 }
 
-// The encoding of a block whose units were staged with its cutoff and ranges and an exponent none of its own exceeds.
-int launch_real_enc_infer(const float *a_ik, const float *rpos, const float *tvecs, const int64_t *pairs, int64_t U, int64_t H,
-                          int64_t K, int64_t D, double dist_max, double wscale, const void *packed, const float *rvlen,
-                          float cutoff, int lattice_range, int min_range, double weakest, int64_t limit, const void *staged,
-                          float *z, float *v, hipStream_t st)
+// The encoding, for the pairs of a slice, of a block whose units were staged with its cutoff and ranges and an exponent none of
+// its own exceeds.
+int launch_real_enc_infer(const float *a_ik, const float *rpos, const float *tvecs, const int64_t *pairs, int64_t U,
+                          int64_t before, int64_t slice, int64_t H, int64_t K, int64_t D, double dist_max, double wscale,
+                          const void *packed, const float *rvlen, float cutoff, int lattice_range, int min_range,
+                          double weakest, const void *staged, float *z, float *v, hipStream_t st)
 {
     const bool boxes = rvlen && cutoff != 0.0f;
-    const Carved m = carve_units(const_cast<void *>(staged), U, boxes, limit);
+    const Carved m = carve_units(const_cast<void *>(staged), slice, boxes);
     InferArgs x{};
-    x.a_ik = a_ik; x.rpos = rpos; x.tvecs = tvecs; x.rvlen = rvlen; x.pairs = pairs;
-    x.units = m.units; x.d2 = m.d2; x.n = m.n; x.capacity = m.capacity;
+    x.a_ik = a_ik; x.rpos = rpos; x.tvecs = tvecs; x.rvlen = rvlen; x.pairs = pairs + before * PAIR_FIELDS;
+    x.units = m.units; x.d2 = m.d2; x.n = m.n; x.capacity = capacity_of(boxes);
     x.weights = (const int4_t *)packed; x.z = z; x.v = v;
-    x.U = U; x.live_U = live_units(U);
+    x.U = slice; x.before = before; x.live_U = live_units(U);
     x.H = (int)H; x.D = (int)D; x.heads = heads_of(H);
     x.lattice_range = lattice_range; x.min_range = min_range; x.cutoff = cutoff;
     x.bin_step = 1.0f / ((float)wscale * sqrtf(2.0f)) * sqrtf(LOG2E);
     x.s_scale = x.bin_step / ((float)dist_max / (float)K);
     x.inv_bin_step = 1.0f / x.bin_step;
     x.reach = -40.0f / fminf((float)weakest * LOG2E, LEAST_A2);
-    x.rounds_per_group = (int)((U + WPB - 1) / WPB);
+    x.rounds_per_group = (int)((slice + WPB - 1) / WPB);
     const int blocks = x.rounds_per_group * (x.heads / 8);
 #define CF_INFER(NTV, DTV)                                                                  \
     do {                                                                                    \

@@ -29,9 +29,15 @@ from .latticeformer import Latticeformer, is_plain_head
 from .lib import device_guard, stream_handle
 
 
-# What the staged translations of a forward may take: 700 MB for 890 thousand atom pairs in the fixed cube; with adaptive boxes
-# the capacity of a pair follows from it (256 translations there, 832 below 320 thousand pairs).
-STAGED_UNITS_MAX_BYTES = 3 << 29
+# What the staged translations of a forward may take: with adaptive boxes 5024 bytes an atom pair, all at once for 1.28 million
+# pairs, in the fixed cube 544.  Where they take more they are staged in slices, by every block; results don't depend on it.  An
+# `ops.STAGED_RINGS_MAX_BYTES` below its default bounds these too.
+STAGED_UNITS_MAX_BYTES = 6 << 30
+
+
+def _unit_limit() -> int:
+    return STAGED_UNITS_MAX_BYTES if ops.STAGED_RINGS_MAX_BYTES >= 1 << 30 \
+        else min(STAGED_UNITS_MAX_BYTES, ops.STAGED_RINGS_MAX_BYTES)
 
 
 def _hooked(module: nn.Module) -> bool:
@@ -268,7 +274,7 @@ def _run(encoder: nn.Module, src: Tensor, pos: Tensor, batch: Tensor, trans: Ten
     sched = ops._scheduling_words(dev) if ops.DYNAMIC_ROUNDS else None
     args = _lib.ForwardArgs(
         N, layout.num_edges, sizes.numel(), len(blocks), H, width, ff, KM.LATTICE_RANGE, KM.MINIMUM_RANGE, 1,
-        int(store), int(KM.STAGED_RINGS), int(KM.ADAPTIVE_RINGS), STAGED_UNITS_MAX_BYTES, hidden,
+        int(store), int(KM.STAGED_RINGS), int(KM.ADAPTIVE_RINGS), ops.STAGED_RINGS_MAX_BYTES, _unit_limit(), hidden,
         targets, embed.in_features if embed else 0, src.data_ptr(), pos.data_ptr(), trans.data_ptr(),
         layout.batch.data_ptr(), layout.atom_start.data_ptr(), layout.edge_start.data_ptr(), layout.edges.data_ptr(),
         layout.e_start.data_ptr(), layout.pairs.data_ptr(),

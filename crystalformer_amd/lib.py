@@ -38,7 +38,7 @@ class ForwardArgs(ctypes.Structure):
     """``cf_forward_args`` of include/crystalformer_hip.h."""
     _fields_ = ([(n, _i64) for n in ("N", "E", "B", "layers", "H", "width", "ff", "lattice_range", "minimum_range",
                                      "adaptive", "update_stats", "staged_rings", "adaptive_rings", "ring_limit_bytes",
-                                     "hidden", "targets", "embed_width")]
+                                     "unit_limit_bytes", "hidden", "targets", "embed_width")]
                 + [(n, _ptr) for n in ("x", "pos", "tvecs", "batch", "atom_start", "edge_start", "edges", "e_start",
                                        "pairs", "sched", "w_head", "b_head", "w_last", "b_last", "w_embed", "b_embed",
                                        "out")])

@@ -510,7 +510,10 @@ typedef struct {
     int64_t adaptive;                 /* 0: cutoffs are ignored, every box is the fixed cube */
     int64_t update_stats;             /* training mode without gradients: store the exponent statistics */
     int64_t staged_rings, adaptive_rings, ring_limit_bytes;   /* whether blocks (with adaptive boxes too) share staged
-                                         translations, and how many bytes these may take */
+                                         translations, and how many bytes cf_real_enc_ring_stage's may take */
+    int64_t unit_limit_bytes;         /* the same for those of the encoding of its own: 544 bytes a pair in the fixed cube,
+                                         5024 in adaptive boxes; where these are more they are staged in slices of pairs,
+                                         by every block (results stay the same); below 4096 pairs' it is not used */
     int64_t hidden, targets;          /* head: width -> hidden (ReLU) -> targets; hidden 0: width -> targets;
                                          targets 0: out takes the encoder's output (N, width) */
     int64_t embed_width;

@@ -6,7 +6,8 @@ import dataclasses
 import pytest
 import torch
 
-from crystalformer_amd import executor, hip_funcs
+from crystalformer_amd import executor, hip_funcs, ops
+from crystalformer_amd.graphs import GraphedForward
 from crystalformer_amd.latticeformer import default_params
 from crystalformer_amd.synthetic import CrystalBatch, lattice_from_parameters
 from oracle import torch_model as om
@@ -69,14 +70,48 @@ def test_boxes_along_each_axis(dev, length):
     compare(dev, crystals([list(length)] * 3, [4, 9, 1], angles=[[80.0, 95.0, 110.0]] * 3), scale_real=[3.0])
 
 
-def test_less_room_than_units_need(dev, monkeypatch):
-    """The least capacity, which most of these units exceed, and none at all."""
-    b = crystals([[4.0, 4.0, 5.0], [9.0, 9.0, 9.0]], [12, 10])
-    units = 12 * 13 // 2 + 10 * 11 // 2
-    for limit in (units * 128 * 6, units * 128 * 6 - 1, 0):
-        monkeypatch.setattr(executor, "STAGED_UNITS_MAX_BYTES", limit)
-        compare(dev, b, scale_real=[3.0])
-        compare(dev, b, scale_real=[3.0], adaptive_cutoff_sigma=0.0)
+LEAST_BYTES = 4096 * (32 + 832 * 6)                        # (of a slice in adaptive boxes; the fixed cube's entries are fewer)
+
+
+@pytest.mark.parametrize("adaptive", [-3.5, 0.0])
+@pytest.mark.parametrize("owner", ["STAGED_UNITS_MAX_BYTES", "STAGED_RINGS_MAX_BYTES"])
+def test_less_room_than_units_need(dev, monkeypatch, adaptive, owner):
+    """As many slices of pairs as the room asks for give the same bits as one; below the least slice's the operators'
+    kernels serve."""
+    b = crystals([[4.0, 4.0, 5.0], [9.0, 9.0, 9.0], [2.4, 2.5, 2.6], [3.0, 12.0, 7.0]], [92, 90, 91, 34]).to(dev)
+    units = int((b.sizes * (b.sizes + 1)).sum()) // 2
+    assert units > 3 * 4096 and units % 8
+    model = scaled(default_params(num_layers=2, scale_real=[3.0], adaptive_cutoff_sigma=adaptive)).to(dev).eval()
+    whole, modules = both_ways(model, b)
+    assert_close(whole, modules, "encoder", atol=atol_rows(modules))
+    least = LEAST_BYTES if adaptive else 4096 * (32 + 128 * 4)
+    for limit in (least, 5 * least // 2, least - 1, 0):
+        monkeypatch.setattr(executor if owner == "STAGED_UNITS_MAX_BYTES" else ops, owner, limit)
+        sliced, _ = both_ways(model, b)
+        if limit >= least:
+            assert torch.equal(sliced, whole)
+        else:
+            assert_close(sliced, modules, "encoder", atol=atol_rows(modules))
+
+
+@pytest.mark.parametrize("crystals_", [5, 150])
+def test_a_capacity_graph_has_the_eager_bits_whatever_its_capacity(dev, monkeypatch, crystals_):
+    """Units with more entries than a large capacity's share of the room, in a graph and eagerly; crystals by themselves too."""
+    monkeypatch.setattr(executor, "STAGED_UNITS_MAX_BYTES", LEAST_BYTES)
+    b = crystals([[4.0, 4.0, 5.0], [3.0, 3.5, 4.0], [2.4, 2.5, 2.6], [3.0, 12.0, 7.0]], [12, 10, 7, 5]).to(dev)
+    model = scaled(default_params(num_layers=2, scale_real=[3.0]))
+    with torch.no_grad():
+        for layer in model.encoder.layers:
+            layer.self_attn.gauss_scale.copy_(torch.tensor([0.8, -0.1]))
+    model = model.to(dev).eval()
+    graph = GraphedForward(model, b, capacity=(crystals_, 12 * crystals_, 144 * crystals_))
+    with torch.no_grad():
+        eager = model(b).clone()
+        for _ in range(3):
+            assert torch.equal(graph(b), eager)
+        n = int(b.sizes[0])
+        alone = model(CrystalBatch(b.x[:n], b.pos[:n], b.batch[:n], b.trans_vec[:1], b.sizes[:1]))
+    assert torch.equal(alone, eager[:1])
 
 
 @pytest.mark.parametrize("adaptive", [-3.5, 0.0])

@@ -426,8 +426,8 @@ def main() -> int:
                     help="batches in flight: the step's HIP graph is replayed round robin on this many "
                          "streams (default priority), each with its own copy of the batch; 1 = one after the other")
     ap.add_argument("--launch-share", type=float, default=0.75,
-                    help="with several steps in flight: share of the GPU one periodic-encoding launch "
-                         "occupies (384 of its 512 work-groups by default)")
+                    help="with several steps in flight: share of the GPU one persistent encoding launch occupies (the "
+                         "staging of the translations; the blocks' encodings are short work-groups and take no share)")
     ap.add_argument("--two-launch-blocks", action="store_true",
                     help="blocks without value bins: run bias and attention as two operators instead of one launch")
     ap.add_argument("--no-staged-rings", action="store_true",
@@ -788,7 +788,7 @@ def main() -> int:
                    "submission": "eager launches" if args.no_graph else (
                        "one HIP graph replay per step" if args.inflight <= 1 else
                        f"one HIP graph replay per step, {args.inflight} steps in flight on {args.inflight} streams, "
-                       f"encoding launches at {args.launch_share:g} of the GPU each")},
+                       f"staging launches at {args.launch_share:g} of the GPU each")},
         "single_stream": None if args.no_graph else single,
         "eager": {"value": round(B * args.steps / eager_elapsed, 2),
                   "ms_per_step": round(eager_elapsed / args.steps * 1e3, 4)},

@@ -65,9 +65,11 @@ class GraphedForward:
     :meth:`overflowed` reports it.
 
     ``launch_share`` (0 < share <= 1) is for several graphs replayed concurrently on
-    different streams: the periodic-encoding launches of this graph then take that share
-    of the GPU each (:class:`crystalformer_amd.ops.launch_share`), which lengthens one
-    replay on its own and shortens the steps when several are in flight.
+    different streams: the persistent periodic-encoding launches of this graph then take that
+    share of the GPU each (:class:`crystalformer_amd.ops.launch_share`), which lengthens one
+    replay on its own and leaves room for the others.  In a forward that runs as one native call
+    this is the staging of the translations; its blocks' encodings are short work-groups that
+    leave room by themselves.
     """
 
     def __init__(self, model: torch.nn.Module, batch: CrystalBatch, warmup: int = 3,

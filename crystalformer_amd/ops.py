@@ -53,9 +53,9 @@ def count_translation_evals(a_ik: Tensor, rvlen_n: Optional[Tensor], batch_i: Te
 
 
 class launch_share:
-    """Context manager: within it, forward launches of the periodic encoding made by this
-    thread occupy at most ``share`` of the GPU (``cf_set_launch_share``), so that kernels of
-    other streams run beside them.  For callers that keep several forwards in flight; a
+    """Context manager: within it, persistent forward launches of the periodic encoding made by
+    this thread (the operators', and the staging of a native forward) occupy at most ``share`` of
+    the GPU (``cf_set_launch_share``), so that kernels of other streams run beside them.  For callers that keep several forwards in flight; a
     graph captured inside keeps the share.  Results do not depend on it."""
 
     def __init__(self, share: float):

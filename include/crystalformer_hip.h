@@ -40,14 +40,16 @@ const char *cf_last_error(void);
 int cf_max_translation_range(void);
 
 /*
- * Share of the GPU that one forward launch of the periodic encoding may occupy, for the
- * calling thread (default 1).  The forward pair kernel is persistent: it launches two
- * work-groups per CU, which hold the CU's whole register file, so kernels of other streams
- * wait for it to drain.  A caller that keeps several streams busy (several forwards in
- * flight) sets a share below 1: the kernel launches that fraction of its work-groups, runs
- * longer on its own, and leaves room beside it; results are bit-identical.  Read at launch
- * (a captured graph keeps the share it was captured with).  The backward kernel ignores
- * it.  No counterpart in the reference, whose launches are sized by the problem alone
+ * Share of the GPU that one persistent forward launch of the periodic encoding may occupy, for
+ * the calling thread (default 1): those of cf_real_enc_fwd, cf_real_enc_fwd_rings and
+ * cf_real_enc_ring_stage, and the staging launch of cf_forward.  They hold what they take until
+ * they end, two work-groups per CU the CU's whole register file, so kernels of other streams
+ * wait.  A caller that keeps several streams busy sets a share below 1: such a kernel launches
+ * that fraction of its work-groups, runs longer on its own, and leaves room beside it; results
+ * are bit-identical.  Read at launch (a captured graph keeps the share it was captured with).
+ * The backward kernel ignores it, and so does cf_forward's own encoding of a block, whose
+ * work-groups last a few microseconds each and let others in as they end (held to three of the
+ * four that fit a CU, four forwards in flight take 806 us instead of 780).  No counterpart in the reference, whose launches are sized by the problem alone
  * (models/cuda_funcs/real_space_enc_proj.py:75-96).
  */
 int cf_set_launch_share(double share);

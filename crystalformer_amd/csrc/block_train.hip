@@ -4,7 +4,7 @@
 // Four operators a block each way, every one with its checks, allocations and an autograd node of its own, took 200 us of host
 // time forward and 140 backward; as one node and two calls it is 65 and 85, most of it the launches.  A step of four blocks on
 // an ever new batch of 61 crystals, whose kernels take 0.79 ms, waited for the host: 2.44 -> 1.66 ms.
-// What is kept for the backward call lies in one piece of memory, what either call needs for itself in another.
+// What is kept for the backward call lies in two pieces of memory, what either call needs for itself in another.
 #include "cf_common.h"
 
 namespace {
@@ -25,29 +25,34 @@ struct Carve {
     float *rows(int64_t n, int64_t width) { return take(n * width * 4); }
 };
 
-// att, s and h first, at multiples of whole rows: the weight gradients read them.
+// What the caller's weight gradients read, rows of whole 256 bytes, and what only the backward call does: two pieces, since the
+// first lives on until the weight gradients of all blocks are formed.
 struct Saved {
-    float *att, *s, *h, *q, *qs, *k, *v, *a, *alpha_n, *used, *z, *val, *prob;
+    float *att, *s, *h;
     int64_t bytes;
+    float *q, *qs, *k, *v, *a, *alpha_n, *used, *z, *val, *prob;
+    int64_t more_bytes;
 };
-Saved carve_saved(const cf_block_train &f, void *base)
+Saved carve_saved(const cf_block_train &f, void *base, void *more)
 {
-    Carve c{(char *)base};
     Saved r{};
+    Carve c{(char *)base};
     r.att = c.rows(f.N, W);
     r.s = c.rows(f.N, W);
     r.h = c.rows(f.N, FF);
-    r.q = c.rows(f.N, W);
-    r.qs = c.rows(f.N, W);
-    r.k = c.rows(f.N, W);
-    r.v = c.rows(f.N, W);
-    r.a = c.rows(f.N, f.H);
-    r.alpha_n = c.rows(f.N, f.H);
-    r.used = c.take(8);
-    r.z = c.rows(f.E, f.H);
-    r.val = f.bins > 0 ? c.rows(f.E, W) : nullptr;
-    r.prob = c.rows(f.E, f.H);
     r.bytes = c.at;
+    Carve m{(char *)more};
+    r.q = m.rows(f.N, W);
+    r.qs = m.rows(f.N, W);
+    r.k = m.rows(f.N, W);
+    r.v = m.rows(f.N, W);
+    r.a = m.rows(f.N, f.H);
+    r.alpha_n = m.rows(f.N, f.H);
+    r.used = m.take(8);
+    r.z = m.rows(f.E, f.H);
+    r.val = f.bins > 0 ? m.rows(f.E, W) : nullptr;
+    r.prob = m.rows(f.E, f.H);
+    r.more_bytes = m.at;
     return r;
 }
 
@@ -67,9 +72,9 @@ ForwardScratch carve_forward(const cf_block_train &f, void *base)
     return r;
 }
 
-// gq, gk, gv, gs, gx, gh, gw_pos: what the caller goes on with, at multiples of whole rows.
+// gq, gk, gv, gs, gx, gh: what the caller goes on with, at multiples of whole rows.
 struct Kept {
-    float *gq, *gk, *gv, *gs, *gx, *gh, *gw_pos;
+    float *gq, *gk, *gv, *gs, *gx, *gh;
     int64_t bytes;
 };
 Kept carve_kept(const cf_block_train &f, void *base)
@@ -82,7 +87,6 @@ Kept carve_kept(const cf_block_train &f, void *base)
     r.gs = c.rows(f.N, W);
     r.gx = c.rows(f.N, W);
     r.gh = c.rows(f.N, FF);
-    r.gw_pos = c.rows(1, W);
     r.bytes = c.at;
     return r;
 }
@@ -123,7 +127,7 @@ int check_block(const cf_block_train *args, const char *who)
 int check_pointers(const cf_block_train &f, const char *who)
 {
     CF_REQUIRE(f.x && f.w_pos && f.rpos && f.tvecs && f.batch && f.edges && f.e_start && f.atom_start &&
-                   f.edge_start && f.pairs && f.saved && f.scratch && (f.bins == 0 || f.w_pe) &&
+                   f.edge_start && f.pairs && f.saved && f.saved_more && f.scratch && (f.bins == 0 || f.w_pe) &&
                    (f.cutoff == 0.0 || f.rvlen), CF_ERR_INVALID_ARGUMENT, "%s: null pointer", who);
     CF_REQUIRE(!cf_get_size_header(), CF_ERR_UNSUPPORTED, "%s: not under a size header", who);
     return CF_OK;
@@ -131,15 +135,17 @@ int check_pointers(const cf_block_train &f, const char *who)
 
 }  // namespace
 
-extern "C" int cf_block_train_bytes(const cf_block_train *args, int64_t *bytes_4)
+extern "C" int cf_block_train_bytes(const cf_block_train *args, int64_t *bytes_5)
 {
     const int rc = check_block(args, "cf_block_train_bytes");
     if (rc) return rc;
-    CF_REQUIRE(bytes_4, CF_ERR_INVALID_ARGUMENT, "cf_block_train_bytes: null pointer");
-    bytes_4[0] = carve_saved(*args, nullptr).bytes;
-    bytes_4[1] = carve_forward(*args, nullptr).bytes;
-    bytes_4[2] = carve_kept(*args, nullptr).bytes;
-    bytes_4[3] = carve_backward(*args, nullptr).bytes;
+    CF_REQUIRE(bytes_5, CF_ERR_INVALID_ARGUMENT, "cf_block_train_bytes: null pointer");
+    const Saved b = carve_saved(*args, nullptr, nullptr);
+    bytes_5[0] = b.bytes;
+    bytes_5[1] = b.more_bytes;
+    bytes_5[2] = carve_forward(*args, nullptr).bytes;
+    bytes_5[3] = carve_kept(*args, nullptr).bytes;
+    bytes_5[4] = carve_backward(*args, nullptr).bytes;
     return CF_OK;
 }
 
@@ -149,7 +155,7 @@ extern "C" int cf_block_train_fwd(const cf_block_train *args, void *stream)
     if (rc || (rc = check_pointers(*args, "cf_block_train_fwd"))) return rc;
     const cf_block_train &f = *args;
     CF_REQUIRE(f.packed && f.counter && f.gauss_scale && f.y, CF_ERR_INVALID_ARGUMENT, "cf_block_train_fwd: null pointer");
-    const Saved b = carve_saved(f, f.saved);
+    const Saved b = carve_saved(f, f.saved, f.saved_more);
     const ForwardScratch t = carve_forward(f, f.scratch);
     const int64_t D = W / f.H;
     if ((rc = cf_block_head(f.x, f.N, f.H, f.packed, f.b_in, f.w_pos, f.gauss_scale, (int)f.normalize, (int)f.update_stats,
@@ -175,9 +181,9 @@ extern "C" int cf_block_train_bwd(const cf_block_train *args, void *stream)
     int rc = check_block(args, "cf_block_train_bwd");
     if (rc || (rc = check_pointers(*args, "cf_block_train_bwd"))) return rc;
     const cf_block_train &f = *args;
-    CF_REQUIRE(f.packed_bwd && f.gy && f.kept && (!f.want_gw_pe || f.gw_pe), CF_ERR_INVALID_ARGUMENT,
+    CF_REQUIRE(f.packed_bwd && f.gy && f.kept && f.gw_pos && (!f.want_gw_pe || f.gw_pe), CF_ERR_INVALID_ARGUMENT,
                "cf_block_train_bwd: null pointer");
-    const Saved b = carve_saved(f, f.saved);
+    const Saved b = carve_saved(f, f.saved, f.saved_more);
     const Kept g = carve_kept(f, f.kept);
     const BackwardScratch t = carve_backward(f, f.scratch);
     const int64_t D = W / f.H;
@@ -198,5 +204,5 @@ extern "C" int cf_block_train_bwd(const cf_block_train *args, void *stream)
     if (rc) return rc;
     return cf_block_head_bwd(t.ga, t.gqs, g.gk, g.gv, g.gs, b.q, f.w_pos, b.alpha_n, f.normalize ? b.used : nullptr, f.N, f.H,
                              f.packed_bwd, (int)f.positive_func, (float)f.beta, (float)f.lower_bound, (float)f.coef,
-                             (float)f.q_scale, t.g_alpha, g.gq, g.gx, g.gw_pos, stream);
+                             (float)f.q_scale, t.g_alpha, g.gq, g.gx, f.gw_pos, stream);
 }

@@ -773,19 +773,21 @@ class BlockTrainHIP(torch.autograd.Function):
             f[10], f[12], shared.rpos.data_ptr(), shared.tvecs.data_ptr(), shared.rvlen.data_ptr(), lay.batch.data_ptr(),
             lay.edges.data_ptr(), lay.e_start.data_ptr(), lay.atom_start.data_ptr(), lay.edge_start.data_ptr(),
             lay.pairs.data_ptr(), _lib.ptr(rings), _lib.ptr(sched), pack.counters.data_ptr() + 4 * i, y.data_ptr())
-        need = (c_int64 * 4)()
+        need = (c_int64 * 5)()
         L = _lib.load()
         _lib.check(L.cf_block_train_bytes(byref(args), need), "cf_block_train_bytes")
+        # (deferred weight gradients hold on to the first piece until the end: the tensors per edge are not in it)
+        # (and this call's own scratch, some bytes a pair, lies behind the second)
         saved = torch.empty(need[0] // 4, dtype=torch.float32, device=dev)
-        scratch = torch.empty(max(need[1], 1), dtype=torch.uint8, device=dev)
-        args.saved, args.scratch = saved.data_ptr(), scratch.data_ptr()
+        more = torch.empty((need[1] + need[2]) // 4, dtype=torch.float32, device=dev)
+        args.saved, args.saved_more, args.scratch = saved.data_ptr(), more.data_ptr(), more.data_ptr() + need[1]
         with _lib.device_guard(dev):
             rc = L.cf_block_train_fwd(byref(args), _lib.stream_handle(dev))
         _lib.check(rc, "cf_block_train_fwd")
-        ctx.save_for_backward(x, wq, wk, wv, w_pos, w_pe, wo, w1, w2, saved, pack.backward[floats * i:floats * (i + 1)],
+        ctx.save_for_backward(x, wq, wk, wv, w_pos, w_pe, wo, w1, w2, saved, more, pack.backward[floats * i:floats * (i + 1)],
                               shared.rpos, shared.tvecs, shared.rvlen, lay.batch, lay.edges)
         # (what the backward call starts from, as above)
-        ctx.conf, ctx.layout = (conf, reals), lay
+        ctx.conf, ctx.layout, ctx.more = (conf, reals), lay, more.numel()
         ctx.rings = rings if cutoff == 0.0 and bins <= 64 and x.shape[1] // H <= 16 else None
         ctx.leaves = tuple(_leaf(t) for t in (wq, wk, wv, b_in, wo, bo, w1, b1, w2, b2))
         ctx.has_bias = tuple(t is not None for t in (b_in, bo, b1, b2))
@@ -794,12 +796,13 @@ class BlockTrainHIP(torch.autograd.Function):
     @staticmethod
     def backward(ctx, gy):
         from ctypes import byref, c_int64
-        (x, wq, wk, wv, w_pos, w_pe, wo, w1, w2, saved, packed_bwd, rpos, tvecs, rvlen, batch, edges) = ctx.saved_tensors
+        (x, wq, wk, wv, w_pos, w_pe, wo, w1, w2, saved, more, packed_bwd, rpos, tvecs, rvlen, batch,
+         edges) = ctx.saved_tensors
         ops._refuse_live_sizes("a training block's backward pass")
         # (whatever a saved-tensor hook brought back: the same values, in the same place and type)
-        dev = ops.require_device(gy, x, w_pos, w_pe, saved, packed_bwd, rpos, tvecs, rvlen, batch, edges)
-        gy, x, w_pos, w_pe, saved, packed_bwd, rpos, tvecs, rvlen = (
-            ops._f32(t, "saved operand") for t in (gy, x, w_pos, w_pe, saved, packed_bwd, rpos, tvecs, rvlen))
+        dev = ops.require_device(gy, x, w_pos, w_pe, saved, more, packed_bwd, rpos, tvecs, rvlen, batch, edges)
+        gy, x, w_pos, w_pe, saved, more, packed_bwd, rpos, tvecs, rvlen = (
+            ops._f32(t, "saved operand") for t in (gy, x, w_pos, w_pe, saved, more, packed_bwd, rpos, tvecs, rvlen))
         batch, edges = ops._i64(batch, "batch"), ops._i64(edges, "edges")
         conf, reals = ctx.conf
         lay, rings = ctx.layout, ctx.rings
@@ -811,26 +814,27 @@ class BlockTrainHIP(torch.autograd.Function):
             raise _lib.CrystalformerHipError("a training block's saved operands have other shapes than its forward pass's")
         need = ctx.needs_input_grad
         gw_pe = torch.empty_like(w_pe) if w_pe is not None and need[6] else None
+        gw_pos = torch.empty_like(w_pos)        # (a parameter's gradient, which outlives the rest)
         args = _lib.BlockTrain(
             *conf, int(gw_pe is not None), *reals, x.data_ptr(), None, packed_bwd.data_ptr(), None, w_pos.data_ptr(), None,
             _lib.ptr(w_pe), None, None, None, rpos.data_ptr(), tvecs.data_ptr(), rvlen.data_ptr(), batch.data_ptr(),
             edges.data_ptr(), lay.e_start.data_ptr(), lay.atom_start.data_ptr(), lay.edge_start.data_ptr(),
-            lay.pairs.data_ptr(), _lib.ptr(rings), None, None, None, saved.data_ptr(), None, gy.data_ptr(), None,
-            _lib.ptr(gw_pe))
-        bytes_ = (c_int64 * 4)()
+            lay.pairs.data_ptr(), _lib.ptr(rings), None, None, None, saved.data_ptr(), more.data_ptr(), None, gy.data_ptr(),
+            None, gw_pos.data_ptr(), _lib.ptr(gw_pe))
+        bytes_ = (c_int64 * 5)()
         L = _lib.load()
         _lib.check(L.cf_block_train_bytes(byref(args), bytes_), "cf_block_train_bytes")
-        if saved.numel() * 4 != bytes_[0]:
+        if saved.numel() * 4 != bytes_[0] or more.numel() != ctx.more:
             raise _lib.CrystalformerHipError("a training block's saved operands have other shapes than its forward pass's")
-        kept = torch.empty(bytes_[2] // 4, dtype=torch.float32, device=dev)
-        scratch = torch.empty(bytes_[3], dtype=torch.uint8, device=dev)
+        kept = torch.empty(bytes_[3] // 4, dtype=torch.float32, device=dev)
+        scratch = torch.empty(bytes_[4], dtype=torch.uint8, device=dev)
         args.kept, args.scratch = kept.data_ptr(), scratch.data_ptr()
         with _lib.device_guard(dev):
             rc = L.cf_block_train_bwd(byref(args), _lib.stream_handle(dev))
         _lib.check(rc, "cf_block_train_bwd")
         n = N * W
         gq, gk, gv, gs, gx = (kept.as_strided((N, W), (W, 1), k * n) for k in range(5))
-        gh, gw_pos = kept.as_strided((N, 4 * W), (4 * W, 1), 5 * n), kept.as_strided((W,), (1,), 9 * n)
+        gh = kept.as_strided((N, 4 * W), (4 * W, 1), 5 * n)
         att, s, h = (saved.as_strided((N, c), (c, 1), at) for c, at in ((W, 0), (W, n), (4 * W, 2 * n)))
         lq, lk, lv, b_in, lo, bo, l1, b1, l2, b2 = ctx.leaves
         has_in, has_o, has_1, has_2 = ctx.has_bias
@@ -847,7 +851,7 @@ class BlockTrainHIP(torch.autograd.Function):
         got = _weight_gradients([(g, x, w, leaf, b_in, i * W, need[1 + i], want_b)
                                  for i, (g, w, leaf) in enumerate(zip((gq, gk, gv), (wq, wk, wv), head))])
         gb = torch.cat([b for _, b in got]) if want_b and got[0][1] is not None else None
-        return (gx if need[0] else None, *(w for w, _ in got), gb, gw_pos.view(w_pos.shape) if need[5] else None, gw_pe,
+        return (gx if need[0] else None, *(w for w, _ in got), gb, gw_pos if need[5] else None, gw_pe,
                 *(t for pair in tail for t in pair), None, None)
 
 

@@ -51,7 +51,8 @@ class BlockTrain(ctypes.Structure):
                 + [(n, _dbl) for n in ("dist_max", "wscale", "cutoff", "beta", "lower_bound", "coef", "q_scale")]
                 + [(n, _ptr) for n in ("x", "packed", "packed_bwd", "b_in", "w_pos", "gauss_scale", "w_pe", "bo", "b1", "b2",
                                        "rpos", "tvecs", "rvlen", "batch", "edges", "e_start", "atom_start", "edge_start",
-                                       "pairs", "rings", "sched", "counter", "y", "saved", "scratch", "gy", "kept", "gw_pe")])
+                                       "pairs", "rings", "sched", "counter", "y", "saved", "saved_more", "scratch", "gy", "kept",
+                                       "gw_pos", "gw_pe")])
 
 
 # name -> (restype, argtypes); mirrors include/crystalformer_hip.h

@@ -587,10 +587,11 @@ int cf_block_head_bwd(const float *ga, const float *gqs, const float *gk, const 
  * attention, models/indexed_lattice_multi_head_attention_cuda.py:636-790 and the encoder layer around it) as one call
  * forward and one backward: the launches of cf_block_head, cf_real_enc_fwd(_rings), cf_fused_dpa_fwd, cf_block_tail and of
  * their backward calls, on dense edge lists, results the same to the bit.  Not under a size header.
- *   saved    written forward, read backward: att (N,128), s (N,128), h (N,512) at its start, rows of whole 256 bytes
- *   kept     written backward: gq, gk, gv, gs, gx (N,128), gh (N,512), gw_pos (128), in this order
- *   bytes_4  sizes of saved, forward scratch, kept, backward scratch (256-byte aligned memory; by sizes, bins, normalize,
- *            cutoff, rings and want_gw_pe)
+ *   saved       written forward, read backward: att (N,128), s (N,128), h (N,512), in this order
+ *   saved_more  the same, the backward call's own (queries, keys, values, exponents; per edge biases, values, weights)
+ *   kept        written backward: gq, gk, gv, gs, gx (N,128), gh (N,512), in this order
+ *   bytes_5     sizes of saved, saved_more, forward scratch, kept, backward scratch (256-byte aligned memory, multiples of
+ *               256; by sizes, bins, normalize, cutoff, rings and want_gw_pe)
  */
 typedef struct {
     int64_t N, E, B, U, H, bins, lattice_range, minimum_range, normalize, update_stats, positive_func, want_gw_pe;
@@ -603,13 +604,13 @@ typedef struct {
     const void *rings;                                                    /* cf_real_enc_ring_stage, nullable */
     int32_t *sched, *counter;
     float *y;
-    void *saved, *scratch;
+    void *saved, *saved_more, *scratch;
     const float *gy;                                                      /* backward: from here */
     void *kept;
-    float *gw_pe;
+    float *gw_pos, *gw_pe;                                                /* (128); as w_pe */
 } cf_block_train;
 
-int cf_block_train_bytes(const cf_block_train *args, int64_t *bytes_4);
+int cf_block_train_bytes(const cf_block_train *args, int64_t *bytes_5);
 int cf_block_train_fwd(const cf_block_train *args, void *stream);
 int cf_block_train_bwd(const cf_block_train *args, void *stream);
 

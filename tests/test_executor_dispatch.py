@@ -395,6 +395,6 @@ def test_a_training_block_has_a_row_an_atom(rows, served):
     got = executor.native_training(model.encoder, torch.zeros(N + rows, 128), pack, layout, torch.zeros(E, 3),
                                    b.trans_vec, torch.zeros(B, 3))
     assert (got is not None) == served
-    need = (ctypes.c_int64 * 4)()
+    need = (ctypes.c_int64 * 5)()
     args = lib.BlockTrain(N + rows, E, B, (E + N) // 2, 8, 64)
     assert (lib.load().cf_block_train_bytes(ctypes.byref(args), need) == 0) == served

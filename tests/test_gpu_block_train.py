@@ -126,6 +126,23 @@ def test_a_parameter_changed_in_between_is_noticed(dev, monkeypatch):
         loss.backward()
 
 
+def test_what_outlives_a_block(dev, monkeypatch):
+    """A gradient holds its own memory alone, and what deferred weight gradients wait with is rows, not edges."""
+    b = labelled([60, 60], dev)
+    model = scaled(default_params(num_layers=2)).to(dev).train()
+    monkeypatch.setattr(hip_funcs, "USE_LINEAR_FUNCTION", True)
+    with hip_funcs.deferred_weight_grads():
+        (model(b)[:, 0] - b.y).abs().mean().backward()
+        waiting = {t.untyped_storage().data_ptr(): t.untyped_storage().nbytes()
+                   for entry in hip_funcs._deferred for t in entry[:2]}
+    atoms, rows = 120, 128 * 4
+    # (per block: att, s, h and gq, gk, gv, gs, gx, gh; the block inputs and the gradient behind the last block)
+    assert sum(waiting.values()) < (2 * (6 + 9) + 4) * atoms * rows, waiting
+    for name, p in model.named_parameters():
+        if p.grad is not None and "lattice_pos_weights" in name:
+            assert p.grad.untyped_storage().nbytes() == rows
+
+
 def test_graph_replays_and_eager_steps(dev, monkeypatch):
     """The captured step, replayed with eager work in between, has the eager step's bits."""
     b = labelled([9, 20, 3], dev)

@@ -38,12 +38,11 @@ struct PackArgs {
     PackSource block[PACK_BLOCKS];
     int blocks, embed_width;
     const float *w_embed;                     // (128, embed_width <= 128), nullable
-    float *packed, *packed_embed;             // blocks x PACKED_BLOCK floats; 128 x 128
+    float *packed, *packed_embed;             // blocks x PACKED_BLOCK (the prologue: SPLIT_BLOCK) floats; 128 x 129
     float *packed_bwd;                        // nullable: as packed, for the backward kernels
     unsigned *zero;                           // words to clear, nullable
     int64_t words;
 };
-int launch_pack_weights(const PackArgs &p, hipStream_t st);
 
 struct PrologueArgs {
     int64_t B, E;

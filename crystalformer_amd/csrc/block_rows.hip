@@ -386,17 +386,8 @@ __device__ __forceinline__ void pack_weights(const PackArgs &p, int x, int l, bo
     const int u = x / (UNIT_FLOATS / 1024);
     if (p.zero && x == 0 && l == 0 && !transposed)
         for (int64_t t = threadIdx.x; t < p.words; t += 256) p.zero[t] = 0u;
-    if (l == p.blocks && u > 0) return;
     const int at = 4 * (int)(x % (UNIT_FLOATS / 1024) * 256 + threadIdx.x);             // first of four floats of the unit
     const int wave = at / 2048, k = at / 256 % 8 * 16 + at / 64 % 4 * 4, col = 16 * wave + at / 4 % 16;
-    if (l == p.blocks) {                                        // the embedding, filled up with zeros
-        const float *we = p.w_embed + col * p.embed_width;
-        float4_t v;
-#pragma unroll
-        for (int i = 0; i < 4; i++) v[i] = k + i < p.embed_width ? we[k + i] : 0.f;
-        *reinterpret_cast<float4_t *>(p.packed_embed + at) = v;
-        return;
-    }
     const PackSource &w = p.block[l];
     if (transposed) {                                           // units 0-3 W2, 4-7 W1, 8 Wo, 9-11 Wq, Wk, Wv
         const float *t;
@@ -1144,14 +1135,6 @@ bool block_rows_served(int64_t width, int64_t ff, int64_t H)
     return width == RW && ff == RF && H >= 1 && RW % H == 0 && (RW / H) % 4 == 0;
 }
 
-int launch_pack_weights(const PackArgs &p, hipStream_t st)
-{
-    const dim3 grid(PACK_GRID, (unsigned)(p.blocks + (p.w_embed ? 1 : 0)), p.packed_bwd ? 2 : 1);
-    pack_weights_kernel<<<grid, 256, 0, st>>>(p);
-    CF_CHECK_LAUNCH("packing of the weights");
-    return CF_OK;
-}
-
 int launch_forward_prologue(const PackArgs &k, PrologueArgs p, hipStream_t st)
 {
     p.live_E = live_edges(p.E);
@@ -1225,8 +1208,9 @@ extern "C" int cf_pack_blocks(int64_t blocks, const float *const *weights, float
             a.zero = (unsigned *)zero_words;
             a.words = words;
         }
-        const int rc = cf::launch_pack_weights(a, (hipStream_t)stream);
-        if (rc) return rc;
+        const dim3 grid(PACK_GRID, (unsigned)a.blocks, a.packed_bwd ? 2 : 1);
+        pack_weights_kernel<<<grid, 256, 0, (hipStream_t)stream>>>(a);
+        CF_CHECK_LAUNCH("cf_pack_blocks");
     }
     return CF_OK;
 }

@@ -49,7 +49,8 @@ bool staged_block(const cf_forward_args &f, const cf_forward_block &p)
                         f.unit_limit_bytes);
 }
 
-// Whether the other blocks with value bins start from staged rings, and the bytes these take.
+// Whether the other blocks with value bins -- adaptive boxes below that line, and all where a caller leaves the units no room --
+// start from staged rings.
 bool use_rings(const cf_forward_args &f, int64_t U)
 {
     if (!f.staged_rings || U < 1) return false;

@@ -36,15 +36,19 @@ struct Buffers {
 };
 
 // How a block with value bins is encoded: from units staged by real_enc_infer.hip wherever that is served.  Adaptive boxes are
-// staged in the box of the weakest exponent the positive map allows, which grows as the lower bound to the power -3/2.  Four
-// blocks, 128 crystals of up to 64 atoms, staged against not: bound 0.2 288 and 379 us a forward (r0 = 1.4 A), 625 and 802 (3 A);
-// 0.05 333 and 382, 690 and 803.  Below, boxes meet the largest range and images their capacity.
+// staged in the box of the weakest exponent the positive map allows, which grows as the lower bound to the power -3/2, while the
+// blocks' own boxes hardly do.  Four blocks, staged against not, us a forward by bound (r0 = 1.4 A unless said):
+//   128 crystals of up to 64 atoms:          0.1 325 / 392, 0.05 344 / 393, 0.02 369 / 391, 0.01 422 / 389, 0.005 571 / 395
+//     with r0 = 3 A:                         0.1 650 / 808, 0.05 694 / 809, 0.03 780 / 810, 0.02 902 / 811
+//   4 of 200 to 400 in large skewed cells:   0.5 538 / 633, 0.25 588 / 660, 0.1 669 / 668, 0.07 746 / 675, 0.05 836 / 693
+//   16 of them:                              0.5 3390 / 4707, 0.1 4080 / 4706, 0.05 4519 / 4705
+// So from a tenth on, where staging is nowhere slower.
 bool boxes_of(const cf_forward_args &f, const cf_forward_block &p) { return f.adaptive != 0 && p.cutoff != 0.0; }
 int64_t real_heads(const cf_forward_args &f, const cf_forward_block &p) { return p.coef_reci != 0.0 ? f.H / 2 : f.H; }
 bool staged_block(const cf_forward_args &f, const cf_forward_block &p)
 {
     const bool boxes = boxes_of(f, p);
-    return p.bins > 0 && f.staged_rings && (!boxes || (f.adaptive_rings && (p.cutoff > 0.0 || p.lower_bound >= 0.05))) &&
+    return p.bins > 0 && f.staged_rings && (!boxes || (f.adaptive_rings && (p.cutoff > 0.0 || p.lower_bound >= 0.1))) &&
            infer_served(f.N, f.E, real_heads(f, p), p.bins, f.width / f.H, boxes, (int)f.lattice_range, p.weakest,
                         f.unit_limit_bytes);
 }

@@ -179,6 +179,14 @@ extern "C" int64_t cf_forward_workspace(const cf_forward_args *f, const cf_forwa
     return carve(*f, blocks, nullptr, b);
 }
 
+extern "C" int64_t cf_forward_staged(const cf_forward_args *f, const cf_forward_block *blocks)
+{
+    if (check_args(f, blocks)) return -1;
+    int64_t count = 0;
+    for (int64_t l = 0; l < f->layers; l++) count += staged_block(*f, blocks[l]);
+    return count;
+}
+
 extern "C" int cf_forward(const cf_forward_args *f_, const cf_forward_block *blocks, void *workspace,
                           int64_t workspace_bytes, void *stream)
 {

@@ -111,6 +111,7 @@ SIGNATURES = {
     "cf_block_tail_bwd": (_int, [_ptr, _ptr, _i64, _ptr, _ptr, _ptr, _ptr, _ptr]),
     "cf_block_head_bwd": (_int, [_ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _i64, _i64, _ptr, _int, _f32, _f32,
                                  _f32, _f32, _ptr, _ptr, _ptr, _ptr, _ptr]),
+    "cf_forward_staged": (_i64, [_ptr, _ptr]),
     "cf_forward": (_int, [_ptr, _ptr, _ptr, _i64, _ptr]),
     "cf_block_train_bytes": (_int, [_ptr, _ptr]),
     "cf_block_train_fwd": (_int, [_ptr, _ptr]),

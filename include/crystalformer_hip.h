@@ -529,6 +529,8 @@ typedef struct {
 } cf_forward_args;
 
 int64_t cf_forward_workspace(const cf_forward_args *args, const cf_forward_block *blocks);
+/* how many of the blocks are encoded from translations staged for them (under unit_limit_bytes); reads no device memory */
+int64_t cf_forward_staged(const cf_forward_args *args, const cf_forward_block *blocks);
 int cf_forward(const cf_forward_args *args, const cf_forward_block *blocks, void *workspace,
                int64_t workspace_bytes, void *stream);
 

@@ -1,12 +1,13 @@
 """The encoding of an inference forward (``csrc/real_enc_infer.hip``: units staged once, split matrix products) against the
 operators' kernels, which have the reference's sums in fp32, and against the oracle in float64: the edges of its groups
 (16), chunks (64) and images (832), of its bin and row tiles, and the units its staging leaves to the blocks."""
+import contextlib
 import dataclasses
 
 import pytest
 import torch
 
-from crystalformer_amd import executor, hip_funcs, ops
+from crystalformer_amd import executor, hip_funcs, lib, ops
 from crystalformer_amd.graphs import GraphedForward
 from crystalformer_amd.latticeformer import default_params
 from crystalformer_amd.synthetic import CrystalBatch, lattice_from_parameters
@@ -32,9 +33,34 @@ def crystals(lengths, sizes, seed=1, angles=None, shift=0):
     return CrystalBatch(x, pos, batch, trans, s)
 
 
-def compare(dev, b, rtol=RTOL, **options):
+@contextlib.contextmanager
+def blocks_staged():
+    """Within it, how many blocks of each native forward were encoded from staged units, and of how many."""
+    counts, real = [], lib.load()
+
+    class Asked:
+        def __getattr__(self, name):
+            return getattr(real, name)
+
+        def cf_forward(self, args, blocks, *rest):
+            counts.append((real.cf_forward_staged(args, blocks), len(blocks)))
+            return real.cf_forward(args, blocks, *rest)
+    with pytest.MonkeyPatch.context() as m:
+        m.setattr(executor._lib, "load", Asked)
+        yield counts
+
+
+def served(model, b, staged=True):
+    """``both_ways``, whose native call must have taken the staged encoding in every block (or in none)."""
+    with blocks_staged() as counts:
+        both = both_ways(model, b)
+    assert counts and all(got == (of if staged else 0) for got, of in counts), counts
+    return both
+
+
+def compare(dev, b, rtol=RTOL, staged=True, **options):
     model = scaled(default_params(num_layers=2, **options)).to(dev).eval()
-    native, modules = both_ways(model, b.to(dev))
+    native, modules = served(model, b.to(dev), staged)
     assert_close(native, modules, "encoder", rtol=rtol, atol=atol_rows(modules))
 
 
@@ -82,12 +108,12 @@ def test_less_room_than_units_need(dev, monkeypatch, adaptive, owner):
     units = int((b.sizes * (b.sizes + 1)).sum()) // 2
     assert units > 3 * 4096 and units % 8
     model = scaled(default_params(num_layers=2, scale_real=[3.0], adaptive_cutoff_sigma=adaptive)).to(dev).eval()
-    whole, modules = both_ways(model, b)
+    whole, modules = served(model, b)
     assert_close(whole, modules, "encoder", atol=atol_rows(modules))
     least = LEAST_BYTES if adaptive else 4096 * (32 + 128 * 4)
     for limit in (least, 5 * least // 2, least - 1, 0):
         monkeypatch.setattr(executor if owner == "STAGED_UNITS_MAX_BYTES" else ops, owner, limit)
-        sliced, _ = both_ways(model, b)
+        sliced, _ = served(model, b, staged=limit >= least)
         if limit >= least:
             assert torch.equal(sliced, whole)
         else:
@@ -105,8 +131,9 @@ def test_a_capacity_graph_has_the_eager_bits_whatever_its_capacity(dev, monkeypa
             layer.self_attn.gauss_scale.copy_(torch.tensor([0.8, -0.1]))
     model = model.to(dev).eval()
     graph = GraphedForward(model, b, capacity=(crystals_, 12 * crystals_, 144 * crystals_))
-    with torch.no_grad():
+    with torch.no_grad(), blocks_staged() as counts:
         eager = model(b).clone()
+        assert counts == [(2, 2)]
         for _ in range(3):
             assert torch.equal(graph(b), eager)
         n = int(b.sizes[0])
@@ -128,20 +155,22 @@ def test_skewed_cells_with_and_without_a_floor(dev, floor, monkeypatch):
     model = scaled(default_params(num_layers=2, scale_real=[2.0])).to(dev).eval()
     if not floor:
         monkeypatch.setattr(hip_funcs.KernelManager, "MINIMUM_RANGE", 0)
-    native, modules = both_ways(model, b.to(dev))
+    native, modules = served(model, b.to(dev))
     assert_close(native, modules, "encoder", atol=atol_rows(modules))
 
 
-@pytest.mark.parametrize("bound", [0.0, 0.04, 0.05, 0.1, 0.25, 0.9])
+@pytest.mark.parametrize("bound", [0.0, 0.05, 0.099, 0.1, 0.25, 0.9])
 @pytest.mark.parametrize("adaptive", [-3.5, 0.0])
 def test_bounds_of_the_exponents(dev, bound, adaptive):
-    compare(dev, batch_of([5, 14]), gauss_lb_real=bound, positive_func="abs", adaptive_cutoff_sigma=adaptive)
+    # (staged in the box of the weakest exponent, which only a bound holds down)
+    compare(dev, batch_of([5, 14]), staged=adaptive == 0.0 or bound >= 0.1, gauss_lb_real=bound, positive_func="abs",
+            adaptive_cutoff_sigma=adaptive)
 
 
 def test_blocks_that_share_units_and_blocks_that_do_not(dev):
     compare(dev, batch_of([12, 3, 25]), scale_real=[1.4, 3.0])
     model = scaled(default_params(num_layers=34, t_fixup_init=True)).to(dev).eval()    # (more blocks than are packed at once)
-    native, modules = both_ways(model, batch_of([9, 5]).to(dev))
+    native, modules = served(model, batch_of([9, 5]).to(dev))
     assert_close(native, modules, "encoder of 34 blocks", rtol=34 * RTOL)
 
 
@@ -158,7 +187,7 @@ def test_no_further_from_float64_than_the_operators(dev, r0):
         x = torch.nn.functional.linear(b64.x, P["input_embeddings.weight"])
         want = om.encoder_forward(P, cfg, x, b64.pos, b64.batch, b64.trans_vec, b64.sizes)
     want = want[0] if isinstance(want, tuple) else want
-    native, modules = both_ways(model.to(dev).eval(), b.to(dev))
+    native, modules = served(model.to(dev).eval(), b.to(dev))
     err = [float((t.cpu().double() - want).square().mean().sqrt()) for t in (native, modules)]
     print("\nrms from float64: staged %.3e, operators %.3e" % tuple(err), flush=True)
     assert err[0] <= 1.1 * err[1], err
@@ -174,7 +203,7 @@ def distances_from_float64(dev, cfg, change, b):
         x = torch.nn.functional.linear(b.x.double(), P["input_embeddings.weight"])
         want = om.encoder_forward(P, cfg, x, b.pos.double(), b.batch, b.trans_vec.double(), b.sizes)
     want = want[0] if isinstance(want, tuple) else want
-    return [float((t.cpu().double() - want).square().mean().sqrt()) for t in both_ways(model.to(dev).eval(), b.to(dev))]
+    return [float((t.cpu().double() - want).square().mean().sqrt()) for t in served(model.to(dev).eval(), b.to(dev))]
 
 
 # Bins whose weights are up to 2^24 apart: within a tenth of the fp32 products' own distance.
@@ -194,6 +223,6 @@ def test_infinite_projection_weights(dev):
         model.encoder.layers[0].self_attn.pe_dist_proj[0, 3, 5, 20] = float("inf")
         model.encoder.layers[0].self_attn.out_proj.weight[:, 3 * 16 + 5] = 0.0
         model.encoder.layers[0].self_attn.out_proj.weight[7, 3 * 16 + 5] = 1.0
-    native, modules = both_ways(model, batch_of([1, 7, 20]).to(dev))
+    native, modules = served(model, batch_of([1, 7, 20]).to(dev))
     for same in (torch.isposinf, torch.isneginf, torch.isnan):
         assert torch.equal(same(native), same(modules))

@@ -9,9 +9,11 @@ inputs resident in HBM.  Metric: crystals/s.
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--config NAME] [--rule A|B]
 
 Prints one JSON line.  The step is submitted as one HIP graph replay (the eager
-figure is reported beside it).  `roofline` describes the periodic-encoding kernel: the
-launches of one forward (one per block, with that block's real inputs) re-issued back to
-back, each timed with a pair of HIP events on its launch stream; `cpu_baseline`
+figure is reported beside it).  `roofline` describes the periodic-encoding kernel of the
+timed steps, by a kernel trace of replays after them, and `roofline.operators` the kernel that
+training and callers of the operators run: the launches of one forward (one per block, with
+that block's real inputs) re-issued back to back, each timed with a pair of HIP events on its
+launch stream; `cpu_baseline`
 times the CPU oracle (the restated PyTorch path of the reference) on the host
 cores for the same batch and weights and checks the GPU output against it.
 """
@@ -34,12 +36,13 @@ PEAK_HBM_GBS = 8000.0
 PROFILE_FILE = os.path.join(ROOT, "profiles", "traffic.json")
 KERNEL_SOURCES = {"fwd": ("real_enc_ring.hip", "real_enc_mfma.hip", "real_enc_pair_fwd.h", "real_enc_pair.h", "cf_common.h",
                           "cf_index_rules.h"),
-                  "bwd": ("real_enc_mfma_bwd.hip", "real_enc_pair.h", "cf_common.h", "cf_index_rules.h")}
+                  "bwd": ("real_enc_mfma_bwd.hip", "real_enc_pair.h", "cf_common.h", "cf_index_rules.h"),
+                  "infer": ("real_enc_infer.hip", "split_f16.h", "real_enc_pair.h", "cf_common.h", "cf_index_rules.h")}
 
 
 def kernel_fingerprint(direction: str) -> str:
-    """SHA-256 (first 16 hex digits) of the sources of the periodic-encoding pair kernel of one
-    direction ("fwd" / "bwd"): stored beside hardware counters when they are taken, compared
+    """SHA-256 (first 16 hex digits) of the sources of the periodic-encoding kernel of one
+    direction ("fwd" / "bwd"; "infer" the native forward's): stored beside hardware counters when they are taken, compared
     when they are used."""
     import hashlib
     h = hashlib.sha256()
@@ -106,6 +109,33 @@ def executed_work(c: dict, launch_ms: float) -> dict:
             "valu_insts": c["valu"], "mfma_insts": c["mfma"]}
 
 
+def issued_work(c: dict, launch_ms: float) -> dict:
+    """The native forward's encoding against the rate at which vector instructions (matrix ones among them) can be issued:
+    one per SIMD and four cycles.  Its products are split f16 ones, whose matrix instructions run beside vector work, so
+    flop are not what bounds it."""
+    peak = c.get("cus", 256) * 4 * c.get("clock_ghz", 2.4) / 4.0                 # 10^9 wave instructions a second
+    rate = c["valu"] / (launch_ms * 1e-3) / 1e9
+    return {"achieved": round(rate, 1), "peak": round(peak, 1), "frac": round(rate / peak, 4),
+            "valu_insts": c["valu"], "mfma_insts": c.get("mfma_f16"), "salu_insts": c.get("salu"),
+            "mfma_f16_tflops": None if "mfma_mops_f16" not in c else
+            round(c["mfma_mops_f16"] * 512.0 / (launch_ms * 1e-3) / 1e12, 1)}
+
+
+def kernel_times(run, passes: int = 10):
+    """{kernel name: (launches, mean microseconds)} over ``passes`` calls of ``run``, by torch's profiler; None under another
+    profiler (rocprofv3), which has the runtime's hooks already."""
+    import torch
+    if any(k.startswith(("ROCPROF", "ROCP_")) for k in os.environ) or "rocprof" in os.environ.get("LD_PRELOAD", ""):
+        return None
+    from torch.profiler import ProfilerActivity, profile
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CUDA]) as p:
+        for _ in range(passes):
+            run()
+        torch.cuda.synchronize()
+    return {e.key: (e.count, e.device_time) for e in p.key_averages() if e.device_time}
+
+
 def host_description() -> dict:
     model = "unknown"
     try:
@@ -158,7 +188,8 @@ def ingest_counters(directory: str, key: str, kernel: str) -> int:
     k = {c: mean(v) for c, v in agg["kernel"].items()}
     names = {"SQ_INSTS_VALU": "valu", "SQ_INSTS_VALU_MFMA_F32": "mfma", "SQ_INSTS_VALU_FMA_F32": "fma",
              "SQ_INSTS_VALU_ADD_F32": "add", "SQ_INSTS_VALU_MUL_F32": "mul", "SQ_INSTS_VALU_TRANS_F32": "trans",
-             "SQ_INSTS_VALU_MFMA_MOPS_F32": "mfma_mops_f32", "SQ_WAVES": "waves", "SQ_INSTS_SALU": "salu",
+             "SQ_INSTS_VALU_MFMA_MOPS_F32": "mfma_mops_f32", "SQ_INSTS_VALU_MFMA_F16": "mfma_f16",
+             "SQ_INSTS_VALU_MFMA_MOPS_F16": "mfma_mops_f16", "SQ_INSTS_SMEM": "smem", "SQ_WAVES": "waves", "SQ_INSTS_SALU": "salu",
              "SQ_INSTS_LDS": "lds"}
     entry = {short: round(k[c], 1) for c, short in names.items() if c in k}
     copy_kib = 256.0 * 1024.0
@@ -443,9 +474,9 @@ def main() -> int:
     ap.add_argument("--train", action="store_true",
                     help="time full training steps (forward + backward + AdamW) instead of forwards")
     ap.add_argument("--profile-kernel", action="store_true",
-                    help="counter-collection helper: launch only a 256 MiB device copy (calibration) and the "
-                         "periodic-encoding kernel on the workload (with --train: its backward), 5 times each, "
-                         "and exit")
+                    help="counter-collection helper: launch only a 256 MiB device copy (calibration), the operators' "
+                         "periodic-encoding kernel on the workload and native forwards (with --train: the backward "
+                         "kernel), 5 times each, and exit")
     ap.add_argument("--no-counters", action="store_true",
                     help="do not require stored hardware counters for this workload: roofline.frac is then null")
     ap.add_argument("--ingest-counters", metavar="DIR",
@@ -546,6 +577,10 @@ def main() -> int:
                 if nm == "staged_rings":
                     ops._ring_cache.clear()
                 originals[nm](*a, **kw)
+        if not args.train:                               # the native forward's own encoding
+            with torch.no_grad():
+                for _ in range(5):
+                    model(data)
         torch.cuda.synchronize()
         print(json.dumps({"profile_kernel": True, "copy_bytes_read": src.numel() * 4,
                           "copy_bytes_written": src.numel() * 4, "edges": E, "atoms": N}))
@@ -604,8 +639,7 @@ def main() -> int:
     ms_per_step = elapsed / args.steps * 1e3
     value = B * args.steps / elapsed
 
-    # ---- roofline of the operators' encoding kernel, forward (the timed steps' native call has an encoding of its own, whose
-    # products are split f16 ones; training and callers of the operators run this one)
+    # ---- roofline of the operators' encoding kernel, forward
     enc_ms = [s.elapsed_time(e) for (name, s, e, info) in log if name == "real_enc_fwd"]
     dpa_ms = [s.elapsed_time(e) for (name, s, e, info) in log if name == "fused_dpa_fwd"]
     stage_ms = [s.elapsed_time(e) for (name, s, e, info) in log if name == "real_enc_ring_stage"]
@@ -668,6 +702,35 @@ def main() -> int:
                                      "avg_launch_ms": round(dpa_avg_ms, 4),
                                      "note": "the operator, which stores the weights; a forward without gradients "
                                              "leaves them out"}
+
+    # ---- and of the timed steps' own, where the native call has one
+    with torch.no_grad():
+        traced = kernel_times((lambda: model(data)) if args.no_graph else graphed)
+    own = [(n, *v) for n, v in (traced or {}).items() if "real_enc_infer_kernel" in n]
+    if own:
+        us = sum(count * mean for _, count, mean in own) / sum(count for _, count, _ in own)
+        stage_us = [mean for n, (_, mean) in traced.items() if "infer_stage_kernel" in n]
+        counters = None if args.domain != "real" else stored_counters(f"{args.config}:{args.rule}:infer",
+                                                                      required=not args.no_counters)
+        work = issued_work(counters, us * 1e-3) if counters else None
+        roofline = {
+            "kernel": "real_enc_infer_kernel (periodic encoding of the native forward: translations staged once for all blocks, "
+                      "split f16 products, projection fused)",
+            "bound": "valu issue",
+            "achieved": work["achieved"] if work else None, "peak": work["peak"] if work else None,
+            "unit": "G vector instructions/s", "frac": work["frac"] if work else None,
+            "executed": work,
+            "counters_from": None if not counters else {k: counters.get(k) for k in
+                                                        ("commit", "date", "kernel_sha16", "current")},
+            "traffic": counters.get("hbm_bytes") if counters else None,
+            "traffic_note": "HBM bytes per launch from the stored rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE runs "
+                            "(not measured in this run)" if counters else None,
+            "launches_timed": sum(count for _, count, _ in own),
+            "avg_launch_ms": round(us * 1e-3, 4),
+            "stage_avg_ms": round(stage_us[0] * 1e-3, 4) if stage_us else None,
+            "algorithmic_equivalent": {"tflops": round(flop_launch / (us * 1e-6) / 1e12, 3)},
+            "operators": roofline,
+        }
 
     # ---- forwards over batches never seen before: every step a batch with other crystal sizes.
     # One captured graph with capacity buffers serves them all (the index structure and the counts
@@ -781,6 +844,8 @@ def main() -> int:
         "scaling": "weak",
         "vs_baseline": None,
         "dtype": "f32",
+        "products": None if traced is None else "fp32 sums of split f16 products, 22 bits of either factor"
+                    if own or any("block_rows_kernel" in n for n in traced) else "fp32",
         "data": "synthetic",
         "config": {"workload": args.config, "crystals": B, "atoms": N, "edges": E, "blocks": cfg.num_layers,
                    "heads": H, "value_pe_bins": K, "translation_rule": args.rule,

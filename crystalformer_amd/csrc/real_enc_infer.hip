@@ -10,15 +10,17 @@
 // v_mfma_f32_16x16x4_f32 takes 32 cycles in which no vector instruction runs (measured: 32.2 alone, 57.0 beside eight
 // v_fma), v_mfma_f32_16x16x16_f16 16 that hide behind them (17.2 alone, 33.7 beside the same eight).  So here
 //   * both factors of a matrix product are split in two halves of 11 bits, x 2^15 = hi + lo, and all four products
-//     summed in fp32: 22 bits and a sign of each factor.  A split costs two instructions a value;
+//     summed in fp32: 22 bits and a sign of each factor.  A split costs two instructions a value.  Weights and Gaussians,
+//     none above 1, share one fixed scale: below 2^-17 a factor is off by up to 2^-40, the bound on what is left out;
 //   * a translation enters only if its weight exceeds 2^-40 of the leading one in some column, by the block's own
 //     exponents (a prefix of the order), and a 16-bin tile only if weight x Gaussian can exceed 2^-40: 17 translations and
 //     4.5 tiles of 16 a pair with r0 = 1.4 A where the others evaluate 32 and 16 of 4, 64 and 10 where 98 and 47 with 3 A;
 //   * square roots, column lookups and tile tests are made for these only, lane = translation;
 //   * nothing about the pair passes through vector registers: its 32 bytes are scalar loads.
-// What bounds a block now is the issue of vector instructions, 843 a pair at the largest, slots 84 % busy.  Measured, pair and
-// ring kernels -> this, a block: 28 thousand pairs in the fixed cube 43.5 -> 33.8 us, in boxes 45.4 and 9.4 for the lists ->
-// 38.1, 294 thousand (mean of seven blocks) 440 and 15 -> 276, 958 thousand 3060 -> 1570.
+// What bounds a block now is the issue of vector instructions: 851 a pair at the largest (52 of them matrix ones) take 86 % of the
+// slots, 339 a pair with r0 = 1.4 A in the cube half of them, the rest going on the launch's start, its last round and waits.
+// Measured, pair and ring kernels -> this, a block: 28 thousand pairs in the fixed cube 43.5 -> 33.8 us, in boxes 45.4 and 9.4 for
+// the lists -> 38.1, 147 thousand (mean of seven blocks) 440 and 15 -> 276, 958 thousand 3060 -> 1540.
 //
 // Lane roles of the accumulation (q = lane / 16, c = lane % 16): lane (q, c) holds translations 4 q .. 4 q + 3 of a group of
 // 16: column c's weights (B operand) and the Gaussians of bin 16 m + c of every tile m in reach (A operand).  Projection
@@ -289,7 +291,7 @@ __global__ __launch_bounds__(STAGE_WAVES * 64) void infer_stage_kernel(StageArgs
         } else {
             // A lane has a place (two of the three numbers) and walks along the third axis, the one that leaves the fewest
             // steps of 64 places: 15 instructions a step.  (All three numbers of 64 consecutive translations, carried from
-            // step to step, took 45: 958 thousand pairs with 232 of them staged 1030 us, so 915, with the ranking below 770.)
+            // step to step, took 45: 958 thousand pairs with 132 of them staged 1030 us, so 915, with the ranking below 770.)
             const int S1 = 2 * bx.U1 + 1;
             const int s1 = ((bx.S2 * bx.S3 + 63) >> 6) * S1, s2 = ((S1 * bx.S3 + 63) >> 6) * bx.S2,
                       s3 = ((S1 * bx.S2 + 63) >> 6) * bx.S3;
@@ -751,8 +753,9 @@ __global__ __launch_bounds__(512, DT > 1 || NT > 4 ? 6 : 8) void real_enc_infer_
     }
 }
 
-// Entries a unit may have: all of a small fixed cube, else 832 (what leaves six staging work-groups a CU: seven blocks on 256
-// crystals, r0 = 3 A, have 232 in the mean and one unit in a hundred above 700).  The same whatever the batch: a unit that has
+// Entries a unit may have: all of a small fixed cube, else 832 (what leaves six staging work-groups a CU).  Units under the weakest
+// exponent have 31 in the mean with r0 = 1.4 A, 230 with 3 A in small cells (an eighth above 512, two in a thousand above 832),
+// 132 and none above 256 in large skewed ones.  The same whatever the batch: a unit that has
 // more is formed by the blocks, in another order, and its bits must not depend on what else is in the batch, nor on the capacity
 // of a graph that serves it.
 constexpr int capacity_of(bool boxes) { return boxes ? MOST_STAGED : 128; }

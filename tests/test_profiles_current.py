@@ -14,7 +14,8 @@ def test_stored_counters_match_the_kernel_sources():
     with open(bench.PROFILE_FILE) as f:
         stored = json.load(f)
     keys = [k for k in stored if not k.startswith("_")]
-    assert "cfg2_default_b128:A:fwd" in keys and "cfg4_train_b128:A:bwd" in keys
+    assert {"cfg2_default_b128:A:fwd", "cfg4_train_b128:A:bwd", "cfg2_default_b128:A:infer",
+            "cfg2_default_b128:B:infer"} <= set(keys)
     for key in keys:
         now = bench.kernel_fingerprint(key.rsplit(":", 1)[1])
         assert stored[key].get("kernel_sha16") == now, \

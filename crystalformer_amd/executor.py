@@ -29,10 +29,10 @@ from .latticeformer import Latticeformer, is_plain_head
 from .lib import device_guard, stream_handle
 
 
-# What the staged translations of a forward may take: with adaptive boxes 5024 bytes an atom pair, all at once for 1.28 million
+# What the staged translations of a forward may take: with adaptive boxes 5024 bytes an atom pair, all at once for 1.7 million
 # pairs, in the fixed cube 544.  Where they take more they are staged in slices, by every block; results don't depend on it.  An
 # `ops.STAGED_RINGS_MAX_BYTES` below its default bounds these too.
-STAGED_UNITS_MAX_BYTES = 6 << 30
+STAGED_UNITS_MAX_BYTES = 8 << 30
 
 
 def _unit_limit() -> int:

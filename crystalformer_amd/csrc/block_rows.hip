@@ -18,8 +18,8 @@
 // bounds a launch now is the chain of one tile: 16 rows are staged in 2.5 us, each of the twelve units of 128 columns takes
 // 0.5, each of the four splits 0.3, output and exponents 0.9.  Without the weights' loads it would be 10.4 us at 12 rows; five
 // buffers of weights instead of three: 0.9 us slower.
-// Measured, tail and head in a forward, fp32 products -> these: 12 rows 13.7 -> 12.7 us, 1774 rows 17.6 -> 13.6 (0.70 GFLOP: 51
-// TFLOP/s), 4096 rows 25.8 -> 17.1, 5.2 thousand rows 40 -> 21.5 (95 TFLOP/s).  One scale a row instead of one a piece, and first
+// Measured, tail and head in a forward, fp32 products -> these: 12 rows 13.7 -> 12.5 us, 1774 rows 17.6 -> 13.7 (0.70 GFLOP: 51
+// TFLOP/s), 4096 rows 25.8 -> 16.9, 5.2 thousand rows 40 -> 21.5 (95 TFLOP/s).  One scale a row instead of one a piece, and first
 // and second halves scaled alike, made it 12.2, 13.4, 16.8 and 20.0, and lost what lies below 2^-16 of a row's largest.
 // Operands of v_mfma_f32_16x16x32_f16, lane (q, c) = (lane / 16, lane % 16), reduction step s of 32:
 //   A: 16 bytes of row c at k = 32 s + 8 q, hi or lo;  B: the same of column c's weights;  D: row 4 q + r, column c.
@@ -97,77 +97,90 @@ __device__ __forceinline__ void multiply(float4_t (&acc)[T], const Weights &b, c
     }
 }
 
-// The largest of 32 adjacent lanes' magnitudes, in each of them.  By the bits: of floats >= 0 the order of the integers is
+// The largest of 8 or 32 adjacent lanes' magnitudes, in each of them.  By the bits: of floats >= 0 the order of the integers is
 // theirs (as floats every step costs a canonicalising instruction beside the one on the DPP path).
 template <int CTRL>
 __device__ __forceinline__ int dpp_max(int v)
 {
     return max(v, __builtin_amdgcn_update_dpp(v, v, CTRL, 0xF, 0xF, false));
 }
-__device__ __forceinline__ int magnitude_bits(float x) { return __float_as_int(x) & 0x7FFFFFFF; }
-__device__ __forceinline__ int half_wave_max(int v)
+template <int LANES>
+__device__ __forceinline__ int lanes_max(int v)
 {
     v = dpp_max<DPP_QUAD_1032>(v);
     v = dpp_max<DPP_QUAD_2301>(v);
+    if (LANES == 8) return dpp_max<0x141>(v);                   // row_half_mirror: the other four of eight
     v = dpp_max<DPP_ROW_ROR4>(v);
     v = dpp_max<DPP_ROW_ROR8>(v);
     const uint2_cf r = __builtin_amdgcn_permlane16_swap((unsigned)v, (unsigned)v, false, false);
     return max((int)r[0], (int)r[1]);
 }
+__device__ __forceinline__ int magnitude_bits(float x) { return __float_as_int(x) & 0x7FFFFFFF; }
 
-// Four values of each of L pieces of 128 columns of a row, scaled by the largest magnitude of the row's piece and split
-// (split2_far): of every eight values (32 bytes) the eight his, then the eight los.  32 threads a row, thread j has columns
-// 4 j .. 4 j + 3; the exponent of piece l goes to exp[l * stride].
-template <int L>
-__device__ __forceinline__ void split_row(float4_t (&v)[L], float *row, int j, int *exp, int stride)
+// 4 L values of a piece of 128 columns of a row, whose other values LANES - 1 adjacent lanes hold, scaled by the piece's largest
+// magnitude and split (split2_far): of every eight values (32 bytes) the eight his, then the eight los.  v[l] are the columns
+// from at(l) on, a multiple of 4; every lane of the piece gives its exponent's place.
+template <int L, class Place>
+__device__ __forceinline__ void split_piece(float4_t (&v)[L], float *piece, Place at, bool first, int *exp)
 {
+    constexpr int LANES = RW / (4 * L);
     float zero = 0.f;
     asm volatile("" : "+v"(zero));
-    float *hi = row + 8 * (j / 2) + 2 * (j % 2);
-    int top[L], all = 0;
+    int top = 0;
 #pragma unroll
-    for (int l = 0; l < L; l++) {
-        top[l] = max(max(magnitude_bits(v[l][0]), magnitude_bits(v[l][1])), max(magnitude_bits(v[l][2]), magnitude_bits(v[l][3])));
-        top[l] = half_wave_max(top[l]);
-        all = max(all, top[l]);
-    }
-    if (__builtin_expect(__ballot(all >= 0x7F800000) != 0ull, 0)) {              // infinities, or not a number
+    for (int l = 0; l < L; l++)
 #pragma unroll
-        for (int l = 0; l < L; l++) {
-            float t = 0.f;
+        for (int i = 0; i < 4; i++) top = max(top, magnitude_bits(v[l][i]));
+    top = lanes_max<LANES>(top);
+    if (__builtin_expect(__ballot(top >= 0x7F800000) != 0ull, 0)) {              // infinities, or not a number
+        float t = 0.f;
+#pragma unroll
+        for (int l = 0; l < L; l++)
 #pragma unroll
             for (int i = 0; i < 4; i++) t = fmaxf(t, finite_magnitude(v[l][i]));
-            top[l] = half_wave_max(__float_as_int(t));
-        }
+        top = lanes_max<LANES>(__float_as_int(t));
     }
-    int e[L];
-#pragma unroll
-    for (int l = 0; l < L; l++) {
-        e[l] = __builtin_amdgcn_frexp_expf(__int_as_float(top[l]));              // (0 for 0)
-        if (j == 0) exp[l * stride] = e[l];
-    }
+    const int e = __builtin_amdgcn_frexp_expf(__int_as_float(top));              // (0 for 0)
+    if (first) *exp = e;
 #pragma unroll
     for (int l = 0; l < L; l++) {
 #pragma unroll
-        for (int i = 0; i < 4; i++) v[l][i] = ldexpf(v[l][i], 26 - e[l]);
+        for (int i = 0; i < 4; i++) v[l][i] = ldexpf(v[l][i], 26 - e);
         const Split2 a = split2_far(v[l][0], v[l][1], zero), b = split2_far(v[l][2], v[l][3], zero);
-        *reinterpret_cast<int2_t *>(hi + RW * l) = int2_t{a.hi, b.hi};
-        *reinterpret_cast<int2_t *>(hi + RW * l + 4) = int2_t{a.lo, b.lo};
+        const int c = at(l);
+        float *hi = piece + (c & ~7) + (c & 4) / 2;
+        *reinterpret_cast<int2_t *>(hi) = int2_t{a.hi, b.hi};
+        *reinterpret_cast<int2_t *>(hi + 4) = int2_t{a.lo, b.lo};
     }
 }
 
-// The rows of an LDS buffer split in place (a group's two lanes have read both before either writes); exps: M a piece.
-template <int M, int L>
-__device__ __forceinline__ void split_rows(float *xs, int ld, int *exps)
+// The rows of an LDS buffer split in place (the lanes of a piece have read it before any writes), 32 threads a row.
+template <int M>
+__device__ __forceinline__ void split_rows(float *xs, int *exps)
 {
     const int j = threadIdx.x % 32;
 #pragma unroll
     for (int r0 = 0; r0 < M; r0 += RT / 32) {
         const int r = r0 + threadIdx.x / 32;
-        float4_t v[L];
+        float4_t v[1] = {*reinterpret_cast<const float4_t *>(xs + r * LDX + 4 * j)};
+        split_piece<1>(v, xs + r * LDX, [&](int) { return 4 * j; }, j == 0, exps + r);
+    }
+}
+// The hidden units, four pieces a row with exponents M apart.  Eight lanes a piece, each with four times four columns 32 apart; every
+// other piece starts with its second 32, so that 16 lanes' reads cover all banks.
+template <int M>
+__device__ __forceinline__ void split_hidden(float *hs, int *exps)
+{
+    const int p = threadIdx.x / 8 % 4, k = threadIdx.x % 8;
+    auto at = [&](int l) { return 4 * k + 32 * l + (l % 2 ? -32 : 32) * (p & 1); };
 #pragma unroll
-        for (int l = 0; l < L; l++) v[l] = *reinterpret_cast<const float4_t *>(xs + r * ld + 4 * j + RW * l);
-        split_row<L>(v, xs + r * ld, j, exps + r, M);
+    for (int r0 = 0; r0 < M; r0 += RT / 32) {
+        const int r = r0 + threadIdx.x / 32;
+        float *piece = hs + r * LDH + p * RW;
+        float4_t v[4];
+#pragma unroll
+        for (int l = 0; l < 4; l++) v[l] = *reinterpret_cast<const float4_t *>(piece + at(l));
+        split_piece<4>(v, piece, at, k == 0, exps + p * M + r);
     }
 }
 
@@ -609,7 +622,7 @@ __global__ __launch_bounds__(RT, 2) void block_rows_kernel(RowsArgs p)
 #pragma unroll
         for (int t = 0; t < PASSES; t++) {
             const int r = 16 * t + threadIdx.x / 32;
-            split_row<1>(in[t], b2 + r * LDX, j, x_exp + r, M);
+            split_piece<1>(in[t], b2 + r * LDX, [&](int) { return 4 * j; }, j == 0, x_exp + r);
             if (SRC == ROWS_TAIL) *reinterpret_cast<float4_t *>(b1 + r * LDX + 4 * j) = residual[t];
         }
         __syncthreads();
@@ -629,7 +642,7 @@ __global__ __launch_bounds__(RT, 2) void block_rows_kernel(RowsArgs p)
                     b0[at + (16 * t + r) * LDX] = v;
                 }
             __syncthreads();
-            split_rows<M, 1>(b0, LDX, x_exp);
+            split_rows<M>(b0, x_exp);
             __syncthreads();
             // hidden units, four tiles on one read of the rows
             read_rows(x, b0, LDX, lane);
@@ -645,7 +658,7 @@ __global__ __launch_bounds__(RT, 2) void block_rows_kernel(RowsArgs p)
                     }
             }
             __syncthreads();
-            split_rows<M, 4>(hs, LDH, x_exp);
+            split_hidden<M>(hs, x_exp);
             __syncthreads();
             float y[T][4];
             Rows<T> ahead;                                      // (read a unit before it is multiplied)
@@ -688,7 +701,7 @@ __global__ __launch_bounds__(RT, 2) void block_rows_kernel(RowsArgs p)
         }
         if (HEAD) {
             if (SRC != ROWS_PLAIN) {
-                split_rows<M, 1>(b2, LDX, x_exp);
+                split_rows<M>(b2, x_exp);
                 __syncthreads();
             }
             read_rows(x, b2, LDX, lane);
@@ -1153,7 +1166,7 @@ int launch_block_rows(RowsArgs p, hipStream_t st)
     const int64_t cus = device_cu_count();
     // 32 rows a tile beyond one round of 16 (a tile a CU): 257 to 512 tiles of 16 are two rounds, the second short of
     // work, and ask for the weights twice as often.  At 5.2 thousand rows 21.5 us a launch against 28.6; up to one round 16 are
-    // better, with all CUs at work (1774 rows: 13.6 us, on 111 of them, and a tile of 32 is the 21.5).
+    // better, with all CUs at work (1774 rows: 13.7 us, on 111 of them, and a tile of 32 is the 21.5).
     // (Live rows are somewhere below the capacity; a tile has at most 256 exponents, see complete_groups.)
     const int T = !p.live_N && p.N > 16 * cus && p.H <= 8 ? 2 : 1;
     int64_t grid = (p.N + 16 * T - 1) / (16 * T);

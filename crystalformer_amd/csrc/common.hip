@@ -63,7 +63,7 @@ int64_t *size_header_for_layout(int64_t N, int64_t E)
 
 }  // namespace cf
 
-extern "C" int cf_version(void) { return 101; }
+extern "C" int cf_version(void) { return 102; }
 
 extern "C" int cf_set_size_header(int64_t *header_4, int64_t N_cap, int64_t E_cap)
 {
